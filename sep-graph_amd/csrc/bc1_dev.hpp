@@ -131,7 +131,7 @@ __device__ __forceinline__ double wave_level_sum(const uint32_t *adj, const uint
     const int ln = lane();
     const uint32_t r = e - b;
     const uint32_t incl = wave_incl_scan(r);
-    const uint32_t total = shfl(incl, kWave - 1);
+    const uint32_t total = lane_value(incl, kWave - 1);
     const uint32_t excl = incl - r;
     double acc = 0.0;
     for (uint32_t jb = 0; jb < total; jb += U * kWave) {
@@ -156,12 +156,7 @@ __device__ __forceinline__ double wave_level_sum(const uint32_t *adj, const uint
         for (int s = 0; s < U; s++) {
             // segmented sum over the lanes of one owner (owners are contiguous)
             double y = x[s];
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-                const double t = __shfl_up(y, d, kWave);
-                const int ko = __shfl_up(k[s], d, kWave);
-                if (ln >= d && ko == k[s]) y += t;
-            }
+            y = wave_seg_scan(y, (uint32_t)k[s], [](double lo, double hi) { return lo + hi; });
             // this lane's vertex covers positions [excl, incl) of the concatenation
             const uint32_t base = jb + (uint32_t)(s * kWave);
             const uint32_t lo = min(max(excl, base), base + 64u) - base;
@@ -194,8 +189,8 @@ __device__ __forceinline__ double wave_chunk_sum(const uint32_t *adj, const uint
         for (int q = 0; q < Q; q++) {
             t[q] = todo ? first_lane(todo) : -1;
             todo &= todo - 1;
-            cb[q] = t[q] >= 0 ? shfl(b, t[q]) : 0u;
-            ce[q] = t[q] >= 0 ? shfl(e, t[q]) : 0u;
+            cb[q] = t[q] >= 0 ? lane_value(b, t[q]) : 0u;
+            ce[q] = t[q] >= 0 ? lane_value(e, t[q]) : 0u;
         }
         double acc[Q];
 #pragma unroll
@@ -240,7 +235,7 @@ __device__ __forceinline__ void wave_level_push(const uint32_t *adj, uint32_t b,
     const int ln = lane();
     const uint32_t r = e - b;
     const uint32_t incl = wave_incl_scan(r);
-    const uint32_t total = shfl(incl, kWave - 1);
+    const uint32_t total = lane_value(incl, kWave - 1);
     const uint32_t excl = incl - r;
     for (uint32_t jb = 0; jb < total; jb += U * kWave) {
         uint32_t u[U];
@@ -328,8 +323,7 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
             if (vv)
                 lane_level_vol(s_vol, true, (uint32_t)l, g.row[v + 1] - g.row[v], g.cstart[v + 1] - g.cstart[v]);
         }
-#pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) lmax = max(lmax, (uint32_t)__shfl_xor(lmax, d, kWave));
+        lmax = wave_max_u32(lmax);
         if (ln == 0) atomicMax(&s_max, lmax);
         __syncthreads();
         const uint32_t top = min(s_max, kBcLdsLevels - 1);
@@ -476,9 +470,7 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
                 if (ln == 0) cur[w] = m;
                 const uint32_t deg = at ? g.cstart[v + 1] - g.cstart[v] : 0u;
                 const bool light = at && deg <= kPullHubDegree;  // in-hubs: the chunk pass below
-                uint32_t rows = light ? deg : 0u;
-#pragma unroll
-                for (int d = kWave / 2; d > 0; d >>= 1) rows = max(rows, (uint32_t)__shfl_xor(rows, d, kWave));
+                const uint32_t rows = wave_max_u32(light ? deg : 0u);
                 if (!rows) continue;
                 const uint32_t *S = g.sell_src + g.sell_off[w] + ln;
                 constexpr int U = kLevelSteps;

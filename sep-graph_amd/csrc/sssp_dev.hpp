@@ -189,7 +189,7 @@ __device__ __forceinline__ void push_expand(Round &R, bool valid, uint32_t u)
     }
     defer(R, later, u, du);
     const uint32_t incl = wave_incl_scan(d);
-    const uint32_t total = shfl(incl, kWave - 1);
+    const uint32_t total = lane_value(incl, kWave - 1);
     const uint32_t off = b - (incl - d);
     const int ln = lane();
     for (uint32_t jb = 0; jb < total; jb += kWave) {
@@ -226,8 +226,7 @@ __device__ __forceinline__ void push_expand_serial(Round &R, bool valid, uint32_
     }
     defer(R, later, u, du);
     uint32_t dmax = d;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) dmax = max(dmax, (uint32_t)__shfl_xor(dmax, o, kWave));
+    dmax = wave_max_u32(dmax);
     for (uint32_t j = 0; j < dmax; j++) {
         const bool act = j < d;
         uint32_t v = 0, nd = kInf;
@@ -301,7 +300,7 @@ __device__ __forceinline__ void pull_word(Round &R, uint32_t w)
     for (;;) {
         const uint32_t r = e - b;
         const uint32_t incl = wave_incl_scan(r);
-        const uint32_t total = shfl(incl, kWave - 1);
+        const uint32_t total = lane_value(incl, kWave - 1);
         if (total == 0) break;
         const uint32_t excl = incl - r;
         int k[U];
@@ -326,12 +325,7 @@ __device__ __forceinline__ void pull_word(Round &R, uint32_t w)
             // segmented minimum over lanes with the same owner (owners are
             // contiguous), then each vertex takes the last lane of its run
             uint32_t m = du[s] != kInf ? sat_add(du[s], wt[s]) : kInf;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-                const uint32_t y = __shfl_up(m, d, kWave);
-                const int ko = __shfl_up(k[s], d, kWave);
-                if (ln >= d && ko == k[s]) m = min(m, y);
-            }
+            m = wave_seg_scan(m, (uint32_t)k[s], [](uint32_t x, uint32_t y) { return min(x, y); });
             const uint32_t base = (uint32_t)(s * kWave);
             const uint32_t lo = min(max(excl, base), base + 64u) - base;
             const uint32_t hi = min(max(incl, base), base + 64u) - base;
@@ -521,8 +515,7 @@ __device__ __forceinline__ void pull_hubs(Round &R, uint32_t first, uint32_t str
 #pragma unroll
             for (int s = 0; s < U; s++)
                 if (du[i][s] != kInf) m = min(m, sat_add(du[i][s], wt[i][s]));
-#pragma unroll
-            for (int d = kWave / 2; d > 0; d >>= 1) m = min(m, (uint32_t)__shfl_xor(m, d, kWave));
+            m = wave_min_u32(m);
             // dv is this chunk's earlier read of the hub: a candidate not
             // below it cannot lower the hub
             const bool issue = dsc[i].x != kInf && m < dv[i];
@@ -606,8 +599,7 @@ __device__ __forceinline__ void pull_hubs_sorted(Round &R, uint32_t first, uint3
 #pragma unroll
             for (int s = 0; s < U; s++)
                 if (du[i][s] != kInf) m = min(m, sat_add(du[i][s], wt[i][s]));
-#pragma unroll
-            for (int d = kWave / 2; d > 0; d >>= 1) m = min(m, (uint32_t)__shfl_xor(m, d, kWave));
+            m = wave_min_u32(m);
             const bool issue = hv[i] != kInf && m < dv[i];
             pv[i] = issue ? hv[i] : kInf;
             pm[i] = m;
@@ -735,7 +727,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
                 while (mm) {
                     const int t = first_lane(mm);
                     mm &= mm - 1;
-                    const uint32_t u = shfl(dsc.x, t), beg = shfl(dsc.y, t);
+                    const uint32_t u = lane_value(dsc.x, t), beg = lane_value(dsc.y, t);
                     const uint32_t end = min(g.row[u + 1], beg + kHugeChunk);
                     const uint32_t du = a.dist[u];
                     // a deferred hub is carried by its queue entry
@@ -818,8 +810,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
             // block minimum of the queued distances, one atomic per block
             // (the priority threshold and the settled test of pull rounds)
             uint32_t m = R.minv;
-#pragma unroll
-            for (int d = kWave / 2; d > 0; d >>= 1) m = min(m, (uint32_t)__shfl_xor(m, d, kWave));
+            m = wave_min_u32(m);
             if (threadIdx.x == 0) s_bmin = kInf;
             __syncthreads();
             if (ln == 0 && m != kInf) atomicMin(&s_bmin, m);
