@@ -15,8 +15,8 @@ __global__ SG_BFS_BOUNDS(BS) void k_bfs(BfsArgs a)
         return;
     }
     const uint32_t xcc = xcc_id();
-    BarState gen = bar_begin(a.bar, xcc);
-    bfs_run<BS, kStage>(a, blockIdx.x, gridDim.x, xcc, gen);
+    BarState gen = bar_begin<!kStage>(a.bar, xcc);
+    bfs_run<BS, kStage, !kStage, !kStage>(a, blockIdx.x, gridDim.x, xcc, gen);
 }
 
 
@@ -88,6 +88,7 @@ int bfs_launch(sg_engine *e, uint32_t source, int32_t *out, bool traced)
     a.max_rounds = (uint32_t)o.max_iteration;
     a.lb_push_none = o.lb_push == SG_LB_NONE;
     a.lb_pull_none = o.lb_pull == SG_LB_NONE;
+    a.team = a.lb_push_none || a.lb_pull_none ? 0u : e->g->relabeled ? 1u : 2u;
     e->last_algo = 0;
     const int bs = o.block_size ? o.block_size : 1024;
     switch (bs) {
@@ -255,6 +256,7 @@ extern "C" int sg_bfs_noalloc(const sg_graph *g, uint32_t source, int32_t *level
     a.max_rounds = (uint32_t)o.max_iteration;
     a.lb_push_none = o.lb_push == SG_LB_NONE;
     a.lb_pull_none = o.lb_pull == SG_LB_NONE;
+    a.team = a.lb_push_none || a.lb_pull_none ? 0u : g->relabeled ? 1u : 2u;
     if (!d.ptr && (rc = na_setup(d, g, s, a))) return rc;
 
     uint64_t *bm = (uint64_t *)(d.ptr + kNaOffBitmaps);

@@ -36,12 +36,28 @@
 // vertex stops at its first parent (the reference's early break,
 // pull_functor.h:138-188). Pull rounds write whole words of the next frontier
 // bitmap and of a visited filter, so they need no atomics.
+//
+// Rounds with little work, and whole queries on small graphs, run on the blocks
+// of one XCD, the team, with a barrier inside its L2 (bfs_team_phase,
+// bfs_whole; team_exchange in sg_device.hpp).
 #pragma once
 
 #include "frontier.hpp"
 
 using namespace sg;
 
+// Rounds a team runs: push rounds of at most this many edges (see
+// bfs_team_fits), and every round of a graph of at most this many words and
+// edges (see bfs_whole).
+#ifndef SG_TEAM_PUSH_EDGES
+#define SG_TEAM_PUSH_EDGES 16384
+#endif
+#ifndef SG_TEAM_WORDS
+#define SG_TEAM_WORDS 256
+#endif
+#ifndef SG_TEAM_EDGES
+#define SG_TEAM_EDGES 1000000
+#endif
 // Words of 64 vertices a wave works on at once in a pull round.
 #ifndef SG_PULL_GROUP
 #define SG_PULL_GROUP 2
@@ -56,6 +72,12 @@ namespace {
 namespace bfsk {
 
 constexpr int kPullGroup = SG_PULL_GROUP;
+constexpr uint32_t kTeamPushEdges = SG_TEAM_PUSH_EDGES, kTeamPushNodes = SG_TEAM_PUSH_EDGES;
+constexpr uint32_t kTeamWords = SG_TEAM_WORDS;
+constexpr uint64_t kTeamEdges = SG_TEAM_EDGES;
+static_assert(kTeamPushEdges <= kTeamSegment && kTeamWords * 64 <= kTeamSegment, "a team round fits its segments");
+// Rounds of one team phase: bounds the other blocks' wait.
+constexpr uint32_t kTeamRounds = 8192;
 
 struct BfsArgs {
     DevGraph g;
@@ -86,6 +108,8 @@ struct BfsArgs {
     // LoadBalancing::NONE (one lane per vertex, its edges in order, no hub
     // chunks) for push / pull rounds; otherwise the balanced schedulers
     uint32_t lb_push_none, lb_pull_none;
+    uint32_t team;  // rounds with little work may run on one XCD's blocks:
+                    // 1 (skewed graphs) after the first pull round, 2 from the start
 };
 
 // Hub chunks whose heads a block stages in LDS at a time (with 64-edge
@@ -306,6 +330,400 @@ __device__ __forceinline__ void pull_group(Round &R, const uint32_t (&wg)[G], co
     }
 }
 
+// ------------------------------------------------------------ team rounds
+// A graph so small that the team runs all of its rounds. Every member then
+// keeps the visited filter and the round's frontier in LDS (2 x 4 KiB), and the
+// rounds meet only in the next frontier's bitmap: atomics on the few cache
+// lines such bitmaps fill serialise (6-15 ns each on one line), so a bit set in
+// a member's own copy is claimed there first.
+__device__ __forceinline__ bool bfs_team_graph(const DevGraph &g)
+{
+    return g.words <= kTeamWords && g.m <= kTeamEdges;
+}
+
+// Whether round L, of a grid round's frontier, starts a team phase; evaluated
+// alike by every block. Only narrow push rounds do: on the 2048 x 2048 grid
+// (2668 rounds of at most 10.6 K edges) they take 4.4-6.1 us on the team and
+// 10.2-11.4 on the whole grid, 33.6 -> 16.3 ms a query; with the limit at 8 K
+// edges it takes 17.3 ms, at 4 K 24.5, and no measured graph had a round between
+// 16 K and 32 K that told them apart.
+// On a skewed graph only once its peak is past: before it a
+// narrow frontier's next one is seldom narrow, and ending a phase costs a
+// barrier and a frontier read back from its bitmap.
+__device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const DirectionPolicy &pol, uint32_t L,
+                                              uint32_t pulls, const RoundCounts &rc)
+{
+    if (!a.team) return false;
+    DirectionPolicy p = pol;
+    return (a.team == 2 || pulls) && !rc.has_huge && rc.count <= kTeamPushNodes && rc.scout <= kTeamPushEdges &&
+           !p.next(L, rc.count, rc.scout);
+}
+
+// What the rounds of a phase share: the member's place, and the frontier as
+// segments of a queue, one per block that found its vertices (lane k holds the
+// entries up to the end of segment k).
+struct BfsTeam {
+    uint32_t members, rank, tag;
+    uint32_t gwave, nwaves;
+    uint32_t L;
+    uint32_t incl, total;    // segment ends (by lane), entries in all
+    const uint32_t *qin;
+    uint32_t *qout;          // this block's segment of the next queue
+    uint32_t seg;            // entries per segment
+    uint64_t *fnext;
+    uint64_t *s_vis;         // whole-graph phases: the visited filter and
+    uint64_t *s_front;       // frontier L in LDS
+};
+
+// A vertex found for level L+1: its level and its place in the next queue.
+// `dv`: its out-degree.
+__device__ __forceinline__ void team_found(const BfsArgs &a, const BfsTeam &T, TeamLds &t, uint32_t v, uint32_t id,
+                                           uint32_t dv)
+{
+    a.level[id] = (int32_t)T.L + 1;
+    const unsigned long long old = atomicAdd(&t.acc, (1ull << kTeamCountShift) | dv);
+    if (dv > kHugeDegree) t.flag = 1u;
+    T.qout[(uint32_t)(old >> kTeamCountShift)] = v;
+}
+
+// Edge -> v for `act` lanes. One atomicOr claims an unvisited head (heads of a
+// narrow round seldom share a word, so runs are not gathered first); the loads
+// a discovery needs travel with it.
+template <bool kWhole>
+__device__ __forceinline__ void team_visit(const BfsArgs &a, const BfsTeam &T, TeamLds &t, bool act, uint32_t v)
+{
+    if (!act) return;
+    const uint32_t w = v >> 6;
+    const uint64_t bit = 1ull << (v & 63);
+    uint64_t old;
+    if constexpr (kWhole) {
+        if (T.s_vis[w] & bit) return;
+        if (atomicOr((unsigned long long *)&T.s_vis[w], (unsigned long long)bit) & bit) return;
+        old = atomicOr((unsigned long long *)&T.fnext[w], (unsigned long long)bit);
+    } else {
+        if (load_team(a.vis + w) & bit) return;
+        old = atomicOr((unsigned long long *)&a.vis[w], (unsigned long long)bit);
+    }
+    const uint32_t rb = a.g.row[v], re = a.g.row[v + 1];
+    const uint32_t id = caller_id(a, v);
+    if (!(old & bit)) team_found(a, T, t, v, id, re - rb);
+}
+
+// Push: `width` lanes per queue entry (a power of two, 4 to 64, as many as the
+// team has for the frontier), each taking every width-th out-edge, so a
+// narrow frontier needs no edge scheduling across the wave.
+template <bool kWhole>
+__device__ __forceinline__ void team_push(const BfsArgs &a, const BfsTeam &T, TeamLds &t, bool hubs)
+{
+    const DevGraph &g = a.g;
+    const int ln = lane();
+    if (kWhole && hubs) {
+        // out-degrees above kHugeDegree by the chunk list
+        for (uint32_t c0 = 0; c0 < g.nhuge; c0 += T.nwaves * kWave) {
+            const uint32_t c = c0 + (uint32_t)ln * T.nwaves + T.gwave;
+            uint2 dsc = make_uint2(0u, 0u);
+            uint32_t end = 0;
+            bool mem = false;
+            if (c < g.nhuge) {
+                dsc = g.huge[c];
+                end = g.huge_end[c];
+                mem = test_bit(T.s_front, dsc.x);
+            }
+            uint64_t mm = ballot(mem);
+            while (mm) {
+                const int k = first_lane(mm);
+                mm &= mm - 1;
+                const uint32_t beg = lane_value(dsc.y, k), stop = lane_value(end, k);
+                for (uint32_t e = beg + (uint32_t)ln; e < stop; e += kWave)
+                    team_visit<kWhole>(a, T, t, true, g.col[e]);
+            }
+        }
+    }
+    uint32_t shift = 6;
+    while (shift > 2 && ((uint64_t)T.total << shift) > (uint64_t)T.nwaves * kWave) shift--;
+    const uint32_t width = 1u << shift, groups = kWave >> shift;
+    const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
+    for (uint32_t i0 = T.gwave * groups; i0 < T.total; i0 += T.nwaves * groups) {
+        const uint32_t i = i0 + grp;
+        // the segment holding entry i: uniform for i0, stepped on from there
+        int k = __popcll(ballot(T.incl <= i0));
+        for (;;) {
+            const uint32_t stop = shfl(T.incl, k);
+            const bool past = i < T.total && i >= stop;
+            if (!ballot(past)) break;
+            k += past;
+        }
+        const uint32_t before = shfl(T.incl, k > 0 ? k - 1 : 0);
+        uint32_t e = 0, end = 0;
+        if (i < T.total) {
+            const uint32_t u = load_team(T.qin + (size_t)k * T.seg + (i - (k > 0 ? before : 0u)));
+            e = g.row[u];
+            end = g.row[u + 1];
+            if (end - e > kHugeDegree) end = e;
+            e += sub;
+        }
+        for (; ballot(e < end); e += 2 * width) {
+            const bool p = e < end, q = e + width < end;
+            const uint32_t v = p ? g.col[e] : 0u, w = q ? g.col[e + width] : 0u;
+            team_visit<kWhole>(a, T, t, p, v);
+            team_visit<kWhole>(a, T, t, q, w);
+        }
+    }
+}
+
+// Pull (whole-graph phases): an in-hub per wave, 256 of its in-edges in flight,
+// then `width` lanes per other unvisited vertex, a wave's vertices adjacent so
+// that it sets their next-frontier bits with one atomic. Each stops at a
+// first parent.
+__device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, TeamLds &t)
+{
+    const DevGraph &g = a.g;
+    const uint32_t n = g.n;
+    const int ln = lane();
+    constexpr int K = 4;
+    for (uint32_t h = T.gwave; h < g.nhubin; h += T.nwaves) {
+        const uint2 first = g.hugein[g.hubin[h].x];
+        const uint32_t v = first.x, stop = g.cstart[v + 1];
+        if (test_bit(T.s_vis, v)) continue;
+        for (uint32_t e0 = first.y; e0 < stop; e0 += K * kWave) {
+            uint32_t u[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const uint32_t e = e0 + (uint32_t)(k * kWave + ln);
+                u[k] = e < stop ? g.csrc[e] : 0xFFFFFFFFu;
+            }
+            bool hit = false;
+#pragma unroll
+            for (int k = 0; k < K; k++) hit |= u[k] != 0xFFFFFFFFu && test_bit(T.s_front, u[k]);
+            if (!ballot(hit)) continue;
+            if (ln == 0) {
+                atomicOr((unsigned long long *)&T.fnext[v >> 6], 1ull << (v & 63));
+                team_found(a, T, t, v, caller_id(a, v), g.row[v + 1] - g.row[v]);
+            }
+            break;
+        }
+    }
+    uint32_t shift = 6;
+    while (shift > 2 && ((uint64_t)n << shift) > (uint64_t)T.nwaves * kWave) shift--;
+    const uint32_t width = 1u << shift, groups = kWave >> shift;
+    const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
+    const uint64_t gmask = (shift == 6 ? ~0ull : (1ull << width) - 1) << (grp << shift);
+    for (uint32_t v0 = T.gwave * groups; v0 < n; v0 += T.nwaves * groups) {
+        const uint32_t v = v0 + grp;
+        const bool want = v < n && !test_bit(T.s_vis, v);
+        if (!ballot(want)) continue;
+        uint32_t e = 0, end = 0, dv = 0, id = 0;
+        if (want) {
+            e = g.cstart[v];
+            end = g.cstart[v + 1];
+            if (end - e > kPullHubDegree) end = e;
+            e += sub;
+            dv = g.row[v + 1] - g.row[v];
+            id = caller_id(a, v);
+        }
+        bool found = false;
+        while (ballot(e < end)) {
+            uint32_t u[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) u[k] = e + k * width < end ? g.csrc[e + k * width] : 0xFFFFFFFFu;
+            bool hit = false;
+#pragma unroll
+            for (int k = 0; k < K; k++) hit |= u[k] != 0xFFFFFFFFu && test_bit(T.s_front, u[k]);
+            found |= (ballot(hit) & gmask) != 0;
+            e = found ? end : e + K * width;
+        }
+        found = found && sub == 0;
+        if (!ballot(found)) continue;
+        const uint64_t bits = wave_reduce(found ? 1ull << (v & 63) : 0ull, 0ull, [](uint64_t x, uint64_t y) { return x | y; });
+        if (ln == 0) atomicOr((unsigned long long *)&T.fnext[v0 >> 6], (unsigned long long)bits);
+        if (found) team_found(a, T, t, v, id, dv);
+    }
+}
+
+// The members' words after an exchange: segment ends and entries in all.
+__device__ __forceinline__ uint64_t team_segments(BfsTeam &T, const TeamLds &t)
+{
+    const uint64_t w = (uint32_t)lane() < kTeamMax ? t.slot[lane()] : 0ull;
+    T.incl = wave_incl_scan((uint32_t)((w >> kTeamCountShift) & kTeamCountMask));
+    T.total = lane_value(T.incl, kWave - 1);
+    return w;
+}
+
+// A team phase: rounds from L on, by this member of the team, while they stay
+// small (kWhole, a graph the team runs whole: to the end). The state it leaves
+// is what a grid round expects: frontier L as a bitmap, counters saying that no
+// queue holds it; after the last round, what the epilogue leaves. Returns
+// false when a wait expired; `more`: rounds are left. At most `cap` rounds;
+// `t_start` is the trace's time 0.
+template <int BS, bool kWhole>
+__device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t members,
+                                               uint32_t rank, uint32_t &tag, DirectionPolicy &pol, uint32_t &L,
+                                               const RoundCounts &rc, uint32_t &pushes, uint32_t &pulls,
+                                               unsigned long long &ptrace, long long t_start, uint32_t cap,
+                                               bool &more)
+{
+    constexpr int WPB = BS / kWave;
+    const uint32_t W = a.g.words;
+    const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
+    const bool lead = rank == 0 && threadIdx.x == 0;
+    BfsTeam T;
+    T.members = members;
+    T.rank = rank;
+    T.tag = tag;
+    T.gwave = rank * WPB + threadIdx.x / kWave;
+    T.nwaves = members * WPB;
+    T.seg = a.qcap / members;
+    T.s_vis = s_bits;
+    T.s_front = s_bits + kTeamWords;
+    if (kWhole)
+        for (uint32_t w = threadIdx.x; w < W; w += BS) T.s_vis[w] = load_team(a.vis + w);
+    bool ok = true;
+    if (pol.pull_prev || rc.overflow) {
+        // no queue: each member gathers its share of the bitmap into its segment
+        const uint64_t *fl = a.fbit + (size_t)(L % 3) * W;
+        uint32_t *q = a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg;
+        for (uint32_t w = tid; w < W; w += nthreads) {
+            uint64_t x = load_team(fl + w);
+            if (!x) continue;
+            const unsigned long long old =
+                atomicAdd(&t.acc, (unsigned long long)__popcll(x) << kTeamCountShift);
+            uint32_t at = (uint32_t)(old >> kTeamCountShift);
+            for (; x; x &= x - 1) q[at++] = w * 64 + (uint32_t)first_lane(x);
+        }
+        ok = team_exchange(a.bar, t, members, rank, T.tag, a.abort);
+        team_segments(T, t);
+    } else {
+        T.incl = T.total = rc.qlen;  // the grid's queue is one segment
+    }
+    unsigned long long count = rc.count, scout = rc.scout;
+    bool hubs = rc.has_huge;
+    // a phase of narrow rounds keeps no bitmaps and leaves all three clear meanwhile
+    if (!kWhole)
+        for (uint32_t w = tid; w < W; w += nthreads) {
+            a.fbit[(size_t)(L % 3) * W + w] = 0;
+            a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
+        }
+    more = ok;
+    for (uint32_t r = 0; more && r < cap; r++) {
+        const bool pull = pol.next(L, count, scout);
+        pulls += pull;
+        pushes += !pull;
+        if (pull && L < 64) ptrace |= 1ull << L;
+        if (lead) write_trace(a.trace, L, pull, count, scout, t_start);
+        T.L = L;
+        T.qin = a.queue + (size_t)(L % 3) * a.qcap;
+        T.qout = a.queue + (size_t)((L + 1) % 3) * a.qcap + (size_t)rank * T.seg;
+        T.fnext = a.fbit + (size_t)((L + 1) % 3) * W;
+        if constexpr (kWhole) {
+            for (uint32_t w = tid; w < W; w += nthreads) a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
+            for (uint32_t w = threadIdx.x; w < W; w += BS) {
+                const uint64_t x = load_team(a.fbit + (size_t)(L % 3) * W + w);
+                T.s_front[w] = x;
+                T.s_vis[w] |= x;
+            }
+            __syncthreads();
+            if (pull) team_pull(a, T, t);
+            else team_push<true>(a, T, t, hubs);
+        } else {
+            team_push<false>(a, T, t, false);
+        }
+        pol.pull_prev = pull;
+        L++;
+        ok = team_exchange(a.bar, t, members, rank, T.tag, a.abort);
+        if (!ok) break;
+        const uint64_t w = team_segments(T, t);
+        count = T.total;
+        scout = wave_sum_u64(w & 0xFFFFFFFFu);
+        hubs = ballot((w >> kTeamFlagShift) & 1) != 0;
+        more = count != 0 && !(a.max_rounds && L >= a.max_rounds);
+        if (more && !kWhole) {
+            DirectionPolicy p = pol;
+            if (hubs || count > kTeamPushNodes || scout > kTeamPushEdges || p.next(L, count, scout)) break;
+        }
+    }
+    tag = T.tag;
+    if (!ok) return false;
+    uint64_t *fl = a.fbit + (size_t)(L % 3) * W;
+    if (!more) {
+        // the last round: bitmaps and counters are left clear for the next query
+        for (uint32_t w = tid; w < 3 * W && kWhole; w += nthreads) a.fbit[w] = 0;
+    } else if (kWhole) {
+        // the filter in memory takes frontier L and all before it
+        if (rank == 0)
+            for (uint32_t w = threadIdx.x; w < W; w += BS) a.vis[w] = T.s_vis[w] | load_team(fl + w);
+    } else {
+        const uint32_t own = (uint32_t)((t.slot[rank] >> kTeamCountShift) & kTeamCountMask);
+        const uint32_t *q = a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg;
+        for (uint32_t i = threadIdx.x; i < own; i += BS) {
+            const uint32_t u = load_team(q + i);
+            atomicOr((unsigned long long *)&fl[u >> 6], 1ull << (u & 63));
+        }
+    }
+    if (rank == 0) {
+        for (int i = 0; i < 3; i++) clear_ctr(&a.ctr[i]);
+        block_sync_global();
+        if (threadIdx.x == 0 && more) {
+            FrontierCtr &c = a.ctr[L % 3];
+            c.overflow = 1;
+            c.has_huge = hubs;
+            c.stripe[0].scout = scout;
+            c.stripe[0].count = count;
+        }
+    }
+    return true;
+}
+
+// The whole query on the team, for a graph it runs whole: the other blocks
+// return after the census, so no grid barrier is taken. Every state the next
+// query expects is left as the grid's own path leaves it. A query by grid
+// rounds and by this path: RMAT graphs of 4096 vertices 56 and 37 us, of 8001 62
+// and 41, of 16001 67 and 51, of 32001 70 and 84 (one XCD's caches and CUs
+// no longer suffice), so the line lies at 16384 vertices.
+template <int BS>
+__device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t sdeg, uint32_t xcc,
+                                          BarState &gen, long long t_start)
+{
+    __shared__ uint32_t s_m[3];
+    const DevGraph &g = a.g;
+    const uint32_t W = g.words, src = a.source;
+    if (threadIdx.x == 0) {
+        s_m[2] = bar_census(a.bar, xcc, gen, a.abort);
+        s_m[0] = min(gen.cnt, kTeamMax);
+        s_m[1] = xcc == gen.first && gen.rank < kTeamMax ? gen.rank : ~0u;
+    }
+    __syncthreads();
+    const uint32_t members = s_m[0], rank = s_m[1];
+    uint32_t tag = 0, L = 0, pushes = 0, pulls = 0;
+    unsigned long long ptrace = 0;
+    bool ok = s_m[2] != 0u, more = true;
+    if (ok && rank == ~0u) return true;
+    if (ok) {
+        const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
+        for (uint32_t i = tid; i < g.n; i += nthreads) a.level[i] = i == a.source_id ? 0 : -1;
+        for (uint32_t w = tid; w < W; w += nthreads) {
+            const uint64_t sb = w == (src >> 6) ? 1ull << (src & 63) : 0ull;
+            const uint64_t inert = g.inert ? g.inert[w] : 0ull;
+            a.vis[w] = inert | sb;
+            a.vis_idle[w] = inert;
+            a.fbit[w] = sb;
+            a.fbit[(size_t)W + w] = 0;
+            a.fbit[2 * (size_t)W + w] = 0;
+        }
+        if (tid == 0) a.queue[0] = src;
+        ok = team_exchange(a.bar, t, members, rank, tag, a.abort);
+    }
+    if (ok) {
+        DirectionPolicy pol{a.alpha, a.beta, a.total_workload0, g.n, a.force};
+        const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
+        ok = bfs_team_phase<BS, true>(a, t, s_bits, members, rank, tag, pol, L, rc, pushes, pulls, ptrace, t_start, ~0u,
+                                      more);
+    }
+    // (after a failed census every block's rank is unknown: block 0 reports)
+    if (threadIdx.x == 0 && (s_m[2] ? rank == 0 : blockIdx.x == 0))
+        write_final(a.trace, a.stats, L, pushes, pulls, ptrace, ok, t_start);
+    return ok;
+}
+
 #if SG_BFS_WAVES
 #define SG_BFS_BOUNDS(BS) __launch_bounds__(BS, SG_BFS_WAVES)
 #else
@@ -320,7 +738,11 @@ __device__ __forceinline__ void pull_group(Round &R, const uint32_t (&wg)[G], co
 // kStage: push rounds stage hub neighbour lists in LDS (the engine option
 // stage_hubs; a separate instantiation, so the default path keeps its
 // register budget).
-template <int BS, bool kStage = false>
+// kTeamOk: rounds with little work may run on the team (a.team; needs `gen`
+// from bar_begin<true> on a.bar, whose first barrier takes the census).
+// kLeave: nothing follows the traversal, so blocks may return before every
+// block has seen its end.
+template <int BS, bool kStage = false, bool kTeamOk = false, bool kLeave = false>
 __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32_t nblocks, uint32_t xcc,
                                         BarState &gen)
 {
@@ -337,12 +759,20 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
 
     __shared__ unsigned long long s_red[2][WPB];
     __shared__ unsigned long long s_lvl[5];
-    __shared__ uint32_t s_q[kLdsQ];
+    alignas(8) __shared__ uint32_t s_q[kLdsQ];
     __shared__ uint32_t s_qn, s_flush[2];
     // hub round: the block's member chunks (first edge, end) and their staged heads
     __shared__ uint2 s_hc[kStage ? kHubList : 1];
     __shared__ uint32_t s_he[kStage ? kStageChunks * kHugeChunk : 1];
     __shared__ uint32_t s_hn;
+    __shared__ TeamLds s_t;
+    __shared__ uint32_t s_team[2], s_note[8];
+    static_assert(sizeof(s_q) >= 2 * kTeamWords * 8, "a team's bitmaps fit the queue's LDS");
+    if (kTeamOk && threadIdx.x == 0) {
+        s_t.acc = 0;
+        s_t.flag = 0;
+    }
+    uint32_t phase = 0, tag = 0;
 
     // ---- prologue: reset the levels (caller order) and seed the source.
     // The previous query left the frontier bitmaps and counters zeroed, and
@@ -352,6 +782,11 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
     const uint32_t src = a.source;
     const uint32_t sbeg = g.row[src], sdeg = g.row[src + 1] - sbeg;
     const uint64_t sbit = 1ull << (src & 63);
+    if constexpr (kLeave) {
+        if (a.team && bfs_team_graph(g))
+            return bfs_whole<BS>(a, s_t, (uint64_t *)s_q, sdeg, xcc, gen, t_start);
+    }
+    if (kTeamOk && gtid == 0) *(long long *)(a.bar.words + kBarNote + 8) = t_start;
     for (uint32_t i = gtid; i < n; i += nthreads) a.level[i] = (i == a.source_id) ? 0 : -1;
     for (uint32_t w = gtid; w < W; w += nthreads) a.vis_idle[w] = g.inert ? g.inert[w] : 0ull;
     DirectionPolicy pol{a.alpha, a.beta, a.total_workload0, n, a.force};  // replicated in every block
@@ -430,6 +865,65 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         }
         if (rc.count == 0) break;
         if (a.max_rounds && L >= a.max_rounds) break;
+
+        if (kTeamOk && bfs_team_fits(a, pol, L, pulls, rc)) {
+            if (threadIdx.x == 0) {
+                s_team[0] = min(gen.cnt, kTeamMax);
+                s_team[1] = xcc == gen.first && gen.rank < kTeamMax ? gen.rank : ~0u;
+            }
+            __syncthreads();
+            const uint32_t members = s_team[0], rank = s_team[1];
+            // two notes in turn: a block may still be reading the last
+            // phase's when the next phase's is written
+            uint32_t *note = a.bar.words + kBarNote + 16 * (phase++ & 1u);
+            bool more = true;
+            if (rank != ~0u) {
+                // a failed wait set the abort flag, which ends the others' wait
+                const long long t0 = rank == 0 && threadIdx.x == 0
+                                         ? (long long)load_team((const uint64_t *)(a.bar.words + kBarNote + 8))
+                                         : 0ll;
+                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, members, rank, tag, pol, L, rc, pushes, pulls,
+                                               ptrace, t0, kTeamRounds, more);
+                if (!ok) break;
+                if (rank == 0 && threadIdx.x == 0) {
+                    note[0] = L;
+                    note[1] = pol.total_wl;
+                    note[2] = pol.pull_prev;
+                    note[3] = pushes;
+                    note[4] = pulls;
+                    note[5] = (uint32_t)ptrace;
+                    note[6] = (uint32_t)(ptrace >> 32);
+                    note[7] = more;
+                    if (kLeave && !more) write_final(a.trace, a.stats, L, pushes, pulls, ptrace, true, t_start);
+                }
+            }
+            // the phase's barrier. After the last round a member leaves once it
+            // has arrived, and the others as soon as they see the note, with no
+            // acquire (they read nothing more).
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                const uint32_t gen0 = grid_arrive(a.bar, xcc, gen);
+                if (kLeave && !more) {
+                    s_note[7] = 0;
+                } else {
+                    s_team[0] = spin_wait<true>(a.bar.words + kBarGen, gen0, true, a.bar.spin_limit, a.abort);
+                    for (int i = 0; i < 8; i++) s_note[i] = poll_load(note + i);
+                    if (!kLeave || s_note[7]) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                    __builtin_amdgcn_s_waitcnt(0);
+                }
+            }
+            __syncthreads();
+            ok = s_team[0] != 0u;
+            if (kLeave && ok && !s_note[7]) return true;
+            L = s_note[0];
+            pol.total_wl = s_note[1];
+            pol.pull_prev = s_note[2] != 0u;
+            pushes = s_note[3];
+            pulls = s_note[4];
+            ptrace = (unsigned long long)s_note[6] << 32 | s_note[5];
+            continue;
+        }
 
         const bool pull = pol.next(L, rc.count, rc.scout);
         if (pull) {

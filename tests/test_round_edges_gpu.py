@@ -36,3 +36,70 @@ def test_pagerank_in_degree_edges(sg, orc, gpu, degrees, mode):
     ref = ref[0] if isinstance(ref, tuple) else ref
     # FP32 ranks: one rounding each, sums compensated
     assert np.abs(got - ref).sum() / ref.sum() < 1e-6
+
+
+def path_graph(sg, n):
+    v = np.arange(n - 1, dtype=np.uint32)
+    row, col = sg.build_csr(n, v, v + 1, symmetrize=True)
+    return sg.HostGraph(n, row, col, None, undirected=True)
+
+
+def random_graph(sg, n, degree, seed, weights=None):
+    rng = np.random.default_rng(seed)
+    src = rng.integers(0, n, n * degree).astype(np.uint32)
+    dst = rng.integers(0, n, n * degree).astype(np.uint32)
+    row, col = sg.build_csr(n, src, dst)
+    w = None if weights is None else rng.integers(weights[0], weights[1], len(col)).astype(np.uint32)
+    return sg.HostGraph(n, row, col, w)
+
+
+def star_chain(sg, n, leaves):
+    """A path whose every 50th vertex also has `leaves` leaves."""
+    hubs = np.arange(0, n, 50)
+    src = np.concatenate([np.arange(n - 1), np.repeat(hubs, leaves)]).astype(np.uint32)
+    dst = np.concatenate([np.arange(1, n), n + np.arange(len(hubs) * leaves)]).astype(np.uint32)
+    total = n + len(hubs) * leaves
+    row, col = sg.build_csr(total, src, dst, symmetrize=True)
+    return sg.HostGraph(total, row, col, None, undirected=True)
+
+
+SMALL_ROUND_GRAPHS = {
+    # the whole query on one XCD's blocks: words and their remainders, the limit, hubs
+    "n1": lambda sg: sg.HostGraph(1, np.zeros(2, np.uint32), np.zeros(0, np.uint32), None),
+    "n63": lambda sg: random_graph(sg, 63, 3, 1),
+    "n64": lambda sg: random_graph(sg, 64, 3, 2),
+    "n65": lambda sg: random_graph(sg, 65, 3, 3),
+    "n16384": lambda sg: random_graph(sg, 16384, 8, 4),
+    "n16385": lambda sg: random_graph(sg, 16385, 8, 5),
+    "stars": lambda sg: star_chain(sg, 300, 257),
+    "path9000": lambda sg: path_graph(sg, 9000),
+    "rmat13": lambda sg: sg.rmat_graph(13, 16, symmetrize=True, seed=6),
+    # narrow rounds of a larger graph: more rounds than one phase holds, a
+    # frontier that outgrows the limit and shrinks again, hubs on the way
+    "path20000": lambda sg: path_graph(sg, 20000),
+    "random": lambda sg: random_graph(sg, 60000, 3, 7),
+    "dense": lambda sg: random_graph(sg, 40000, 40, 8),
+    "stars-long": lambda sg: star_chain(sg, 17000, 300),
+    "grid": lambda sg: sg.grid_graph(131, 257, 0.1, seed=9, weights=None),
+    "rmat17": lambda sg: sg.rmat_graph(17, 16, symmetrize=False, seed=10),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opts", [{}, {"block_size": 256}, {"grid_blocks": 1}, {"force_variant": "async_pull_dd"},
+                                  {"force_variant": "async_push_dd"}, {"max_iteration": 3}])
+@pytest.mark.parametrize("name", list(SMALL_ROUND_GRAPHS))
+def test_bfs_small_rounds(sg, orc, gpu, name, opts):
+    if name in ("path9000", "path20000", "stars-long") and opts and "max_iteration" not in opts:
+        pytest.skip("long traversal: default schedule and round limit only")
+    hg = SMALL_ROUND_GRAPHS[name](sg)
+    e = sg.Engine(sg.Graph(hg), **opts)
+    for s in sorted({0, hg.n // 2, hg.n - 1}):
+        e.bfs(s)
+        got = e.gather(np.int32)
+        ref = orc.bfs(hg.row, hg.col, s)
+        cap = opts.get("max_iteration")
+        if cap:
+            ref = np.where(ref > cap, -1, ref)
+        assert np.array_equal(got, ref), s
+        assert e.stats()["rounds"] == (min(cap, ref.max() + 1) if cap else ref.max() + 1)
