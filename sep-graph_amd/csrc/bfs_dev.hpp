@@ -46,18 +46,6 @@
 
 using namespace sg;
 
-// Rounds a team runs: push rounds of at most this many edges (see
-// bfs_team_fits), and every round of a graph of at most this many words and
-// edges (see bfs_whole).
-#ifndef SG_TEAM_PUSH_EDGES
-#define SG_TEAM_PUSH_EDGES 16384
-#endif
-#ifndef SG_TEAM_WORDS
-#define SG_TEAM_WORDS 256
-#endif
-#ifndef SG_TEAM_EDGES
-#define SG_TEAM_EDGES 1000000
-#endif
 // Words of 64 vertices a wave works on at once in a pull round.
 #ifndef SG_PULL_GROUP
 #define SG_PULL_GROUP 2
@@ -72,12 +60,6 @@ namespace {
 namespace bfsk {
 
 constexpr int kPullGroup = SG_PULL_GROUP;
-constexpr uint32_t kTeamPushEdges = SG_TEAM_PUSH_EDGES, kTeamPushNodes = SG_TEAM_PUSH_EDGES;
-constexpr uint32_t kTeamWords = SG_TEAM_WORDS;
-constexpr uint64_t kTeamEdges = SG_TEAM_EDGES;
-static_assert(kTeamPushEdges <= kTeamSegment && kTeamWords * 64 <= kTeamSegment, "a team round fits its segments");
-// Rounds of one team phase: bounds the other blocks' wait.
-constexpr uint32_t kTeamRounds = 8192;
 
 struct BfsArgs {
     DevGraph g;
@@ -331,15 +313,11 @@ __device__ __forceinline__ void pull_group(Round &R, const uint32_t (&wg)[G], co
 }
 
 // ------------------------------------------------------------ team rounds
-// A graph so small that the team runs all of its rounds. Every member then
-// keeps the visited filter and the round's frontier in LDS (2 x 4 KiB), and the
-// rounds meet only in the next frontier's bitmap: atomics on the few cache
-// lines such bitmaps fill serialise (6-15 ns each on one line), so a bit set in
-// a member's own copy is claimed there first.
-__device__ __forceinline__ bool bfs_team_graph(const DevGraph &g)
-{
-    return g.words <= kTeamWords && g.m <= kTeamEdges;
-}
+// On a graph that the team runs whole, every member keeps the visited filter
+// and the round's frontier in LDS (2 x 2 KiB), and the rounds meet only in the
+// next frontier's bitmap: atomics on the few cache lines such bitmaps fill
+// serialise (6-15 ns each on one line), so a bit set in a member's own copy
+// is claimed there first.
 
 // Whether round L, of a grid round's frontier, starts a team phase; evaluated
 // alike by every block. Only narrow push rounds do: on the 2048 x 2048 grid
@@ -350,26 +328,17 @@ __device__ __forceinline__ bool bfs_team_graph(const DevGraph &g)
 // On a skewed graph only once its peak is past: before it a
 // narrow frontier's next one is seldom narrow, and ending a phase costs a
 // barrier and a frontier read back from its bitmap.
-__device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const DirectionPolicy &pol, uint32_t L,
-                                              uint32_t pulls, const RoundCounts &rc)
+__device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const RoundState &S, const RoundCounts &rc)
 {
     if (!a.team) return false;
-    DirectionPolicy p = pol;
-    return (a.team == 2 || pulls) && !rc.has_huge && rc.count <= kTeamPushNodes && rc.scout <= kTeamPushEdges &&
-           !p.next(L, rc.count, rc.scout);
+    DirectionPolicy p = S.pol;
+    return (a.team == 2 || S.pulls) && !rc.has_huge && rc.count <= kTeamPushNodes && rc.scout <= kTeamPushEdges &&
+           !p.next(S.L, rc.count, rc.scout);
 }
 
-// What the rounds of a phase share: the member's place, and the frontier as
-// segments of a queue, one per block that found its vertices (lane k holds the
-// entries up to the end of segment k).
-struct BfsTeam {
-    uint32_t members, rank, tag;
-    uint32_t gwave, nwaves;
+// What the rounds of a phase share.
+struct BfsTeam : TeamFront {
     uint32_t L;
-    uint32_t incl, total;    // segment ends (by lane), entries in all
-    const uint32_t *qin;
-    uint32_t *qout;          // this block's segment of the next queue
-    uint32_t seg;            // entries per segment
     uint64_t *fnext;
     uint64_t *s_vis;         // whole-graph phases: the visited filter and
     uint64_t *s_front;       // frontier L in LDS
@@ -381,9 +350,8 @@ __device__ __forceinline__ void team_found(const BfsArgs &a, const BfsTeam &T, T
                                            uint32_t dv)
 {
     a.level[id] = (int32_t)T.L + 1;
-    const unsigned long long old = atomicAdd(&t.acc, (1ull << kTeamCountShift) | dv);
     if (dv > kHugeDegree) t.flag = 1u;
-    T.qout[(uint32_t)(old >> kTeamCountShift)] = v;
+    team_append(T, t, v, dv);
 }
 
 // Edge -> v for `act` lanes. One atomicOr claims an unvisited head (heads of a
@@ -439,24 +407,14 @@ __device__ __forceinline__ void team_push(const BfsArgs &a, const BfsTeam &T, Te
             }
         }
     }
-    uint32_t shift = 6;
-    while (shift > 2 && ((uint64_t)T.total << shift) > (uint64_t)T.nwaves * kWave) shift--;
+    const uint32_t shift = team_width(T, T.total);
     const uint32_t width = 1u << shift, groups = kWave >> shift;
     const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
     for (uint32_t i0 = T.gwave * groups; i0 < T.total; i0 += T.nwaves * groups) {
         const uint32_t i = i0 + grp;
-        // the segment holding entry i: uniform for i0, stepped on from there
-        int k = __popcll(ballot(T.incl <= i0));
-        for (;;) {
-            const uint32_t stop = shfl(T.incl, k);
-            const bool past = i < T.total && i >= stop;
-            if (!ballot(past)) break;
-            k += past;
-        }
-        const uint32_t before = shfl(T.incl, k > 0 ? k - 1 : 0);
+        const uint32_t u = team_entry(T, i0, i);
         uint32_t e = 0, end = 0;
         if (i < T.total) {
-            const uint32_t u = load_team(T.qin + (size_t)k * T.seg + (i - (k > 0 ? before : 0u)));
             e = g.row[u];
             end = g.row[u + 1];
             if (end - e > kHugeDegree) end = e;
@@ -503,8 +461,7 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
             break;
         }
     }
-    uint32_t shift = 6;
-    while (shift > 2 && ((uint64_t)n << shift) > (uint64_t)T.nwaves * kWave) shift--;
+    const uint32_t shift = team_width(T, n);
     const uint32_t width = 1u << shift, groups = kWave >> shift;
     const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
     const uint64_t gmask = (shift == 6 ? ~0ull : (1ull << width) - 1) << (grp << shift);
@@ -540,15 +497,6 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
     }
 }
 
-// The members' words after an exchange: segment ends and entries in all.
-__device__ __forceinline__ uint64_t team_segments(BfsTeam &T, const TeamLds &t)
-{
-    const uint64_t w = (uint32_t)lane() < kTeamMax ? t.slot[lane()] : 0ull;
-    T.incl = wave_incl_scan((uint32_t)((w >> kTeamCountShift) & kTeamCountMask));
-    T.total = lane_value(T.incl, kWave - 1);
-    return w;
-}
-
 // A team phase: rounds from L on, by this member of the team, while they stay
 // small (kWhole, a graph the team runs whole: to the end). The state it leaves
 // is what a grid round expects: frontier L as a bitmap, counters saying that no
@@ -557,10 +505,8 @@ __device__ __forceinline__ uint64_t team_segments(BfsTeam &T, const TeamLds &t)
 // `t_start` is the trace's time 0.
 template <int BS, bool kWhole>
 __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t members,
-                                               uint32_t rank, uint32_t &tag, DirectionPolicy &pol, uint32_t &L,
-                                               const RoundCounts &rc, uint32_t &pushes, uint32_t &pulls,
-                                               unsigned long long &ptrace, long long t_start, uint32_t cap,
-                                               bool &more)
+                                               uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
+                                               long long t_start, uint32_t cap, bool &more)
 {
     constexpr int WPB = BS / kWave;
     const uint32_t W = a.g.words;
@@ -578,18 +524,11 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
     if (kWhole)
         for (uint32_t w = threadIdx.x; w < W; w += BS) T.s_vis[w] = load_team(a.vis + w);
     bool ok = true;
-    if (pol.pull_prev || rc.overflow) {
+    uint32_t &L = S.L;
+    if (S.pol.pull_prev || rc.overflow) {
         // no queue: each member gathers its share of the bitmap into its segment
-        const uint64_t *fl = a.fbit + (size_t)(L % 3) * W;
-        uint32_t *q = a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg;
-        for (uint32_t w = tid; w < W; w += nthreads) {
-            uint64_t x = load_team(fl + w);
-            if (!x) continue;
-            const unsigned long long old =
-                atomicAdd(&t.acc, (unsigned long long)__popcll(x) << kTeamCountShift);
-            uint32_t at = (uint32_t)(old >> kTeamCountShift);
-            for (; x; x &= x - 1) q[at++] = w * 64 + (uint32_t)first_lane(x);
-        }
+        team_gather(t, a.fbit + (size_t)(L % 3) * W, W, a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg, tid,
+                    nthreads);
         ok = team_exchange(a.bar, t, members, rank, T.tag, a.abort);
         team_segments(T, t);
     } else {
@@ -605,10 +544,7 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
         }
     more = ok;
     for (uint32_t r = 0; more && r < cap; r++) {
-        const bool pull = pol.next(L, count, scout);
-        pulls += pull;
-        pushes += !pull;
-        if (pull && L < 64) ptrace |= 1ull << L;
+        const bool pull = S.next(count, scout);
         if (lead) write_trace(a.trace, L, pull, count, scout, t_start);
         T.L = L;
         T.qin = a.queue + (size_t)(L % 3) * a.qcap;
@@ -627,7 +563,7 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
         } else {
             team_push<false>(a, T, t, false);
         }
-        pol.pull_prev = pull;
+        S.pol.pull_prev = pull;
         L++;
         ok = team_exchange(a.bar, t, members, rank, T.tag, a.abort);
         if (!ok) break;
@@ -637,7 +573,7 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
         hubs = ballot((w >> kTeamFlagShift) & 1) != 0;
         more = count != 0 && !(a.max_rounds && L >= a.max_rounds);
         if (more && !kWhole) {
-            DirectionPolicy p = pol;
+            DirectionPolicy p = S.pol;
             if (hubs || count > kTeamPushNodes || scout > kTeamPushEdges || p.next(L, count, scout)) break;
         }
     }
@@ -683,19 +619,14 @@ template <int BS>
 __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t sdeg, uint32_t xcc,
                                           BarState &gen, long long t_start)
 {
-    __shared__ uint32_t s_m[3];
+    __shared__ uint32_t s_ok;
     const DevGraph &g = a.g;
     const uint32_t W = g.words, src = a.source;
-    if (threadIdx.x == 0) {
-        s_m[2] = bar_census(a.bar, xcc, gen, a.abort);
-        s_m[0] = min(gen.cnt, kTeamMax);
-        s_m[1] = xcc == gen.first && gen.rank < kTeamMax ? gen.rank : ~0u;
-    }
-    __syncthreads();
-    const uint32_t members = s_m[0], rank = s_m[1];
-    uint32_t tag = 0, L = 0, pushes = 0, pulls = 0;
-    unsigned long long ptrace = 0;
-    bool ok = s_m[2] != 0u, more = true;
+    if (threadIdx.x == 0) s_ok = bar_census(a.bar, xcc, gen, a.abort);
+    uint32_t members, rank, tag = 0;
+    team_place(xcc, gen, members, rank);
+    RoundState S{{a.alpha, a.beta, a.total_workload0, g.n, a.force}, 0, 0, 0, 0};
+    bool ok = s_ok != 0u, more = true;
     if (ok && rank == ~0u) return true;
     if (ok) {
         const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
@@ -713,14 +644,12 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint64_t
         ok = team_exchange(a.bar, t, members, rank, tag, a.abort);
     }
     if (ok) {
-        DirectionPolicy pol{a.alpha, a.beta, a.total_workload0, g.n, a.force};
         const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
-        ok = bfs_team_phase<BS, true>(a, t, s_bits, members, rank, tag, pol, L, rc, pushes, pulls, ptrace, t_start, ~0u,
-                                      more);
+        ok = bfs_team_phase<BS, true>(a, t, s_bits, members, rank, tag, S, rc, t_start, ~0u, more);
     }
     // (after a failed census every block's rank is unknown: block 0 reports)
-    if (threadIdx.x == 0 && (s_m[2] ? rank == 0 : blockIdx.x == 0))
-        write_final(a.trace, a.stats, L, pushes, pulls, ptrace, ok, t_start);
+    if (threadIdx.x == 0 && (s_ok ? rank == 0 : blockIdx.x == 0))
+        write_final(a.trace, a.stats, S.L, S.pushes, S.pulls, S.ptrace, ok, t_start);
     return ok;
 }
 
@@ -766,12 +695,8 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
     __shared__ uint32_t s_he[kStage ? kStageChunks * kHugeChunk : 1];
     __shared__ uint32_t s_hn;
     __shared__ TeamLds s_t;
-    __shared__ uint32_t s_team[2], s_note[8];
     static_assert(sizeof(s_q) >= 2 * kTeamWords * 8, "a team's bitmaps fit the queue's LDS");
-    if (kTeamOk && threadIdx.x == 0) {
-        s_t.acc = 0;
-        s_t.flag = 0;
-    }
+    if (kTeamOk && threadIdx.x == 0) s_t.reset();
     uint32_t phase = 0, tag = 0;
 
     // ---- prologue: reset the levels (caller order) and seed the source.
@@ -783,16 +708,14 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
     const uint32_t sbeg = g.row[src], sdeg = g.row[src + 1] - sbeg;
     const uint64_t sbit = 1ull << (src & 63);
     if constexpr (kLeave) {
-        if (a.team && bfs_team_graph(g))
+        if (a.team && team_whole_graph(g))
             return bfs_whole<BS>(a, s_t, (uint64_t *)s_q, sdeg, xcc, gen, t_start);
     }
-    if (kTeamOk && gtid == 0) *(long long *)(a.bar.words + kBarNote + 8) = t_start;
+    if (kTeamOk && gtid == 0) team_clock_set(a.bar, t_start);
     for (uint32_t i = gtid; i < n; i += nthreads) a.level[i] = (i == a.source_id) ? 0 : -1;
     for (uint32_t w = gtid; w < W; w += nthreads) a.vis_idle[w] = g.inert ? g.inert[w] : 0ull;
-    DirectionPolicy pol{a.alpha, a.beta, a.total_workload0, n, a.force};  // replicated in every block
-    unsigned long long ptrace = 0;
-    uint32_t pushes = 0, pulls = 0;
-    uint32_t L = 0;
+    RoundState S{{a.alpha, a.beta, a.total_workload0, n, a.force}, 0, 0, 0, 0};  // replicated in every block
+    uint32_t &L = S.L;
     const bool local0 = !a.full_init && a.force != 1 && sdeg <= kLocalRound0;
     if (!local0) {
         // state of unknown content (first query, other work since), a wide
@@ -845,8 +768,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
     }
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
     if (local0) {
-        pol.next(0, 1, sdeg);  // push, as every round 0
-        pushes = 1;
+        S.next(1, sdeg);  // push, as every round 0
         if (gtid == 0) write_trace(a.trace, 0, false, 1, sdeg, t_start);
         L = 1;
     }
@@ -866,72 +788,24 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         if (rc.count == 0) break;
         if (a.max_rounds && L >= a.max_rounds) break;
 
-        if (kTeamOk && bfs_team_fits(a, pol, L, pulls, rc)) {
-            if (threadIdx.x == 0) {
-                s_team[0] = min(gen.cnt, kTeamMax);
-                s_team[1] = xcc == gen.first && gen.rank < kTeamMax ? gen.rank : ~0u;
-            }
-            __syncthreads();
-            const uint32_t members = s_team[0], rank = s_team[1];
-            // two notes in turn: a block may still be reading the last
-            // phase's when the next phase's is written
-            uint32_t *note = a.bar.words + kBarNote + 16 * (phase++ & 1u);
-            bool more = true;
+        if (kTeamOk && bfs_team_fits(a, S, rc)) {
+            uint32_t members, rank;
+            team_place(xcc, gen, members, rank);
+            bool more = true, left;
             if (rank != ~0u) {
                 // a failed wait set the abort flag, which ends the others' wait
-                const long long t0 = rank == 0 && threadIdx.x == 0
-                                         ? (long long)load_team((const uint64_t *)(a.bar.words + kBarNote + 8))
-                                         : 0ll;
-                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, members, rank, tag, pol, L, rc, pushes, pulls,
-                                               ptrace, t0, kTeamRounds, more);
+                const long long t0 = rank == 0 && threadIdx.x == 0 ? team_clock(a.bar) : 0ll;
+                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, members, rank, tag, S, rc, t0, kTeamRounds, more);
                 if (!ok) break;
-                if (rank == 0 && threadIdx.x == 0) {
-                    note[0] = L;
-                    note[1] = pol.total_wl;
-                    note[2] = pol.pull_prev;
-                    note[3] = pushes;
-                    note[4] = pulls;
-                    note[5] = (uint32_t)ptrace;
-                    note[6] = (uint32_t)(ptrace >> 32);
-                    note[7] = more;
-                    if (kLeave && !more) write_final(a.trace, a.stats, L, pushes, pulls, ptrace, true, t_start);
-                }
+                if (kLeave && !more && rank == 0 && threadIdx.x == 0)
+                    write_final(a.trace, a.stats, L, S.pushes, S.pulls, S.ptrace, true, t0);
             }
-            // the phase's barrier. After the last round a member leaves once it
-            // has arrived, and the others as soon as they see the note, with no
-            // acquire (they read nothing more).
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                const uint32_t gen0 = grid_arrive(a.bar, xcc, gen);
-                if (kLeave && !more) {
-                    s_note[7] = 0;
-                } else {
-                    s_team[0] = spin_wait<true>(a.bar.words + kBarGen, gen0, true, a.bar.spin_limit, a.abort);
-                    for (int i = 0; i < 8; i++) s_note[i] = poll_load(note + i);
-                    if (!kLeave || s_note[7]) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                    __builtin_amdgcn_s_waitcnt(0);
-                }
-            }
-            __syncthreads();
-            ok = s_team[0] != 0u;
-            if (kLeave && ok && !s_note[7]) return true;
-            L = s_note[0];
-            pol.total_wl = s_note[1];
-            pol.pull_prev = s_note[2] != 0u;
-            pushes = s_note[3];
-            pulls = s_note[4];
-            ptrace = (unsigned long long)s_note[6] << 32 | s_note[5];
+            ok = team_rejoin<kLeave>(a.bar, xcc, gen, a.abort, phase++, rank, more, S, left);
+            if (ok && left) return true;
             continue;
         }
 
-        const bool pull = pol.next(L, rc.count, rc.scout);
-        if (pull) {
-            pulls++;
-            if (L < 64) ptrace |= 1ull << L;
-        } else {
-            pushes++;
-        }
+        const bool pull = S.next(rc.count, rc.scout);
         if (gtid == 0) write_trace(a.trace, L, pull, rc.count, rc.scout, t_start);
         if (brank == 0) clear_ctr(&a.ctr[(L + 2) % 3]);
 
@@ -1027,7 +901,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
             }
             // (2) the rest of the frontier: from the queue after a push round,
             //     from the bitmap after a pull round or if the queue overflowed.
-            if (pol.pull_prev || rc.overflow) {
+            if (S.pol.pull_prev || rc.overflow) {
                 // words dealt round-robin: in a degree-ordered graph adjacent
                 // words hold vertices of similar degree
                 for (uint32_t wb = 0; wb < W; wb += nwaves * kWave) {
@@ -1094,7 +968,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         // flush waits for its position
         publish_counts<WPB>(R.S.nxt, R.scout, R.count, R.huge, s_red);
         flush_stage(R.S, s_flush);
-        pol.pull_prev = pull;
+        S.pol.pull_prev = pull;
         L++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
@@ -1110,7 +984,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
             clear_ctr(&a.ctr[2]);
         }
     }
-    if (gtid == 0) write_final(a.trace, a.stats, L, pushes, pulls, ptrace, ok, t_start);
+    if (gtid == 0) write_final(a.trace, a.stats, L, S.pushes, S.pulls, S.ptrace, ok, t_start);
     return ok;
 }
 

@@ -415,6 +415,123 @@ __device__ __forceinline__ void write_final(DevTrace *trace, DevStats *stats, ui
     *stats = s;
 }
 
+// Rounds a team runs: push rounds of at most this many edges (see
+// bfs_team_fits), and every round of a graph of at most this many words and
+// edges (see bfs_whole).
+#ifndef SG_TEAM_PUSH_EDGES
+#define SG_TEAM_PUSH_EDGES 16384
+#endif
+#ifndef SG_TEAM_WORDS
+#define SG_TEAM_WORDS 256
+#endif
+#ifndef SG_TEAM_EDGES
+#define SG_TEAM_EDGES 1000000
+#endif
+constexpr uint32_t kTeamPushEdges = SG_TEAM_PUSH_EDGES, kTeamPushNodes = SG_TEAM_PUSH_EDGES;
+constexpr uint32_t kTeamWords = SG_TEAM_WORDS;
+constexpr uint64_t kTeamEdges = SG_TEAM_EDGES;
+static_assert(kTeamPushEdges <= kTeamSegment && kTeamWords * 64 <= kTeamSegment, "a team round fits its segments");
+// Rounds of one team phase: bounds the other blocks' wait.
+constexpr uint32_t kTeamRounds = 8192;
+
+// A graph so small that the team runs all of its rounds.
+__device__ __forceinline__ bool team_whole_graph(const DevGraph &g)
+{
+    return g.words <= kTeamWords && g.m <= kTeamEdges;
+}
+
+// What a traversal carries from round to round, alike in every block.
+struct RoundState {
+    DirectionPolicy pol;
+    uint32_t L, pushes, pulls;
+    unsigned long long ptrace;  // bit r: round r pulled
+
+    // The direction of round L, counted.
+    __device__ __forceinline__ bool next(unsigned long long count, unsigned long long scout)
+    {
+        const bool pull = pol.next(L, count, scout);
+        pulls += pull;
+        pushes += !pull;
+        if (pull && L < 64) ptrace |= 1ull << L;
+        return pull;
+    }
+};
+
+// Where this block stands in the team of its launch: members of it, and this
+// block's rank (~0 when it is none). After the first barrier of a launch.
+__device__ __forceinline__ void team_place(uint32_t xcc, const BarState &gen, uint32_t &members, uint32_t &rank)
+{
+    __shared__ uint32_t s_team[2];
+    if (threadIdx.x == 0) {
+        s_team[0] = min(gen.cnt, kTeamMax);
+        s_team[1] = xcc == gen.first && gen.rank < kTeamMax ? gen.rank : ~0u;
+    }
+    __syncthreads();
+    members = s_team[0];
+    rank = s_team[1];
+}
+
+// The launch's time 0, left for the team's lead by block 0 before the first barrier.
+__device__ __forceinline__ void team_clock_set(const GridBarrier &gb, long long t)
+{
+    *(long long *)(gb.words + kBarNote + 8) = t;
+}
+__device__ __forceinline__ long long team_clock(const GridBarrier &gb)
+{
+    return (long long)load_team((const uint64_t *)(gb.words + kBarNote + 8));
+}
+
+// The grid barrier that ends team phase number `phase`: the member of rank 0
+// leaves the rounds' state in a note (two in turn: a block may still be reading
+// the last phase's when the next phase's is written), from which every block
+// goes on. `more` (members): rounds are left. With kLeave, nothing follows the
+// last round: a member is done once it has arrived, and the others as soon as
+// they see the note, with no acquire; `left` tells them so. False when the wait
+// expired or a block aborted.
+template <bool kLeave>
+__device__ __forceinline__ bool team_rejoin(const GridBarrier &gb, uint32_t xcc, BarState &gen, uint32_t *abort,
+                                            uint32_t phase, uint32_t rank, bool more, RoundState &S, bool &left)
+{
+    __shared__ uint32_t s_note[8], s_ok;
+    uint32_t *note = gb.words + kBarNote + 16 * (phase & 1u);
+    if (rank == 0 && threadIdx.x == 0) {
+        note[0] = S.L;
+        note[1] = S.pol.total_wl;
+        note[2] = S.pol.pull_prev;
+        note[3] = S.pushes;
+        note[4] = S.pulls;
+        note[5] = (uint32_t)S.ptrace;
+        note[6] = (uint32_t)(S.ptrace >> 32);
+        note[7] = more;
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t gen0 = grid_arrive(gb, xcc, gen);
+        s_ok = 1u;
+        if (kLeave && rank != ~0u && !more) {
+            s_note[7] = 0;
+        } else {
+            s_ok = spin_wait<true>(gb.words + kBarGen, gen0, true, gb.spin_limit, abort);
+            for (int i = 0; i < 8; i++) s_note[i] = poll_load(note + i);
+            if (!kLeave || s_note[7]) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            __builtin_amdgcn_s_waitcnt(0);
+        }
+    }
+    __syncthreads();
+    left = kLeave && !s_note[7];
+    if (!s_ok) return false;
+    if (!left) {
+        S.L = s_note[0];
+        S.pol.total_wl = s_note[1];
+        S.pol.pull_prev = s_note[2] != 0u;
+        S.pushes = s_note[3];
+        S.pulls = s_note[4];
+        S.ptrace = (unsigned long long)s_note[6] << 32 | s_note[5];
+    }
+    return true;
+}
+
 // Map the engine's variant option onto a forced direction (-1 = auto).
 inline int forced_direction(const sg_engine_options &o)
 {

@@ -183,7 +183,7 @@ __device__ __forceinline__ void wave_append(bool pred, uint32_t v, uint32_t *q, 
 // launch depends on how blocks were dispatched in an earlier one.
 constexpr int kBarLine = 32;      // uint32 per 128-byte line
 constexpr int kMaxXcd = 16;       // XCC_ID is 4 bits wide
-constexpr int kBarWords = kBarLine * (13 + 4 * kMaxXcd);
+constexpr int kBarWords = kBarLine * (21 + 4 * kMaxXcd);
 
 // Word offsets inside the barrier area.
 constexpr int kBarGen = 0;
@@ -199,9 +199,9 @@ __host__ __device__ constexpr int bar_reg(int set, int x) { return kBarLine * (4
 // team rounds: the members' words, per launch parity and round parity, and the
 // notes a team leaves for the rest of the grid when its phase ends
 constexpr uint32_t kTeamMax = 32;
-__host__ __device__ constexpr int bar_slots(int set) { return kBarLine * (4 + 4 * kMaxXcd + 4 * set); }
-constexpr int kBarNote = kBarLine * (12 + 4 * kMaxXcd);
-static_assert(bar_slots(1) - bar_slots(0) == 2 * kTeamMax * 2, "team words layout");
+__host__ __device__ constexpr int bar_slots(int set) { return kBarLine * (4 + 4 * kMaxXcd + 8 * set); }
+constexpr int kBarNote = kBarLine * (20 + 4 * kMaxXcd);
+static_assert(bar_slots(1) - bar_slots(0) == 2 * 2 * kTeamMax * 2, "team words layout");
 static_assert(kBarNote + kBarLine <= kBarWords, "barrier layout");
 
 struct GridBarrier {
@@ -277,7 +277,7 @@ template <bool kTeam = false>
 __device__ __forceinline__ BarState bar_begin(const GridBarrier &gb, uint32_t xcc)
 {
     BarState s{0u, 0u, 0u, 0u, 0u};
-    if (kTeam && blockIdx.x == 0 && threadIdx.x < 2 * kTeamMax)
+    if (kTeam && blockIdx.x == 0 && threadIdx.x < 4 * kTeamMax)
         ((uint64_t *)(gb.words + bar_slots((int)(gb.rset & 1u) ^ 1)))[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
         uint32_t *w = gb.words;
@@ -452,16 +452,26 @@ constexpr uint64_t kTeamCountMask = (1ull << (kTeamFlagShift - kTeamCountShift))
 
 // LDS of a team round.
 struct TeamLds {
-    unsigned long long slot[kTeamMax];  // every member's word of the last round
-    unsigned long long acc;             // this round: sum in bits 0..31, count above
-    uint32_t flag, ok;
+    unsigned long long slot[2 * kTeamMax];  // every member's words of the last round
+    unsigned long long acc;                 // this round: sum in bits 0..31, count above
+    uint32_t flag, mn, ok;
+
+    // by thread 0, before the launch's first block barrier
+    __device__ __forceinline__ void reset()
+    {
+        acc = 0;
+        flag = 0;
+        mn = ~0u;
+    }
 };
 
-// Ends a team round: publishes this block's sums (acc, flag, which it resets) and
-// waits for every member's, left in t.slot. The words double as the barrier:
-// one store and one poll of two cache lines, no atomics and no separate
-// read of the counters. Two sets of words in turn, as a member may still be
-// polling the last round's. False when the wait expired or a block aborted.
+// Ends a team round: publishes this block's sums (acc, flag and, with kMin, the
+// minimum mn), which it resets, and waits for every member's, left in t.slot
+// (the minima from kTeamMax on). The words double as the barrier: one store
+// and one poll of a few cache lines, no atomics and no separate read of the
+// counters. Two sets of words in turn, as a member may still be polling the
+// last round's. False when the wait expired or a block aborted.
+template <bool kMin = false>
 __device__ __forceinline__ bool team_exchange(const GridBarrier &gb, TeamLds &t, uint32_t members, uint32_t rank,
                                               uint32_t &tag, uint32_t *abort)
 {
@@ -469,19 +479,19 @@ __device__ __forceinline__ bool team_exchange(const GridBarrier &gb, TeamLds &t,
     __syncthreads();
     tag++;
     if (threadIdx.x < kWave) {
-        uint64_t *slots = (uint64_t *)(gb.words + bar_slots((int)(gb.rset & 1u))) + (tag & 1u) * kTeamMax;
+        uint64_t *slots = (uint64_t *)(gb.words + bar_slots((int)(gb.rset & 1u))) + (tag & 1u) * 2 * kTeamMax;
         const uint64_t want = tag & 0xFFFu;
         const uint32_t ln = threadIdx.x;
-        if (ln == 0) {
-            const uint64_t mine = t.acc | (uint64_t)(t.flag != 0u) << kTeamFlagShift | want << kTeamTagShift;
-            __hip_atomic_store(slots + rank, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            t.acc = 0;
-            t.flag = 0;
+        if (ln == 0 || (kMin && ln == kTeamMax)) {
+            const uint64_t mine = ln ? (uint64_t)t.mn : t.acc | (uint64_t)(t.flag != 0u) << kTeamFlagShift;
+            __hip_atomic_store(slots + ln + rank, mine | want << kTeamTagShift, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
         }
+        const bool read = ln % kTeamMax < members && (kMin || ln < kTeamMax);
         uint32_t polls = 0, ok = 1u;
         uint64_t v;
         for (;;) {
-            v = ln < members ? load_team(slots + ln) : want << kTeamTagShift;
+            v = read ? load_team(slots + ln) : want << kTeamTagShift;
             if (!ballot(v >> kTeamTagShift != want)) break;
             if ((++polls & 255) == 0 && poll_load(abort)) {
                 ok = 0u;
@@ -493,11 +503,81 @@ __device__ __forceinline__ bool team_exchange(const GridBarrier &gb, TeamLds &t,
                 break;
             }
         }
-        if (ln < kTeamMax) t.slot[ln] = ln < members ? v : 0ull;
-        if (ln == 0) t.ok = ok;
+        t.slot[ln] = read ? v : ln < kTeamMax ? 0ull : ~0ull;
+        if (ln == 0) {
+            t.reset();
+            t.ok = ok;
+        }
     }
     __syncthreads();
     return t.ok != 0;
+}
+
+// A member's place in a team phase, and the frontier as segments of a queue,
+// one per block that found its vertices (lane k holds the entries up to the
+// end of segment k).
+struct TeamFront {
+    uint32_t members, rank, tag;
+    uint32_t gwave, nwaves;
+    uint32_t incl, total;  // segment ends (by lane), entries in all
+    uint32_t seg;          // entries per segment
+    const uint32_t *qin;
+    uint32_t *qout;        // this block's segment of the next queue
+};
+
+// What an exchange left: segment ends, entries in all; returned: this lane's word.
+__device__ __forceinline__ uint64_t team_segments(TeamFront &T, const TeamLds &t)
+{
+    const uint64_t w = (uint32_t)lane() < kTeamMax ? t.slot[lane()] : 0ull;
+    T.incl = wave_incl_scan((uint32_t)((w >> kTeamCountShift) & kTeamCountMask));
+    T.total = lane_value(T.incl, kWave - 1);
+    return w;
+}
+
+// Queue entry i of each lane (i >= T.total: 0), i0 the wave's lowest. The
+// segment is found for i0 by one ballot and stepped on from there.
+// Wave-convergent.
+__device__ __forceinline__ uint32_t team_entry(const TeamFront &T, uint32_t i0, uint32_t i)
+{
+    int k = __popcll(ballot(T.incl <= i0));
+    for (;;) {
+        const uint32_t stop = shfl(T.incl, k);
+        const bool past = i < T.total && i >= stop;
+        if (!ballot(past)) break;
+        k += past;
+    }
+    const uint32_t before = shfl(T.incl, k > 0 ? k - 1 : 0);
+    return i < T.total ? load_team(T.qin + (size_t)k * T.seg + (i - (k > 0 ? before : 0u))) : 0u;
+}
+
+// Lanes per item (a power of two from 4 to 64, as its logarithm) that give
+// `items` the team's lanes once over.
+__device__ __forceinline__ uint32_t team_width(const TeamFront &T, uint32_t items)
+{
+    uint32_t shift = 6;
+    while (shift > 2 && ((uint64_t)items << shift) > (uint64_t)T.nwaves * kWave) shift--;
+    return shift;
+}
+
+// Adds v (out-degree dv) to this block's segment of the next queue.
+__device__ __forceinline__ void team_append(const TeamFront &T, TeamLds &t, uint32_t v, uint32_t dv)
+{
+    const unsigned long long old = atomicAdd(&t.acc, (1ull << kTeamCountShift) | dv);
+    T.qout[(uint32_t)(old >> kTeamCountShift)] = v;
+}
+
+// This member's share of the frontier bitmap `bits` into its segment `q`; an
+// exchange follows.
+__device__ __forceinline__ void team_gather(TeamLds &t, const uint64_t *bits, uint32_t words, uint32_t *q, uint32_t tid,
+                                            uint32_t nthreads)
+{
+    for (uint32_t w = tid; w < words; w += nthreads) {
+        uint64_t x = load_team(bits + w);
+        if (!x) continue;
+        const unsigned long long old = atomicAdd(&t.acc, (unsigned long long)__popcll(x) << kTeamCountShift);
+        uint32_t at = (uint32_t)(old >> kTeamCountShift);
+        for (; x; x &= x - 1) q[at++] = w * 64 + (uint32_t)first_lane(x);
+    }
 }
 
 }  // namespace sg

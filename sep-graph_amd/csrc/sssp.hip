@@ -22,9 +22,9 @@ __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
         return;
     }
     const uint32_t xcc = xcc_id();
-    BarState st = bar_begin(a.bar, xcc);
+    BarState st = bar_begin<true>(a.bar, xcc);
     if (!a.grouped) {
-        sssp_run<BS>(a, blockIdx.x, gridDim.x, xcc, st);
+        sssp_run<BS, SG_FRONT_LDS * BS, true>(a, blockIdx.x, gridDim.x, xcc, st);
         return;
     }
     // Grouped: the census of this launch decides which XCD runs which query.
@@ -58,12 +58,13 @@ __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
     b.stats = a.stats + q;
     b.trace = nullptr;
     b.source = a.gr.source[q];
+    b.team = 0;  // already on one XCD
     // the XCD's own barrier area (after the whole-grid one), whose census is
     // the one just taken: all s_cnt blocks of the XCD, on one XCD
     b.bar.words = a.bar.words + (size_t)(xcc + 1) * kBarWords;
     BarState xs{0u, s_cnt, 1u, s_rank};
     if (threadIdx.x == 0) xs.gen = poll_load(b.bar.words + kBarGen);
-    sssp_run<BS>(b, s_rank, s_cnt, xcc, xs);
+    sssp_run<BS, SG_FRONT_LDS * BS, true>(b, s_rank, s_cnt, xcc, xs);
     if (s_rank == 0 && threadIdx.x == 0) atomicMin(a.gr.status, b.stats->status);
 }
 
@@ -132,6 +133,7 @@ int sssp_args(sg_engine *e, SsspArgs &a)
     a.max_rounds = (uint32_t)o.max_iteration;
     a.lb_push_none = o.lb_push == SG_LB_NONE;
     a.lb_pull_none = o.lb_pull == SG_LB_NONE;
+    a.team = a.lb_push_none || a.lb_pull_none ? 0u : e->g->relabeled ? 1u : 2u;
     if (o.priority == SG_PRIO_LOW_HIGH) {
         // two-level priority (the reference's SetTwoLevelBasedPriority,
         // algo_variants.cuh:605-685) runs push rounds only; the bucket width

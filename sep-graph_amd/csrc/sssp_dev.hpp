@@ -85,6 +85,8 @@ struct SsspArgs {
     // LoadBalancing::NONE (one lane per vertex, its edges in order, no hub
     // chunks) for push / pull rounds; otherwise the balanced schedulers
     uint32_t lb_push_none, lb_pull_none;
+    uint32_t team;  // rounds with little work may run on one XCD's blocks:
+                    // 1 (skewed graphs) after the first pull round, 2 from the start
 };
 
 struct Round {
@@ -609,12 +611,332 @@ __device__ __forceinline__ void pull_hubs_sorted(Round &R, uint32_t first, uint3
     finish_merges<NC>(R, pv, pm, pold);
 }
 
+// ------------------------------------------------------------ team rounds
+// As for BFS (bfs_dev.hpp): narrow push rounds, and every round on a small graph,
+// on the blocks of one XCD. A vertex is queued by the lane that sets its bit
+// in the next frontier's bitmap, as in a grid round; the bits of the
+// frontier being expanded are cleared entry by entry, so the three bitmaps
+// rotate without being swept.
+
+// Whether round S.L, of a grid round's frontier, starts a team phase; evaluated
+// alike by every block. A round queues at most the heads of its edges and the
+// vertices it defers, which is what a segment holds. 1024 x 1024 grid with the
+// priority schedule (1844 rounds, up to 13 K edges): 11.6-14.9 us a round on the
+// whole grid, 4.6-8.1 on the team, 23.3 -> 11.6 ms a query.
+__device__ __forceinline__ bool sssp_team_fits(const SsspArgs &a, const RoundState &S, unsigned long long count,
+                                               unsigned long long scout, bool hubs)
+{
+    if (!a.team || !(a.team == 2 || S.pulls) || hubs || count + scout > kTeamSegment) return false;
+    DirectionPolicy p = S.pol;
+    return !p.next(S.L, count, scout);
+}
+
+struct SsspTeam : TeamFront {
+    uint64_t *fcur, *fnext;
+    uint64_t *s_front;  // whole-graph phases: frontier L, and the bits this block
+    uint64_t *s_next;   // has set in the next one, in LDS
+    uint32_t thr;       // entries with dist >= thr are deferred (priority mode)
+    uint32_t fmin;      // no distance in this round's frontier is below this
+    uint32_t minv;      // smallest distance this lane queued for the next round
+};
+
+// v, at distance d, into the next frontier, unless it is in it already.
+template <bool kWhole>
+__device__ __forceinline__ void team_queue(const SsspArgs &a, SsspTeam &T, TeamLds &t, uint32_t v, uint32_t d,
+                                           uint32_t dv)
+{
+    const uint64_t bit = 1ull << (v & 63);
+    T.minv = min(T.minv, d);
+    if (kWhole && (atomicOr((unsigned long long *)&T.s_next[v >> 6], (unsigned long long)bit) & bit)) return;
+    if (atomicOr((unsigned long long *)&T.fnext[v >> 6], (unsigned long long)bit) & bit) return;
+    if (dv > kHugeDegree) t.flag = 1u;
+    team_append(T, t, v, dv);
+}
+
+// Edge -> v with candidate distance nd, for `act` lanes.
+template <bool kWhole>
+__device__ __forceinline__ void team_relax(const SsspArgs &a, SsspTeam &T, TeamLds &t, bool act, uint32_t v, uint32_t nd)
+{
+    if (!act || nd >= load_team(a.dist + v)) return;
+    const uint32_t old = atomicMin(&a.dist[v], nd);
+    const uint32_t dv = a.g.row[v + 1] - a.g.row[v];  // travels with the atomic
+    if (nd < old) team_queue<kWhole>(a, T, t, v, nd, dv);
+}
+
+// Push, as BFS's team_push: 4 to 64 lanes per queue entry.
+template <bool kWhole>
+__device__ __forceinline__ void team_push(const SsspArgs &a, SsspTeam &T, TeamLds &t, bool hubs)
+{
+    const DevGraph &g = a.g;
+    const int ln = lane();
+    if (kWhole && hubs) {
+        for (uint32_t c0 = 0; c0 < g.nhuge; c0 += T.nwaves * kWave) {
+            const uint32_t c = c0 + (uint32_t)ln * T.nwaves + T.gwave;
+            uint2 dsc = make_uint2(0u, 0u);
+            uint32_t end = 0;
+            bool mem = false;
+            if (c < g.nhuge) {
+                dsc = g.huge[c];
+                end = g.huge_end[c];
+                mem = test_bit(T.s_front, dsc.x);
+            }
+            uint64_t mm = ballot(mem);
+            while (mm) {
+                const int k = first_lane(mm);
+                mm &= mm - 1;
+                const uint32_t du = load_team(a.dist + lane_value(dsc.x, k));
+                const uint32_t beg = lane_value(dsc.y, k), stop = lane_value(end, k);
+                if (du >= T.thr) continue;  // carried over by its queue entry
+                for (uint32_t e = beg + (uint32_t)ln; e < stop; e += kWave)
+                    team_relax<kWhole>(a, T, t, true, g.col[e], sat_add(du, edge_w(g.w, e)));
+            }
+        }
+    }
+    const uint32_t shift = team_width(T, T.total);
+    const uint32_t width = 1u << shift, groups = kWave >> shift;
+    const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
+    for (uint32_t i0 = T.gwave * groups; i0 < T.total; i0 += T.nwaves * groups) {
+        const uint32_t i = i0 + grp;
+        const uint32_t u = team_entry(T, i0, i);
+        uint32_t e = 0, end = 0, du = kInf;
+        if (i < T.total) {
+            e = g.row[u];
+            end = g.row[u + 1];
+            du = load_team(a.dist + u);
+            const uint32_t deg = end - e;
+            if (!kWhole && sub == 0) T.fcur[u >> 6] = 0ull;
+            const bool later = du >= T.thr;
+            if (later && sub == 0) team_queue<kWhole>(a, T, t, u, du, deg);
+            if (later || deg > kHugeDegree) end = e;
+            e += sub;
+        }
+        for (; ballot(e < end); e += 2 * width) {
+            const bool p = e < end, q = e + width < end;
+            uint32_t v = 0, w = 0, nv = kInf, nw = kInf;
+            if (p) {
+                v = g.col[e];
+                nv = sat_add(du, edge_w(g.w, e));
+            }
+            if (q) {
+                w = g.col[e + width];
+                nw = sat_add(du, edge_w(g.w, e + width));
+            }
+            team_relax<kWhole>(a, T, t, p, v, nv);
+            team_relax<kWhole>(a, T, t, q, w, nw);
+        }
+    }
+}
+
+// Pull (whole-graph phases), as BFS's team_pull: an in-hub per wave, then 4 to
+// 64 lanes per other vertex. A vertex has one writer, so no atomics on it.
+__device__ __forceinline__ void team_pull(const SsspArgs &a, SsspTeam &T, TeamLds &t)
+{
+    const DevGraph &g = a.g;
+    const uint32_t n = g.n;
+    const int ln = lane();
+    constexpr int K = 4;
+    // the smallest candidate over in-edges e, e + step, ... (K of them) below `stop`
+    auto pull = [&](uint32_t e, uint32_t step, uint32_t stop, uint32_t best) {
+        uint32_t u[K], wt[K], du[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const bool in = e + k * step < stop;
+            u[k] = in ? g.csrc[e + k * step] : kInf;
+            wt[k] = in ? edge_w(g.cw, e + k * step) : 0u;
+        }
+        // (a weight that alone cannot beat the best skips the distance read)
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const bool f = u[k] != kInf && sat_add(T.fmin, wt[k]) < best && test_bit(T.s_front, u[k]);
+            du[k] = f ? load_team(a.dist + u[k]) : kInf;
+        }
+        uint32_t m = kInf;
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (du[k] != kInf) m = min(m, sat_add(du[k], wt[k]));
+        return m;
+    };
+    auto lower_bound = [&](uint32_t v) {
+        const uint32_t mw = g.cminw ? g.cminw[v] : (g.cw ? 0u : 1u);
+        return sat_add(T.fmin, mw);
+    };
+    auto lower = [&](uint32_t v, uint32_t d) {
+        a.dist[v] = d;
+        T.minv = min(T.minv, d);
+        const uint32_t dv = g.row[v + 1] - g.row[v];
+        if (dv > kHugeDegree) t.flag = 1u;
+        team_append(T, t, v, dv);
+    };
+    for (uint32_t h = T.gwave; h < g.nhubin; h += T.nwaves) {
+        const uint2 first = g.hugein[g.hubin[h].x];
+        const uint32_t v = first.x, stop = g.cstart[v + 1];
+        const uint32_t d0 = load_team(a.dist + v);
+        uint32_t best = d0;
+        if (d0 != kInf && d0 <= lower_bound(v)) continue;  // no frontier vertex can lower it
+        for (uint32_t e0 = first.y; e0 < stop; e0 += K * kWave)
+            best = min(best, wave_min_u32(pull(e0 + (uint32_t)ln, kWave, stop, best)));
+        if (best < d0 && ln == 0) {
+            lower(v, best);
+            atomicOr((unsigned long long *)&T.fnext[v >> 6], 1ull << (v & 63));
+        }
+    }
+    const uint32_t shift = team_width(T, n);
+    const uint32_t width = 1u << shift, groups = kWave >> shift;
+    const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
+    for (uint32_t v0 = T.gwave * groups; v0 < n; v0 += T.nwaves * groups) {
+        const uint32_t v = v0 + grp;
+        uint32_t e = 0, end = 0, d0 = 0;
+        if (v < n) {
+            e = g.cstart[v];
+            end = g.cstart[v + 1];
+            d0 = load_team(a.dist + v);
+            if (end - e > kPullHubDegree || (d0 != kInf && d0 <= lower_bound(v))) end = e;
+            e += sub;
+        }
+        uint32_t best = d0;
+        for (; ballot(e < end); e += K * width) best = min(best, pull(e, width, end, best));
+        for (uint32_t o = 1; o < width; o <<= 1) best = min(best, (uint32_t)__shfl_xor(best, (int)o, kWave));
+        const bool found = best < d0 && sub == 0;
+        if (!ballot(found)) continue;
+        const uint64_t bits =
+            wave_reduce(found ? 1ull << (v & 63) : 0ull, 0ull, [](uint64_t x, uint64_t y) { return x | y; });
+        if (ln == 0) atomicOr((unsigned long long *)&T.fnext[v0 >> 6], (unsigned long long)bits);
+        if (found) lower(v, best);
+    }
+}
+
+// A team phase: see bfs_team_phase. `cmin`: the smallest distance in frontier
+// S.L. Leaves the bitmaps and counters that a grid round expects.
+template <int BS, bool kWhole>
+__device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t members,
+                                                uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
+                                                uint32_t cmin, long long t_start, uint32_t cap, bool &more)
+{
+    constexpr int WPB = BS / kWave;
+    const uint32_t W = a.g.words;
+    const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
+    const bool lead = rank == 0 && threadIdx.x == 0;
+    uint32_t &L = S.L;
+    SsspTeam T;
+    T.members = members;
+    T.rank = rank;
+    T.tag = tag;
+    T.gwave = rank * WPB + threadIdx.x / kWave;
+    T.nwaves = members * WPB;
+    T.seg = a.qcap / members;
+    T.s_front = s_bits;
+    T.s_next = s_bits + kTeamWords;
+    // the bitmap after next still holds frontier L - 1
+    if (!kWhole)
+        for (uint32_t w = tid; w < W; w += nthreads) a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
+    bool ok = true;
+    if (S.pol.pull_prev || rc.overflow) {
+        team_gather(t, a.fbit + (size_t)(L % 3) * W, W, a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg, tid,
+                    nthreads);
+        ok = team_exchange<true>(a.bar, t, members, rank, T.tag, a.abort);
+        team_segments(T, t);
+    } else {
+        T.incl = T.total = rc.qlen;  // the grid's queue is one segment
+    }
+    unsigned long long count = rc.count, scout = rc.scout;
+    bool hubs = rc.has_huge;
+    more = ok;
+    for (uint32_t r = 0; more && r < cap; r++) {
+        const bool pull = S.next(count, scout);
+        if (lead && a.trace) write_trace(a.trace, L, pull, count, scout, t_start);
+        T.qin = a.queue + (size_t)(L % 3) * a.qcap;
+        T.qout = a.queue + (size_t)((L + 1) % 3) * a.qcap + (size_t)rank * T.seg;
+        T.fcur = a.fbit + (size_t)(L % 3) * W;
+        T.fnext = a.fbit + (size_t)((L + 1) % 3) * W;
+        T.fmin = cmin;
+        T.minv = kInf;
+        T.thr = kInf;
+        if (a.delta) T.thr = (uint32_t)min(((uint64_t)cmin / a.delta + 1) * a.delta, (uint64_t)kInf);
+        if constexpr (kWhole) {
+            for (uint32_t w = tid; w < W; w += nthreads) a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
+            for (uint32_t w = threadIdx.x; w < W; w += BS) {
+                T.s_front[w] = load_team(T.fcur + w);
+                T.s_next[w] = 0;
+            }
+            __syncthreads();
+        }
+        if (kWhole && pull) team_pull(a, T, t);
+        else team_push<kWhole>(a, T, t, hubs);
+        const uint32_t m = wave_min_u32(T.minv);
+        if (lane() == 0 && m != kInf) atomicMin(&t.mn, m);
+        S.pol.pull_prev = pull;
+        L++;
+        ok = team_exchange<true>(a.bar, t, members, rank, T.tag, a.abort);
+        if (!ok) break;
+        const uint64_t w = team_segments(T, t);
+        count = T.total;
+        scout = wave_sum_u64(w & 0xFFFFFFFFu);
+        hubs = ballot((w >> kTeamFlagShift) & 1) != 0;
+        cmin = wave_min_u32((uint32_t)lane() < kTeamMax ? (uint32_t)t.slot[kTeamMax + lane()] : kInf);
+        more = count != 0 && !(a.max_rounds && L >= a.max_rounds);
+        if (more && !kWhole && !sssp_team_fits(a, S, count, scout, hubs)) break;
+    }
+    tag = T.tag;
+    if (!ok) return false;
+    if (rank == 0) {
+        for (int i = 0; i < 3; i++) clear_ctr(&a.ctr[i]);
+        block_sync_global();
+        if (threadIdx.x == 0 && more) {
+            FrontierCtr &c = a.ctr[L % 3];
+            c.overflow = 1;
+            c.has_huge = hubs;
+            c.stripe[0].scout = scout;
+            c.stripe[0].count = count;
+            slot_cmin(&c) = ~cmin;
+        }
+    }
+    return true;
+}
+
+// The whole query on the team (see bfs_whole). By grid rounds and by this path:
+// RMAT graphs of 1024 vertices 181 and 77 us, of 4096 213 and 95, of 16001 205
+// and 125; a 120 x 120 grid 2027 and 934.
+template <int BS>
+__device__ __forceinline__ bool sssp_whole(const SsspArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t xcc, BarState &gen,
+                                           long long t_start)
+{
+    __shared__ uint32_t s_ok;
+    const DevGraph &g = a.g;
+    const uint32_t W = g.words, src = a.source;
+    const uint32_t sdeg = g.row[src + 1] - g.row[src];
+    if (threadIdx.x == 0) s_ok = bar_census(a.bar, xcc, gen, a.abort);
+    uint32_t members, rank, tag = 0;
+    team_place(xcc, gen, members, rank);
+    RoundState S{{a.alpha, a.beta, a.total_workload0, g.n, a.force}, 0, 0, 0, 0};
+    bool ok = s_ok != 0u, more = true;
+    if (ok && rank == ~0u) return true;
+    const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
+    if (ok) {
+        for (uint32_t i = tid; i < g.n; i += nthreads) a.dist[i] = i == src ? 0u : kInf;
+        for (uint32_t w = tid; w < 3 * W; w += nthreads) a.fbit[w] = w == (src >> 6) ? 1ull << (src & 63) : 0ull;
+        if (tid == 0) a.queue[0] = src;
+        ok = team_exchange<true>(a.bar, t, members, rank, tag, a.abort);
+    }
+    if (ok) {
+        const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
+        ok = sssp_team_phase<BS, true>(a, t, s_bits, members, rank, tag, S, rc, 0, t_start, ~0u, more);
+    }
+    // the last exchange ordered every distance before this
+    if (ok && a.out)
+        for (uint32_t v = tid; v < g.n; v += nthreads) a.out[v] = load_team(a.dist + a.inv[v]);
+    if (threadIdx.x == 0 && (s_ok ? rank == 0 : blockIdx.x == 0))
+        write_final(a.trace, a.stats, S.L, S.pushes, S.pulls, S.ptrace, ok, t_start);
+    return ok;
+}
+
 // `gen`: the block's barrier state (from bar_begin, or the census of a
 // grouped launch); `brank` of `nblocks` ranks the block in the query's grid.
 // Returns false when a bounded wait expired (the run then stopped). `gen`
 // is advanced by every barrier. kFrontWords: frontier bitmap words a pull
-// round copies into LDS (the first kFrontWords * 64 vertex ids).
-template <int BS, uint32_t kFrontWords = SG_FRONT_LDS * BS>
+// round copies into LDS (the first kFrontWords * 64 vertex ids). kTeamOk:
+// rounds with little work may run on the team (a.team; needs `gen` from
+// bar_begin<true> on a.bar).
+template <int BS, uint32_t kFrontWords = SG_FRONT_LDS * BS, bool kTeamOk = false>
 __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint32_t nblocks, uint32_t xcc,
                                          BarState &gen)
 {
@@ -635,6 +957,14 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
     __shared__ uint32_t s_qn, s_flush[2], s_cmin, s_bmin;
     constexpr uint32_t kFrontLds = kFrontWords;  // frontier words cached in LDS by pull rounds
     __shared__ uint64_t s_fb[kFrontLds];
+    __shared__ TeamLds s_t;
+    static_assert(!kTeamOk || kFrontLds >= 2 * kTeamWords, "a team's bitmaps fit the frontier's LDS");
+    uint32_t phase = 0, tag = 0;
+    if constexpr (kTeamOk) {
+        if (threadIdx.x == 0) s_t.reset();
+        if (a.team && team_whole_graph(g)) return sssp_whole<BS>(a, s_t, s_fb, xcc, gen, t_start);
+        if (gtid == 0) team_clock_set(a.bar, t_start);
+    }
 
     const uint32_t src = a.source;
     for (uint32_t i = gtid; i < n; i += nthreads) a.dist[i] = (i == src) ? 0u : kInf;
@@ -658,10 +988,8 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
     }
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
 
-    DirectionPolicy pol{a.alpha, a.beta, a.total_workload0, n, a.force};
-    unsigned long long ptrace = 0;
-    uint32_t pushes = 0, pulls = 0;
-    uint32_t L = 0;
+    RoundState S{{a.alpha, a.beta, a.total_workload0, n, a.force}, 0, 0, 0, 0};
+    uint32_t &L = S.L;
     while (ok) {
         read_counts(&a.ctr[L % 3], s_lvl);
         if (threadIdx.x == 0) {
@@ -680,13 +1008,23 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
         if (rc.count == 0) break;
         if (a.max_rounds && L >= a.max_rounds) break;
 
-        const bool pull = pol.next(L, rc.count, rc.scout);
-        if (pull) {
-            pulls++;
-            if (L < 64) ptrace |= 1ull << L;
-        } else {
-            pushes++;
+        if constexpr (kTeamOk) {
+            if (sssp_team_fits(a, S, rc.count, rc.scout, rc.has_huge)) {
+                uint32_t members, rank;
+                team_place(xcc, gen, members, rank);
+                bool more = true, left;
+                if (rank != ~0u) {
+                    // a failed wait set the abort flag, which ends the others' wait
+                    const long long t0 = rank == 0 && threadIdx.x == 0 ? team_clock(a.bar) : 0ll;
+                    ok = sssp_team_phase<BS, false>(a, s_t, nullptr, members, rank, tag, S, rc,
+                                                    s_cmin ? ~s_cmin : 0u, t0, kTeamRounds, more);
+                    if (!ok) break;
+                }
+                ok = team_rejoin<false>(a.bar, xcc, gen, a.abort, phase++, rank, more, S, left);
+                continue;
+            }
         }
+        const bool pull = S.next(rc.count, rc.scout);
         if (gtid == 0 && a.trace) write_trace(a.trace, L, pull, rc.count, rc.scout, t_start);
         if (brank == 0) clear_ctr(&a.ctr[(L + 2) % 3]);
 
@@ -744,10 +1082,10 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
                     }
                 }
             }
-            if (pol.pull_prev) {
-                // after a pull round, from its bitmap, words dealt round-robin
-                // (in a degree-ordered graph adjacent words hold vertices of
-                // similar degree)
+            if (S.pol.pull_prev || rc.overflow) {
+                // no queue (after a pull round, or it overflowed): from the
+                // bitmap, words dealt round-robin (in a degree-ordered graph
+                // adjacent words hold vertices of similar degree)
                 for (uint32_t wb = 0; wb < W; wb += nwaves * kWave) {
                     const uint32_t w = wb + (uint32_t)ln * nwaves + gwave;
                     const uint64_t fl = w < W ? R.fcur[w] : 0ull;
@@ -756,7 +1094,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
                         else push_expand(R, valid, u);
                     });
                 }
-            } else if (!rc.overflow) {
+            } else {
                 // the queue, entries dealt round-robin: lane ln of wave gw
                 // takes entry base + ln * nwaves + gw, so no wave gets a run of
                 // entries staged together
@@ -766,12 +1104,6 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
                     if (!ballot(valid)) break;
                     if (a.lb_push_none) push_expand_serial(R, valid, valid ? qin[i] : 0u);
                     else push_expand(R, valid, valid ? qin[i] : 0u);
-                }
-            } else {
-                for (uint32_t w = gwave; w < W; w += nwaves) {
-                    const uint32_t v = w * 64 + ln;
-                    if (a.lb_push_none) push_expand_serial(R, v < n && test_bit(R.fcur, v), v);
-                    else push_expand(R, v < n && test_bit(R.fcur, v), v);
                 }
             }
         } else {
@@ -818,7 +1150,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
             if (threadIdx.x == 0 && s_bmin != kInf) atomicMax(&slot_cmin(R.S.nxt), ~s_bmin);
         }
         flush_stage(R.S, s_flush);
-        pol.pull_prev = pull;
+        S.pol.pull_prev = pull;
         L++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
@@ -826,7 +1158,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
     // distances in the caller's vertex order: every block left the loop after
     // the same barrier, which made the last round's distances visible
     if (ok && a.out) gather_caller_order(a.out, a.dist, a.inv, n, gtid, nthreads);
-    if (gtid == 0) write_final(a.trace, a.stats, L, pushes, pulls, ptrace, ok, t_start);
+    if (gtid == 0) write_final(a.trace, a.stats, L, S.pushes, S.pulls, S.ptrace, ok, t_start);
     return ok;
 }
 

@@ -103,3 +103,41 @@ def test_bfs_small_rounds(sg, orc, gpu, name, opts):
             ref = np.where(ref > cap, -1, ref)
         assert np.array_equal(got, ref), s
         assert e.stats()["rounds"] == (min(cap, ref.max() + 1) if cap else ref.max() + 1)
+
+
+def weighted(sg, hg, lo, hi, seed):
+    w = sg.gen_weights(hg.row, hg.col, lo, hi, seed=seed, symmetric=hg.undirected)
+    return sg.HostGraph(hg.n, hg.row, hg.col, w, undirected=hg.undirected)
+
+
+def distances(orc, hg, w, s, weights):
+    """Shortest distances; where sums pass 2^32, which the oracle's 32-bit sums
+    would wrap, 64-bit ones cut off at the unreached mark, as the engine's."""
+    if weights is None or weights[1] < 1 << 20:
+        return orc.sssp_dijkstra(hg.row, hg.col, w, s)
+    from scipy.sparse import csr_matrix
+    from scipy.sparse.csgraph import dijkstra
+
+    g = csr_matrix((w.astype(np.float64), hg.col.astype(np.int64), hg.row.astype(np.int64)), shape=(hg.n, hg.n))
+    return np.minimum(dijkstra(g, indices=s), 2.0**32 - 1).astype(np.uint32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opts", [{}, {"priority": 1}, {"block_size": 256}, {"grid_blocks": 1},
+                                  {"force_variant": "async_pull_dd"}, {"priority": 1, "priority_threshold": 3.0}])
+@pytest.mark.parametrize("weights", [None, (1, 64), (0, 3), (1 << 30, 1 << 31)])
+@pytest.mark.parametrize("name", list(SMALL_ROUND_GRAPHS))
+def test_sssp_small_rounds(sg, orc, gpu, name, weights, opts):
+    if name in ("path9000", "path20000", "stars-long") and (opts or weights != (1, 64)):
+        pytest.skip("long traversal: default schedule and one weight range only")
+    hg = SMALL_ROUND_GRAPHS[name](sg)
+    if weights:
+        hg = weighted(sg, hg, *weights, seed=3)
+    e = sg.Engine(sg.Graph(hg), **opts)
+    w = hg.w if weights else np.ones(hg.m, np.uint32)
+    for s in sorted({0, hg.n - 1}):
+        e.sssp(s)
+        assert np.array_equal(e.gather(np.uint32), distances(orc, hg, w, s, weights)), s
+        # and a BFS on the same engine in between
+        e.bfs(s)
+        assert np.array_equal(e.gather(np.int32), orc.bfs(hg.row, hg.col, s)), s
