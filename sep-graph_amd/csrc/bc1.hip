@@ -16,7 +16,26 @@ struct Bc1KArgs {
     uint32_t probe;
 };
 
-template <int BS>
+// The run's summary into the call's (the thread that wrote the run's).
+__device__ __forceinline__ void fold_stats(const Bc1KArgs &a)
+{
+    const DevStats f = *a.b.f.stats;
+    DevStats s = a.b.first ? DevStats{} : *a.acc;
+    s.rounds += f.rounds;
+    s.push_rounds += f.push_rounds;
+    s.pull_rounds += f.pull_rounds;
+    s.trace = f.trace;
+    s.max_depth = max(s.max_depth, f.max_depth);
+    s.iterations += 1;
+    if (s.status == SG_OK) s.status = f.status;
+    *a.acc = s;
+}
+
+// kTeam: levels with little work run on one XCD's blocks (bc_phase). Skewed
+// graphs have a handful of levels, seldom three narrow ones in a row, and the code
+// alone held them up (RMAT-20 425 us without, 433 with): they take the
+// kernel without.
+template <int BS, bool kTeam>
 __global__ __launch_bounds__(BS) void k_bc1(Bc1KArgs a)
 {
     if (a.probe) {
@@ -24,39 +43,50 @@ __global__ __launch_bounds__(BS) void k_bc1(Bc1KArgs a)
         return;
     }
     const uint32_t xcc = xcc_id();
-    BarState gen = bar_begin(a.b.f.bar, xcc);
-    bc1_run<BS>(a.b, blockIdx.x, gridDim.x, xcc, gen);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const DevStats f = *a.b.f.stats;  // written by this thread
-        DevStats s = a.b.first ? DevStats{} : *a.acc;
-        s.rounds += f.rounds;
-        s.push_rounds += f.push_rounds;
-        s.pull_rounds += f.pull_rounds;
-        s.trace = f.trace;
-        s.max_depth = max(s.max_depth, f.max_depth);
-        s.iterations += 1;
-        if (s.status == SG_OK) s.status = f.status;
-        *a.acc = s;
+    BarState gen = bar_begin<kTeam>(a.b.f.bar, xcc);
+    bc1_run<BS, kTeam>(a.b, blockIdx.x, gridDim.x, xcc, gen);
+    if (blockIdx.x == 0 && threadIdx.x == 0) fold_stats(a);
+}
+
+// A query on a graph that one XCD's blocks run whole (bc1_whole).
+template <int BS>
+__global__ __launch_bounds__(BS) void k_bc1_whole(Bc1KArgs a)
+{
+    if (a.probe) {
+        residency_probe(a.b.f.bar.words, 1u << 20);
+        return;
     }
+    const uint32_t xcc = xcc_id();
+    BarState gen = bar_begin<true>(a.b.f.bar, xcc);
+    bool lead;
+    bc1_whole<BS>(a.b, xcc, gen, lead);
+    if (lead) fold_stats(a);
 }
 
 template <int BS>
 int launch_bc1(sg_engine *e, Bc1KArgs &a)
 {
+    // (a forced push fixes the direction of every level pass: grid passes only)
+    void (*kernel)(Bc1KArgs) = a.b.f.team && a.b.f.force != 0 ? k_bc1<BS, true> : k_bc1<BS, false>;
+    int most = 0;
+    if (a.b.f.force != 0 && team_whole_graph(a.b.f.g)) {
+        kernel = k_bc1_whole<BS>;
+        most = e->g->num_cus;
+    }
     sg_engine::PGrid *pg = nullptr;
-    auto probe = [e, a](int blocks, uint32_t *words) -> int {
+    auto probe = [e, a, kernel](int blocks, uint32_t *words) -> int {
         Bc1KArgs p = a;
         p.probe = 1;
         p.b.f.bar.words = words;
-        hipLaunchKernelGGL(k_bc1<BS>, dim3(blocks), dim3(BS), 0, e->stream, p);
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(BS), 0, e->stream, p);
         SG_HIP(hipGetLastError());
         return SG_OK;
     };
-    int rc = engine_persistent_grid(e, (const void *)k_bc1<BS>, BS, probe, &pg);
+    int rc = engine_persistent_grid(e, (const void *)kernel, BS, probe, &pg, most);
     if (rc) return rc;
     bind_barrier(pg, a.b.f.bar);
     return engine_launch_persistent(e, [&]() -> int {
-        hipLaunchKernelGGL(k_bc1<BS>, dim3(pg->blocks), dim3(BS), 0, e->stream, a);
+        hipLaunchKernelGGL(kernel, dim3(pg->blocks), dim3(BS), 0, e->stream, a);
         SG_HIP(hipGetLastError());
         pg->launches++;
         return SG_OK;
@@ -95,6 +125,7 @@ int bc1_launch(sg_engine *e, uint32_t dev_source, float *dep, const uint32_t *pe
     a.b.first = first;
     a.b.last = last;
     a.acc = e->stats;
+    a.b.f.team = e->g->relabeled ? 0u : 2u;
     const int bs = e->opt.block_size ? e->opt.block_size : 1024;
     switch (bs) {
     case 256: return launch_bc1<256>(e, a);

@@ -272,7 +272,292 @@ __device__ __forceinline__ void lane_level_vol(uint32_t *vol, bool valid, uint32
     if (id > kPullHubDegree) atomicAdd(&vol[3 * kBcVolLevels + l], 1u);
 }
 
+// 0.5 delta(v) into the outputs asked for.
+__device__ __forceinline__ void bc_output(const Bc1Args &a, uint32_t v, double h)
+{
+    if (a.dep) a.dep[a.perm ? a.perm[v] : v] = (float)h;
+    if (a.bcsum) {
+        const double t = a.first ? h : a.bcsum[v] + h;
+        a.bcsum[v] = t;
+        if (a.last && a.bcout) a.bcout[v] = (float)t;
+    }
+}
+
+// ------------------------------------------------------------ team levels
+// Levels with few vertices, and whole queries on small graphs, on the blocks of
+// one XCD (the team, sg_device.hpp). A level's vertices get 4 to 64 lanes
+// each, pulling over in-edges (sigma) or out-edges (dependencies); a neighbour
+// is tested by its level, so no bitmap is kept. Everything but sigma and
+// acc is fixed by then, so the next level's lists, edges and tests are loaded
+// while the members wait for each other. 400 x 400 grid (two passes over ~800
+// levels beside the traversal): 10 us a level by grid passes, 21.7 ms a query;
+// 6.3 ms by the team.
+
+// Vertices of a narrow level, and its edges where they are counted.
+constexpr uint32_t kBcTeamNodes = 8192, kBcTeamEdges = 32768;
+// Edges above which a whole wave sums one vertex.
+constexpr uint32_t kBcTeamBig = 64;
+
+// Whether level l, of `count` vertices, is summed by the team (over in- or
+// out-edges). Deeper than kBcVolLevels no volume is known: only a graph without
+// hubs on that side has narrow levels there.
+template <bool kIn>
+__device__ __forceinline__ bool bc_narrow(const Bc1Args &a, uint32_t l, uint32_t count)
+{
+    if (a.f.force == 0 || count > kBcTeamNodes) return false;
+    if (l < kBcVolLevels) return a.lvol[(kIn ? kBcVolLevels : 0) + l] <= kBcTeamEdges;
+    return kIn ? a.f.g.nhubin == 0 : a.f.g.nhuge == 0;
+}
+
+// The narrow ones of levels 1 .. min(D, 63), a bit each, found once: asked for
+// before every level, their counts cost a trip to memory each time (6-8 us a
+// query). Wave-convergent.
+template <bool kIn>
+__device__ __forceinline__ uint64_t bc_narrow_mask(const Bc1Args &a, uint32_t D)
+{
+    const uint32_t l = (uint32_t)lane();
+    return ballot(l >= 1 && l <= D && bc_narrow<kIn>(a, l, a.loff[l + 1] - a.loff[l]));
+}
+
+// Whether a phase of team levels starts at level l, with at least kBcTeamRun
+// narrow ones ahead: a phase ends with a grid barrier and the bits of a level.
+constexpr uint32_t kBcTeamRun = 3;
+template <bool kIn>
+__device__ __forceinline__ bool bc_phase_fits(const Bc1Args &a, uint32_t l, uint32_t D, uint64_t narrow)
+{
+    if ((kIn ? D + 1 - l : l) < kBcTeamRun) return false;
+    const uint32_t low = kIn ? l : l - (kBcTeamRun - 1);
+    constexpr uint64_t run = (1ull << kBcTeamRun) - 1;
+    if (low + kBcTeamRun <= kBcVolLevels) return ((narrow >> low) & run) == run;
+    for (uint32_t r = 0; r < kBcTeamRun; r++) {
+        const uint32_t k = kIn ? l + r : l - r;
+        if (!bc_narrow<kIn>(a, k, a.loff[k + 1] - a.loff[k])) return false;
+    }
+    return true;
+}
+
+// A lane's share of a level: its group's vertex, and its first edge.
+struct BcItem {
+    uint32_t i0, end, shift;  // the wave's first position, the level's end, lanes per vertex (log)
+    uint32_t v, e, stop;      // vertex, this lane's first edge, end of its edges
+    uint32_t u;               // neighbour of that edge
+    bool on;                  // it counts
+};
+
+struct BcTeam : TeamFront {
+    const uint32_t *off, *adj;  // of the pass: CSC (sigma) or CSR (dependencies)
+};
+
+// Whether u is at level `l`: fixed by the traversal, which a whole query's
+// other members ran with no invalidation since.
+template <bool kWhole>
+__device__ __forceinline__ bool bc_at(const Bc1Args &a, uint32_t u, int32_t l)
+{
+    return (kWhole ? load_team(a.f.level + u) : a.f.level[u]) == l;
+}
+
+// The items of positions i0 + (group) in [., end): everything before sigma or acc.
+template <bool kWhole>
+__device__ __forceinline__ void bc_load(const Bc1Args &a, const BcTeam &T, BcItem &x, int32_t target)
+{
+    const uint32_t width = 1u << x.shift, grp = (uint32_t)lane() >> x.shift, sub = (uint32_t)lane() & (width - 1);
+    x.e = x.stop = x.v = x.u = 0;
+    x.on = false;
+    if (x.i0 + grp >= x.end) return;
+    x.v = load_team(a.order + x.i0 + grp);
+    const uint32_t b = T.off[x.v];
+    x.stop = T.off[x.v + 1];
+    x.e = b + sub;
+    if (x.stop - b > kBcTeamBig) {
+        x.e = b;  // the wave's (bc_sum)
+    } else if (x.e < x.stop) {
+        x.u = T.adj[x.e];
+        x.on = bc_at<kWhole>(a, x.u, target);
+    }
+}
+
+// Sums val over the items' neighbours at level `target` into dst[2 v].
+template <bool kWhole, typename Val>
+__device__ __forceinline__ void bc_sum(const Bc1Args &a, const BcTeam &T, const BcItem &x, int32_t target, double *dst,
+                                       Val val)
+{
+    const int ln = lane();
+    const uint32_t width = 1u << x.shift, grp = (uint32_t)ln >> x.shift, sub = (uint32_t)ln & (width - 1);
+    const bool in = x.i0 + grp < x.end;
+    const bool big = in && (sub == 0 ? x.stop - x.e > kBcTeamBig : false);
+    const uint64_t bigs = ballot(big);
+    const bool mine = in && !((bigs >> (grp << x.shift)) & 1);
+    double sum = mine && x.on ? val(x.u) : 0.0;
+    for (uint32_t e = x.e + width; ballot(mine && e < x.stop); e += width)
+        if (mine && e < x.stop) {
+            const uint32_t u = T.adj[e];
+            if (bc_at<kWhole>(a, u, target)) sum += val(u);
+        }
+    sum = wave_seg_scan(sum, grp, [](double p, double q) { return p + q; });
+    if (mine && sub == width - 1) dst[2 * (size_t)x.v] = sum;
+    for (uint64_t todo = bigs; todo; todo &= todo - 1) {
+        const int k = first_lane(todo);
+        const uint32_t v = lane_value(x.v, k), b = lane_value(x.e, k), stop = lane_value(x.stop, k);
+        constexpr int K = 4;
+        double s = 0.0;
+        for (uint32_t e0 = b; e0 < stop; e0 += K * kWave) {
+            uint32_t u[K];
+            bool on[K];
+#pragma unroll
+            for (int q = 0; q < K; q++) {
+                const uint32_t e = e0 + (uint32_t)(q * kWave + ln);
+                on[q] = e < stop;
+                u[q] = on[q] ? T.adj[e] : 0u;
+            }
+#pragma unroll
+            for (int q = 0; q < K; q++) on[q] = on[q] && bc_at<kWhole>(a, u[q], target);
+#pragma unroll
+            for (int q = 0; q < K; q++) s += on[q] ? val(u[q]) : 0.0;
+        }
+        s = wave_sum_f64(s);
+        if (ln == 0) dst[2 * (size_t)v] = s;
+    }
+}
+
+// Team passes from level l in steps of kStep (1: sigma, -1: dependencies) while
+// levels are narrow (kWhole: to `last`). Returns false when a wait expired; l is
+// the first level not done.
+template <int BS, bool kWhole, int kStep>
+__device__ __forceinline__ bool bc_team_levels(const Bc1Args &a, TeamLds &t, BcTeam &T, uint32_t &l, uint32_t last,
+                                               uint32_t cap)
+{
+    constexpr bool kIn = kStep > 0;
+    const DevGraph &g = a.f.g;
+    T.off = kIn ? g.cstart : g.row;
+    T.adj = kIn ? g.csrc : g.col;
+    double *dst = kIn ? &a.sa[0].x : &a.sa[0].y;
+    auto sigma = [&](uint32_t u) { return load_team(&a.sa[u].x); };
+    auto psi = [&](uint32_t w) { return 1.0 / load_team(&a.sa[w].x) + load_team(&a.sa[w].y); };
+    // the level's items for this wave's first sweep
+    auto take = [&](uint32_t lv, BcItem &x) {
+        const uint32_t b = load_team(a.loff + lv);
+        x.end = load_team(a.loff + lv + 1);
+        x.shift = team_width(T, x.end - b);
+        x.i0 = b + T.gwave * (kWave >> x.shift);
+        bc_load<kWhole>(a, T, x, (int32_t)lv - kStep);
+        return x.end - b;
+    };
+    BcItem x;
+    take(l, x);
+    for (uint32_t r = 0;; r++) {
+        const int32_t target = (int32_t)l - kStep;
+        for (;;) {
+            if constexpr (kIn) bc_sum<kWhole>(a, T, x, target, dst, sigma);
+            else bc_sum<kWhole>(a, T, x, target, dst, psi);
+            x.i0 += T.nwaves * (kWave >> x.shift);
+            if (x.i0 >= x.end) break;
+            bc_load<kWhole>(a, T, x, target);
+        }
+        team_arrive(a.f.bar, t, T.rank, T.tag);
+        const bool end = l == last;
+        l += kStep;
+        uint32_t count = 0;
+        if (!end) count = take(l, x);
+        if (!team_wait(a.f.bar, t, T.members, T.tag, a.f.abort)) return false;
+        if (end || r + 1 >= cap || (!kWhole && !bc_narrow<kIn>(a, l, count))) return true;
+    }
+}
+
+// Clears or sets the bits of levels [l0, l1]'s vertices in the rotating level
+// bitmaps, so that a phase of team levels, which keeps none, starts and ends
+// with what a grid pass expects.
+__device__ __forceinline__ void bc_level_bits(const Bc1Args &a, uint32_t l0, uint32_t l1, bool set, uint32_t tid,
+                                              uint32_t nthreads)
+{
+    for (uint32_t l = l0; l <= l1; l++) {
+        uint64_t *bm = a.lbm + (size_t)(l % 3) * a.f.g.words;
+        for (uint32_t i = a.loff[l] + tid; i < a.loff[l + 1]; i += nthreads) {
+            const uint32_t v = a.order[i];
+            if (set) atomicOr((unsigned long long *)&bm[v >> 6], 1ull << (v & 63));
+            else bm[v >> 6] = 0ull;
+        }
+    }
+}
+
+// One phase of narrow levels from l on, for every block: the team's share, or
+// the wait for it.
+template <int BS, int kStep>
+__device__ __forceinline__ bool bc_phase(const Bc1Args &a, TeamLds &t, uint32_t &tag, uint32_t &phase, uint32_t &l,
+                                         uint32_t last, uint32_t D, uint32_t xcc, BarState &gen)
+{
+    uint32_t members, rank;
+    team_place(xcc, gen, members, rank);
+    RoundState S{};
+    bool ok = true, left;
+    if (rank != ~0u) {
+        const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
+        BcTeam T;
+        T.members = members;
+        T.rank = rank;
+        T.tag = tag;
+        T.gwave = rank * (BS / kWave) + threadIdx.x / kWave;
+        T.nwaves = members * (BS / kWave);
+        bc_level_bits(a, kStep > 0 ? l - min(l, 2u) : l, kStep > 0 ? l - 1 : min(D, l + 2), false, tid, nthreads);
+        ok = bc_team_levels<BS, false, kStep>(a, t, T, l, last, kTeamRounds);
+        tag = T.tag;
+        if (!ok) return false;  // the abort flag ends the other blocks' wait
+        // (the exchanges ordered the clearing before this)
+        bc_level_bits(a, l - kStep, l - kStep, true, tid, nthreads);
+        S.L = l;
+    }
+    ok = team_rejoin<false>(a.f.bar, xcc, gen, a.f.abort, phase++, rank, true, S, left);
+    l = S.L;
+    return ok;
+}
+
+// The whole query on the team (see bfs_whole), the traversal leaving its level
+// lists. `lead`: set in the one thread that wrote the run's stats. By grid
+// passes and by this path: RMAT graphs of 1024 vertices 188 and 84 us, of 4096
+// 223 and 102, of 16001 247 and 199; a 60 x 60 grid 2904 and 678.
 template <int BS>
+__device__ __forceinline__ bool bc1_whole(const Bc1Args &a, uint32_t xcc, BarState &gen, bool &lead)
+{
+    __shared__ TeamLds t;
+    const uint32_t n = a.f.g.n, src = a.f.source;
+    uint32_t members, rank, tag;
+    bool ok = bfs_whole<BS>(a.f, t, xcc, gen, members, rank, tag, a.order, a.loff);
+    lead = rank == 0 && threadIdx.x == 0;
+    if (!ok || rank == ~0u) return ok;
+    const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
+    // (written by the lead; levels 0 .. D hold vertices)
+    __shared__ uint32_t s_D;
+    for (uint32_t v = tid; v < n; v += nthreads) a.sa[v] = make_double2(v == src ? 1.0 : 0.0, 0.0);
+    ok = team_exchange(a.f.bar, t, members, rank, tag, a.f.abort);
+    if (threadIdx.x == 0) s_D = load_team(&a.f.stats->max_depth);
+    __syncthreads();
+    const uint32_t D = s_D;
+    BcTeam T;
+    T.members = members;
+    T.rank = rank;
+    T.tag = tag;
+    T.gwave = rank * (BS / kWave) + threadIdx.x / kWave;
+    T.nwaves = members * (BS / kWave);
+    if (ok && D >= 1) {
+        uint32_t l = 1;
+        ok = bc_team_levels<BS, true, 1>(a, t, T, l, D, ~0u);
+    }
+    if (ok && D >= 2) {
+        uint32_t l = D - 1;
+        ok = bc_team_levels<BS, true, -1>(a, t, T, l, 1, ~0u);
+    }
+    if (ok)
+        for (uint32_t v = tid; v < n; v += nthreads) {
+            double h = 0.0;
+            if (load_team(a.f.level + v) > 0) h = 0.5 * load_team(&a.sa[v].x) * load_team(&a.sa[v].y);
+            bc_output(a, v, h);
+        }
+    if (!ok && lead) a.f.stats->status = SG_ERR_TIMEOUT;
+    return ok;
+}
+
+// kTeamOk: levels with little work may run on the team (needs `gen` from
+// bar_begin<true> on f.bar).
+template <int BS, bool kTeamOk = false>
 __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32_t nblocks, uint32_t xcc,
                                         BarState &gen)
 {
@@ -289,7 +574,9 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
     __shared__ uint32_t s_hist[kBcLdsLevels];
     __shared__ uint32_t s_max, s_scan[BS / kWave], s_D;
     __shared__ uint32_t s_vol[4 * kBcVolLevels];
+    __shared__ TeamLds s_t;
 
+    uint32_t tag = 0, phase = 0;
     // level counters start at zero (the BFS's first barrier publishes this)
     for (uint32_t i = gtid; i <= kBcMaxDepth; i += nthreads) {
         a.lcnt[i] = 0;
@@ -300,7 +587,7 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
         a.ctl[0] = 0;
         a.ctl[1] = 0;
     }
-    bool ok = bfs_run<BS>(a.f, brank, nblocks, xcc, gen);
+    bool ok = bfs_run<BS, false, kTeamOk>(a.f, brank, nblocks, xcc, gen, &s_t, &tag, &phase);
     int32_t status = ok ? SG_OK : SG_ERR_TIMEOUT;
 
     // ---- per-level counts: block histograms, one atomic per block and level
@@ -406,8 +693,14 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
     const uint32_t D = ok ? s_D : 0u;
     // ---- sigma, level by level
     const uint32_t W = g.words;
+    uint64_t narrow = kTeamOk && ok ? bc_narrow_mask<true>(a, D) : 0ull;
     for (uint32_t L = 1; ok && L <= D; L++) {
         const uint32_t b0 = a.loff[L], e0 = a.loff[L + 1];
+        if (kTeamOk && bc_phase_fits<true>(a, L, D, narrow)) {
+            ok = bc_phase<BS, 1>(a, s_t, tag, phase, L, D, D, xcc, gen);
+            L--;  // (the loop counts it)
+            continue;
+        }
         const uint64_t *up = a.lbm + (size_t)((L - 1) % 3) * W;  // level L-1
         uint64_t *cur = a.lbm + (size_t)(L % 3) * W;             // level L, set now
         uint64_t *old = a.lbm + (size_t)((L + 1) % 3) * W;       // level L-2, cleared now
@@ -532,8 +825,14 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
     }
     // ---- dependencies, from the deepest level up (the deepest has no
     // successors: acc stays 0); the source's level needs none
+    narrow = kTeamOk && ok ? bc_narrow_mask<false>(a, D) : 0ull;
     for (uint32_t L = D; ok && L-- > 1;) {
         const uint32_t b0 = a.loff[L], e0 = a.loff[L + 1];
+        if (kTeamOk && bc_phase_fits<false>(a, L, D, narrow)) {
+            ok = bc_phase<BS, -1>(a, s_t, tag, phase, L, 1, D, xcc, gen);
+            L++;  // (the loop counts it)
+            continue;
+        }
         const uint64_t *down = a.lbm + (size_t)((L + 1) % 3) * W;  // level L+1
         uint64_t *cur = a.lbm + (size_t)(L % 3) * W;               // level L, set now
         uint64_t *old = a.lbm + (size_t)((L + 2) % 3) * W;         // level L+2, cleared now
@@ -633,12 +932,7 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
                 const double2 x = a.sa[v];
                 h = 0.5 * x.x * x.y;
             }
-            if (a.dep) a.dep[a.perm ? a.perm[v] : v] = (float)h;
-            if (a.bcsum) {
-                const double t = a.first ? h : a.bcsum[v] + h;
-                a.bcsum[v] = t;
-                if (a.last && a.bcout) a.bcout[v] = (float)t;
-            }
+            bc_output(a, v, h);
         }
     }
     if (!ok && status == SG_OK) status = SG_ERR_TIMEOUT;

@@ -20,24 +20,45 @@ __global__ SG_BFS_BOUNDS(BS) void k_bfs(BfsArgs a)
 }
 
 
+// A query on a graph that one XCD's blocks run whole (bfs_whole).
+template <int BS>
+__global__ SG_BFS_BOUNDS(BS) void k_bfs_whole(BfsArgs a)
+{
+    if (a.probe) {
+        residency_probe(a.bar.words, 1u << 20);
+        return;
+    }
+    __shared__ TeamLds s_t;
+    uint32_t members, rank, tag;
+    const uint32_t xcc = xcc_id();
+    BarState gen = bar_begin<true>(a.bar, xcc);
+    bfs_whole<BS>(a, s_t, xcc, gen, members, rank, tag);
+}
+
 template <int BS, bool kStage>
 int launch_bfs(sg_engine *e, BfsArgs &args, bool timed)
 {
+    void (*kernel)(BfsArgs) = k_bfs<BS, kStage>;
+    int most = 0;
+    if (!kStage && args.team && team_whole_graph(args.g)) {
+        kernel = k_bfs_whole<BS>;
+        most = e->g->num_cus;
+    }
     sg_engine::PGrid *pg = nullptr;
-    auto probe = [e, args](int blocks, uint32_t *words) -> int {
+    auto probe = [e, args, kernel](int blocks, uint32_t *words) -> int {
         BfsArgs p = args;
         p.probe = 1;
         p.bar.words = words;
-        hipLaunchKernelGGL((k_bfs<BS, kStage>), dim3(blocks), dim3(BS), 0, e->stream, p);
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(BS), 0, e->stream, p);
         SG_HIP(hipGetLastError());
         return SG_OK;
     };
-    int rc = engine_persistent_grid(e, (const void *)k_bfs<BS, kStage>, BS, probe, &pg);
+    int rc = engine_persistent_grid(e, (const void *)kernel, BS, probe, &pg, most);
     if (rc) return rc;
     bind_barrier(pg, args.bar);
     return engine_launch_persistent(e, [&]() -> int {
         if (timed) SG_HIP(hipEventRecord(e->ev0, e->stream));
-        hipLaunchKernelGGL((k_bfs<BS, kStage>), dim3(pg->blocks), dim3(BS), 0, e->stream, args);
+        hipLaunchKernelGGL(kernel, dim3(pg->blocks), dim3(BS), 0, e->stream, args);
         SG_HIP(hipGetLastError());
         pg->launches++;
         if (timed) SG_HIP(hipEventRecord(e->ev1, e->stream));
@@ -269,7 +290,9 @@ extern "C" int sg_bfs_noalloc(const sg_graph *g, uint32_t source, int32_t *level
     a.bar.rset = (uint32_t)(d.launches & 1u);
     a.abort = (uint32_t *)(d.ptr + kNaOffAbort);
     a.stats = (DevStats *)(d.ptr + kNaOffStats);
-    hipLaunchKernelGGL((k_bfs<kNaBlock, false>), dim3(d.blocks), dim3(kNaBlock), 0, s, a);
+    // (k_bfs_whole takes fewer registers and less LDS: k_bfs's grid is resident for it too)
+    void (*kernel)(BfsArgs) = a.team && team_whole_graph(dg) ? k_bfs_whole<kNaBlock> : k_bfs<kNaBlock, false>;
+    hipLaunchKernelGGL(kernel, dim3(d.blocks), dim3(kNaBlock), 0, s, a);
     SG_HIP(hipGetLastError());
     d.launches++;
     int32_t status = 0;

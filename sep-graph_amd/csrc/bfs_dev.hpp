@@ -327,12 +327,15 @@ __device__ __forceinline__ void pull_group(Round &R, const uint32_t (&wg)[G], co
 // 16 K and 32 K that told them apart.
 // On a skewed graph only once its peak is past: before it a
 // narrow frontier's next one is seldom narrow, and ending a phase costs a
-// barrier and a frontier read back from its bitmap.
+// barrier and a frontier read back from its bitmap; and only when nothing
+// follows the traversal (kLeave): its last one to three rounds do not earn
+// the barrier back (the BFS of a BC query on 32 001 vertices: 230 us without, 238 with).
+template <bool kLeave>
 __device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const RoundState &S, const RoundCounts &rc)
 {
     if (!a.team) return false;
     DirectionPolicy p = S.pol;
-    return (a.team == 2 || S.pulls) && !rc.has_huge && rc.count <= kTeamPushNodes && rc.scout <= kTeamPushEdges &&
+    return (a.team == 2 || (kLeave && S.pulls)) && !rc.has_huge && rc.count <= kTeamPushNodes && rc.scout <= kTeamPushEdges &&
            !p.next(S.L, rc.count, rc.scout);
 }
 
@@ -502,11 +505,13 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
 // is what a grid round expects: frontier L as a bitmap, counters saying that no
 // queue holds it; after the last round, what the epilogue leaves. Returns
 // false when a wait expired; `more`: rounds are left. At most `cap` rounds;
-// `t_start` is the trace's time 0.
+// `t_start` is the trace's time 0. `order` (from level 0): receives the reached
+// vertices level by level, loff[l] the first position of level l.
 template <int BS, bool kWhole>
 __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t members,
                                                uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
-                                               long long t_start, uint32_t cap, bool &more)
+                                               long long t_start, uint32_t cap, bool &more, uint32_t *order = nullptr,
+                                               uint32_t *loff = nullptr)
 {
     constexpr int WPB = BS / kWave;
     const uint32_t W = a.g.words;
@@ -536,6 +541,7 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
     }
     unsigned long long count = rc.count, scout = rc.scout;
     bool hubs = rc.has_huge;
+    uint32_t placed = 1;  // (level 0 is the source)
     // a phase of narrow rounds keeps no bitmaps and leaves all three clear meanwhile
     if (!kWhole)
         for (uint32_t w = tid; w < W; w += nthreads) {
@@ -571,6 +577,14 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
         count = T.total;
         scout = wave_sum_u64(w & 0xFFFFFFFFu);
         hubs = ballot((w >> kTeamFlagShift) & 1) != 0;
+        if (kWhole && order) {
+            // level L: this block's entries after those of the members before it
+            const uint32_t own = (uint32_t)((t.slot[rank] >> kTeamCountShift) & kTeamCountMask);
+            const uint32_t at = placed + lane_value(T.incl, (int)rank) - own;
+            for (uint32_t i = threadIdx.x; i < own; i += BS) order[at + i] = load_team(T.qout + i);
+            placed += T.total;
+            if (lead) loff[L + 1] = placed;
+        }
         more = count != 0 && !(a.max_rounds && L >= a.max_rounds);
         if (more && !kWhole) {
             DirectionPolicy p = S.pol;
@@ -615,15 +629,22 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
 // rounds and by this path: RMAT graphs of 4096 vertices 56 and 37 us, of 8001 62
 // and 41, of 16001 67 and 51, of 32001 70 and 84 (one XCD's caches and CUs
 // no longer suffice), so the line lies at 16384 vertices.
+// `t` is reset here; members, rank (~0: none) and tag are this block's place
+// for what follows the traversal; `order`, `loff`: see bfs_team_phase.
 template <int BS>
-__device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t sdeg, uint32_t xcc,
-                                          BarState &gen, long long t_start)
+__device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint32_t xcc, BarState &gen, uint32_t &members,
+                                          uint32_t &rank, uint32_t &tag, uint32_t *order = nullptr,
+                                          uint32_t *loff = nullptr)
 {
     __shared__ uint32_t s_ok;
+    __shared__ uint64_t s_bits[2 * kTeamWords];
+    const long long t_start = wall_clock64();
     const DevGraph &g = a.g;
     const uint32_t W = g.words, src = a.source;
+    const uint32_t sdeg = g.row[src + 1] - g.row[src];
+    tag = 0;
+    if (threadIdx.x == 0) t.reset();
     if (threadIdx.x == 0) s_ok = bar_census(a.bar, xcc, gen, a.abort);
-    uint32_t members, rank, tag = 0;
     team_place(xcc, gen, members, rank);
     RoundState S{{a.alpha, a.beta, a.total_workload0, g.n, a.force}, 0, 0, 0, 0};
     bool ok = s_ok != 0u, more = true;
@@ -640,15 +661,23 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint64_t
             a.fbit[(size_t)W + w] = 0;
             a.fbit[2 * (size_t)W + w] = 0;
         }
-        if (tid == 0) a.queue[0] = src;
+        if (tid == 0) {
+            a.queue[0] = src;
+            if (order) {
+                order[0] = src;
+                loff[0] = 0;
+                loff[1] = 1;
+            }
+        }
         ok = team_exchange(a.bar, t, members, rank, tag, a.abort);
     }
     if (ok) {
         const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
-        ok = bfs_team_phase<BS, true>(a, t, s_bits, members, rank, tag, S, rc, t_start, ~0u, more);
+        ok = bfs_team_phase<BS, true>(a, t, s_bits, members, rank, tag, S, rc, t_start, ~0u, more, order, loff);
     }
-    // (after a failed census every block's rank is unknown: block 0 reports)
-    if (threadIdx.x == 0 && (s_ok ? rank == 0 : blockIdx.x == 0))
+    // (after a failed census no block's place is known: block 0 reports)
+    if (!s_ok) rank = blockIdx.x ? ~0u : 0u;
+    if (rank == 0 && threadIdx.x == 0)
         write_final(a.trace, a.stats, S.L, S.pushes, S.pulls, S.ptrace, ok, t_start);
     return ok;
 }
@@ -670,10 +699,12 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint64_t
 // kTeamOk: rounds with little work may run on the team (a.team; needs `gen`
 // from bar_begin<true> on a.bar, whose first barrier takes the census).
 // kLeave: nothing follows the traversal, so blocks may return before every
-// block has seen its end.
+// block has seen its end. team, team_tag, team_phase: the caller's own team
+// state, when its team goes on after the traversal.
 template <int BS, bool kStage = false, bool kTeamOk = false, bool kLeave = false>
 __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32_t nblocks, uint32_t xcc,
-                                        BarState &gen)
+                                        BarState &gen, TeamLds *team = nullptr, uint32_t *team_tag = nullptr,
+                                        uint32_t *team_phase = nullptr)
 {
     constexpr int WPB = BS / kWave;
     constexpr uint32_t kLdsQ = 8u * BS;
@@ -688,16 +719,17 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
 
     __shared__ unsigned long long s_red[2][WPB];
     __shared__ unsigned long long s_lvl[5];
-    alignas(8) __shared__ uint32_t s_q[kLdsQ];
+    __shared__ uint32_t s_q[kLdsQ];
     __shared__ uint32_t s_qn, s_flush[2];
     // hub round: the block's member chunks (first edge, end) and their staged heads
     __shared__ uint2 s_hc[kStage ? kHubList : 1];
     __shared__ uint32_t s_he[kStage ? kStageChunks * kHugeChunk : 1];
     __shared__ uint32_t s_hn;
-    __shared__ TeamLds s_t;
-    static_assert(sizeof(s_q) >= 2 * kTeamWords * 8, "a team's bitmaps fit the queue's LDS");
+    __shared__ TeamLds s_own;
+    TeamLds &s_t = team ? *team : s_own;
+    uint32_t phase0 = 0, tag0 = 0;
+    uint32_t &phase = team_phase ? *team_phase : phase0, &tag = team_tag ? *team_tag : tag0;
     if (kTeamOk && threadIdx.x == 0) s_t.reset();
-    uint32_t phase = 0, tag = 0;
 
     // ---- prologue: reset the levels (caller order) and seed the source.
     // The previous query left the frontier bitmaps and counters zeroed, and
@@ -707,10 +739,6 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
     const uint32_t src = a.source;
     const uint32_t sbeg = g.row[src], sdeg = g.row[src + 1] - sbeg;
     const uint64_t sbit = 1ull << (src & 63);
-    if constexpr (kLeave) {
-        if (a.team && team_whole_graph(g))
-            return bfs_whole<BS>(a, s_t, (uint64_t *)s_q, sdeg, xcc, gen, t_start);
-    }
     if (kTeamOk && gtid == 0) team_clock_set(a.bar, t_start);
     for (uint32_t i = gtid; i < n; i += nthreads) a.level[i] = (i == a.source_id) ? 0 : -1;
     for (uint32_t w = gtid; w < W; w += nthreads) a.vis_idle[w] = g.inert ? g.inert[w] : 0ull;
@@ -788,7 +816,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         if (rc.count == 0) break;
         if (a.max_rounds && L >= a.max_rounds) break;
 
-        if (kTeamOk && bfs_team_fits(a, S, rc)) {
+        if (kTeamOk && bfs_team_fits<kLeave>(a, S, rc)) {
             uint32_t members, rank;
             team_place(xcc, gen, members, rank);
             bool more = true, left;

@@ -434,8 +434,9 @@ static_assert(kTeamPushEdges <= kTeamSegment && kTeamWords * 64 <= kTeamSegment,
 // Rounds of one team phase: bounds the other blocks' wait.
 constexpr uint32_t kTeamRounds = 8192;
 
-// A graph so small that the team runs all of its rounds.
-__device__ __forceinline__ bool team_whole_graph(const DevGraph &g)
+// A graph so small that the team runs all of its rounds (kernels of their own:
+// a query this short is held up by code it does not run).
+__host__ __device__ __forceinline__ bool team_whole_graph(const DevGraph &g)
 {
     return g.words <= kTeamWords && g.m <= kTeamEdges;
 }

@@ -690,7 +690,7 @@ static int size_grid(sg_engine *e, sg_engine::PGrid &pg, int per_cu)
 }
 
 int engine_persistent_grid(sg_engine *e, const void *fn, int bs, const std::function<int(int, uint32_t *)> &probe,
-                           sg_engine::PGrid **out)
+                           sg_engine::PGrid **out, int most)
 {
     e->launch_seq++;  // any persistent kernel may overwrite the BFS state
     if (e->needs_bar_reset) {
@@ -709,7 +709,7 @@ int engine_persistent_grid(sg_engine *e, const void *fn, int bs, const std::func
         SG_HIP(hipMemsetAsync(e->abort_flag, 0, 4, e->stream));
         e->needs_bar_reset = false;
     }
-    const int cap = std::max(0, e->opt.grid_blocks);
+    const int cap = e->opt.grid_blocks > 0 ? e->opt.grid_blocks : most;
     for (int i = 0; i < e->ngrids; i++) {
         if (e->grids[i].fn == fn && e->grids[i].bs == bs && e->grids[i].cap == cap) {
             *out = &e->grids[i];

@@ -465,28 +465,36 @@ struct TeamLds {
     }
 };
 
-// Ends a team round: publishes this block's sums (acc, flag and, with kMin, the
-// minimum mn), which it resets, and waits for every member's, left in t.slot
-// (the minima from kTeamMax on). The words double as the barrier: one store
-// and one poll of a few cache lines, no atomics and no separate read of the
-// counters. Two sets of words in turn, as a member may still be polling the
-// last round's. False when the wait expired or a block aborted.
+// First half of a team round's end: publishes this block's sums (acc, flag
+// and, with kMin, the minimum mn), its stores before. Two sets of words in
+// turn, as a member may still be polling the last round's.
 template <bool kMin = false>
-__device__ __forceinline__ bool team_exchange(const GridBarrier &gb, TeamLds &t, uint32_t members, uint32_t rank,
-                                              uint32_t &tag, uint32_t *abort)
+__device__ __forceinline__ void team_arrive(const GridBarrier &gb, const TeamLds &t, uint32_t rank, uint32_t &tag)
 {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     tag++;
-    if (threadIdx.x < kWave) {
+    const uint32_t ln = threadIdx.x;
+    if (ln == 0 || (kMin && ln == kTeamMax)) {
         uint64_t *slots = (uint64_t *)(gb.words + bar_slots((int)(gb.rset & 1u))) + (tag & 1u) * 2 * kTeamMax;
+        const uint64_t mine = ln ? (uint64_t)t.mn : t.acc | (uint64_t)(t.flag != 0u) << kTeamFlagShift;
+        __hip_atomic_store(slots + ln + rank, mine | (uint64_t)(tag & 0xFFFu) << kTeamTagShift, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+// Second half: waits for every member's words, left in t.slot (the minima from
+// kTeamMax on), and resets this block's sums. The words double as the
+// barrier: one store and one poll of a few cache lines, no atomics and no
+// separate read of the counters. False when the wait expired or a block aborted.
+template <bool kMin = false>
+__device__ __forceinline__ bool team_wait(const GridBarrier &gb, TeamLds &t, uint32_t members, uint32_t tag,
+                                          uint32_t *abort)
+{
+    if (threadIdx.x < kWave) {
+        const uint64_t *slots = (const uint64_t *)(gb.words + bar_slots((int)(gb.rset & 1u))) + (tag & 1u) * 2 * kTeamMax;
         const uint64_t want = tag & 0xFFFu;
         const uint32_t ln = threadIdx.x;
-        if (ln == 0 || (kMin && ln == kTeamMax)) {
-            const uint64_t mine = ln ? (uint64_t)t.mn : t.acc | (uint64_t)(t.flag != 0u) << kTeamFlagShift;
-            __hip_atomic_store(slots + ln + rank, mine | want << kTeamTagShift, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
         const bool read = ln % kTeamMax < members && (kMin || ln < kTeamMax);
         uint32_t polls = 0, ok = 1u;
         uint64_t v;
@@ -511,6 +519,15 @@ __device__ __forceinline__ bool team_exchange(const GridBarrier &gb, TeamLds &t,
     }
     __syncthreads();
     return t.ok != 0;
+}
+
+// Ends a team round.
+template <bool kMin = false>
+__device__ __forceinline__ bool team_exchange(const GridBarrier &gb, TeamLds &t, uint32_t members, uint32_t rank,
+                                              uint32_t &tag, uint32_t *abort)
+{
+    team_arrive<kMin>(gb, t, rank, tag);
+    return team_wait<kMin>(gb, t, members, tag, abort);
 }
 
 // A member's place in a team phase, and the frontier as segments of a queue,

@@ -297,9 +297,10 @@ int engine_alloc(void **p, uint64_t bytes);
 // Grid for a persistent kernel: the largest blocks-per-CU x CUs (starting
 // from the occupancy API's figure) whose blocks all turn out to be resident
 // when the kernel is launched in probe mode, with the barrier's per-XCD block
-// counts from that probe. Barriers are re-zeroed after an aborted run.
+// counts from that probe. Barriers are re-zeroed after an aborted run. `most`:
+// no more blocks than that, unless options.grid_blocks says otherwise (0: fill).
 int engine_persistent_grid(sg_engine *e, const void *fn, int bs,
-                           const std::function<int(int, uint32_t *)> &probe, sg_engine::PGrid **out);
+                           const std::function<int(int, uint32_t *)> &probe, sg_engine::PGrid **out, int most = 0);
 // Point a launch's barrier at the grid's words, with the registration set of
 // the grid's next launch; the caller counts the launch (pg->launches++) once
 // it has been enqueued.

@@ -68,6 +68,19 @@ __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
     if (s_rank == 0 && threadIdx.x == 0) atomicMin(a.gr.status, b.stats->status);
 }
 
+// A query on a graph that one XCD's blocks run whole (sssp_whole).
+template <int BS>
+__global__ __launch_bounds__(BS) void k_sssp_whole(SsspArgs a)
+{
+    if (a.probe) {
+        residency_probe(a.bar.words, 1u << 20);
+        return;
+    }
+    const uint32_t xcc = xcc_id();
+    BarState gen = bar_begin<true>(a.bar, xcc);
+    sssp_whole<BS>(a, xcc, gen);
+}
+
 // Persistent grid for k_sssp<BS>; grouped launches take the barrier area
 // `group_words` ((1 + kMaxXcd) areas) and give the XCDs holding blocks one
 // query each, in XCD order.
@@ -77,17 +90,23 @@ int launch_sssp(sg_engine *e, SsspArgs &args, uint32_t *group_words)
     if (!args.abort || !args.stats || (!args.dist && !args.grouped) || !args.fbit || !args.queue ||
         !args.ctr || (args.grouped && (!group_words || !args.gr.status)))
         SG_FAIL(SG_ERR_STATE, "sg_sssp: launch with unset device state");
+    void (*kernel)(SsspArgs) = k_sssp<BS>;
+    int most = 0;
+    if (!args.grouped && args.team && team_whole_graph(args.g)) {
+        kernel = k_sssp_whole<BS>;
+        most = e->g->num_cus;
+    }
     sg_engine::PGrid *pg = nullptr;
-    auto probe = [e, args](int blocks, uint32_t *words) -> int {
+    auto probe = [e, args, kernel](int blocks, uint32_t *words) -> int {
         SsspArgs p = args;
         p.probe = 1;
         p.grouped = 0;
         p.bar.words = words;
-        hipLaunchKernelGGL(k_sssp<BS>, dim3(blocks), dim3(BS), 0, e->stream, p);
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(BS), 0, e->stream, p);
         SG_HIP(hipGetLastError());
         return SG_OK;
     };
-    int rc = engine_persistent_grid(e, (const void *)k_sssp<BS>, BS, probe, &pg);
+    int rc = engine_persistent_grid(e, (const void *)kernel, BS, probe, &pg, most);
     if (rc) return rc;
     if (args.grouped) {
         args.bar.words = group_words;
@@ -96,7 +115,7 @@ int launch_sssp(sg_engine *e, SsspArgs &args, uint32_t *group_words)
         bind_barrier(pg, args.bar);
     }
     return engine_launch_persistent(e, [&]() -> int {
-        hipLaunchKernelGGL(k_sssp<BS>, dim3(pg->blocks), dim3(BS), 0, e->stream, args);
+        hipLaunchKernelGGL(kernel, dim3(pg->blocks), dim3(BS), 0, e->stream, args);
         SG_HIP(hipGetLastError());
         if (args.grouped) e->group_launches++;
         else pg->launches++;

@@ -897,10 +897,13 @@ __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, u
 // RMAT graphs of 1024 vertices 181 and 77 us, of 4096 213 and 95, of 16001 205
 // and 125; a 120 x 120 grid 2027 and 934.
 template <int BS>
-__device__ __forceinline__ bool sssp_whole(const SsspArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t xcc, BarState &gen,
-                                           long long t_start)
+__device__ __forceinline__ bool sssp_whole(const SsspArgs &a, uint32_t xcc, BarState &gen)
 {
     __shared__ uint32_t s_ok;
+    __shared__ TeamLds t;
+    __shared__ uint64_t s_bits[2 * kTeamWords];
+    const long long t_start = wall_clock64();
+    if (threadIdx.x == 0) t.reset();
     const DevGraph &g = a.g;
     const uint32_t W = g.words, src = a.source;
     const uint32_t sdeg = g.row[src + 1] - g.row[src];
@@ -958,11 +961,9 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
     constexpr uint32_t kFrontLds = kFrontWords;  // frontier words cached in LDS by pull rounds
     __shared__ uint64_t s_fb[kFrontLds];
     __shared__ TeamLds s_t;
-    static_assert(!kTeamOk || kFrontLds >= 2 * kTeamWords, "a team's bitmaps fit the frontier's LDS");
     uint32_t phase = 0, tag = 0;
     if constexpr (kTeamOk) {
         if (threadIdx.x == 0) s_t.reset();
-        if (a.team && team_whole_graph(g)) return sssp_whole<BS>(a, s_t, s_fb, xcc, gen, t_start);
         if (gtid == 0) team_clock_set(a.bar, t_start);
     }
 

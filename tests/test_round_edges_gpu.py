@@ -141,3 +141,29 @@ def test_sssp_small_rounds(sg, orc, gpu, name, weights, opts):
         # and a BFS on the same engine in between
         e.bfs(s)
         assert np.array_equal(e.gather(np.int32), orc.bfs(hg.row, hg.col, s)), s
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opts", [{}, {"block_size": 256}, {"grid_blocks": 1}, {"force_variant": "async_pull_dd"},
+                                  {"force_variant": "async_push_dd"}])
+@pytest.mark.parametrize("name", [n for n in SMALL_ROUND_GRAPHS if n != "n1"])
+def test_bc_small_levels(sg, orc, gpu, name, opts):
+    if name in ("path9000", "path20000", "stars-long") and opts:
+        pytest.skip("long traversal: default schedule only")
+    hg = SMALL_ROUND_GRAPHS[name](sg)
+    e = sg.Engine(sg.Graph(hg), **opts)
+    sources = sorted({0, hg.n // 3, hg.n - 1})
+    e.bc_dependency(sources, 1)
+    got = e.gather(np.float32).reshape(len(sources), hg.n)
+    st = e.stats()
+    total = np.zeros(hg.n)
+    depth = 0
+    for i, s in enumerate(sources):
+        ref, _ = orc.bc_single(hg.row, hg.col, s)
+        total += ref
+        depth = max(depth, int(orc.bfs(hg.row, hg.col, s).max()))
+        # FP64 sums, one rounding to FP32
+        np.testing.assert_allclose(got[i], ref, rtol=1e-6, atol=1e-6)
+    assert st["iterations"] == len(sources) and st["max_depth"] == depth
+    e.bc(sources, 1)
+    np.testing.assert_allclose(e.gather(np.float32), total, rtol=1e-6, atol=1e-6)
