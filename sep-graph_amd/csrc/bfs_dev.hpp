@@ -314,10 +314,17 @@ __device__ __forceinline__ void pull_group(Round &R, const uint32_t (&wg)[G], co
 
 // ------------------------------------------------------------ team rounds
 // On a graph that the team runs whole, every member keeps the visited filter
-// and the round's frontier in LDS (2 x 2 KiB), and the rounds meet only in the
+// and the round's frontier in LDS (2 x 2 KiB; the frontier's vertices are counted
+// off its bitmap, so there is no queue), and the rounds meet only in the
 // next frontier's bitmap: atomics on the few cache lines such bitmaps fill
 // serialise (6-15 ns each on one line), so a bit set in a member's own copy
 // is claimed there first.
+
+// Edges of a narrow push round at most.
+#ifndef SG_TEAM_PUSH_EDGES
+#define SG_TEAM_PUSH_EDGES 16384
+#endif
+constexpr uint32_t kTeamPushEdges = SG_TEAM_PUSH_EDGES;
 
 // Whether round L, of a grid round's frontier, starts a team phase; evaluated
 // alike by every block. Only narrow push rounds do: on the 2048 x 2048 grid
@@ -334,8 +341,9 @@ template <bool kLeave>
 __device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const RoundState &S, const RoundCounts &rc)
 {
     if (!a.team) return false;
+    const uint32_t limit = team_limit(a.qcap, kTeamPushEdges);
     DirectionPolicy p = S.pol;
-    return (a.team == 2 || (kLeave && S.pulls)) && !rc.has_huge && rc.count <= kTeamPushNodes && rc.scout <= kTeamPushEdges &&
+    return (a.team == 2 || (kLeave && S.pulls)) && !rc.has_huge && rc.count <= limit && rc.scout <= limit &&
            !p.next(S.L, rc.count, rc.scout);
 }
 
@@ -343,18 +351,20 @@ __device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const RoundState
 struct BfsTeam : TeamFront {
     uint32_t L;
     uint64_t *fnext;
-    uint64_t *s_vis;         // whole-graph phases: the visited filter and
-    uint64_t *s_front;       // frontier L in LDS
+    TeamBits *front;         // whole-graph phases: frontier L and the visited
+    uint64_t *s_vis;         // filter in LDS
 };
 
-// A vertex found for level L+1: its level and its place in the next queue.
-// `dv`: its out-degree.
+// A vertex found for level L+1: its level, its share of the sums and its place
+// in the next queue (a whole-graph phase has none). `dv`: its out-degree.
+template <bool kWhole>
 __device__ __forceinline__ void team_found(const BfsArgs &a, const BfsTeam &T, TeamLds &t, uint32_t v, uint32_t id,
                                            uint32_t dv)
 {
     a.level[id] = (int32_t)T.L + 1;
     if (dv > kHugeDegree) t.flag = 1u;
-    team_append(T, t, v, dv);
+    if (kWhole) atomicAdd(&t.acc, (1ull << kTeamCountShift) | dv);
+    else team_append(T, t, v, dv);
 }
 
 // Edge -> v for `act` lanes. One atomicOr claims an unvisited head (heads of a
@@ -377,7 +387,7 @@ __device__ __forceinline__ void team_visit(const BfsArgs &a, const BfsTeam &T, T
     }
     const uint32_t rb = a.g.row[v], re = a.g.row[v + 1];
     const uint32_t id = caller_id(a, v);
-    if (!(old & bit)) team_found(a, T, t, v, id, re - rb);
+    if (!(old & bit)) team_found<kWhole>(a, T, t, v, id, re - rb);
 }
 
 // Push: `width` lanes per queue entry (a power of two, 4 to 64, as many as the
@@ -398,7 +408,7 @@ __device__ __forceinline__ void team_push(const BfsArgs &a, const BfsTeam &T, Te
             if (c < g.nhuge) {
                 dsc = g.huge[c];
                 end = g.huge_end[c];
-                mem = test_bit(T.s_front, dsc.x);
+                mem = test_bit(T.front->word, dsc.x);
             }
             uint64_t mm = ballot(mem);
             while (mm) {
@@ -415,9 +425,10 @@ __device__ __forceinline__ void team_push(const BfsArgs &a, const BfsTeam &T, Te
     const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
     for (uint32_t i0 = T.gwave * groups; i0 < T.total; i0 += T.nwaves * groups) {
         const uint32_t i = i0 + grp;
-        const uint32_t u = team_entry(T, i0, i);
-        uint32_t e = 0, end = 0;
+        uint32_t u = 0, e = 0, end = 0;
+        if (!kWhole) u = team_entry(T, i0, i);
         if (i < T.total) {
+            if (kWhole) u = team_bits_entry(*T.front, i);
             e = g.row[u];
             end = g.row[u + 1];
             if (end - e > kHugeDegree) end = e;
@@ -455,11 +466,11 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
             }
             bool hit = false;
 #pragma unroll
-            for (int k = 0; k < K; k++) hit |= u[k] != 0xFFFFFFFFu && test_bit(T.s_front, u[k]);
+            for (int k = 0; k < K; k++) hit |= u[k] != 0xFFFFFFFFu && test_bit(T.front->word, u[k]);
             if (!ballot(hit)) continue;
             if (ln == 0) {
                 atomicOr((unsigned long long *)&T.fnext[v >> 6], 1ull << (v & 63));
-                team_found(a, T, t, v, caller_id(a, v), g.row[v + 1] - g.row[v]);
+                team_found<true>(a, T, t, v, caller_id(a, v), g.row[v + 1] - g.row[v]);
             }
             break;
         }
@@ -488,7 +499,7 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
             for (int k = 0; k < K; k++) u[k] = e + k * width < end ? g.csrc[e + k * width] : 0xFFFFFFFFu;
             bool hit = false;
 #pragma unroll
-            for (int k = 0; k < K; k++) hit |= u[k] != 0xFFFFFFFFu && test_bit(T.s_front, u[k]);
+            for (int k = 0; k < K; k++) hit |= u[k] != 0xFFFFFFFFu && test_bit(T.front->word, u[k]);
             found |= (ballot(hit) & gmask) != 0;
             e = found ? end : e + K * width;
         }
@@ -496,7 +507,7 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
         if (!ballot(found)) continue;
         const uint64_t bits = wave_reduce(found ? 1ull << (v & 63) : 0ull, 0ull, [](uint64_t x, uint64_t y) { return x | y; });
         if (ln == 0) atomicOr((unsigned long long *)&T.fnext[v0 >> 6], (unsigned long long)bits);
-        if (found) team_found(a, T, t, v, id, dv);
+        if (found) team_found<true>(a, T, t, v, id, dv);
     }
 }
 
@@ -508,7 +519,8 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
 // `t_start` is the trace's time 0. `order` (from level 0): receives the reached
 // vertices level by level, loff[l] the first position of level l.
 template <int BS, bool kWhole>
-__device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t members,
+__device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, TeamBits *front, uint64_t *s_vis,
+                                               uint32_t members,
                                                uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
                                                long long t_start, uint32_t cap, bool &more, uint32_t *order = nullptr,
                                                uint32_t *loff = nullptr)
@@ -524,13 +536,15 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
     T.gwave = rank * WPB + threadIdx.x / kWave;
     T.nwaves = members * WPB;
     T.seg = a.qcap / members;
-    T.s_vis = s_bits;
-    T.s_front = s_bits + kTeamWords;
+    T.front = front;
+    T.s_vis = s_vis;
     if (kWhole)
         for (uint32_t w = threadIdx.x; w < W; w += BS) T.s_vis[w] = load_team(a.vis + w);
     bool ok = true;
     uint32_t &L = S.L;
-    if (S.pol.pull_prev || rc.overflow) {
+    if (kWhole) {
+        T.total = rc.count;
+    } else if (S.pol.pull_prev || rc.overflow) {
         // no queue: each member gathers its share of the bitmap into its segment
         team_gather(t, a.fbit + (size_t)(L % 3) * W, W, a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg, tid,
                     nthreads);
@@ -539,9 +553,10 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
     } else {
         T.incl = T.total = rc.qlen;  // the grid's queue is one segment
     }
+    const uint32_t limit = team_limit(a.qcap, kTeamPushEdges);
     unsigned long long count = rc.count, scout = rc.scout;
     bool hubs = rc.has_huge;
-    uint32_t placed = 1;  // (level 0 is the source)
+    uint32_t placed = 0;  // vertices of the levels before L
     // a phase of narrow rounds keeps no bitmaps and leaves all three clear meanwhile
     if (!kWhole)
         for (uint32_t w = tid; w < W; w += nthreads) {
@@ -560,10 +575,20 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
             for (uint32_t w = tid; w < W; w += nthreads) a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
             for (uint32_t w = threadIdx.x; w < W; w += BS) {
                 const uint64_t x = load_team(a.fbit + (size_t)(L % 3) * W + w);
-                T.s_front[w] = x;
+                T.front->word[w] = x;
                 T.s_vis[w] |= x;
             }
             __syncthreads();
+            if (!pull || order) team_bits_count(*T.front, W);
+            if (order) {
+                for (uint32_t w = tid; w < W; w += nthreads) {
+                    uint32_t at = placed + T.front->before[w];
+                    for (uint64_t x = T.front->word[w]; x; x &= x - 1) order[at++] = w * 64 + (uint32_t)first_lane(x);
+                }
+                if (lead) loff[L] = placed;
+                placed += T.total;
+                if (lead) loff[L + 1] = placed;
+            }
             if (pull) team_pull(a, T, t);
             else team_push<true>(a, T, t, hubs);
         } else {
@@ -577,18 +602,10 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, uin
         count = T.total;
         scout = wave_sum_u64(w & 0xFFFFFFFFu);
         hubs = ballot((w >> kTeamFlagShift) & 1) != 0;
-        if (kWhole && order) {
-            // level L: this block's entries after those of the members before it
-            const uint32_t own = (uint32_t)((t.slot[rank] >> kTeamCountShift) & kTeamCountMask);
-            const uint32_t at = placed + lane_value(T.incl, (int)rank) - own;
-            for (uint32_t i = threadIdx.x; i < own; i += BS) order[at + i] = load_team(T.qout + i);
-            placed += T.total;
-            if (lead) loff[L + 1] = placed;
-        }
         more = count != 0 && !(a.max_rounds && L >= a.max_rounds);
         if (more && !kWhole) {
             DirectionPolicy p = S.pol;
-            if (hubs || count > kTeamPushNodes || scout > kTeamPushEdges || p.next(L, count, scout)) break;
+            if (hubs || count > limit || scout > limit || p.next(L, count, scout)) break;
         }
     }
     tag = T.tag;
@@ -637,7 +654,8 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint32_t
                                           uint32_t *loff = nullptr)
 {
     __shared__ uint32_t s_ok;
-    __shared__ uint64_t s_bits[2 * kTeamWords];
+    __shared__ TeamBits s_front;
+    __shared__ uint64_t s_vis[kTeamWords];
     const long long t_start = wall_clock64();
     const DevGraph &g = a.g;
     const uint32_t W = g.words, src = a.source;
@@ -661,19 +679,11 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint32_t
             a.fbit[(size_t)W + w] = 0;
             a.fbit[2 * (size_t)W + w] = 0;
         }
-        if (tid == 0) {
-            a.queue[0] = src;
-            if (order) {
-                order[0] = src;
-                loff[0] = 0;
-                loff[1] = 1;
-            }
-        }
         ok = team_exchange(a.bar, t, members, rank, tag, a.abort);
     }
     if (ok) {
         const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
-        ok = bfs_team_phase<BS, true>(a, t, s_bits, members, rank, tag, S, rc, t_start, ~0u, more, order, loff);
+        ok = bfs_team_phase<BS, true>(a, t, &s_front, s_vis, members, rank, tag, S, rc, t_start, ~0u, more, order, loff);
     }
     // (after a failed census no block's place is known: block 0 reports)
     if (!s_ok) rank = blockIdx.x ? ~0u : 0u;
@@ -823,7 +833,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
             if (rank != ~0u) {
                 // a failed wait set the abort flag, which ends the others' wait
                 const long long t0 = rank == 0 && threadIdx.x == 0 ? team_clock(a.bar) : 0ll;
-                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, members, rank, tag, S, rc, t0, kTeamRounds, more);
+                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, nullptr, members, rank, tag, S, rc, t0, kTeamRounds, more);
                 if (!ok) break;
                 if (kLeave && !more && rank == 0 && threadIdx.x == 0)
                     write_final(a.trace, a.stats, L, S.pushes, S.pulls, S.ptrace, true, t0);

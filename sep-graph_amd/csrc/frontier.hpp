@@ -415,22 +415,25 @@ __device__ __forceinline__ void write_final(DevTrace *trace, DevStats *stats, ui
     *stats = s;
 }
 
-// Rounds a team runs: push rounds of at most this many edges (see
-// bfs_team_fits), and every round of a graph of at most this many words and
-// edges (see bfs_whole).
-#ifndef SG_TEAM_PUSH_EDGES
-#define SG_TEAM_PUSH_EDGES 16384
-#endif
+// A team runs every round of a graph of at most this many words and edges (see
+// bfs_whole).
 #ifndef SG_TEAM_WORDS
 #define SG_TEAM_WORDS 256
 #endif
 #ifndef SG_TEAM_EDGES
 #define SG_TEAM_EDGES 1000000
 #endif
-constexpr uint32_t kTeamPushEdges = SG_TEAM_PUSH_EDGES, kTeamPushNodes = SG_TEAM_PUSH_EDGES;
 constexpr uint32_t kTeamWords = SG_TEAM_WORDS;
 constexpr uint64_t kTeamEdges = SG_TEAM_EDGES;
-static_assert(kTeamPushEdges <= kTeamSegment && kTeamWords * 64 <= kTeamSegment, "a team round fits its segments");
+
+// What a narrow round may add to the next frontier at most: however it spreads
+// over the members, it has to fit one member's segment of the queue (an engine's
+// queue holds two entries per vertex and 4096).
+__device__ __forceinline__ uint32_t team_limit(uint32_t qcap, uint32_t most)
+{
+    return min(most, qcap / kTeamMax);
+}
+
 // Rounds of one team phase: bounds the other blocks' wait.
 constexpr uint32_t kTeamRounds = 8192;
 
@@ -439,6 +442,44 @@ constexpr uint32_t kTeamRounds = 8192;
 __host__ __device__ __forceinline__ bool team_whole_graph(const DevGraph &g)
 {
     return g.words <= kTeamWords && g.m <= kTeamEdges;
+}
+
+// The frontier of a whole-graph phase as a bitmap in LDS, with the vertices
+// before each word, so that its i-th vertex is found without a queue.
+struct TeamBits {
+    uint64_t word[kTeamWords];
+    uint32_t before[kTeamWords];
+};
+
+// Fills b.before for `words` words (block-wide; the words are in place).
+__device__ __forceinline__ void team_bits_count(TeamBits &b, uint32_t words)
+{
+    constexpr int K = (int)(kTeamWords / kWave);
+    static_assert(kTeamWords % kWave == 0, "whole words per lane");
+    if (threadIdx.x < kWave) {
+        uint32_t c[K], sum = 0;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const uint32_t w = threadIdx.x * K + (uint32_t)k;
+            c[k] = sum;
+            sum += w < words ? (uint32_t)__popcll(b.word[w]) : 0u;
+        }
+        const uint32_t excl = wave_incl_scan(sum) - sum;
+#pragma unroll
+        for (int k = 0; k < K; k++) b.before[threadIdx.x * K + (uint32_t)k] = excl + c[k];
+    }
+    __syncthreads();
+}
+
+// Its i-th vertex, for i below its number of vertices.
+__device__ __forceinline__ uint32_t team_bits_entry(const TeamBits &b, uint32_t i)
+{
+    // the last word with at most i vertices before it
+    uint32_t w = 0;
+#pragma unroll
+    for (uint32_t step = kTeamWords / 2; step > 0; step >>= 1)
+        if (b.before[w + step] <= i) w += step;
+    return w * 64 + nth_set_bit(b.word[w], i - b.before[w]);
 }
 
 // What a traversal carries from round to round, alike in every block.

@@ -883,9 +883,7 @@ int engine_ensure_bfs_state(sg_engine *e)
     if ((rc = alloc((void **)&e->bitmaps, (uint64_t)d.words * 8 * 5))) return rc;
     // Frontier queues may hold a vertex more than once (non-atomic discovery
     // across XCDs); past qcap a round falls back to scanning the level array.
-    // At least what the team rounds' segments take.
-    e->qcap = (uint32_t)std::min<uint64_t>(
-        std::max<uint64_t>(2ull * d.n + 4096, (uint64_t)kTeamMax * std::min(d.n, kTeamSegment)), 0xFFFFFFF0ull);
+    e->qcap = (uint32_t)std::min<uint64_t>(2ull * d.n + 4096, 0xFFFFFFF0ull);
     if ((rc = alloc((void **)&e->queues, (uint64_t)e->qcap * 4 * 3))) return rc;
     if ((rc = alloc((void **)&e->ctr, kCtrBytes))) return rc;
     if ((rc = alloc((void **)&e->abort_flag, 4))) return rc;

@@ -106,10 +106,6 @@ constexpr uint32_t kHugeChunk = SG_HUGE_CHUNK;
 // of kPullChunk.
 constexpr uint32_t kPullHubDegree = 64;
 constexpr uint32_t kPullChunk = 256;
-// Queue entries a team round needs per member, however they spread over the
-// members: no more than the graph's vertices, a narrow round's edges, or the
-// vertices of a graph that the team runs whole.
-constexpr uint32_t kTeamSegment = 24576;
 
 }  // namespace sg
 

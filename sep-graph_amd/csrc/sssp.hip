@@ -177,15 +177,9 @@ struct GroupLayout {
     uint64_t fbit, queue, ctr, stats, bar, status, total;
 };
 
-// Queue entries of each concurrent query (no team rounds: no segments).
-uint32_t group_qcap(const sg_engine *e)
-{
-    return (uint32_t)std::min<uint64_t>(e->qcap, 2ull * e->g->dev.n + 4096);
-}
-
 GroupLayout group_layout(const sg_engine *e)
 {
-    const uint64_t W = e->g->dev.words, qc = group_qcap(e);
+    const uint64_t W = e->g->dev.words, qc = e->qcap;
     auto al = [](uint64_t x) { return (x + 255) / 256 * 256; };
     GroupLayout L;
     L.fbit = 0;
@@ -256,7 +250,7 @@ int sssp_group_launch(sg_engine *e, const uint32_t *sources, int nq, uint32_t *c
     if ((rc = sssp_args(e, a))) return rc;
     a.fbit = (uint64_t *)(base + L.fbit);
     a.queue = (uint32_t *)(base + L.queue);
-    a.qcap = group_qcap(e);
+    a.qcap = e->qcap;
     a.ctr = (FrontierCtr *)(base + L.ctr);
     a.stats = (DevStats *)(base + L.stats);
     a.grouped = 1;

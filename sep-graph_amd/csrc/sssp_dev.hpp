@@ -618,22 +618,25 @@ __device__ __forceinline__ void pull_hubs_sorted(Round &R, uint32_t first, uint3
 // frontier being expanded are cleared entry by entry, so the three bitmaps
 // rotate without being swept.
 
+// Edges and vertices of a narrow push round at most: a round queues no more than
+// the heads of its edges and the vertices it defers.
+constexpr uint32_t kTeamPushWork = 24576;
+
 // Whether round S.L, of a grid round's frontier, starts a team phase; evaluated
-// alike by every block. A round queues at most the heads of its edges and the
-// vertices it defers, which is what a segment holds. 1024 x 1024 grid with the
+// alike by every block. 1024 x 1024 grid with the
 // priority schedule (1844 rounds, up to 13 K edges): 11.6-14.9 us a round on the
 // whole grid, 4.6-8.1 on the team, 23.3 -> 11.6 ms a query.
 __device__ __forceinline__ bool sssp_team_fits(const SsspArgs &a, const RoundState &S, unsigned long long count,
                                                unsigned long long scout, bool hubs)
 {
-    if (!a.team || !(a.team == 2 || S.pulls) || hubs || count + scout > kTeamSegment) return false;
+    if (!a.team || !(a.team == 2 || S.pulls) || hubs || count + scout > team_limit(a.qcap, kTeamPushWork)) return false;
     DirectionPolicy p = S.pol;
     return !p.next(S.L, count, scout);
 }
 
 struct SsspTeam : TeamFront {
     uint64_t *fcur, *fnext;
-    uint64_t *s_front;  // whole-graph phases: frontier L, and the bits this block
+    TeamBits *front;    // whole-graph phases: frontier L, and the bits this block
     uint64_t *s_next;   // has set in the next one, in LDS
     uint32_t thr;       // entries with dist >= thr are deferred (priority mode)
     uint32_t fmin;      // no distance in this round's frontier is below this
@@ -650,7 +653,8 @@ __device__ __forceinline__ void team_queue(const SsspArgs &a, SsspTeam &T, TeamL
     if (kWhole && (atomicOr((unsigned long long *)&T.s_next[v >> 6], (unsigned long long)bit) & bit)) return;
     if (atomicOr((unsigned long long *)&T.fnext[v >> 6], (unsigned long long)bit) & bit) return;
     if (dv > kHugeDegree) t.flag = 1u;
-    team_append(T, t, v, dv);
+    if (kWhole) atomicAdd(&t.acc, (1ull << kTeamCountShift) | dv);
+    else team_append(T, t, v, dv);
 }
 
 // Edge -> v with candidate distance nd, for `act` lanes.
@@ -678,7 +682,7 @@ __device__ __forceinline__ void team_push(const SsspArgs &a, SsspTeam &T, TeamLd
             if (c < g.nhuge) {
                 dsc = g.huge[c];
                 end = g.huge_end[c];
-                mem = test_bit(T.s_front, dsc.x);
+                mem = test_bit(T.front->word, dsc.x);
             }
             uint64_t mm = ballot(mem);
             while (mm) {
@@ -697,9 +701,10 @@ __device__ __forceinline__ void team_push(const SsspArgs &a, SsspTeam &T, TeamLd
     const uint32_t grp = (uint32_t)ln >> shift, sub = (uint32_t)ln & (width - 1);
     for (uint32_t i0 = T.gwave * groups; i0 < T.total; i0 += T.nwaves * groups) {
         const uint32_t i = i0 + grp;
-        const uint32_t u = team_entry(T, i0, i);
-        uint32_t e = 0, end = 0, du = kInf;
+        uint32_t u = 0, e = 0, end = 0, du = kInf;
+        if (!kWhole) u = team_entry(T, i0, i);
         if (i < T.total) {
+            if (kWhole) u = team_bits_entry(*T.front, i);
             e = g.row[u];
             end = g.row[u + 1];
             du = load_team(a.dist + u);
@@ -747,7 +752,7 @@ __device__ __forceinline__ void team_pull(const SsspArgs &a, SsspTeam &T, TeamLd
         // (a weight that alone cannot beat the best skips the distance read)
 #pragma unroll
         for (int k = 0; k < K; k++) {
-            const bool f = u[k] != kInf && sat_add(T.fmin, wt[k]) < best && test_bit(T.s_front, u[k]);
+            const bool f = u[k] != kInf && sat_add(T.fmin, wt[k]) < best && test_bit(T.front->word, u[k]);
             du[k] = f ? load_team(a.dist + u[k]) : kInf;
         }
         uint32_t m = kInf;
@@ -765,7 +770,7 @@ __device__ __forceinline__ void team_pull(const SsspArgs &a, SsspTeam &T, TeamLd
         T.minv = min(T.minv, d);
         const uint32_t dv = g.row[v + 1] - g.row[v];
         if (dv > kHugeDegree) t.flag = 1u;
-        team_append(T, t, v, dv);
+        atomicAdd(&t.acc, (1ull << kTeamCountShift) | dv);
     };
     for (uint32_t h = T.gwave; h < g.nhubin; h += T.nwaves) {
         const uint2 first = g.hugein[g.hubin[h].x];
@@ -808,7 +813,8 @@ __device__ __forceinline__ void team_pull(const SsspArgs &a, SsspTeam &T, TeamLd
 // A team phase: see bfs_team_phase. `cmin`: the smallest distance in frontier
 // S.L. Leaves the bitmaps and counters that a grid round expects.
 template <int BS, bool kWhole>
-__device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, uint64_t *s_bits, uint32_t members,
+__device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, TeamBits *front, uint64_t *s_next,
+                                                uint32_t members,
                                                 uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
                                                 uint32_t cmin, long long t_start, uint32_t cap, bool &more)
 {
@@ -824,13 +830,15 @@ __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, u
     T.gwave = rank * WPB + threadIdx.x / kWave;
     T.nwaves = members * WPB;
     T.seg = a.qcap / members;
-    T.s_front = s_bits;
-    T.s_next = s_bits + kTeamWords;
+    T.front = front;
+    T.s_next = s_next;
     // the bitmap after next still holds frontier L - 1
     if (!kWhole)
         for (uint32_t w = tid; w < W; w += nthreads) a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
     bool ok = true;
-    if (S.pol.pull_prev || rc.overflow) {
+    if (kWhole) {
+        T.total = rc.count;
+    } else if (S.pol.pull_prev || rc.overflow) {
         team_gather(t, a.fbit + (size_t)(L % 3) * W, W, a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg, tid,
                     nthreads);
         ok = team_exchange<true>(a.bar, t, members, rank, T.tag, a.abort);
@@ -855,10 +863,11 @@ __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, u
         if constexpr (kWhole) {
             for (uint32_t w = tid; w < W; w += nthreads) a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
             for (uint32_t w = threadIdx.x; w < W; w += BS) {
-                T.s_front[w] = load_team(T.fcur + w);
+                T.front->word[w] = load_team(T.fcur + w);
                 T.s_next[w] = 0;
             }
             __syncthreads();
+            if (!pull) team_bits_count(*T.front, W);
         }
         if (kWhole && pull) team_pull(a, T, t);
         else team_push<kWhole>(a, T, t, hubs);
@@ -901,7 +910,8 @@ __device__ __forceinline__ bool sssp_whole(const SsspArgs &a, uint32_t xcc, BarS
 {
     __shared__ uint32_t s_ok;
     __shared__ TeamLds t;
-    __shared__ uint64_t s_bits[2 * kTeamWords];
+    __shared__ TeamBits s_front;
+    __shared__ uint64_t s_next[kTeamWords];
     const long long t_start = wall_clock64();
     if (threadIdx.x == 0) t.reset();
     const DevGraph &g = a.g;
@@ -917,12 +927,11 @@ __device__ __forceinline__ bool sssp_whole(const SsspArgs &a, uint32_t xcc, BarS
     if (ok) {
         for (uint32_t i = tid; i < g.n; i += nthreads) a.dist[i] = i == src ? 0u : kInf;
         for (uint32_t w = tid; w < 3 * W; w += nthreads) a.fbit[w] = w == (src >> 6) ? 1ull << (src & 63) : 0ull;
-        if (tid == 0) a.queue[0] = src;
         ok = team_exchange<true>(a.bar, t, members, rank, tag, a.abort);
     }
     if (ok) {
         const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
-        ok = sssp_team_phase<BS, true>(a, t, s_bits, members, rank, tag, S, rc, 0, t_start, ~0u, more);
+        ok = sssp_team_phase<BS, true>(a, t, &s_front, s_next, members, rank, tag, S, rc, 0, t_start, ~0u, more);
     }
     // the last exchange ordered every distance before this
     if (ok && a.out)
@@ -1017,7 +1026,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
                 if (rank != ~0u) {
                     // a failed wait set the abort flag, which ends the others' wait
                     const long long t0 = rank == 0 && threadIdx.x == 0 ? team_clock(a.bar) : 0ll;
-                    ok = sssp_team_phase<BS, false>(a, s_t, nullptr, members, rank, tag, S, rc,
+                    ok = sssp_team_phase<BS, false>(a, s_t, nullptr, nullptr, members, rank, tag, S, rc,
                                                     s_cmin ? ~s_cmin : 0u, t0, kTeamRounds, more);
                     if (!ok) break;
                 }
