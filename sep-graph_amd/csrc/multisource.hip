@@ -178,6 +178,9 @@ __device__ __forceinline__ double masked_row_sum(const uint32_t *adj, const uint
     return acc;
 }
 
+// Slice rows a wave of a pull discovery keeps in flight.
+constexpr int kDiscoverRows = 8;
+
 // Discovery of the next level's masks: Fn[w] gets the bits of sources that
 // reach w for the first time through a level-L vertex. Push expands the
 // level's entries (seg_v/seg_m, len) over out-edges with atomicOr; pull has
@@ -249,13 +252,63 @@ __device__ __forceinline__ void ms_discover(const DevGraph &g, const uint64_t *s
             const uint64_t unseen = bm & ~seen[dsc.x];
             if (!unseen) continue;
             const uint32_t end = min(g.cstart[dsc.x + 1], dsc.y + kPullChunk);
-            uint64_t o = 0;
-            for (uint32_t e0 = dsc.y; e0 < end; e0 += kWave) {
-                const uint32_t e = e0 + ln;
-                if (e < end) o |= Fc[g.csrc[e]];
+            constexpr int K = (int)(kPullChunk / kWave);
+            uint32_t u[K];
+            uint64_t f[K], o = 0;
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const uint32_t e = dsc.y + (uint32_t)(k * kWave + ln);
+                u[k] = e < end ? g.csrc[e] : 0xFFFFFFFFu;
             }
+#pragma unroll
+            for (int k = 0; k < K; k++) f[k] = u[k] != 0xFFFFFFFFu ? Fc[u[k]] : 0ull;
+#pragma unroll
+            for (int k = 0; k < K; k++) o |= f[k];
             o = wave_or_u64(o) & unseen;
             if (ln == 0 && o) atomicOr((unsigned long long *)&Fn[dsc.x], (unsigned long long)o);
+        }
+        // By the sliced in-edges, a lane per vertex and kDiscoverRows rows in
+        // flight, a lane stopping once it has every bit it lacks: a vertex's
+        // OR stays in a register, where scheduling the edges over the wave
+        // took a segmented 64-bit scan per 64 of them. A graph with fewer
+        // words than waves gives each word to `parts` waves, which take its rows
+        // in turn and merge by atomics. 64 BFS on an RMAT graph of 524 288
+        // vertices: its pull rounds 212, 204, 161, 77, 32 us by scheduled edges
+        // and an append atomic per word, 108, 101, 59, 31, 26 by rows and
+        // append_level.
+        if (g.sell_src) {
+            uint32_t parts = 1;
+            while (parts < 16 && (uint64_t)parts * 2 * W <= nwaves) parts <<= 1;
+            for (uint32_t it = gwave; it < W * parts; it += nwaves) {
+                const uint32_t w = it / parts, part = it % parts, v = w * 64 + (uint32_t)ln;
+                uint64_t unseen = 0, acc = 0;
+                uint32_t deg = 0;
+                if (v < n) {
+                    unseen = bm & ~seen[v];
+                    deg = g.cstart[v + 1] - g.cstart[v];
+                    if (deg > kPullHubDegree) deg = 0;
+                }
+                uint32_t j0 = part * kDiscoverRows;
+                bool act = unseen && j0 < deg;
+                if (!ballot(act)) continue;
+                const uint32_t *S = g.sell_src + g.sell_off[w] + ln;
+                for (; ballot(act); j0 += parts * kDiscoverRows) {
+                    uint32_t u[kDiscoverRows];
+                    uint64_t f[kDiscoverRows];
+#pragma unroll
+                    for (int k = 0; k < kDiscoverRows; k++)
+                        u[k] = act && j0 + k < deg ? S[(size_t)(j0 + k) * kWave] : 0xFFFFFFFFu;
+#pragma unroll
+                    for (int k = 0; k < kDiscoverRows; k++) f[k] = u[k] != 0xFFFFFFFFu ? Fc[u[k]] : 0ull;
+#pragma unroll
+                    for (int k = 0; k < kDiscoverRows; k++) acc |= f[k];
+                    act = act && j0 + parts * kDiscoverRows < deg && (acc & unseen) != unseen;
+                }
+                acc &= unseen;
+                if (acc && parts == 1) Fn[v] = acc;
+                else if (acc) atomicOr((unsigned long long *)&Fn[v], (unsigned long long)acc);
+            }
+            return;
         }
         for (uint32_t w = gwave; w < W; w += nwaves) {
             const uint32_t v = w * 64 + ln;
@@ -270,6 +323,54 @@ __device__ __forceinline__ void ms_discover(const DevGraph &g, const uint64_t *s
             const uint64_t o = wave_gather_or(g, Fc, b, e, unseen) & unseen;
             if (o) Fn[v] = o;
         }
+    }
+}
+
+// Appends (v, F[v]) of every vertex with a bit in F to the pair list (vv, mm)
+// whose length is *count, one atomic per block (one per word of vertices, all
+// on the same counter, serialise at 11 ns each: 90 us a level on 2^19
+// vertices): the block's waves count first, then write. s_at: WPB words. Past
+// `cap` entries *overflow is set.
+template <int WPB>
+__device__ __forceinline__ void append_level(const uint64_t *F, uint32_t n, uint32_t W, uint32_t gwave, uint32_t nwaves,
+                                             uint32_t *count, uint32_t *vv, uint64_t *mm, uint32_t cap,
+                                             uint32_t *overflow, uint32_t *s_at)
+{
+    const int ln = lane(), wid = threadIdx.x / kWave;
+    uint32_t mine = 0;
+    for (uint32_t w = gwave; w < W; w += nwaves) {
+        const uint32_t v = w * 64 + (uint32_t)ln;
+        mine += (uint32_t)__popcll(ballot(v < n && F[v] != 0));
+    }
+    if (ln == 0) s_at[wid] = mine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t sum = 0;
+        for (int i = 0; i < WPB; i++) sum += s_at[i];
+        uint32_t at = sum ? atomicAdd(count, sum) : 0u;
+        for (int i = 0; i < WPB; i++) {
+            const uint32_t c = s_at[i];
+            s_at[i] = at;
+            at += c;
+        }
+    }
+    __syncthreads();
+    uint32_t at = s_at[wid];
+    if (!mine) return;
+    for (uint32_t w = gwave; w < W; w += nwaves) {
+        const uint32_t v = w * 64 + (uint32_t)ln;
+        const uint64_t x = v < n ? F[v] : 0ull;
+        const uint64_t m = ballot(x != 0);
+        if (x) {
+            const uint32_t pos = at + (uint32_t)rank_in(m);
+            if (pos < cap) {
+                vv[pos] = v;
+                mm[pos] = x;
+            } else {
+                *overflow = 1;
+            }
+        }
+        at += (uint32_t)__popcll(m);
     }
 }
 
@@ -317,7 +418,7 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
 
     __shared__ unsigned long long s_red[2][WPB];
     __shared__ unsigned long long s_lvl[5];
-    __shared__ uint32_t s_len;
+    __shared__ uint32_t s_len, s_at[WPB];
 
     // ---- prologue: clear masks; zero the rows hub chunks accumulate into
     for (uint32_t v = gtid; v < n; v += nthreads) {
@@ -411,21 +512,33 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
 
         // (2) the new level: seen, stack, sigma from predecessors on level L
         unsigned long long scout = 0, cnt = 0;
+        append_level<WPB>(Fn, n, W, gwave, nwaves, &a.ctl[0], a.stk_v, a.stk_m, a.cap, &a.ctl[1], s_at);
         for (uint32_t w = gwave; w < W; w += nwaves) {
             const uint32_t v = w * 64 + ln;
+            const uint64_t nw = v < n ? Fn[v] : 0ull;
+            if (nw) {
+                a.seen[v] |= nw;
+                scout += g.row[v + 1] - g.row[v];
+                cnt++;
+            }
+        }
+        // a wave sums one vertex at a time: a graph with fewer words than
+        // waves gives each word's vertices to `parts` waves (2^16 vertices, 64
+        // sources: 1024 words had kept three of four waves idle)
+        uint32_t parts = 1;
+        while (parts < 64 && (uint64_t)parts * 2 * W <= nwaves) parts <<= 1;
+        const uint32_t span = 64 / parts;
+        for (uint32_t it = gwave; it < W * parts; it += nwaves) {
+            const uint32_t w = it / parts, first = it % parts * span;
+            const uint32_t v = w * 64 + ln;
+            const bool in = (uint32_t)ln - first < span && v < n;
             uint64_t nw = 0;
             uint32_t b = 0, e = 0;
-            if (v < n) {
-                nw = Fn[v];
-                if (nw) {
-                    a.seen[v] |= nw;
-                    b = g.cstart[v];
-                    e = g.cstart[v + 1];
-                    scout += g.row[v + 1] - g.row[v];
-                    cnt++;
-                }
+            if (in) nw = Fn[v];
+            if (nw) {
+                b = g.cstart[v];
+                e = g.cstart[v + 1];
             }
-            append_pair(&a.ctl[0], a.stk_v, a.stk_m, a.cap, &a.ctl[1], nw != 0, v, nw);
             uint64_t cand = ballot(nw != 0 && e - b <= kPullHubDegree);
             while (cand) {
                 const int t = first_lane(cand);
@@ -465,11 +578,21 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
             const uint32_t fb = a.lvl[l + 2], fe = a.lvl[l + 3];
             for (uint32_t i = fb + gtid; i < fe; i += nthreads) Af[a.stk_v[i]] = 0;
         }
-        for (uint32_t i = sb + gwave; i < se; i += nwaves) {
-            const uint32_t v = a.stk_v[i];
-            const uint32_t rb = g.row[v], re = g.row[v + 1];
+        // (the entry after next and the next one's edge range are read while
+        // this one is summed)
+        uint32_t i = sb + gwave;
+        uint32_t v1 = i < se ? a.stk_v[i] : 0u, v2 = i + nwaves < se ? a.stk_v[i + nwaves] : 0u;
+        uint32_t rb1 = g.row[v1], re1 = g.row[v1 + 1];
+        uint64_t mv1 = i < se ? a.stk_m[i] : 0ull;
+        for (; i < se; i += nwaves) {
+            const uint32_t v = v1, rb = rb1, re = re1;
+            const uint64_t mv = mv1;
+            v1 = v2;
+            v2 = i + 2 * nwaves < se ? a.stk_v[i + 2 * nwaves] : 0u;
+            rb1 = g.row[v1];
+            re1 = g.row[v1 + 1];
+            mv1 = i + nwaves < se ? a.stk_m[i + nwaves] : 0ull;
             if (re - rb > kHugeDegree) continue;
-            const uint64_t mv = a.stk_m[i];
             const double acc = masked_row_sum(g.col, An, a.psi, rb, re, mv);
             double dl = 0.0;
             if ((mv >> ln) & 1) {
@@ -581,17 +704,13 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
 
     __shared__ unsigned long long s_red[2][WPB];
     __shared__ unsigned long long s_lvl[5];
-    __shared__ uint32_t s_len;
+    __shared__ uint32_t s_len, s_at[WPB];
 
     for (uint32_t v = gtid; v < n; v += nthreads) {
         a.seen[v] = 0;
         a.F[v] = 0;
         a.F[(size_t)n + v] = 0;
         a.F[2 * (size_t)n + v] = 0;
-    }
-    for (uint32_t s = 0; s < a.nsrc; s++) {
-        int32_t *row = a.out + out_row(a.orow, s, n);
-        for (uint32_t v = gtid; v < n; v += nthreads) row[v] = -1;
     }
     if (blockIdx.x == 0) {
         clear_ctr(&a.ctr[0]);
@@ -667,18 +786,16 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
         if (!ok) break;
 
         unsigned long long scout = 0, cnt = 0;
+        append_level<WPB>(Fn, n, W, gwave, nwaves, &a.ctl[2 + ((L + 1) & 1)], a.ring_v + other, a.ring_m + other, n,
+                          &a.ctl[1], s_at);
         for (uint32_t w = gwave; w < W; w += nwaves) {
             const uint32_t v = w * 64 + ln;
-            uint64_t nw = 0;
-            if (v < n) {
-                nw = Fn[v];
-                if (nw) {
-                    a.seen[v] |= nw;
-                    scout += g.row[v + 1] - g.row[v];
-                    cnt++;
-                }
+            const uint64_t nw = v < n ? Fn[v] : 0ull;
+            if (nw) {
+                a.seen[v] |= nw;
+                scout += g.row[v + 1] - g.row[v];
+                cnt++;
             }
-            append_pair(&a.ctl[2 + ((L + 1) & 1)], a.ring_v + other, a.ring_m + other, n, &a.ctl[1], nw != 0, v, nw);
             // one pass per source present in this word: lanes write consecutive vertices
             uint64_t any = wave_or_u64(nw);
             while (any) {
@@ -693,6 +810,19 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
         L++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
+    // -1 where no query of the batch came by (every block left the loop after
+    // the same barrier, and `seen` holds all levels)
+    if (ok)
+        for (uint32_t w = gwave; w < W; w += nwaves) {
+            const uint32_t v = w * 64 + ln;
+            const uint64_t not_seen = v < n ? bm & ~a.seen[v] : 0ull;
+            uint64_t any = wave_or_u64(not_seen);
+            while (any) {
+                const int s = first_lane(any);
+                any &= any - 1;
+                if ((not_seen >> s) & 1) a.out[out_row(a.orow, s, n) + v] = -1;
+            }
+        }
     if (gtid == 0) {
         DevStats s = *a.stats;
         s.rounds += L;

@@ -167,3 +167,23 @@ def test_bc_small_levels(sg, orc, gpu, name, opts):
     assert st["iterations"] == len(sources) and st["max_depth"] == depth
     e.bc(sources, 1)
     np.testing.assert_allclose(e.gather(np.float32), total, rtol=1e-6, atol=1e-6)
+
+
+BATCH_GRAPHS = ["n65", "n16385", "stars", "rmat13", "rmat17", "dense", "grid"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [1, 2, 9, 33, 64, 70])
+@pytest.mark.parametrize("name", BATCH_GRAPHS)
+def test_bfs_batches(sg, orc, gpu, name, k):
+    hg = SMALL_ROUND_GRAPHS[name](sg)
+    e = sg.Engine(sg.Graph(hg))
+    src = np.random.default_rng(k).integers(0, hg.n, k)  # repeats among them
+    e.bfs_multi(src)
+    got = e.gather(np.int32).reshape(k, hg.n)
+    for i in sorted({0, k // 2, k - 1}):
+        assert np.array_equal(got[i], orc.bfs(hg.row, hg.col, int(src[i]))), i
+    assert e.stats()["status"] == 0
+    e.bc(src)
+    # FP64 sums, one rounding to FP32
+    np.testing.assert_allclose(e.gather(np.float32), orc.bc(hg.row, hg.col, src), rtol=1e-5, atol=1e-5)
