@@ -838,24 +838,31 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
 
 // ----------------------------------------------------------- multi-source SSSP
 // Up to 64 independent SSSP queries in one launch. Distances live as rows
-// dist[v][64] (lane q = query q), so relaxing an edge for every query whose
-// frontier holds its tail is one coalesced row access and at most one
-// atomicMin per improving lane. A round pushes from every vertex whose mask
-// (queries that lowered its distance last round) is non-zero; a vertex enters
-// the next round's entry list when the first bit of its next mask is set
-// (the atomicOr returns 0). Results are written transposed, one contiguous
-// n-vector per query, equal to sg_sssp from that source.
+// dist[v][2^qbits] (the batch rounded up to a power of two; lane q of a group
+// of 2^qbits = query q), so an edge's end is one coalesced row for every
+// query. A vertex's mask holds the queries that lowered its distance last
+// round. A push round relaxes the out-edges of every vertex with a mask: a row
+// read, an atomicMin per improving lane and one on the head's mask per edge; a
+// vertex enters the next round's entry list when the first bit of its next
+// mask is set (the atomicOr returns 0). A pull round has every vertex take the
+// minimum over its in-edges from vertices with a mask, its row in registers:
+// no atomics but for in-hubs split into chunks. Results leave
+// transposed, one contiguous n-vector per query in the order asked for, equal
+// to sg_sssp from that source.
 struct MsSsspArgs {
     DevGraph g;
     const uint32_t *src;
     uint32_t nsrc;
-    uint32_t *dist;       // [n][64]
+    uint32_t *dist;       // [n][2^qbits]
     uint64_t *F;          // 3 x n masks, round r in F + (r % 3) n
     uint32_t *out;        // distances of source q in row out_row(orow, q)
     const uint32_t *orow;
+    const uint32_t *inv;  // out[v] is device vertex inv[v]'s (null: v's)
+    int32_t force;        // 0: push rounds only
     uint32_t *ring;       // 3 x n: entries of round r in third r % 3
-    uint32_t *ctl;        // [1] overflow, [2 + t] entries in third t
-    FrontierCtr *ctr;     // 3 slots: count / out-degree of each round's entries
+    uint32_t *cmin;       // 3 x 64: smallest distance queued for round r by each
+                          // query, complemented (0: none), in third r % 3
+    FrontierCtr *ctr;     // 3 slots: entries / out-degree of each round
     GridBarrier bar;
     uint32_t *abort;
     DevStats *stats;
@@ -867,10 +874,11 @@ struct MsSsspArgs {
 struct MsRelax {
     const MsSsspArgs *a;
     uint64_t *Fn;
-    uint32_t *ring_next;
-    uint32_t *cnt_next;
+    Stager S;        // the next round's entries
     uint32_t qbits;  // queries of the batch fit in 2^qbits lanes
     unsigned long long scout, count;
+    uint32_t fmin;   // this lane's query has no frontier distance below this
+    uint32_t minv;   // smallest distance this lane queued for the next round
 };
 
 // Edge steps a group of lanes keeps in flight in the batched relaxation.
@@ -880,13 +888,12 @@ struct MsRelax {
 constexpr int kMsRelaxSteps = SG_MS_RELAX_STEPS;
 
 // Relax the out-edges [b, e) of u for the queries in `mask`. The wave is
-// split into 64 / 2^qbits groups of 2^qbits lanes (lane q of a group = query
-// q); each group takes kMsRelaxSteps edges per step, with the loads and
-// atomics of all of them issued before any result is used, so a batch of B
-// queries keeps about 64 / B x kMsRelaxSteps edges in flight per wave. A
-// group's leader publishes the queries whose distance it lowered into the
-// next round's mask of the edge's head; the wave queues the heads whose mask
-// it was first to set, with one append per wave and step.
+// split into 64 / 2^qbits groups; each group takes kMsRelaxSteps edges per
+// step, with the loads and atomics of all of them issued before any result is
+// used, so a batch of B queries keeps about 64 / B x kMsRelaxSteps edges in
+// flight per wave. A group's leader publishes the queries whose distance it
+// lowered into the next round's mask of the edge's head; the heads whose mask
+// it was first to set are staged for the next round's entries.
 __device__ __forceinline__ void ms_relax_range(MsRelax &R, uint32_t u, uint32_t b, uint32_t e, uint64_t mask)
 {
     constexpr int U = kMsRelaxSteps;
@@ -897,7 +904,7 @@ __device__ __forceinline__ void ms_relax_range(MsRelax &R, uint32_t u, uint32_t 
     const uint32_t q = (uint32_t)ln & ((1u << qb) - 1), grp = (uint32_t)ln >> qb, ngrp = 64u >> qb;
     const uint64_t gmask = qb == 6 ? ~0ull : ((1ull << (1u << qb)) - 1);
     const bool mine = (mask >> q) & 1;
-    const uint32_t du = mine ? a.dist[(size_t)u * 64 + q] : 0xFFFFFFFFu;
+    const uint32_t du = mine ? a.dist[((size_t)u << qb) + q] : 0xFFFFFFFFu;
     for (uint32_t e0 = b; e0 < e; e0 += ngrp * U) {
         uint32_t v[U], nd[U], cur[U];
         bool act[U];
@@ -911,47 +918,217 @@ __device__ __forceinline__ void ms_relax_range(MsRelax &R, uint32_t u, uint32_t 
             act[s] = act[s] && mine;
         }
 #pragma unroll
-        for (int s = 0; s < U; s++) cur[s] = act[s] ? a.dist[(size_t)v[s] * 64 + q] : 0u;
+        for (int s = 0; s < U; s++) cur[s] = act[s] ? a.dist[((size_t)v[s] << qb) + q] : 0u;
         // every atomic of the step is issued before any result is read (a
         // result consumed inside its own branch makes each one wait in turn)
         uint32_t old[U];
 #pragma unroll
         for (int s = 0; s < U; s++) {
             old[s] = 0xFFFFFFFFu;
-            if (act[s] && nd[s] < cur[s]) old[s] = atomicMin(&a.dist[(size_t)v[s] * 64 + q], nd[s]);
+            if (act[s] && nd[s] < cur[s]) old[s] = atomicMin(&a.dist[((size_t)v[s] << qb) + q], nd[s]);
         }
         unsigned long long fo[U];
 #pragma unroll
         for (int s = 0; s < U; s++) {
             const bool imp = act[s] && nd[s] < cur[s] && nd[s] < old[s];
+            if (imp) R.minv = min(R.minv, nd[s]);
             const uint64_t im = ballot(imp);
             const uint64_t gm = (im >> (grp << qb)) & gmask;
             fo[s] = ~0ull;
             if (q == 0 && gm) fo[s] = atomicOr((unsigned long long *)&R.Fn[v[s]], (unsigned long long)gm);
         }
-        // heads whose mask this wave set first: one append for the whole step
-        uint64_t fm[U];
-        uint32_t tot = 0;
+        // heads whose mask this wave set first, staged in the block's LDS: an
+        // append per wave and step to one global counter had serialised at
+        // 11 ns each (131 K entries: 580 us a round)
 #pragma unroll
         for (int s = 0; s < U; s++) {
-            fm[s] = ballot(fo[s] == 0);
-            tot += (uint32_t)__popcll(fm[s]);
-        }
-        if (!tot) continue;
-        uint32_t base = 0;
-        if (ln == 0) base = atomicAdd(R.cnt_next, tot);
-        base = lane_value(base, 0);
-#pragma unroll
-        for (int s = 0; s < U; s++) {
-            if (fo[s] == 0) {
-                const uint32_t pos = base + (uint32_t)rank_in(fm[s]);
-                if (pos < g.n) R.ring_next[pos] = v[s];
-                else a.ctl[1] = 1;
+            const bool fresh = fo[s] == 0;
+            if (fresh) {
                 R.scout += g.row[v[s] + 1] - g.row[v[s]];
                 R.count++;
             }
-            base += (uint32_t)__popcll(fm[s]);
+            stage(R.S, fresh, v[s]);
         }
+    }
+}
+
+// Rows a group keeps in flight in a pull round.
+constexpr int kMsPullRows = 8;
+// A round pulls when its entries' out-edges number at least 1/kMsPullRatio of
+// all edges, and when the batch fills groups of at least 2^kMsPullBits lanes: a
+// pull round reads every vertex's in-edges, but a row only where it can still
+// lower something, and without atomics. 24 queries on 230 017 vertices, 3.4 M
+// edges: 500 us a dense round by pushing, 250 falling to 180 by pulling; whole
+// call 3180 us without pull rounds, 1759 with a ratio of 4, 1621 with 16, 1569
+// with 32 (64: 1541, but a 150 x 200 grid loses what that gains). Narrow groups walk too
+// few edges at a time: 8 queries on 60 001 vertices take 602 us pushing and 702
+// pulling, 16 take 859 and 703.
+#ifndef SG_MS_PULL_RATIO
+#define SG_MS_PULL_RATIO 32
+#endif
+constexpr uint32_t kMsPullRatio = SG_MS_PULL_RATIO;
+#ifndef SG_MS_PULL_BITS
+#define SG_MS_PULL_BITS 4
+#endif
+constexpr uint32_t kMsPullBits = SG_MS_PULL_BITS;
+
+// In-edges a group is about to read the far ends of: one per lane.
+struct MsEdges {
+    uint32_t u, w;
+    bool in;
+};
+
+__device__ __forceinline__ MsEdges ms_edges(const DevGraph &g, uint32_t ed, uint32_t e)
+{
+    MsEdges x{0u, 0u, ed < e};
+    if (x.in) {
+        x.u = g.csrc[ed];
+        x.w = g.cw ? g.cw[ed] : 1u;
+    }
+    return x;
+}
+
+// Smallest candidate below `best` of this lane's query over the edges `x` from
+// vertices with a mask in Fc, or `best`. A row is read by the lanes whose query
+// the edge can still improve (every frontier distance is at least fmin).
+// Wave-convergent.
+__device__ __forceinline__ uint32_t ms_pull_edges(const MsRelax &R, const uint64_t *Fc, const MsEdges &x, uint32_t best)
+{
+    const MsSsspArgs &a = *R.a;
+    const int ln = lane();
+    const uint32_t qb = R.qbits, width = 1u << qb;
+    const uint32_t q = (uint32_t)ln & (width - 1);
+    const int base = ln & ~(int)(width - 1);  // the group's first lane
+    const uint64_t gmask = qb == 6 ? ~0ull : ((1ull << width) - 1);
+    const uint64_t f = x.in ? Fc[x.u] : 0ull;
+    uint64_t live = (ballot(f != 0) >> base) & gmask;  // the group's edges to read
+    while (ballot(live != 0)) {
+        uint32_t d[kMsPullRows], wt[kMsPullRows];
+#pragma unroll
+        for (int k = 0; k < kMsPullRows; k++) {
+            const bool on = live != 0;
+            const int j = base + (on ? first_lane(live) : 0);
+            live &= live - 1;
+            const uint32_t uj = shfl(x.u, j);
+            const uint64_t fj = shfl(f, j);
+            wt[k] = shfl(x.w, j);
+            const bool can = on && ((fj >> q) & 1) && (uint64_t)R.fmin + wt[k] < best;
+            d[k] = can ? a.dist[((size_t)uj << qb) + q] : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (int k = 0; k < kMsPullRows; k++) best = min(best, d[k] > 0xFFFFFFFFu - wt[k] ? 0xFFFFFFFFu : d[k] + wt[k]);
+    }
+    return best;
+}
+
+// A pull round: in-hubs by the chunk list, a chunk per group merged with
+// atomicMin, then every other vertex, a group each. Either way a group stops at
+// once where no query of it can be lowered (see sssp_dev.hpp's settled()).
+__device__ __forceinline__ void ms_pull(MsRelax &R, const uint64_t *Fc, uint32_t nsrc, uint32_t gwave, uint32_t nwaves)
+{
+    const MsSsspArgs &a = *R.a;
+    const DevGraph &g = a.g;
+    const int ln = lane();
+    const uint32_t qb = R.qbits, width = 1u << qb, ngrp = 64u >> qb;
+    const uint32_t q = (uint32_t)ln & (width - 1), grp = (uint32_t)ln >> qb;
+    const uint64_t gmask = qb == 6 ? ~0ull : ((1ull << width) - 1);
+    const bool has = q < nsrc;
+    // whether some query of the group can be lowered below its d
+    auto open = [&](uint32_t d, uint32_t mw) {
+        return ((ballot(has && (uint64_t)R.fmin + mw < d) >> (grp << qb)) & gmask) != 0;
+    };
+    // the group's lowered queries into v's next mask, v into the next entries
+    auto publish = [&](bool low, uint32_t v, uint32_t d, bool shared) {
+        if (low) R.minv = min(R.minv, d);
+        const uint64_t bits = (ballot(low) >> (grp << qb)) & gmask;
+        bool fresh = false;
+        if (q == 0 && bits) {
+            if (shared) {
+                fresh = atomicOr((unsigned long long *)&R.Fn[v], (unsigned long long)bits) == 0;
+            } else {
+                R.Fn[v] = bits;
+                fresh = true;
+            }
+        }
+        if (fresh) {
+            R.scout += g.row[v + 1] - g.row[v];
+            R.count++;
+        }
+        stage(R.S, fresh, v);
+    };
+    const uint32_t step = nwaves * ngrp;
+    for (uint32_t c0 = gwave * ngrp; c0 < g.nhugein; c0 += step) {
+        const uint32_t c = c0 + grp;
+        uint32_t v = 0, b = 0, e = 0, d0 = 0, mw = 0;
+        if (c < g.nhugein) {
+            const uint2 dsc = g.hugein[c];
+            v = dsc.x;
+            b = dsc.y;
+            e = min(g.cstart[v + 1], b + kPullChunk);
+            d0 = a.dist[((size_t)v << qb) + q];
+            mw = g.cminw ? g.cminw[v] : (g.cw ? 0u : 1u);
+        }
+        if (!open(d0, mw)) e = b;
+        uint32_t best = d0;
+        MsEdges x = ms_edges(g, b + q, e);
+        for (; ballot(b < e); b += width) {
+            const MsEdges y = ms_edges(g, b + width + q, e);  // the next ones, while these are worked
+            best = ms_pull_edges(R, Fc, x, best);
+            x = y;
+        }
+        bool low = has && best < d0;
+        if (low) low = best < atomicMin(&a.dist[((size_t)v << qb) + q], best);
+        publish(low, v, best, true);
+    }
+    // Every other vertex: the next one's row, first edges and smallest weight are
+    // read while this one is worked, the edge range of the one after it too.
+    auto range = [&](uint32_t v, uint32_t &b, uint32_t &e) {
+        b = e = 0;
+        if (v < g.n) {
+            b = g.cstart[v];
+            e = g.cstart[v + 1];
+            if (e - b > kPullHubDegree) e = b;
+        }
+    };
+    auto head = [&](uint32_t v, uint32_t b, uint32_t e, uint32_t &d, uint32_t &mw, MsEdges &x) {
+        d = mw = 0;
+        x = ms_edges(g, b + q, e);
+        if (b < e) {
+            d = a.dist[((size_t)v << qb) + q];
+            mw = g.cminw ? g.cminw[v] : (g.cw ? 0u : 1u);
+        }
+    };
+    uint32_t v = gwave * ngrp + grp, b, e, b1, e1, d0, mw;
+    MsEdges x;
+    range(v, b, e);
+    range(v + step, b1, e1);
+    head(v, b, e, d0, mw, x);
+    for (uint32_t v0 = gwave * ngrp; v0 < g.n; v0 += step, v += step) {
+        uint32_t b2, e2, d1, mw1;
+        MsEdges x1;
+        range(v + 2 * step, b2, e2);
+        head(v + step, b1, e1, d1, mw1, x1);
+        if (!open(d0, mw)) {
+            e = b;
+            x.in = false;
+        }
+        uint32_t best = d0;
+        for (; ballot(b < e); b += width) {
+            best = ms_pull_edges(R, Fc, x, best);
+            x = ms_edges(g, b + width + q, e);
+        }
+        const bool low = has && best < d0;
+        if (ballot(low)) {
+            if (low) a.dist[((size_t)v << qb) + q] = best;
+            publish(low, v, best, false);
+        }
+        b = b1;
+        e = e1;
+        b1 = b2;
+        e1 = e2;
+        d0 = d1;
+        mw = mw1;
+        x = x1;
     }
 }
 
@@ -978,20 +1155,17 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
 
     __shared__ unsigned long long s_red[2][WPB];
     __shared__ unsigned long long s_lvl[5];
-    __shared__ uint32_t s_len;
+    constexpr uint32_t kLdsQ = 8u * BS;
+    __shared__ uint32_t s_q[kLdsQ];
+    __shared__ uint32_t s_qn, s_flush[2], s_min[64];
 
-    for (size_t i = gtid; i < (size_t)n * 64; i += nthreads) a.dist[i] = 0xFFFFFFFFu;
+    for (size_t i = gtid; i < (size_t)n << qbits; i += nthreads) a.dist[i] = 0xFFFFFFFFu;
     for (size_t i = gtid; i < 3 * (size_t)n; i += nthreads) a.F[i] = 0;
     if (blockIdx.x == 0) {
         clear_ctr(&a.ctr[0]);
         clear_ctr(&a.ctr[1]);
         clear_ctr(&a.ctr[2]);
-        if (threadIdx.x == 0) {
-            a.ctl[1] = 0;
-            a.ctl[2] = 0;
-            a.ctl[3] = 0;
-            a.ctl[4] = 0;
-        }
+        if (threadIdx.x < 3 * 64) a.cmin[threadIdx.x] = threadIdx.x < 64 ? ~0u : 0u;  // round 0: distance 0
     }
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
     if (ok && blockIdx.x == 0 && threadIdx.x < kWave) {
@@ -1007,73 +1181,116 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
             }
         }
         const bool lead = has && firstl == ln;
-        if (has) a.dist[(size_t)v * 64 + ln] = 0;
+        if (has) a.dist[((size_t)v << qbits) + ln] = 0;
         if (lead) a.F[v] = m;
         const uint64_t lm = ballot(lead);
         if (lead) a.ring[rank_in(lm)] = v;
         const uint32_t dv = lead ? g.row[v + 1] - g.row[v] : 0u;
         const unsigned long long sc = wave_sum_u64(dv);
         if (ln == 0) {
-            a.ctl[2] = (uint32_t)__popcll(lm);
+            a.ctr[0].qlen = (uint32_t)__popcll(lm);
             a.ctr[0].stripe[0].scout = sc;
             a.ctr[0].stripe[0].count = (unsigned long long)__popcll(lm);
         }
     }
     if (ok) ok = grid_sync(a.bar, xcc, gen, a.abort);
 
-    uint32_t r = 0, prev_len = 0;
+    uint32_t r = 0, prev_len = 0, pulls = 0;
+    unsigned long long ptrace = 0;
     while (ok) {
         read_counts(&a.ctr[r % 3], s_lvl);
-        if (threadIdx.x == 0) s_len = __hip_atomic_load(&a.ctl[2 + r % 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x == 0) s_qn = 0;
         __syncthreads();
-        const RoundCounts rc = unpack_counts(s_lvl, 0xFFFFFFFFu);
-        const uint32_t len = min(s_len, n);
+        const RoundCounts rc = unpack_counts(s_lvl, n);
+        const uint32_t len = rc.qlen;
         __syncthreads();
         if (rc.count == 0 || (a.max_rounds && r >= a.max_rounds)) break;
-        if (gtid == 0) {
-            a.ctl[2 + (r + 2) % 3] = 0;  // held round r-1, read by every block a round ago
-            write_trace(a.trace, r, false, rc.count, rc.scout, t_start);
+        const bool pull = a.force != 0 && qbits >= kMsPullBits && rc.scout * kMsPullRatio >= g.m;
+        pulls += pull;
+        if (pull && r < 64) ptrace |= 1ull << r;
+        if (gtid == 0) write_trace(a.trace, r, pull, rc.count, rc.scout, t_start);
+        if (blockIdx.x == 0) {
+            clear_ctr(&a.ctr[(r + 2) % 3]);
+            if (threadIdx.x < 64) a.cmin[(r + 2) % 3 * 64 + threadIdx.x] = 0;
         }
-        if (blockIdx.x == 0) clear_ctr(&a.ctr[(r + 2) % 3]);
+        if (threadIdx.x < 64) s_min[threadIdx.x] = 0xFFFFFFFFu;  // (a barrier of the round's end orders this)
         const uint64_t *Fc = a.F + (size_t)(r % 3) * n;
         uint64_t *Ff = a.F + (size_t)((r + 2) % 3) * n;
         const uint32_t *cur = a.ring + (size_t)(r % 3) * n;
         const uint32_t *old = a.ring + (size_t)((r + 2) % 3) * n;
         for (uint32_t i = gtid; i < prev_len; i += nthreads) Ff[old[i]] = 0;
 
-        MsRelax R{&a, a.F + (size_t)((r + 1) % 3) * n, a.ring + (size_t)((r + 1) % 3) * n, &a.ctl[2 + (r + 1) % 3],
-                  qbits, 0, 0};
+        // (a vertex enters a round's entries once, so n entries hold them all)
+        MsRelax R{&a, a.F + (size_t)((r + 1) % 3) * n,
+                  Stager{a.ring + (size_t)((r + 1) % 3) * n, n, &a.ctr[(r + 1) % 3], s_q, &s_qn, kLdsQ}, qbits, 0, 0, 0, 0xFFFFFFFFu};
+        const uint32_t q = (uint32_t)ln & ((1u << qbits) - 1);
+        R.fmin = ~__hip_atomic_load(&a.cmin[r % 3 * 64 + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (pull) ms_pull(R, Fc, a.nsrc, gwave, nwaves);
         // hubs through the static chunk list
-        for (uint32_t c = gwave; c < g.nhuge; c += nwaves) {
+        for (uint32_t c = gwave; !pull && c < g.nhuge; c += nwaves) {
             const uint2 dsc = g.huge[c];
             const uint64_t mk = Fc[dsc.x];
             if (mk) ms_relax_range(R, dsc.x, dsc.y, min(g.row[dsc.x + 1], dsc.y + kHugeChunk), mk);
         }
-        for (uint32_t i = gwave; i < len; i += nwaves) {
-            const uint32_t u = cur[i];
-            const uint32_t b = g.row[u], e = g.row[u + 1];
+        // (the entry after next, and the next one's edge range and mask, are
+        // read while this one is relaxed)
+        uint32_t i = pull ? len : gwave;
+        uint32_t u1 = i < len ? cur[i] : 0u, u2 = i + nwaves < len ? cur[i + nwaves] : 0u;
+        uint32_t b1 = g.row[u1], e1 = g.row[u1 + 1];
+        uint64_t m1 = Fc[u1];
+        for (; i < len; i += nwaves) {
+            const uint32_t u = u1, b = b1, e = e1;
+            const uint64_t mk = m1;
+            u1 = u2;
+            u2 = i + 2 * nwaves < len ? cur[i + 2 * nwaves] : 0u;
+            b1 = g.row[u1];
+            e1 = g.row[u1 + 1];
+            m1 = Fc[u1];
             if (e - b > kHugeDegree) continue;
-            ms_relax_range(R, u, b, e, Fc[u]);
+            ms_relax_range(R, u, b, e, mk);
         }
         publish_counts<WPB>(&a.ctr[(r + 1) % 3], R.scout, R.count, false, s_red);
+        if (R.minv != 0xFFFFFFFFu) atomicMin(&s_min[q], R.minv);
+        flush_stage(R.S, s_flush);
+        if (threadIdx.x < 64 && s_min[threadIdx.x] != 0xFFFFFFFFu)
+            atomicMax(&a.cmin[(r + 1) % 3 * 64 + threadIdx.x], ~s_min[threadIdx.x]);
         prev_len = len;
         r++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
-    // results, one contiguous row per query
+    // results, one contiguous row per query: tiles of 64 vertices go through
+    // the block's LDS, rows read and written whole (the caller's order is a
+    // permutation of rows here, and costs no pass of its own)
     if (ok) {
-        for (uint32_t v = gtid; v < n; v += nthreads) {
-            const uint32_t *row = a.dist + (size_t)v * 64;
-            for (uint32_t q = 0; q < a.nsrc; q++) a.out[out_row(a.orow, q, n) + v] = row[q];
+        static_assert(kLdsQ >= 64 * 9, "a tile of eight queries fits");
+        constexpr uint32_t kTileQ = kLdsQ / 64 - 1 < 64 ? kLdsQ / 64 - 1 : 64;  // queries a tile holds
+        const uint32_t qn = 1u << qbits;
+        for (uint32_t v0 = blockIdx.x * 64; v0 < n; v0 += gridDim.x * 64) {
+            for (uint32_t q0 = 0; q0 < a.nsrc; q0 += kTileQ) {
+                const uint32_t qc = min(kTileQ, a.nsrc - q0);
+                __syncthreads();
+                for (uint32_t i = threadIdx.x; i < 64 * qn; i += BS) {
+                    const uint32_t v = v0 + (i >> qbits), q = i & (qn - 1);
+                    if (v < n && q - q0 < qc)
+                        s_q[(q - q0) * 65 + (i >> qbits)] = a.dist[((size_t)(a.inv ? a.inv[v] : v) << qbits) + q];
+                }
+                __syncthreads();
+                for (uint32_t i = threadIdx.x; i < 64 * qc; i += BS) {
+                    const uint32_t v = v0 + (i & 63), q = i >> 6;
+                    if (v < n) a.out[out_row(a.orow, q0 + q, n) + v] = s_q[q * 65 + (i & 63)];
+                }
+            }
         }
     }
     if (gtid == 0) {
         DevStats s = *a.stats;
         s.rounds += r;
-        s.push_rounds += r;
+        s.push_rounds += r - pulls;
+        s.pull_rounds += pulls;
+        s.trace = ptrace;
         s.max_depth = max(s.max_depth, r);
         s.iterations += 1;
-        if (s.status == SG_OK) s.status = ok ? (a.ctl[1] ? SG_ERR_CAPACITY : SG_OK) : SG_ERR_TIMEOUT;
+        if (s.status == SG_OK) s.status = ok ? SG_OK : SG_ERR_TIMEOUT;
         *a.stats = s;
     }
 }
@@ -1111,7 +1328,7 @@ MsLayout ms_layout(int kind, uint64_t n)
         put(0, n * 64 * 4); // dist rows
         put(1, 3 * n * 8);  // F
         put(2, 3 * n * 4);  // ring
-        put(4, 256);        // ctl
+        put(4, 3 * 64 * 4); // cmin
     } else {
         const uint64_t cap = std::min<uint64_t>(n * 64 + 4096, 0xFFFFFFF0ull);
         put(0, n * 8);                             // seen
@@ -1175,7 +1392,7 @@ int ms_prepare(sg_engine *e, int kind)
 }
 
 int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, void *out, const uint32_t *dev_orow,
-              bool first, bool last)
+              bool first, bool last, const uint32_t *inv)
 {
     if (nsrc < 1 || nsrc > 64) SG_FAIL(SG_ERR_RANGE, "batched launch: 1..64 sources");
     const uint64_t n = e->g->dev.n;
@@ -1219,9 +1436,11 @@ int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, vo
         a.dist = (uint32_t *)(base + L.off[0]);
         a.F = (uint64_t *)(base + L.off[1]);
         a.ring = (uint32_t *)(base + L.off[2]);
-        a.ctl = (uint32_t *)(base + L.off[4]);
         a.out = (uint32_t *)out;
         a.orow = dev_orow;
+        a.inv = inv;
+        a.cmin = (uint32_t *)(base + L.off[4]);
+        a.force = force;
         a.max_rounds = (uint32_t)o.max_iteration;
         const void *fn = bs == 256 ? (const void *)k_mssssp<256> : bs == 512 ? (const void *)k_mssssp<512> : (const void *)k_mssssp<1024>;
         return launch_grid(e, fn, bs, a);
@@ -1283,7 +1502,14 @@ int ms_run(sg_engine *e, int kind, const uint32_t *sources, int32_t k, int32_t b
     const uint64_t n = d.n;
     const uint64_t rows = kind == kMsBcSum ? 1 : (uint64_t)k;
     void *res = nullptr;
-    if ((rc = engine_result_rows(e, rows, &res))) return rc;
+    // batched SSSP writes the caller's order itself
+    const bool direct = kind == kMsSssp;
+    if (direct) {
+        if ((rc = engine_ensure_value(e, rows * n * 4))) return rc;
+        res = e->value;
+    } else if ((rc = engine_result_rows(e, rows, &res))) {
+        return rc;
+    }
     if ((rc = engine_ensure_srcbuf(e, (uint64_t)k))) return rc;
     std::vector<uint32_t> dsrc(k);
     for (int32_t i = 0; i < k; i++) dsrc[i] = dev_vertex(e->g, sources[i]);
@@ -1309,11 +1535,12 @@ int ms_run(sg_engine *e, int kind, const uint32_t *sources, int32_t k, int32_t b
     for (int i = 0; i < nb; i++) {
         const uint32_t ns = (uint32_t)std::min(batch, k - i * batch);
         void *out = kind == kMsBcSum ? res : (void *)((uint32_t *)res + (size_t)i * batch * n);
-        rc = ms_launch(e, kind, e->srcbuf + (size_t)i * batch, ns, out, nullptr, i == 0, i == nb - 1);
+        rc = ms_launch(e, kind, e->srcbuf + (size_t)i * batch, ns, out, nullptr, i == 0, i == nb - 1,
+                       direct && e->g->relabeled ? e->g->d_inv : nullptr);
         if (rc) return rc;
     }
     SG_HIP(hipEventRecord(e->ev1, e->stream));
-    if ((rc = engine_finish(e, rows))) return rc;
+    if (!direct && (rc = engine_finish(e, rows))) return rc;
     e->timed = true;
     return SG_OK;
 }

@@ -187,3 +187,23 @@ def test_bfs_batches(sg, orc, gpu, name, k):
     e.bc(src)
     # FP64 sums, one rounding to FP32
     np.testing.assert_allclose(e.gather(np.float32), orc.bc(hg.row, hg.col, src), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opts", [{}, {"force_variant": "async_push_dd"}, {"block_size": 256}])
+@pytest.mark.parametrize("weights", [None, (0, 3), (1, 64), (1 << 30, 1 << 31)])
+@pytest.mark.parametrize("k", [1, 2, 7, 16, 24, 64, 70])
+@pytest.mark.parametrize("name", BATCH_GRAPHS)
+def test_sssp_batches(sg, orc, gpu, name, k, weights, opts):
+    if opts and (weights != (1, 64) or k not in (16, 64)):
+        pytest.skip("options: one weight range, two batch sizes")
+    hg = SMALL_ROUND_GRAPHS[name](sg)
+    if weights:
+        hg = weighted(sg, hg, *weights, seed=5)
+    w = hg.w if weights else np.ones(hg.m, np.uint32)
+    e = sg.Engine(sg.Graph(hg), **opts)
+    src = np.random.default_rng(k).integers(0, hg.n, k)
+    e.sssp_multi(src)
+    got = e.gather(np.uint32).reshape(k, hg.n)
+    for i in sorted({0, k - 1}):
+        assert np.array_equal(got[i], distances(orc, hg, w, int(src[i]), weights)), i
