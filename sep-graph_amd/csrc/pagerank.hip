@@ -11,23 +11,20 @@
 // The ranks computed here are the normalised PageRank with uniform teleport
 // and uniform redistribution of dangling mass,
 //     x = (1-d)/n + d (P^T x + (sum of x over dangling vertices)/n),
-// stored as FP32. Sums are compensated FP32 (hi + lo, Neumaier): in the pull
-// mode the per-vertex in-edge sums and the dangling mass, in the residual
-// mode the unnormalised ranks, the residuals (each atomic addition's
-// rounding error, recomputed by the adding lane, goes to a second FP32
-// array) and the normalising sum; only the L1 residual (pull) and the
-// residual mass absorbed at the end (DD) are reduced in FP64. In the pull
-// mode every reduction runs in a fixed order for a given grid, so repeated
-// runs give identical bits.
+// stored as FP32. In the pull mode every sum (in-edges, dangling mass, L1
+// residual) is FP64, in a fixed order for a given grid, so repeated runs give
+// identical bits. In the residual mode the unnormalised ranks, the residuals
+// (each atomic addition's rounding error, recomputed by the adding lane, goes
+// to a second FP32 array) and the normalising sum are compensated FP32 (hi +
+// lo, Neumaier); the residual mass absorbed at the end is reduced in FP64.
 //
 // Pull TD: one lane per vertex sums x[u]/outdeg(u) (kept as an FP32 array
 // `contrib`, ping-ponged between iterations) over its in-edges, reading them
 // row by row from the graph's sliced in-edge layout (a lane's own entries,
 // in order; without that layout, the wave walks the concatenated in-edge
-// lists 64 edges per step with a segmented shuffle scan). Vertices with
-// in-degree above kPullHubDegree are summed per 256-edge chunk into
-// compensated slots and finished after a grid barrier, one wave per hub, in
-// chunk order.
+// lists 64 edges per step with a segmented scan). Vertices with in-degree
+// above kPullHubDegree are summed per 256-edge chunk; a hub of one chunk is
+// finished with it, the others after a grid barrier, eight lanes per hub.
 //
 // Residual DD: solves the unnormalised system y = (1-d)/n + d P^T y by
 // residual propagation (dangling mass leaks) and normalises y at the end; for
@@ -179,12 +176,49 @@ __device__ __forceinline__ CSum wave_gather_csum(uint32_t b, uint32_t e, F val)
 
 // ------------------------------------------------------------ pull TD kernel
 
+// Lanes of one row of 16 take each other's sums (every lane has the total).
+__device__ __forceinline__ double row_sum(double x)
+{
+    x += dpp<kDppRowRor + 8>(0.0, x);
+    x += dpp<kDppRowRor + 4>(0.0, x);
+    x += dpp<kDppRowRor + 2>(0.0, x);
+    x += dpp<kDppRowRor + 1>(0.0, x);
+    return x;
+}
+
+// (FP64 adds run at the rate of FP32 ones here: a conversion and an add per
+// in-edge where a compensated FP32 sum takes eight instructions.)
+// Four wave sums together: lane l gets that of s[l % 4]. Halves of the wave,
+// then rows of 16 lanes, trade places between two sums, so that three
+// additions leave one sum per row, where four scans would take 24.
+__device__ __forceinline__ double wave_sum4(const double (&s)[4])
+{
+    auto fold = [](double a, double b, bool half) {
+        uint32_t x[2], y[2];
+        __builtin_memcpy(x, &a, 8);
+        __builtin_memcpy(y, &b, 8);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const auto r = half ? __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false)
+                                : __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+            x[i] = r[0];
+            y[i] = r[1];
+        }
+        __builtin_memcpy(&a, x, 8);
+        __builtin_memcpy(&b, y, 8);
+        return a + b;
+    };
+    // rows of (0, 2): 0 0 2 2; of (1, 3): 1 1 3 3; of both: 0 1 2 3
+    const double t = row_sum(fold(fold(s[0], s[2], true), fold(s[1], s[3], true), false));
+    return shfl(t, (lane() & 3) * 16);
+}
+
 struct PrArgs {
     DevGraph g;
     float *x;          // ranks [n]
-    float *contrib;    // 2 x n: x[u] / outdeg(u) of the current / next iteration
-    CSum *hubpart;     // [nhugein] chunk sums
-    PrPart *part;      // 2 x kMaxBlocks (residual, dangling) partials
+    float *contrib;    // 2 rows: x[u] / outdeg(u) of the current / next iteration
+    double *hubpart;   // [nhugein] chunk sums
+    double2 *part;     // 2 x kMaxBlocks (residual, dangling) partials
     GridBarrier bar;
     uint32_t *abort;
     DevStats *stats;
@@ -194,6 +228,17 @@ struct PrArgs {
     uint32_t probe;
 };
 
+// Floats from one row of contributions to the next: 16-byte aligned rows.
+__host__ __device__ constexpr uint64_t contrib_stride(uint32_t n) { return ((uint64_t)n + 3) / 4 * 4; }
+
+// What bounds an iteration: the in-edges whose source has no place in LDS,
+// each an L2 request for a line of which it needs 4 bytes. RMAT-21 (32.4 M
+// edges, 36 % of them such), 17 iterations: 1800 us, of which 1030 are these
+// reads (11.7 M an iteration at 0.19 T/s; the L2s answer 0.27 T/s at most),
+// 210 the barriers, partial sums and LDS copy, the rest index reads, LDS reads
+// and the vertices' own data. It took 2640 us when each in-edge's LDS or L2 read
+// waited for the one before it, the chunks' bounds were read group by group,
+// and every hub, also one of a single chunk, took a wave after the barrier.
 template <int BS>
 __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
 {
@@ -202,6 +247,7 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         return;
     }
     constexpr int WPB = BS / kWave;
+    constexpr uint32_t kPad = 0xFFFFFFFFu;  // no in-edge
     const DevGraph &g = a.g;
     const uint32_t n = g.n, W = g.words;
     const uint32_t gtid = blockIdx.x * BS + threadIdx.x;
@@ -214,42 +260,72 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
     const long long t_start = wall_clock64();
     const float df = (float)a.damping;
     const float inv_nf = (float)(1.0 / (double)n);
+    const uint64_t stride = contrib_stride(n);
 
-    __shared__ PrPart s_red[WPB];
-    __shared__ PrPart s_glob;
+    __shared__ double2 s_red[WPB];
     // The lowest ids' contributions (in a degree-ordered graph the sources of
     // most in-edges) are copied to LDS each iteration: they are read-only
     // until the next barrier, and the gather reads them there instead of
-    // sending one L2 request per in-edge.
+    // sending one L2 request per in-edge. As many as fit beside the rest: with
+    // 32 per thread RMAT-21 takes 1848 us, with 39 1803.
 #ifndef SG_PR_LDS
-#define SG_PR_LDS 32
+#define SG_PR_LDS 39
 #endif
     constexpr uint32_t kCcLds = SG_PR_LDS * BS;
-    __shared__ float s_cc[kCcLds];
+    __shared__ __align__(16) float s_cc[kCcLds + 4];  // [kCcLds]: 0, read for every other entry
+
+    // the block's (residual, dangling) partials, in a fixed order
+    auto put_part = [&](uint32_t it, double res, double dang) {
+        res = wave_sum_f64(res);
+        dang = wave_sum_f64(dang);
+        if (ln == 0) s_red[threadIdx.x / kWave] = make_double2(res, dang);
+        __syncthreads();
+        if (threadIdx.x < kWave) {
+            const double2 t = ln < WPB ? s_red[ln] : make_double2(0.0, 0.0);
+            res = wave_sum_f64(t.x);
+            dang = wave_sum_f64(t.y);
+            if (ln == 0) a.part[(size_t)(it & 1) * kMaxBlocks + blockIdx.x] = make_double2(res, dang);
+        }
+    };
 
     // x = 1/n; contributions of iteration 0; dangling mass
-    CSum dang{0.f, 0.f};
+    double dang = 0.0;
     for (uint32_t v = gtid; v < n; v += nthreads) {
         a.x[v] = inv_nf;
         const uint32_t dout = g.row[v + 1] - g.row[v];
         a.contrib[v] = dout ? inv_nf / (float)dout : 0.0f;
-        if (!dout) csum_add(dang, inv_nf);
+        if (!dout) dang += (double)inv_nf;
     }
-    {
-        const PrPart t = block_part<WPB>(0.0, dang, s_red);
-        if (threadIdx.x == 0) a.part[blockIdx.x] = t;
-    }
+    if (threadIdx.x == 0) s_cc[kCcLds] = 0.f;
+    put_part(0, 0.0, dang);
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
 
     uint32_t it = 0;
     double res = INFINITY;
     while (ok) {
-        const PrPart gs = grid_part<BS>(a.part + (size_t)(it & 1) * kMaxBlocks, gridDim.x, s_red, &s_glob);
-        if (it > 0) res = gs.res;
+        const float *cc = a.contrib + (size_t)(it & 1) * stride;
+        float *cn = a.contrib + (size_t)((it + 1) & 1) * stride;
+        // the LDS copy's loads are in flight while the partials are added
+        const uint32_t ncc = min(n, kCcLds);
+        constexpr int kFill = (int)((kCcLds / 4 + BS - 1) / BS);
+        float4 fill[kFill];
+#pragma unroll
+        for (int i = 0; i < kFill; i++) {
+            fill[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (4 * threadIdx.x < ncc - min(ncc, (uint32_t)(4 * i * BS))) fill[i] = ((const float4 *)cc + i * BS)[threadIdx.x];
+        }
+        // every wave adds the blocks' partials by itself: no wait for others
+        double2 gs = make_double2(0.0, 0.0);
+        for (uint32_t i = ln; i < gridDim.x; i += kWave) {
+            const double2 q = a.part[(size_t)(it & 1) * kMaxBlocks + i];
+            gs.x += q.x;
+            gs.y += q.y;
+        }
+        gs.x = wave_sum_f64(gs.x);
+        gs.y = wave_sum_f64(gs.y);
+        if (it > 0) res = gs.x;
         if ((it > 0 && res < a.tol) || it >= a.max_iter) break;
-        const float base = (1.0f - df) * inv_nf + df * csum_value(CSum{gs.dhi, gs.dlo}) * inv_nf;
-        const float *cc = a.contrib + (size_t)(it & 1) * n;
-        float *cn = a.contrib + (size_t)((it + 1) & 1) * n;
+        const float base = (1.0f - df) * inv_nf + df * (float)gs.y * inv_nf;
         if (gtid == 0 && it < kTraceRows) {
             DevTrace t;
             t.round = it;
@@ -260,111 +336,230 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
             t.ticks = (unsigned long long)(wall_clock64() - t_start);
             a.trace[it] = t;
         }
-        const uint32_t ncc = min(n, kCcLds);
-        for (uint32_t i = threadIdx.x; i < ncc; i += BS) s_cc[i] = cc[i];
+#pragma unroll
+        for (int i = 0; i < kFill; i++) {
+            if (4 * threadIdx.x < ncc - min(ncc, (uint32_t)(4 * i * BS))) ((float4 *)s_cc + i * BS)[threadIdx.x] = fill[i];
+        }
         __syncthreads();
-        auto contrib = [&](uint32_t u) -> float { return u < ncc ? s_cc[u] : cc[u]; };
-        double r_acc = 0.0;
-        CSum d_acc{0.f, 0.f};
-        // x(v) from its in-edge sum: FP32 ranks and contributions, the
-        // residual |x' - x| summed in FP64
-        auto finish = [&](uint32_t v, const CSum &s) {
-            const float xn = base + df * csum_value(s);
-            r_acc += fabs((double)xn - (double)a.x[v]);
-            a.x[v] = xn;
-            const uint32_t dout = g.row[v + 1] - g.row[v];
-            if (dout) cn[v] = xn / (float)dout;
-            else csum_add(d_acc, xn);
-        };
-        // (A1) chunk sums of the in-hubs, kQ chunks per wave together: every
-        // in-edge load of the kQ chunks is issued before any contribution is
-        // gathered, and every gather before any is added (each lane still
-        // adds its edges of a chunk in edge order, so the sums are the same)
-        constexpr int kQ = 4, kSteps = (int)(kPullChunk / kWave);
-        for (uint32_t c0 = gwave * kQ; c0 < g.nhugein; c0 += nwaves * kQ) {
-            uint32_t cb[kQ], ce[kQ];
+        // contributions of N sources: the loads of those outside LDS are all
+        // issued first, then every entry reads LDS (the zero, if it has no
+        // place there), so no entry waits for the one before it
+        const uint32_t ncold = n > kCcLds ? n - kCcLds : 0u;
+        auto gather = [&](const uint32_t *u, float *c, auto N) {
 #pragma unroll
-            for (int q = 0; q < kQ; q++) {
-                cb[q] = ce[q] = 0;
-                if (c0 + q < g.nhugein) {
-                    const uint2 dsc = g.hugein[c0 + q];
-                    cb[q] = dsc.y;
-                    ce[q] = min(g.cstart[dsc.x + 1], dsc.y + kPullChunk);
-                }
+            for (int q = 0; q < N.value; q++) {
+                c[q] = 0.f;
+                if (u[q] - kCcLds < ncold) c[q] = cc[u[q]];
             }
-            uint32_t u[kQ][kSteps];
 #pragma unroll
-            for (int q = 0; q < kQ; q++)
+            for (int q = 0; q < N.value; q++) c[q] += s_cc[min(u[q], kCcLds)];
+        };
+        double r_acc = 0.0, d_acc = 0.0;
+        // x(v) from its in-edge sum, its last rank and its out-degree: FP32
+        // ranks and contributions, sums and the residual |x' - x| in FP64
+        auto finish = [&](uint32_t v, double s, float xo, uint32_t dout) {
+            const float xn = base + df * (float)s;
+            r_acc += fabs((double)xn - (double)xo);
+            a.x[v] = xn;
+            if (dout) cn[v] = xn / (float)dout;
+            else d_acc += (double)xn;
+        };
+        // (A1) chunk sums of the in-hubs, dealt out one by one. A lane holds
+        // one chunk's bounds and, in the end, its sum; the wave adds kQ
+        // chunks together, the next kQ chunks' in-edges in flight meanwhile.
+        // A hub of one chunk is finished here.
+        constexpr int kQ = 4, kSteps = (int)(kPullChunk / kWave);
+        for (uint32_t first = gwave; first < g.nhugein; first += nwaves * kWave) {
+            const uint32_t cnt = min((uint32_t)kWave, (g.nhugein - first + nwaves - 1) / nwaves);
+            const uint32_t c = first + (uint32_t)ln * nwaves;
+            uint32_t hv = 0, beg = 0, len = 0, dout = 0;
+            float xo = 0.f;
+            bool one = false;
+            if ((uint32_t)ln < cnt) {
+                const uint2 dsc = g.hugein[c];
+                hv = dsc.x;
+                beg = dsc.y;
+                const uint32_t b = g.cstart[hv], e = g.cstart[hv + 1];
+                len = min(e - beg, kPullChunk);
+                one = e - b <= kPullChunk;
+                dout = g.row[hv + 1] - g.row[hv];
+                xo = a.x[hv];
+            }
+            auto load = [&](uint32_t j, uint32_t *u) {
 #pragma unroll
-                for (int t = 0; t < kSteps; t++) {
-                    const uint32_t e = cb[q] + (uint32_t)(t * kWave + ln);
-                    u[q][t] = e < ce[q] ? g.csrc[e] : 0xFFFFFFFFu;
+                for (int q = 0; q < kQ; q++) {
+                    const uint32_t l = lane_value(len, (int)j + q);
+                    const uint32_t *src = g.csrc + lane_value(beg, (int)j + q);
+#pragma unroll
+                    for (int t = 0; t < kSteps; t++) {
+                        const uint32_t k = (uint32_t)(t * kWave + ln);
+                        u[q * kSteps + t] = k < l ? src[k] : kPad;
+                    }
                 }
-            float cv[kQ][kSteps];
+            };
+            double mine = 0.0;
+            uint32_t u[kQ * kSteps], nu[kQ * kSteps];
+            load(0, u);
+            for (uint32_t j = 0; j < cnt; j += kQ) {
+                if (j + kQ < cnt) load(j + kQ, nu);
+                float cv[kQ * kSteps];
+                gather(u, cv, std::integral_constant<int, kQ * kSteps>{});
+                double s[kQ];
 #pragma unroll
-            for (int q = 0; q < kQ; q++)
+                for (int q = 0; q < kQ; q++) {
+                    s[q] = 0.0;
 #pragma unroll
-                for (int t = 0; t < kSteps; t++) cv[q][t] = u[q][t] != 0xFFFFFFFFu ? contrib(u[q][t]) : 0.f;
+                    for (int t = 0; t < kSteps; t++) s[q] += (double)cv[q * kSteps + t];
+                }
+                const double t = wave_sum4(s);
+                if ((uint32_t)ln / kQ == j / kQ) mine = t;
 #pragma unroll
-            for (int q = 0; q < kQ; q++) {
-                if (c0 + q >= g.nhugein) break;  // wave-uniform
-                CSum s{0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < kSteps; t++)
-                    if (u[q][t] != 0xFFFFFFFFu) csum_add(s, cv[q][t]);
-                s = wave_csum(s);
-                if (ln == 0) a.hubpart[c0 + q] = s;
+                for (int q = 0; q < kQ * kSteps; q++) u[q] = nu[q];
+            }
+            if ((uint32_t)ln < cnt) {
+                if (one) finish(hv, mine, xo, dout);
+                else a.hubpart[c] = mine;
             }
         }
+        // in-hubs of several chunks wait for every block's sums: arrive now,
+        // wait once the other vertices are done
+        grid_signal(a.bar, xcc, gen, a.abort);
         // (A2) every other vertex, a 64-vertex word per wave at a time: from
         // the sliced in-edges (each lane sums its own vertex's row entries in
         // order) or, without them, by a scheduled walk of the word's lists
-        for (uint32_t w = gwave; w < W; w += nwaves) {
-            const uint32_t v = w * 64 + ln;
-            uint32_t b = 0, e = 0;
-            bool own = false;
-            if (v < n) {
-                b = g.cstart[v];
-                e = g.cstart[v + 1];
-                own = e - b <= kPullHubDegree;
-                if (!own) b = e;
-            }
-            CSum s{0.f, 0.f};
-            if (g.sell_src) {
-                const uint32_t beg = g.sell_off[w];
-                const uint32_t rows = (g.sell_off[w + 1] - beg) / kWave;
-                const uint32_t *S = g.sell_src + beg + ln;
-                constexpr int U = 4;
-                for (uint32_t j0 = 0; j0 < rows; j0 += U) {
-                    uint32_t u[U];
-#pragma unroll
-                    for (int q = 0; q < U; q++) u[q] = (own && j0 + q < rows) ? S[(size_t)(j0 + q) * kWave] : 0xFFFFFFFFu;
-                    float c[U];
-#pragma unroll
-                    for (int q = 0; q < U; q++) c[q] = u[q] != 0xFFFFFFFFu ? contrib(u[q]) : 0.f;
-#pragma unroll
-                    for (int q = 0; q < U; q++)
-                        if (u[q] != 0xFFFFFFFFu) csum_add(s, c[q]);
+        if (g.sell_src) {
+            constexpr uint32_t U = 4;
+            for (uint32_t first = gwave; first < W; first += nwaves * kWave) {
+                const uint32_t cnt = min((uint32_t)kWave, (W - first + nwaves - 1) / nwaves);
+                // a lane holds one word's rows; what a word's vertices need in
+                // the end is loaded one word ahead, its in-edges one step ahead
+                uint32_t off = 0, nrow = 0;
+                if ((uint32_t)ln < cnt) {
+                    const uint32_t w = first + (uint32_t)ln * nwaves;
+                    off = g.sell_off[w];
+                    nrow = (g.sell_off[w + 1] - off) / kWave;
                 }
-            } else {
-                s = wave_gather_csum(b, e, [&](uint32_t ed) { return contrib(g.csrc[ed]); });
+                struct Own {
+                    uint32_t dout, din;
+                    float xo;
+                };
+                auto load_own = [&](uint32_t i) {
+                    Own o{0u, kPad, 0.f};
+                    const uint32_t v = (first + i * nwaves) * kWave + ln;
+                    if (v < n) {
+                        o.dout = g.row[v + 1] - g.row[v];
+                        o.din = g.cstart[v + 1] - g.cstart[v];
+                        o.xo = a.x[v];
+                    }
+                    return o;
+                };
+                auto load = [&](uint32_t i, uint32_t j, uint32_t *u) {
+                    const uint32_t rows = lane_value(nrow, (int)i);
+                    const uint32_t *S = g.sell_src + lane_value(off, (int)i) + ln;
+#pragma unroll
+                    for (uint32_t q = 0; q < U; q++) {
+                        u[q] = kPad;
+                        if (j + q < rows) u[q] = S[(size_t)(j + q) * kWave];
+                    }
+                };
+                uint32_t i = 0, j = 0, u[U], nu[U];
+                Own own = load_own(0), next = own;
+                load(0, 0, u);
+                double s = 0.0;
+                while (i < cnt) {
+                    if (j == 0 && i + 1 < cnt) next = load_own(i + 1);
+                    const uint32_t rows = lane_value(nrow, (int)i);
+                    const bool last = j + U >= rows;
+                    const uint32_t ni = last ? i + 1 : i, nj = last ? 0u : j + U;
+                    if (ni < cnt) load(ni, nj, nu);
+                    if (rows) {
+                        float cv[U];
+                        gather(u, cv, std::integral_constant<int, (int)U>{});
+#pragma unroll
+                        for (uint32_t q = 0; q < U; q++) s += (double)cv[q];
+                    }
+                    if (last) {
+                        if (own.din <= kPullHubDegree) finish((first + i * nwaves) * kWave + ln, s, own.xo, own.dout);
+                        s = 0.0;
+                        own = next;
+                    }
+#pragma unroll
+                    for (uint32_t q = 0; q < U; q++) u[q] = nu[q];
+                    i = ni;
+                    j = nj;
+                }
             }
-            if (own) finish(v, s);
+        } else {
+            for (uint32_t w = gwave; w < W; w += nwaves) {
+                const uint32_t v = w * kWave + ln;
+                uint32_t b = 0, e = 0;
+                bool own = false;
+                if (v < n) {
+                    b = g.cstart[v];
+                    e = g.cstart[v + 1];
+                    own = e - b <= kPullHubDegree;
+                    if (!own) b = e;
+                }
+                const CSum s = wave_gather_csum(b, e, [&](uint32_t ed) {
+                    const uint32_t u = g.csrc[ed];
+                    return u < ncc ? s_cc[u] : cc[u];
+                });
+                if (own) finish(v, (double)s.hi + (double)s.lo, a.x[v], g.row[v + 1] - g.row[v]);
+            }
         }
-        ok = grid_sync(a.bar, xcc, gen, a.abort);
+        // (B) in-hubs of several chunks, eight lanes each (those of more than
+        // kHubWave chunks: the whole wave), dealt out so that the largest,
+        // which come first, fall to different waves; the first ones' data is
+        // loaded before the wait
+        constexpr uint32_t kHubLanes = 8, kHubs = kWave / kHubLanes, kHubWave = 8 * kHubLanes;
+        struct Hub {
+            uint32_t at, chunks, v, dout;
+            float xo;
+        };
+        auto load_hub = [&](uint32_t h0) {
+            Hub b{0u, 0u, 0u, 0u, 0.f};
+            const uint32_t h = h0 + (uint32_t)ln / kHubLanes * nwaves;
+            if (h < g.nhubin) {
+                const uint2 d = g.hubin[h];
+                b.at = d.x;
+                b.chunks = d.y;
+                if (d.y > 1) {
+                    b.v = g.hugein[d.x].x;
+                    b.dout = g.row[b.v + 1] - g.row[b.v];
+                    b.xo = a.x[b.v];
+                }
+            }
+            return b;
+        };
+        uint32_t h0 = gwave;
+        Hub hb = load_hub(h0);
+        ok = grid_wait(a.bar, gen, a.abort);
         if (!ok) break;
-        // (B) in-hubs: chunk sums in chunk order, one wave per hub
-        for (uint32_t h = gwave; h < g.nhubin; h += nwaves) {
-            const uint2 hb = g.hubin[h];
-            CSum s{0.f, 0.f};
-            for (uint32_t i = ln; i < hb.y; i += kWave) s = csum_merge(s, a.hubpart[hb.x + i]);
-            s = wave_csum(s);
-            if (ln == 0) finish(g.hugein[hb.x].x, s);
+        while (h0 < g.nhubin) {
+            const Hub cur = hb;
+            h0 += nwaves * kHubs;
+            if (h0 < g.nhubin) hb = load_hub(h0);
+            double s = 0.0;
+            if (cur.chunks > 1 && cur.chunks <= kHubWave) {
+#pragma unroll 8
+                for (uint32_t k = (uint32_t)ln % kHubLanes; k < cur.chunks; k += kHubLanes) s += a.hubpart[cur.at + k];
+            }
+            s += dpp<kDppQuad1>(0.0, s);
+            s += dpp<kDppQuad2>(0.0, s);
+            s += dpp<kDppHalfMirror>(0.0, s);
+            uint64_t wide = ballot(cur.chunks > kHubWave);
+            while (wide) {
+                const int l = first_lane(wide);
+                const uint32_t at = lane_value(cur.at, l), chunks = lane_value(cur.chunks, l);
+                double t = 0.0;
+                for (uint32_t k = ln; k < chunks; k += kWave) t += a.hubpart[at + k];
+                t = wave_sum_f64(t);
+                if (ln / (int)kHubLanes == l / (int)kHubLanes) s = t;
+                wide &= ~(0xFFull << l);
+            }
+            if (ln % (int)kHubLanes == 0 && cur.chunks > 1) finish(cur.v, s, cur.xo, cur.dout);
         }
-        {
-            const PrPart t = block_part<WPB>(r_acc, d_acc, s_red);
-            if (threadIdx.x == 0) a.part[(size_t)((it + 1) & 1) * kMaxBlocks + blockIdx.x] = t;
-        }
+        put_part(it + 1, r_acc, d_acc);
         it++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
@@ -1009,8 +1204,8 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
     e->last_algo = 2;
     const uint64_t part_bytes = 2ull * kMaxBlocks * sizeof(double2);
     if (mode == SG_PR_PULL_TD) {
-        // contrib (2n floats) | hubpart | partials
-        const uint64_t off_hub = (2 * n * 4 + 15) / 16 * 16;
+        // contrib (two rows, 16-byte aligned) | hubpart | partials
+        const uint64_t off_hub = 2ull * contrib_stride(d.n) * 4;
         const uint64_t off_part = off_hub + ((uint64_t)d.nhugein * 8 + 15) / 16 * 16;
         if ((rc = engine_ensure_aux(e, off_part + part_bytes))) return rc;
         char *base = (char *)e->aux;
@@ -1018,8 +1213,8 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
         a.g = d;
         a.x = (float *)res;
         a.contrib = (float *)base;
-        a.hubpart = (CSum *)(base + off_hub);
-        a.part = (PrPart *)(base + off_part);
+        a.hubpart = (double *)(base + off_hub);
+        a.part = (double2 *)(base + off_part);
         a.bar.spin_limit = 1u << 22;
         a.abort = e->abort_flag;
         a.stats = e->stats;

@@ -50,9 +50,13 @@ __device__ __forceinline__ T lane_value(T v, int l)
 
 // Data-parallel-primitive controls: a move across lanes inside a vector
 // instruction (a few clocks) where a shuffle goes through LDS (~60 clocks).
+constexpr int kDppQuad1 = 0xB1;        // lanes of a pair trade places
+constexpr int kDppQuad2 = 0x4E;        // pairs of a quad trade places
 constexpr int kDppRowShr = 0x110;      // + k: lane i of a row of 16 takes lane i - k
+constexpr int kDppRowRor = 0x120;      // + k: the same, from the row's end on
 constexpr int kDppWaveShl1 = 0x130;    // lane i takes lane i + 1
 constexpr int kDppWaveShr1 = 0x138;    // lane i takes lane i - 1
+constexpr int kDppHalfMirror = 0x141;  // lane i of 8 takes lane 7 - i
 constexpr int kDppRowBcast15 = 0x142;  // a row takes the last lane of the row before it
 constexpr int kDppRowBcast31 = 0x143;  // rows 2 and 3 take lane 31
 
@@ -217,6 +221,7 @@ struct BarState {
     uint32_t nxcd;  // XCDs holding at least one block of the grid
     uint32_t rank;  // this block's arrival order among its XCD's blocks
     uint32_t first; // lowest XCD holding blocks of the grid (the team's)
+    uint32_t ok;    // what grid_signal found
 };
 
 __device__ __forceinline__ uint32_t xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | 20) & 15; }
@@ -276,7 +281,7 @@ __device__ __forceinline__ bool spin_wait(const uint32_t *p, uint32_t v, bool wa
 template <bool kTeam = false>
 __device__ __forceinline__ BarState bar_begin(const GridBarrier &gb, uint32_t xcc)
 {
-    BarState s{0u, 0u, 0u, 0u, 0u};
+    BarState s{0u, 0u, 0u, 0u, 0u, 0u};
     if (kTeam && blockIdx.x == 0 && threadIdx.x < 4 * kTeamMax)
         ((uint64_t *)(gb.words + bar_slots((int)(gb.rset & 1u) ^ 1)))[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
@@ -389,33 +394,49 @@ __device__ __forceinline__ uint32_t grid_arrive(const GridBarrier &gb, uint32_t 
     return gen0;
 }
 
-// Returns false if the wait timed out or another block aborted; the caller
-// must then leave its loop. `st` is this block's state from bar_begin (only
-// thread 0's copy is used): the first barrier of a launch takes the census,
-// and each barrier advances the generation.
+// The first half of grid_sync: what this block stored before it is there for
+// every block that has returned from the grid_wait that follows. Work between
+// the two hides the wait for the other blocks.
 template <bool kStamp = false>
-__device__ __forceinline__ bool grid_sync(const GridBarrier &gb, uint32_t xcc, BarState &st, uint32_t *abort)
+__device__ __forceinline__ void grid_signal(const GridBarrier &gb, uint32_t xcc, BarState &st, uint32_t *abort)
 {
-    __shared__ uint32_t s_ok;
     // __syncthreads() alone only waits for LDS traffic: every wave must first
     // drain its outstanding global stores/atomics (vmcnt) so they are in the
     // XCD's L2 before the leader writes that L2 back.
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t ok = st.cnt != 0u || bar_census(gb, xcc, st, abort);
-        if (ok) {
-            const uint32_t gen0 = grid_arrive<kStamp>(gb, xcc, st);
-            // every block polls the generation word itself (a relay through a
-            // per-XCD flag costs one more store/poll hop on the critical path)
-            ok = spin_wait(gb.words + kBarGen, gen0, true, gb.spin_limit, abort);
-        }
+        st.ok = st.cnt != 0u || bar_census(gb, xcc, st, abort);
+        if (st.ok) grid_arrive<kStamp>(gb, xcc, st);
+    }
+}
+
+// Returns false if the wait timed out or another block aborted; the caller
+// must then leave its loop.
+__device__ __forceinline__ bool grid_wait(const GridBarrier &gb, BarState &st, uint32_t *abort)
+{
+    __shared__ uint32_t s_ok;
+    if (threadIdx.x == 0) {
+        // every block polls the generation word itself (a relay through a
+        // per-XCD flag costs one more store/poll hop on the critical path)
+        uint32_t ok = st.ok;
+        if (ok) ok = spin_wait(gb.words + kBarGen, st.gen - 1, true, gb.spin_limit, abort);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         __builtin_amdgcn_s_waitcnt(0);
         s_ok = ok;
     }
     __syncthreads();
     return s_ok != 0;
+}
+
+// `st` is this block's state from bar_begin (only thread 0's copy is used):
+// the first barrier of a launch takes the census, and each barrier advances
+// the generation.
+template <bool kStamp = false>
+__device__ __forceinline__ bool grid_sync(const GridBarrier &gb, uint32_t xcc, BarState &st, uint32_t *abort)
+{
+    grid_signal<kStamp>(gb, xcc, st, abort);
+    return grid_wait(gb, st, abort);
 }
 
 // Wall clock recorded by the last stamped barrier (read after it).

@@ -38,6 +38,27 @@ def test_pagerank_in_degree_edges(sg, orc, gpu, degrees, mode):
     assert np.abs(got - ref).sum() / ref.sum() < 1e-6
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("block_size,n", [(256, 9983), (256, 9985), (512, 19969), (1024, 39935), (1024, 39937), (1024, 45001)])
+def test_pagerank_pull_staged_ids_and_hub_chunks(sg, orc, gpu, block_size, n, relabel):
+    """Ids around the last one whose contribution is staged, in-hubs of one
+    chunk, of several, and of more than eight lanes add up."""
+    rng = np.random.default_rng(n)
+    hubs = [d for d in (65, 256, 257, 2048, 2049, 16384, 16385, 30000) if d < n]
+    src = np.concatenate([rng.choice(n, d, replace=False) for d in hubs] + [rng.integers(0, n, 4 * n), np.arange(n)])
+    dst = np.concatenate([np.full(d, i * 7) for i, d in enumerate(hubs)] + [rng.integers(0, n, 4 * n), (np.arange(n) * 5 + 1) % n])
+    row, col = sg.build_csr(n, src.astype(np.uint32), dst.astype(np.uint32))
+    hg = sg.HostGraph(n, row, col, None)
+    e = sg.Engine(sg.Graph(hg, relabel=relabel), block_size=block_size)
+    e.pagerank(0.85, 1e-10, 0, sg.PR_PULL_TD)
+    got = e.gather(np.float32).astype(np.float64)
+    ref = orc.pagerank(hg.row, hg.col, 0.85, 1e-12)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    # three FP32 roundings per rank and iteration, carried on by 1 / (1 - d)
+    assert np.abs(got - ref).sum() / ref.sum() < 3 * 2.0**-24 / 0.15
+
+
 def path_graph(sg, n):
     v = np.arange(n - 1, dtype=np.uint32)
     row, col = sg.build_csr(n, v, v + 1, symmetrize=True)
