@@ -46,6 +46,7 @@ __global__ __launch_bounds__(BS) void k_bc1(Bc1KArgs a)
     BarState gen = bar_begin<kTeam>(a.b.f.bar, xcc);
     bc1_run<BS, kTeam>(a.b, blockIdx.x, gridDim.x, xcc, gen);
     if (blockIdx.x == 0 && threadIdx.x == 0) fold_stats(a);
+    bar_end(a.b.f.bar);
 }
 
 // A query on a graph that one XCD's blocks run whole (bc1_whole).
@@ -61,6 +62,7 @@ __global__ __launch_bounds__(BS) void k_bc1_whole(Bc1KArgs a)
     bool lead;
     bc1_whole<BS>(a.b, xcc, gen, lead);
     if (lead) fold_stats(a);
+    bar_end(a.b.f.bar);
 }
 
 template <int BS>

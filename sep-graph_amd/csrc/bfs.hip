@@ -17,6 +17,7 @@ __global__ SG_BFS_BOUNDS(BS) void k_bfs(BfsArgs a)
     const uint32_t xcc = xcc_id();
     BarState gen = bar_begin<!kStage>(a.bar, xcc);
     bfs_run<BS, kStage, !kStage, !kStage>(a, blockIdx.x, gridDim.x, xcc, gen);
+    bar_end(a.bar);
 }
 
 
@@ -33,10 +34,11 @@ __global__ SG_BFS_BOUNDS(BS) void k_bfs_whole(BfsArgs a)
     const uint32_t xcc = xcc_id();
     BarState gen = bar_begin<true>(a.bar, xcc);
     bfs_whole<BS>(a, s_t, xcc, gen, members, rank, tag);
+    bar_end(a.bar);
 }
 
 template <int BS, bool kStage>
-int launch_bfs(sg_engine *e, BfsArgs &args, bool timed)
+int launch_bfs(sg_engine *e, BfsArgs &args)
 {
     void (*kernel)(BfsArgs) = k_bfs<BS, kStage>;
     int most = 0;
@@ -57,11 +59,9 @@ int launch_bfs(sg_engine *e, BfsArgs &args, bool timed)
     if (rc) return rc;
     bind_barrier(pg, args.bar);
     return engine_launch_persistent(e, [&]() -> int {
-        if (timed) SG_HIP(hipEventRecord(e->ev0, e->stream));
         hipLaunchKernelGGL(kernel, dim3(pg->blocks), dim3(BS), 0, e->stream, args);
         SG_HIP(hipGetLastError());
         pg->launches++;
-        if (timed) SG_HIP(hipEventRecord(e->ev1, e->stream));
         return SG_OK;
     });
 }
@@ -113,15 +113,18 @@ int bfs_launch(sg_engine *e, uint32_t source, int32_t *out, bool traced)
     e->last_algo = 0;
     const int bs = o.block_size ? o.block_size : 1024;
     switch (bs) {
-    case 256: rc = o.stage_hubs ? launch_bfs<256, true>(e, a, traced) : launch_bfs<256, false>(e, a, traced); break;
-    case 512: rc = o.stage_hubs ? launch_bfs<512, true>(e, a, traced) : launch_bfs<512, false>(e, a, traced); break;
-    case 1024: rc = o.stage_hubs ? launch_bfs<1024, true>(e, a, traced) : launch_bfs<1024, false>(e, a, traced); break;
+    case 256: rc = o.stage_hubs ? launch_bfs<256, true>(e, a) : launch_bfs<256, false>(e, a); break;
+    case 512: rc = o.stage_hubs ? launch_bfs<512, true>(e, a) : launch_bfs<512, false>(e, a); break;
+    case 1024: rc = o.stage_hubs ? launch_bfs<1024, true>(e, a) : launch_bfs<1024, false>(e, a); break;
     default: SG_FAIL(SG_ERR_UNSUPPORTED, "sg_bfs: block_size must be 256, 512 or 1024");
     }
     if (rc) return rc;
     e->bfs_token = e->launch_seq;
     e->bfs_parity ^= 1;
-    if (traced) e->timed = true;
+    if (traced) {
+        e->timed = true;
+        e->clocked = e->last_grid;
+    }
     return SG_OK;
 }
 

@@ -542,7 +542,7 @@ extern "C" int sg_engine_destroy(sg_engine *e)
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     engine_forget_stream(e);
     void *ptrs[] = {e->value, e->bitmaps, e->queues, e->ctr,
-                    e->abort_flag, e->stats, e->trace, e->aux, e->srcbuf, e->garena, e->work};
+                    e->abort_flag, e->stats, e->trace, e->aux, e->garena, e->work};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (int i = 0; i < e->ngrids; i++) (void)hipFree(e->grids[i].words);
@@ -712,7 +712,7 @@ int engine_persistent_grid(sg_engine *e, const void *fn, int bs, const std::func
     const int cap = e->opt.grid_blocks > 0 ? e->opt.grid_blocks : most;
     for (int i = 0; i < e->ngrids; i++) {
         if (e->grids[i].fn == fn && e->grids[i].bs == bs && e->grids[i].cap == cap) {
-            *out = &e->grids[i];
+            *out = e->last_grid = &e->grids[i];
             return SG_OK;
         }
     }
@@ -725,18 +725,20 @@ int engine_persistent_grid(sg_engine *e, const void *fn, int bs, const std::func
     pg.bs = bs;
     pg.cap = cap;
     pg.probe = probe;
-    hipError_t err = hipMalloc((void **)&pg.words, kBarWords * 4);
+    const uint64_t most_blocks = std::max((uint64_t)per_cu * e->g->num_cus, (uint64_t)std::max(cap, 0));
+    hipError_t err = hipMalloc((void **)&pg.words, kBarWords * 4 + (1 + most_blocks) * 8);
     if (err != hipSuccess) {
         (void)hipGetLastError();
         SG_FAIL(SG_ERR_NOMEM, "persistent grid: hipMalloc failed");
     }
+    pg.clock = (uint64_t *)(pg.words + kBarWords);
     int rc = size_grid(e, pg, per_cu);
     if (rc) {
         (void)hipFree(pg.words);
         return rc;
     }
     e->grids[e->ngrids] = pg;
-    *out = &e->grids[e->ngrids++];
+    *out = e->last_grid = &e->grids[e->ngrids++];
     return SG_OK;
 }
 
@@ -814,21 +816,6 @@ int engine_run_status(sg_engine *e)
 int engine_finish(sg_engine *e, uint64_t rows)
 {
     return engine_gather_rows(e, e->work, e->value, rows);
-}
-
-int engine_ensure_srcbuf(sg_engine *e, uint64_t entries)
-{
-    if (e->srcbuf && e->srcbuf_cap >= entries) return SG_OK;
-    if (e->srcbuf) {
-        SG_HIP(hipStreamSynchronize(e->stream));
-        (void)hipFree(e->srcbuf);
-        e->srcbuf = nullptr;
-        e->srcbuf_cap = 0;
-    }
-    int rc = engine_alloc((void **)&e->srcbuf, entries * 4);
-    if (rc) return rc;
-    e->srcbuf_cap = entries;
-    return SG_OK;
 }
 
 int engine_ensure_value(sg_engine *e, uint64_t bytes)
@@ -979,7 +966,12 @@ extern "C" int sg_engine_get_stats(sg_engine *e, sg_stats *out)
         out->reached = (uint32_t)h[0];
         out->reached_edges = h[1];
     }
-    if (e->timed) {
+    if (e->timed && e->clocked) {
+        std::vector<uint64_t> t(1 + e->clocked->blocks);
+        SG_HIP(hipMemcpy(t.data(), e->clocked->clock, t.size() * 8, hipMemcpyDeviceToHost));
+        const uint64_t end = *std::max_element(t.begin() + 1, t.end());
+        out->kernel_ms = end > t[0] ? (double)(end - t[0]) / e->wall_khz : 0.0;
+    } else if (e->timed) {
         float ms = 0.f;
         SG_HIP(hipEventElapsedTime(&ms, e->ev0, e->ev1));
         out->kernel_ms = ms;

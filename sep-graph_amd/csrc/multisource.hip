@@ -45,9 +45,16 @@ __device__ __forceinline__ size_t out_row(const uint32_t *orow, uint32_t s, uint
     return (size_t)(orow ? orow[s] : s) * n;
 }
 
+// A batch's sources: handed to the kernel as arguments, or already on the device.
+struct MsSources {
+    const uint32_t *dev;
+    uint32_t v[64];
+    __device__ __forceinline__ uint32_t get(int i) const { return dev ? dev[i] : v[i]; }
+};
+
 struct BcArgs {
     DevGraph g;
-    const uint32_t *src;  // sources of this batch
+    MsSources src;        // sources of this batch
     uint32_t nsrc;
     uint64_t *seen;       // [n]
     uint64_t *F;          // 3 x n: level masks, level L in F + (L % 3) n
@@ -448,7 +455,7 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
     if (ok && blockIdx.x == 0 && threadIdx.x < kWave) {
         // sources: lane s owns source s; a vertex listed twice gets both bits
         const bool has = (uint32_t)ln < a.nsrc;
-        const uint32_t v = has ? a.src[ln] : 0u;
+        const uint32_t v = has ? a.src.get(ln) : 0u;
         uint64_t m = 0;
         int firstl = 64;
         for (int t = 0; t < 64; t++) {
@@ -650,6 +657,7 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
         if (s.status == SG_OK) s.status = !ok ? SG_ERR_TIMEOUT : (overflow || levels + 1 >= kMaxLevels) ? SG_ERR_CAPACITY : SG_OK;
         *a.stats = s;
     }
+    bar_end(a.bar);
 }
 
 // ------------------------------------------------------------ multi-source BFS
@@ -661,7 +669,8 @@ __global__ __launch_bounds__(BS) void k_bc(BcArgs a)
 // (each vertex appears at most once per level).
 struct MsBfsArgs {
     DevGraph g;
-    const uint32_t *src;
+    MsSources src;
+    uint32_t first;       // start the summary (else: add to it)
     uint32_t nsrc;
     uint64_t *seen;       // [n]
     uint64_t *F;          // 3 x n level masks
@@ -725,7 +734,7 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
     if (ok && blockIdx.x == 0 && threadIdx.x < kWave) {
         const bool has = (uint32_t)ln < a.nsrc;
-        const uint32_t v = has ? a.src[ln] : 0u;
+        const uint32_t v = has ? a.src.get(ln) : 0u;
         uint64_t m = 0;
         int firstl = 64;
         for (int t = 0; t < 64; t++) {
@@ -824,7 +833,7 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
             }
         }
     if (gtid == 0) {
-        DevStats s = *a.stats;
+        DevStats s = a.first ? DevStats{} : *a.stats;
         s.rounds += L;
         s.push_rounds += pushes;
         s.pull_rounds += pulls;
@@ -834,6 +843,7 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
         if (s.status == SG_OK) s.status = ok ? (a.ctl[1] ? SG_ERR_CAPACITY : SG_OK) : SG_ERR_TIMEOUT;
         *a.stats = s;
     }
+    bar_end(a.bar);
 }
 
 // ----------------------------------------------------------- multi-source SSSP
@@ -851,7 +861,8 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
 // to sg_sssp from that source.
 struct MsSsspArgs {
     DevGraph g;
-    const uint32_t *src;
+    MsSources src;
+    uint32_t first;       // start the summary (else: add to it)
     uint32_t nsrc;
     uint32_t *dist;       // [n][2^qbits]
     uint64_t *F;          // 3 x n masks, round r in F + (r % 3) n
@@ -1170,7 +1181,7 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
     if (ok && blockIdx.x == 0 && threadIdx.x < kWave) {
         const bool has = (uint32_t)ln < a.nsrc;
-        const uint32_t v = has ? a.src[ln] : 0u;
+        const uint32_t v = has ? a.src.get(ln) : 0u;
         uint64_t m = 0;
         int firstl = 64;
         for (int t = 0; t < 64; t++) {
@@ -1283,7 +1294,7 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
         }
     }
     if (gtid == 0) {
-        DevStats s = *a.stats;
+        DevStats s = a.first ? DevStats{} : *a.stats;
         s.rounds += r;
         s.push_rounds += r - pulls;
         s.pull_rounds += pulls;
@@ -1293,6 +1304,7 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
         if (s.status == SG_OK) s.status = ok ? SG_OK : SG_ERR_TIMEOUT;
         *a.stats = s;
     }
+    bar_end(a.bar);
 }
 
 }  // namespace
@@ -1392,7 +1404,7 @@ int ms_prepare(sg_engine *e, int kind)
 }
 
 int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, void *out, const uint32_t *dev_orow,
-              bool first, bool last, const uint32_t *inv)
+              bool first, bool last, const uint32_t *inv, const uint32_t *host_src)
 {
     if (nsrc < 1 || nsrc > 64) SG_FAIL(SG_ERR_RANGE, "batched launch: 1..64 sources");
     const uint64_t n = e->g->dev.n;
@@ -1408,10 +1420,14 @@ int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, vo
     if (bs != 256 && bs != 512 && bs != 1024) SG_FAIL(SG_ERR_UNSUPPORTED, "batched launch: block_size must be 256, 512 or 1024");
     const double alpha = o.alpha == 0.0 ? 1.0 : o.alpha;
     const double total_wl = (double)e->g->dev.m * o.edge_factor;
+    MsSources src{};
+    src.dev = dev_src;
+    if (!dev_src) std::copy(host_src, host_src + nsrc, src.v);
     if (kind == kMsBfs) {
         MsBfsArgs a{};
         fill_common(e, a);
-        a.src = dev_src;
+        a.src = src;
+        a.first = first;
         a.nsrc = nsrc;
         a.seen = (uint64_t *)(base + L.off[0]);
         a.F = (uint64_t *)(base + L.off[1]);
@@ -1431,7 +1447,8 @@ int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, vo
     if (kind == kMsSssp) {
         MsSsspArgs a{};
         fill_common(e, a);
-        a.src = dev_src;
+        a.src = src;
+        a.first = first;
         a.nsrc = nsrc;
         a.dist = (uint32_t *)(base + L.off[0]);
         a.F = (uint64_t *)(base + L.off[1]);
@@ -1447,7 +1464,7 @@ int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, vo
     }
     BcArgs a{};
     fill_common(e, a);
-    a.src = dev_src;
+    a.src = src;
     a.nsrc = nsrc;
     a.seen = (uint64_t *)(base + L.off[0]);
     a.F = (uint64_t *)(base + L.off[1]);
@@ -1510,38 +1527,35 @@ int ms_run(sg_engine *e, int kind, const uint32_t *sources, int32_t k, int32_t b
     } else if ((rc = engine_result_rows(e, rows, &res))) {
         return rc;
     }
-    if ((rc = engine_ensure_srcbuf(e, (uint64_t)k))) return rc;
+    // (the kernels' arguments carry the sources: nothing is left to wait for)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SG_HIP(hipStreamIsCapturing(e->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) SG_FAIL(SG_ERR_HIP, std::string(name) + ": not on a capturing stream");
     std::vector<uint32_t> dsrc(k);
     for (int32_t i = 0; i < k; i++) dsrc[i] = dev_vertex(e->g, sources[i]);
-    // the source buffer may still be read by an earlier launch on the stream
-    SG_HIP(hipStreamSynchronize(e->stream));
-    SG_HIP(hipMemcpy(e->srcbuf, dsrc.data(), (size_t)k * 4, hipMemcpyHostToDevice));
-    SG_HIP(hipMemsetAsync(e->stats, 0, sizeof(DevStats), e->stream));
     e->last_algo = 3 + kind;
-    SG_HIP(hipEventRecord(e->ev0, e->stream));
-    if (single_bc) {
-        // one source per launch: the single-source kernel (no bit-packed rows)
-        for (int32_t i = 0; i < k; i++) {
+    // one source per launch (the single-source kernel, no bit-packed rows), or
+    // a batch. A single launch's time is the device's clock, several take events.
+    const int per = single_bc ? 1 : batch, nb = (k + per - 1) / per;
+    if (nb > 1) SG_HIP(hipEventRecord(e->ev0, e->stream));
+    for (int i = 0; i < nb; i++) {
+        const bool first = i == 0, last = i == nb - 1;
+        if (single_bc) {
             float *dep = kind == kMsBcDep ? (float *)res + (size_t)i * n : nullptr;
             float *sum = kind == kMsBcSum ? (float *)res : nullptr;
-            if ((rc = bc1_launch(e, dsrc[i], dep, nullptr, sum, i == 0, i == k - 1))) return rc;
+            rc = bc1_launch(e, dsrc[i], dep, nullptr, sum, first, last);
+        } else {
+            const uint32_t ns = (uint32_t)std::min(batch, k - i * batch);
+            void *out = kind == kMsBcSum ? res : (void *)((uint32_t *)res + (size_t)i * batch * n);
+            rc = ms_launch(e, kind, nullptr, ns, out, nullptr, first, last,
+                           direct && e->g->relabeled ? e->g->d_inv : nullptr, dsrc.data() + (size_t)i * batch);
         }
-        SG_HIP(hipEventRecord(e->ev1, e->stream));
-        if ((rc = engine_finish(e, rows))) return rc;
-        e->timed = true;
-        return SG_OK;
-    }
-    const int nb = (k + batch - 1) / batch;
-    for (int i = 0; i < nb; i++) {
-        const uint32_t ns = (uint32_t)std::min(batch, k - i * batch);
-        void *out = kind == kMsBcSum ? res : (void *)((uint32_t *)res + (size_t)i * batch * n);
-        rc = ms_launch(e, kind, e->srcbuf + (size_t)i * batch, ns, out, nullptr, i == 0, i == nb - 1,
-                       direct && e->g->relabeled ? e->g->d_inv : nullptr);
         if (rc) return rc;
     }
-    SG_HIP(hipEventRecord(e->ev1, e->stream));
+    if (nb > 1) SG_HIP(hipEventRecord(e->ev1, e->stream));
     if (!direct && (rc = engine_finish(e, rows))) return rc;
     e->timed = true;
+    e->clocked = nb > 1 ? nullptr : e->last_grid;
     return SG_OK;
 }
 

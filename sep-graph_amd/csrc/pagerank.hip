@@ -580,6 +580,7 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
             a.trace[it] = t;
         }
     }
+    bar_end(a.bar);
 }
 
 // ------------------------------------------------------- residual DD kernel
@@ -1134,6 +1135,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
             a.trace[k] = t;
         }
     }
+    bar_end(a.bar);
 }
 
 template <typename Args, void (*K)(Args)>
@@ -1153,11 +1155,9 @@ int launch_persistent(sg_engine *e, Args &args, int bs)
     if (pg->blocks > (int)kMaxBlocks) SG_FAIL(SG_ERR_STATE, "sg_pagerank: grid exceeds the partial-sum area");
     bind_barrier(pg, args.bar);
     return engine_launch_persistent(e, [&]() -> int {
-        SG_HIP(hipEventRecord(e->ev0, e->stream));
         void *params[] = {&args};
         SG_HIP(hipLaunchKernel((const void *)K, dim3(pg->blocks), dim3(bs), params, 0, e->stream));
         pg->launches++;
-        SG_HIP(hipEventRecord(e->ev1, e->stream));
         return SG_OK;
     });
 }
@@ -1274,5 +1274,6 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
     if (rc) return rc;
     if ((rc = engine_finish(e, 1))) return rc;
     e->timed = true;
+    e->clocked = e->last_grid;
     return SG_OK;
 }

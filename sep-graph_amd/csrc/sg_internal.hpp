@@ -187,8 +187,6 @@ struct sg_engine {
     sg::DevTrace *trace = nullptr;    // kTraceRows rows
     void *aux = nullptr;              // per-algorithm working arrays (PageRank, BC), grown on demand
     uint64_t aux_bytes = 0;
-    uint32_t *srcbuf = nullptr;       // device copy of a batched call's sources
-    uint64_t srcbuf_cap = 0;          // entries
     void *work = nullptr;             // results in device vertex order (relabelled graphs)
     uint64_t work_cap = 0;
     void *garena = nullptr;           // per-query state of concurrent (one per XCD) SSSP
@@ -208,6 +206,7 @@ struct sg_engine {
         int blocks = 0;
         uint64_t launches = 0;  // kernels run on `words` (their parity picks the registration set)
         uint32_t *words = nullptr;
+        uint64_t *clock = nullptr;  // behind `words`: GridBarrier::clock
         // launches the kernel in residency-probe mode with a given grid
         std::function<int(int blocks, uint32_t *words)> probe;
     };
@@ -218,6 +217,8 @@ struct sg_engine {
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool timed = false;
+    PGrid *last_grid = nullptr;  // of the latest launch
+    PGrid *clocked = nullptr;    // whose clock holds the last run's time (null: ev0 to ev1)
 };
 
 namespace sg {
@@ -228,7 +229,6 @@ int engine_ensure_value(sg_engine *e, uint64_t bytes);
 // Grow the engine's auxiliary arena to at least `bytes` (synchronises the
 // stream before replacing a smaller one; contents are not preserved).
 int engine_ensure_aux(sg_engine *e, uint64_t bytes);
-int engine_ensure_srcbuf(sg_engine *e, uint64_t entries);
 
 // Relabelled graphs keep vertices in degree order on the device.
 // The device id of the caller's vertex v.
@@ -248,13 +248,13 @@ int engine_gather_rows(sg_engine *e, const void *src, void *dst, uint64_t rows);
 enum MsKind { kMsBfs = 0, kMsSssp = 1, kMsBcDep = 2, kMsBcSum = 3 };
 // Size the engine's arena for a kind (may synchronise and reallocate).
 int ms_prepare(sg_engine *e, int kind);
-// One batch of nsrc <= 64 device-resident sources, asynchronously on the
-// engine's stream. Results: row dev_orow[i] (or i when null) of `out`, n
+// One batch of nsrc <= 64 sources (on the device, or with dev_src null on the
+// host), asynchronously on the engine's stream. Results: row dev_orow[i] (or i when null) of `out`, n
 // elements per row (int32 levels, uint32 distances, FP32 dependencies); for
 // kMsBcSum, `out` is the n-float BC sum written by the batch with `last`. Rows
 // are in device order; for kMsSssp, `inv` (optional) puts them in the caller's.
 int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, void *out, const uint32_t *dev_orow,
-              bool first, bool last, const uint32_t *inv = nullptr);
+              bool first, bool last, const uint32_t *inv = nullptr, const uint32_t *host_src = nullptr);
 
 // Working arena of one single-source BC run (byte offsets).
 struct Bc1Layout {
@@ -305,6 +305,7 @@ inline void bind_barrier(const sg_engine::PGrid *pg, GridBarrier &bar)
 {
     bar.words = pg->words;
     bar.rset = (uint32_t)(pg->launches & 1u);
+    bar.clock = pg->clock;
 }
 // Concurrent SSSP: size its arena and reset the call's status word
 // (asynchronous), before the call's first sssp_group_launch.

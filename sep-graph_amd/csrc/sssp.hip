@@ -25,6 +25,7 @@ __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
     BarState st = bar_begin<true>(a.bar, xcc);
     if (!a.grouped) {
         sssp_run<BS, SG_FRONT_LDS * BS, true>(a, blockIdx.x, gridDim.x, xcc, st);
+        bar_end(a.bar);
         return;
     }
     // Grouped: the census of this launch decides which XCD runs which query.
@@ -79,6 +80,7 @@ __global__ __launch_bounds__(BS) void k_sssp_whole(SsspArgs a)
     const uint32_t xcc = xcc_id();
     BarState gen = bar_begin<true>(a.bar, xcc);
     sssp_whole<BS>(a, xcc, gen);
+    bar_end(a.bar);
 }
 
 // Persistent grid for k_sssp<BS>; grouped launches take the barrier area
@@ -337,10 +339,9 @@ extern "C" int sg_sssp(sg_engine *e, uint32_t source)
         a.inv = e->g->d_inv;
     }
     e->last_algo = 1;
-    SG_HIP(hipEventRecord(e->ev0, e->stream));
     if ((rc = launch_sssp_bs(e, a, nullptr))) return rc;
-    SG_HIP(hipEventRecord(e->ev1, e->stream));
     e->timed = true;
+    e->clocked = e->last_grid;
     return SG_OK;
 }
 
@@ -371,5 +372,6 @@ extern "C" int sg_sssp_concurrent(sg_engine *e, const uint32_t *sources, int32_t
     SG_HIP(hipEventRecord(e->ev1, e->stream));
     if ((rc = engine_finish(e, (uint64_t)k))) return rc;
     e->timed = true;
+    e->clocked = nullptr;
     return SG_OK;
 }

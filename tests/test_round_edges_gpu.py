@@ -228,3 +228,45 @@ def test_sssp_batches(sg, orc, gpu, name, k, weights, opts):
     got = e.gather(np.uint32).reshape(k, hg.n)
     for i in sorted({0, k - 1}):
         assert np.array_equal(got[i], distances(orc, hg, w, int(src[i]), weights)), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["bfs", "sssp", "pull", "dd", "bfs_multi", "sssp_multi", "bc", "bc_one", "bc_dependency"])
+@pytest.mark.parametrize("k", [1, 5])
+def test_calls_back_to_back_and_their_time(sg, gpu, call, k):
+    """Calls queued one behind the other, each with sources of its own, give
+    what each gives alone; the reported time is within the call's own."""
+    import time
+    hg = random_graph(sg, 5000, 6, 3, weights=(1, 64))
+    graph = sg.Graph(hg)
+    run = {
+        "bfs": lambda e, s: e.bfs(int(s[0])),
+        "sssp": lambda e, s: e.sssp(int(s[0])),
+        "pull": lambda e, s: e.pagerank(0.85, 1e-6, 0, sg.PR_PULL_TD),
+        "dd": lambda e, s: e.pagerank(0.85, 1e-6, 0, sg.PR_PUSH_DD),
+        "bfs_multi": lambda e, s: e.bfs_multi(s, 4),
+        "sssp_multi": lambda e, s: e.sssp_multi(s, 4),
+        "bc": lambda e, s: e.bc(s, 4),
+        "bc_one": lambda e, s: e.bc(s, 1),
+        "bc_dependency": lambda e, s: e.bc_dependency(s, 4),
+    }[call]
+    dtype = np.float32 if call in ("pull", "dd", "bc", "bc_one", "bc_dependency") else np.uint32
+    rng = np.random.default_rng(k)
+    sets = [rng.choice(hg.n, k, replace=False).astype(np.uint32) for _ in range(4)]
+    e = sg.Engine(graph)
+    for s in sets:
+        run(e, s)
+    got = e.gather(dtype)
+    e.stats()
+    t = time.perf_counter()
+    run(e, sets[0])
+    ms = e.stats()["kernel_ms"]
+    wall = (time.perf_counter() - t) * 1e3
+    assert 0.0 < ms < wall
+    alone = sg.Engine(graph)
+    run(alone, sets[-1])
+    want = alone.gather(dtype)
+    if call == "dd" or call.startswith("bc"):  # atomic additions in any order
+        assert np.allclose(got, want, rtol=1e-5, atol=1e-12)
+    else:
+        assert np.array_equal(got, want)
