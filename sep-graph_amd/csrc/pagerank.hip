@@ -33,7 +33,8 @@
 // rounds' worklist holds vertices whose residual crossed theta), moves the
 // residual into y and spreads d r / outdeg along out-edges: with FP32 atomics
 // when the active out-degree is small (push), or by a gather over in-edges
-// from active sources when it exceeds m / alpha (pull).
+// when it exceeds m / alpha (pull, which activates for the next round in the
+// same pass).
 #include "frontier.hpp"
 
 using namespace sg;
@@ -213,6 +214,296 @@ __device__ __forceinline__ double wave_sum4(const double (&s)[4])
     return shfl(t, (lane() & 3) * 16);
 }
 
+// ---------------------------------------------- sums over every in-edge list
+// Both kernels sum one FP32 value per source over all in-edges. The values of
+// the lowest ids (in a degree-ordered graph the sources of most in-edges) are
+// copied to LDS before a pass (they are read-only until the next barrier), and
+// the gather reads them there instead of sending one L2 request per in-edge.
+constexpr uint32_t kNoEdge = 0xFFFFFFFFu;
+
+// Floats from one row of values to the next: 16-byte aligned rows.
+__host__ __device__ constexpr uint64_t contrib_stride(uint32_t n) { return ((uint64_t)n + 3) / 4 * 4; }
+
+// The copy: KF floats per thread, 16 bytes a lane straight from memory into
+// LDS, so that it takes no registers while other loads of the round are waited
+// for. take() starts it (once every wave is done with the last copy), wait()
+// and a __syncthreads() end it.
+template <int BS, int KF>
+struct Staged {
+    static constexpr uint32_t kLds = (uint32_t)KF * BS;
+    static constexpr int kFill = (int)((kLds / 4 + BS - 1) / BS);
+    static __device__ __forceinline__ void take(float *s_cc, const float *cc, uint32_t n)
+    {
+        const uint32_t have = min(n, kLds);
+        const uint32_t wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~(uint32_t)(kWave - 1));
+#pragma unroll
+        for (int i = 0; i < kFill; i++) {
+            if (4 * threadIdx.x < have - min(have, (uint32_t)(4 * i * BS)))
+                __builtin_amdgcn_global_load_lds(
+                    (__attribute__((address_space(1))) void *)((const float4 *)cc + i * BS + threadIdx.x),
+                    (__attribute__((address_space(3))) void *)((float4 *)s_cc + i * BS + wave0), 16, 0, 0);
+        }
+    }
+    static __device__ __forceinline__ void wait() { __builtin_amdgcn_s_waitcnt(0); }
+};
+
+// Values of N sources: the loads of those outside LDS are all issued first,
+// then every entry reads LDS (s_cc[K], a zero, if it has no place there), so
+// no entry waits for the one before it.
+template <uint32_t K>
+struct Gather {
+    const float *cc, *s_cc;
+    uint32_t n;
+    template <int N>
+    __device__ __forceinline__ void get(const uint32_t (&u)[N], float (&c)[N]) const
+    {
+        const uint32_t ncold = n > K ? n - K : 0u;
+#pragma unroll
+        for (int q = 0; q < N; q++) {
+            c[q] = 0.f;
+            if (u[q] - K < ncold) c[q] = cc[u[q]];
+        }
+#pragma unroll
+        for (int q = 0; q < N; q++) c[q] += s_cc[min(u[q], K)];
+    }
+    __device__ __forceinline__ float one(uint32_t u) const { return u < min(n, K) ? s_cc[u] : cc[u]; }
+};
+
+// The bounds a wave starts every pass with: of up to 64 in-hub chunks, of up
+// to 64 words of the sliced layout and of its first in-hubs. They never change, so they are read once per
+// run, not in every round from caches that the barrier before it emptied (RMAT
+// graphs, 17 iterations: 400 001 vertices 477 -> 462 us, 8001 213 -> 209).
+struct Bounds {
+    uint32_t hv, beg, len;  // chunk gwave + lane * nwaves: hub, first in-edge, in-edges
+    bool one;               // the chunk is all of the hub
+    uint32_t off, nrow;     // word gwave + lane * nwaves
+    uint32_t at, chunks, v; // hub gwave + lane / kHubLanes * nwaves, if of several chunks
+
+    static constexpr uint32_t kHubLanes = 8;
+
+    __device__ __forceinline__ void chunk(const DevGraph &g, uint32_t first, uint32_t nwaves)
+    {
+        const uint64_t c = first + (uint64_t)lane() * nwaves;
+        hv = beg = len = 0;
+        one = false;
+        if (c < g.nhugein) {
+            const uint2 dsc = g.hugein[c];
+            hv = dsc.x;
+            beg = dsc.y;
+            const uint32_t b = g.cstart[hv], e = g.cstart[hv + 1];
+            len = min(e - beg, kPullChunk);
+            one = e - b <= kPullChunk;
+        }
+    }
+    __device__ __forceinline__ void word(const DevGraph &g, uint32_t first, uint32_t nwaves)
+    {
+        const uint64_t w = first + (uint64_t)lane() * nwaves;
+        off = nrow = 0;
+        if (g.sell_src && w < g.words) {
+            off = g.sell_off[w];
+            nrow = (g.sell_off[w + 1] - off) / kWave;
+        }
+    }
+    __device__ __forceinline__ void hub(const DevGraph &g, uint32_t first, uint32_t nwaves)
+    {
+        const uint64_t h = first + (uint64_t)(lane() / kHubLanes) * nwaves;
+        at = chunks = v = 0;
+        if (h < g.nhubin) {
+            const uint2 d = g.hubin[h];
+            at = d.x;
+            chunks = d.y;
+            if (d.y > 1) v = g.hugein[d.x].x;
+        }
+    }
+    __device__ __forceinline__ Bounds(const DevGraph &g, uint32_t gwave, uint32_t nwaves)
+    {
+        chunk(g, gwave, nwaves);
+        word(g, gwave, nwaves);
+        hub(g, gwave, nwaves);
+    }
+};
+
+// Chunk sums of the in-hubs, dealt out one by one. A lane holds one chunk's
+// bounds and, in the end, its sum; the wave adds kQ chunks together, the next
+// kQ chunks' in-edges in flight meanwhile. pre(v): what the hub needs in the
+// end, loaded with the bounds (false: no chunk); done(has, c, v, one, own,
+// sum), wave-convergent: `one` if chunk c is all of hub v.
+template <typename G, typename Pre, typename Done>
+__device__ __forceinline__ void hub_chunk_sums(const DevGraph &g, const G &gather, const Bounds &bounds, uint32_t gwave,
+                                               uint32_t nwaves, Pre pre, Done done)
+{
+    constexpr int kQ = 4, kSteps = (int)(kPullChunk / kWave);
+    const int ln = lane();
+    for (uint32_t first = gwave; first < g.nhugein; first += nwaves * kWave) {
+        const uint32_t cnt = min((uint32_t)kWave, (g.nhugein - first + nwaves - 1) / nwaves);
+        const uint32_t c = first + (uint32_t)ln * nwaves;
+        const bool has = (uint32_t)ln < cnt;
+        Bounds bd = bounds;
+        if (first != gwave) bd.chunk(g, first, nwaves);
+        const uint32_t hv = bd.hv, beg = bd.beg, len = bd.len;
+        const bool one = bd.one;
+        const auto own = pre(has, hv);
+        auto load = [&](uint32_t j, uint32_t (&u)[kQ * kSteps]) {
+#pragma unroll
+            for (int q = 0; q < kQ; q++) {
+                const uint32_t l = lane_value(len, (int)j + q);
+                const uint32_t *src = g.csrc + lane_value(beg, (int)j + q);
+#pragma unroll
+                for (int t = 0; t < kSteps; t++) {
+                    const uint32_t k = (uint32_t)(t * kWave + ln);
+                    u[q * kSteps + t] = k < l ? src[k] : kNoEdge;
+                }
+            }
+        };
+        double mine = 0.0;
+        uint32_t u[kQ * kSteps], nu[kQ * kSteps];
+        load(0, u);
+        for (uint32_t j = 0; j < cnt; j += kQ) {
+            if (j + kQ < cnt) load(j + kQ, nu);
+            float cv[kQ * kSteps];
+            gather.get(u, cv);
+            double s[kQ];
+#pragma unroll
+            for (int q = 0; q < kQ; q++) {
+                s[q] = 0.0;
+#pragma unroll
+                for (int t = 0; t < kSteps; t++) s[q] += (double)cv[q * kSteps + t];
+            }
+            const double t = wave_sum4(s);
+            if ((uint32_t)ln / kQ == j / kQ) mine = t;
+#pragma unroll
+            for (int q = 0; q < kQ * kSteps; q++) u[q] = nu[q];
+        }
+        done(has, c, hv, one, own, mine);
+    }
+}
+
+// Sums of every other vertex, a 64-vertex word per wave at a time: from the
+// sliced in-edges (each lane sums its own vertex's row entries in order) or,
+// without them, by a scheduled walk of the word's lists. What a word's
+// vertices need in the end (pre) is loaded one word ahead, its in-edges one
+// step ahead. done(has, v, own, sum), wave-convergent. U rows of in-edges at a
+// time: the steps of a word are a chain, so as many as there are registers for.
+template <uint32_t U, typename G, typename Pre, typename Done>
+__device__ __forceinline__ void word_sums(const DevGraph &g, const G &gather, const Bounds &bounds, uint32_t gwave,
+                                          uint32_t nwaves, Pre pre, Done done)
+{
+    const int ln = lane();
+    const uint32_t n = g.n, W = g.words;
+    if (!g.sell_src) {
+        for (uint32_t w = gwave; w < W; w += nwaves) {
+            const uint32_t v = w * kWave + ln;
+            uint32_t b = 0, e = 0;
+            bool has = false;
+            if (v < n) {
+                b = g.cstart[v];
+                e = g.cstart[v + 1];
+                has = e - b <= kPullHubDegree;
+                if (!has) b = e;
+            }
+            const auto own = pre(has, v);
+            const CSum s = wave_gather_csum(b, e, [&](uint32_t ed) { return gather.one(g.csrc[ed]); });
+            done(has, v, own, (double)s.hi + (double)s.lo);
+        }
+        return;
+    }
+    for (uint32_t first = gwave; first < W; first += nwaves * kWave) {
+        const uint32_t cnt = min((uint32_t)kWave, (W - first + nwaves - 1) / nwaves);
+        Bounds bd = bounds;  // a lane holds one word's rows
+        if (first != gwave) bd.word(g, first, nwaves);
+        const uint32_t off = bd.off, nrow = bd.nrow;
+        auto degree = [&](uint32_t v) { return v < n ? g.cstart[v + 1] - g.cstart[v] : kNoEdge; };
+        auto load = [&](uint32_t i, uint32_t j, uint32_t (&u)[U]) {
+            const uint32_t rows = lane_value(nrow, (int)i);
+            const uint32_t *S = g.sell_src + lane_value(off, (int)i) + ln;
+#pragma unroll
+            for (uint32_t q = 0; q < U; q++) {
+                u[q] = kNoEdge;
+                if (j + q < rows) u[q] = S[(size_t)(j + q) * kWave];
+            }
+        };
+        uint32_t i = 0, j = 0, u[U], nu[U];
+        uint32_t v = first * kWave + ln, nv = v, din = degree(v), ndin = din;
+        auto own = pre(v < n, v), nown = own;
+        load(0, 0, u);
+        double s = 0.0;
+        while (i < cnt) {
+            if (j == 0 && i + 1 < cnt) {
+                nv = v + nwaves * kWave;
+                ndin = degree(nv);
+                nown = pre(nv < n, nv);
+            }
+            const uint32_t rows = lane_value(nrow, (int)i);
+            const bool last = j + U >= rows;
+            const uint32_t ni = last ? i + 1 : i, nj = last ? 0u : j + U;
+            if (ni < cnt) load(ni, nj, nu);
+            if (rows) {
+                float cv[U];
+                gather.get(u, cv);
+#pragma unroll
+                for (uint32_t q = 0; q < U; q++) s += (double)cv[q];
+            }
+            if (last) {
+                done(din <= kPullHubDegree, v, own, s);
+                s = 0.0;
+                v = nv;
+                din = ndin;
+                own = nown;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < U; q++) u[q] = nu[q];
+            i = ni;
+            j = nj;
+        }
+    }
+}
+
+// In-hubs of several chunks, once wait() has seen every block's chunk sums:
+// eight lanes each (those of more than kHubWave chunks: the whole wave), dealt
+// out so that the largest, which come first, fall to different waves; the
+// first ones' data is loaded before the wait. done(has, v, own, sum),
+// wave-convergent. Returns wait()'s result.
+template <typename Wait, typename Pre, typename Done>
+__device__ __forceinline__ bool wide_hub_sums(const DevGraph &g, const double *hubpart, const Bounds &bounds, uint32_t gwave,
+                                              uint32_t nwaves, Wait wait, Pre pre, Done done)
+{
+    constexpr uint32_t kHubLanes = Bounds::kHubLanes, kHubs = kWave / kHubLanes, kHubWave = 8 * kHubLanes;
+    const int ln = lane();
+    Bounds bd = bounds;
+    uint32_t h0 = gwave;
+    auto own = pre(bd.chunks > 1, bd.v);
+    if (!wait()) return false;
+    while (h0 < g.nhubin) {
+        const uint32_t cat = bd.at, cc = bd.chunks, cv = bd.v;
+        const auto cown = own;
+        h0 += nwaves * kHubs;
+        if (h0 < g.nhubin) {
+            bd.hub(g, h0, nwaves);
+            own = pre(bd.chunks > 1, bd.v);
+        }
+        double s = 0.0;
+        if (cc > 1 && cc <= kHubWave) {
+#pragma unroll 8
+            for (uint32_t k = (uint32_t)ln % kHubLanes; k < cc; k += kHubLanes) s += hubpart[cat + k];
+        }
+        s += dpp<kDppQuad1>(0.0, s);
+        s += dpp<kDppQuad2>(0.0, s);
+        s += dpp<kDppHalfMirror>(0.0, s);
+        uint64_t wide = ballot(cc > kHubWave);
+        while (wide) {
+            const int l = first_lane(wide);
+            const uint32_t wat = lane_value(cat, l), wc = lane_value(cc, l);
+            double t = 0.0;
+            for (uint32_t k = ln; k < wc; k += kWave) t += hubpart[wat + k];
+            t = wave_sum_f64(t);
+            if (ln / (int)kHubLanes == l / (int)kHubLanes) s = t;
+            wide &= ~(0xFFull << l);
+        }
+        done(ln % (int)kHubLanes == 0 && cc > 1, cv, cown, s);
+    }
+    return true;
+}
+
 struct PrArgs {
     DevGraph g;
     float *x;          // ranks [n]
@@ -228,12 +519,9 @@ struct PrArgs {
     uint32_t probe;
 };
 
-// Floats from one row of contributions to the next: 16-byte aligned rows.
-__host__ __device__ constexpr uint64_t contrib_stride(uint32_t n) { return ((uint64_t)n + 3) / 4 * 4; }
-
 // What bounds an iteration: the in-edges whose source has no place in LDS,
 // each an L2 request for a line of which it needs 4 bytes. RMAT-21 (32.4 M
-// edges, 36 % of them such), 17 iterations: 1800 us, of which 1030 are these
+// edges, 36 % of them such), 17 iterations: 1750 us, of which 1030 are these
 // reads (11.7 M an iteration at 0.19 T/s; the L2s answer 0.27 T/s at most),
 // 210 the barriers, partial sums and LDS copy, the rest index reads, LDS reads
 // and the vertices' own data. It took 2640 us when each in-edge's LDS or L2 read
@@ -247,7 +535,6 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         return;
     }
     constexpr int WPB = BS / kWave;
-    constexpr uint32_t kPad = 0xFFFFFFFFu;  // no in-edge
     const DevGraph &g = a.g;
     const uint32_t n = g.n, W = g.words;
     const uint32_t gtid = blockIdx.x * BS + threadIdx.x;
@@ -263,16 +550,13 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
     const uint64_t stride = contrib_stride(n);
 
     __shared__ double2 s_red[WPB];
-    // The lowest ids' contributions (in a degree-ordered graph the sources of
-    // most in-edges) are copied to LDS each iteration: they are read-only
-    // until the next barrier, and the gather reads them there instead of
-    // sending one L2 request per in-edge. As many as fit beside the rest: with
-    // 32 per thread RMAT-21 takes 1848 us, with 39 1803.
+    // as many ids in LDS as fit beside the rest: with 32 per thread RMAT-21
+    // took 1848 us, with 39 1803
 #ifndef SG_PR_LDS
 #define SG_PR_LDS 39
 #endif
-    constexpr uint32_t kCcLds = SG_PR_LDS * BS;
-    __shared__ __align__(16) float s_cc[kCcLds + 4];  // [kCcLds]: 0, read for every other entry
+    using Hot = Staged<BS, SG_PR_LDS>;
+    __shared__ __align__(16) float s_cc[Hot::kLds + 4];
 
     // the block's (residual, dangling) partials, in a fixed order
     auto put_part = [&](uint32_t it, double res, double dang) {
@@ -296,24 +580,18 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         a.contrib[v] = dout ? inv_nf / (float)dout : 0.0f;
         if (!dout) dang += (double)inv_nf;
     }
-    if (threadIdx.x == 0) s_cc[kCcLds] = 0.f;
+    if (threadIdx.x == 0) s_cc[Hot::kLds] = 0.f;
     put_part(0, 0.0, dang);
     bool ok = grid_sync(a.bar, xcc, gen, a.abort);
 
+    const Bounds bounds(g, gwave, nwaves);
     uint32_t it = 0;
     double res = INFINITY;
     while (ok) {
         const float *cc = a.contrib + (size_t)(it & 1) * stride;
         float *cn = a.contrib + (size_t)((it + 1) & 1) * stride;
         // the LDS copy's loads are in flight while the partials are added
-        const uint32_t ncc = min(n, kCcLds);
-        constexpr int kFill = (int)((kCcLds / 4 + BS - 1) / BS);
-        float4 fill[kFill];
-#pragma unroll
-        for (int i = 0; i < kFill; i++) {
-            fill[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (4 * threadIdx.x < ncc - min(ncc, (uint32_t)(4 * i * BS))) fill[i] = ((const float4 *)cc + i * BS)[threadIdx.x];
-        }
+        Hot::take(s_cc, cc, n);
         // every wave adds the blocks' partials by itself: no wait for others
         double2 gs = make_double2(0.0, 0.0);
         for (uint32_t i = ln; i < gridDim.x; i += kWave) {
@@ -324,7 +602,10 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         gs.x = wave_sum_f64(gs.x);
         gs.y = wave_sum_f64(gs.y);
         if (it > 0) res = gs.x;
-        if ((it > 0 && res < a.tol) || it >= a.max_iter) break;
+        if ((it > 0 && res < a.tol) || it >= a.max_iter) {
+            Hot::wait();  // no copy into LDS outlives the block
+            break;
+        }
         const float base = (1.0f - df) * inv_nf + df * (float)gs.y * inv_nf;
         if (gtid == 0 && it < kTraceRows) {
             DevTrace t;
@@ -336,229 +617,39 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
             t.ticks = (unsigned long long)(wall_clock64() - t_start);
             a.trace[it] = t;
         }
-#pragma unroll
-        for (int i = 0; i < kFill; i++) {
-            if (4 * threadIdx.x < ncc - min(ncc, (uint32_t)(4 * i * BS))) ((float4 *)s_cc + i * BS)[threadIdx.x] = fill[i];
-        }
+        Hot::wait();
         __syncthreads();
-        // contributions of N sources: the loads of those outside LDS are all
-        // issued first, then every entry reads LDS (the zero, if it has no
-        // place there), so no entry waits for the one before it
-        const uint32_t ncold = n > kCcLds ? n - kCcLds : 0u;
-        auto gather = [&](const uint32_t *u, float *c, auto N) {
-#pragma unroll
-            for (int q = 0; q < N.value; q++) {
-                c[q] = 0.f;
-                if (u[q] - kCcLds < ncold) c[q] = cc[u[q]];
-            }
-#pragma unroll
-            for (int q = 0; q < N.value; q++) c[q] += s_cc[min(u[q], kCcLds)];
-        };
+        const Gather<Hot::kLds> gather{cc, s_cc, n};
+        constexpr uint32_t kRows = 8;  // RMAT-21 1774 us by 4, 1746 by 8; 15 001 vertices 226 and 210
         double r_acc = 0.0, d_acc = 0.0;
-        // x(v) from its in-edge sum, its last rank and its out-degree: FP32
-        // ranks and contributions, sums and the residual |x' - x| in FP64
-        auto finish = [&](uint32_t v, double s, float xo, uint32_t dout) {
-            const float xn = base + df * (float)s;
-            r_acc += fabs((double)xn - (double)xo);
-            a.x[v] = xn;
-            if (dout) cn[v] = xn / (float)dout;
-            else d_acc += (double)xn;
-        };
-        // (A1) chunk sums of the in-hubs, dealt out one by one. A lane holds
-        // one chunk's bounds and, in the end, its sum; the wave adds kQ
-        // chunks together, the next kQ chunks' in-edges in flight meanwhile.
-        // A hub of one chunk is finished here.
-        constexpr int kQ = 4, kSteps = (int)(kPullChunk / kWave);
-        for (uint32_t first = gwave; first < g.nhugein; first += nwaves * kWave) {
-            const uint32_t cnt = min((uint32_t)kWave, (g.nhugein - first + nwaves - 1) / nwaves);
-            const uint32_t c = first + (uint32_t)ln * nwaves;
-            uint32_t hv = 0, beg = 0, len = 0, dout = 0;
-            float xo = 0.f;
-            bool one = false;
-            if ((uint32_t)ln < cnt) {
-                const uint2 dsc = g.hugein[c];
-                hv = dsc.x;
-                beg = dsc.y;
-                const uint32_t b = g.cstart[hv], e = g.cstart[hv + 1];
-                len = min(e - beg, kPullChunk);
-                one = e - b <= kPullChunk;
-                dout = g.row[hv + 1] - g.row[hv];
-                xo = a.x[hv];
-            }
-            auto load = [&](uint32_t j, uint32_t *u) {
-#pragma unroll
-                for (int q = 0; q < kQ; q++) {
-                    const uint32_t l = lane_value(len, (int)j + q);
-                    const uint32_t *src = g.csrc + lane_value(beg, (int)j + q);
-#pragma unroll
-                    for (int t = 0; t < kSteps; t++) {
-                        const uint32_t k = (uint32_t)(t * kWave + ln);
-                        u[q * kSteps + t] = k < l ? src[k] : kPad;
-                    }
-                }
-            };
-            double mine = 0.0;
-            uint32_t u[kQ * kSteps], nu[kQ * kSteps];
-            load(0, u);
-            for (uint32_t j = 0; j < cnt; j += kQ) {
-                if (j + kQ < cnt) load(j + kQ, nu);
-                float cv[kQ * kSteps];
-                gather(u, cv, std::integral_constant<int, kQ * kSteps>{});
-                double s[kQ];
-#pragma unroll
-                for (int q = 0; q < kQ; q++) {
-                    s[q] = 0.0;
-#pragma unroll
-                    for (int t = 0; t < kSteps; t++) s[q] += (double)cv[q * kSteps + t];
-                }
-                const double t = wave_sum4(s);
-                if ((uint32_t)ln / kQ == j / kQ) mine = t;
-#pragma unroll
-                for (int q = 0; q < kQ * kSteps; q++) u[q] = nu[q];
-            }
-            if ((uint32_t)ln < cnt) {
-                if (one) finish(hv, mine, xo, dout);
-                else a.hubpart[c] = mine;
-            }
-        }
-        // in-hubs of several chunks wait for every block's sums: arrive now,
-        // wait once the other vertices are done
-        grid_signal(a.bar, xcc, gen, a.abort);
-        // (A2) every other vertex, a 64-vertex word per wave at a time: from
-        // the sliced in-edges (each lane sums its own vertex's row entries in
-        // order) or, without them, by a scheduled walk of the word's lists
-        if (g.sell_src) {
-            constexpr uint32_t U = 4;
-            for (uint32_t first = gwave; first < W; first += nwaves * kWave) {
-                const uint32_t cnt = min((uint32_t)kWave, (W - first + nwaves - 1) / nwaves);
-                // a lane holds one word's rows; what a word's vertices need in
-                // the end is loaded one word ahead, its in-edges one step ahead
-                uint32_t off = 0, nrow = 0;
-                if ((uint32_t)ln < cnt) {
-                    const uint32_t w = first + (uint32_t)ln * nwaves;
-                    off = g.sell_off[w];
-                    nrow = (g.sell_off[w + 1] - off) / kWave;
-                }
-                struct Own {
-                    uint32_t dout, din;
-                    float xo;
-                };
-                auto load_own = [&](uint32_t i) {
-                    Own o{0u, kPad, 0.f};
-                    const uint32_t v = (first + i * nwaves) * kWave + ln;
-                    if (v < n) {
-                        o.dout = g.row[v + 1] - g.row[v];
-                        o.din = g.cstart[v + 1] - g.cstart[v];
-                        o.xo = a.x[v];
-                    }
-                    return o;
-                };
-                auto load = [&](uint32_t i, uint32_t j, uint32_t *u) {
-                    const uint32_t rows = lane_value(nrow, (int)i);
-                    const uint32_t *S = g.sell_src + lane_value(off, (int)i) + ln;
-#pragma unroll
-                    for (uint32_t q = 0; q < U; q++) {
-                        u[q] = kPad;
-                        if (j + q < rows) u[q] = S[(size_t)(j + q) * kWave];
-                    }
-                };
-                uint32_t i = 0, j = 0, u[U], nu[U];
-                Own own = load_own(0), next = own;
-                load(0, 0, u);
-                double s = 0.0;
-                while (i < cnt) {
-                    if (j == 0 && i + 1 < cnt) next = load_own(i + 1);
-                    const uint32_t rows = lane_value(nrow, (int)i);
-                    const bool last = j + U >= rows;
-                    const uint32_t ni = last ? i + 1 : i, nj = last ? 0u : j + U;
-                    if (ni < cnt) load(ni, nj, nu);
-                    if (rows) {
-                        float cv[U];
-                        gather(u, cv, std::integral_constant<int, (int)U>{});
-#pragma unroll
-                        for (uint32_t q = 0; q < U; q++) s += (double)cv[q];
-                    }
-                    if (last) {
-                        if (own.din <= kPullHubDegree) finish((first + i * nwaves) * kWave + ln, s, own.xo, own.dout);
-                        s = 0.0;
-                        own = next;
-                    }
-#pragma unroll
-                    for (uint32_t q = 0; q < U; q++) u[q] = nu[q];
-                    i = ni;
-                    j = nj;
-                }
-            }
-        } else {
-            for (uint32_t w = gwave; w < W; w += nwaves) {
-                const uint32_t v = w * kWave + ln;
-                uint32_t b = 0, e = 0;
-                bool own = false;
-                if (v < n) {
-                    b = g.cstart[v];
-                    e = g.cstart[v + 1];
-                    own = e - b <= kPullHubDegree;
-                    if (!own) b = e;
-                }
-                const CSum s = wave_gather_csum(b, e, [&](uint32_t ed) {
-                    const uint32_t u = g.csrc[ed];
-                    return u < ncc ? s_cc[u] : cc[u];
-                });
-                if (own) finish(v, (double)s.hi + (double)s.lo, a.x[v], g.row[v + 1] - g.row[v]);
-            }
-        }
-        // (B) in-hubs of several chunks, eight lanes each (those of more than
-        // kHubWave chunks: the whole wave), dealt out so that the largest,
-        // which come first, fall to different waves; the first ones' data is
-        // loaded before the wait
-        constexpr uint32_t kHubLanes = 8, kHubs = kWave / kHubLanes, kHubWave = 8 * kHubLanes;
-        struct Hub {
-            uint32_t at, chunks, v, dout;
+        struct Own {
+            uint32_t dout;
             float xo;
         };
-        auto load_hub = [&](uint32_t h0) {
-            Hub b{0u, 0u, 0u, 0u, 0.f};
-            const uint32_t h = h0 + (uint32_t)ln / kHubLanes * nwaves;
-            if (h < g.nhubin) {
-                const uint2 d = g.hubin[h];
-                b.at = d.x;
-                b.chunks = d.y;
-                if (d.y > 1) {
-                    b.v = g.hugein[d.x].x;
-                    b.dout = g.row[b.v + 1] - g.row[b.v];
-                    b.xo = a.x[b.v];
-                }
-            }
-            return b;
+        auto pre = [&](bool has, uint32_t v) {
+            return has ? Own{g.row[v + 1] - g.row[v], a.x[v]} : Own{0u, 0.f};
         };
-        uint32_t h0 = gwave;
-        Hub hb = load_hub(h0);
-        ok = grid_wait(a.bar, gen, a.abort);
+        // x(v) from its in-edge sum, its last rank and its out-degree: FP32
+        // ranks and contributions, sums and the residual |x' - x| in FP64
+        auto finish = [&](bool has, uint32_t v, const Own &o, double s) {
+            if (!has) return;
+            const float xn = base + df * (float)s;
+            r_acc += fabs((double)xn - (double)o.xo);
+            a.x[v] = xn;
+            if (o.dout) cn[v] = xn / (float)o.dout;
+            else d_acc += (double)xn;
+        };
+        // in-hubs of several chunks wait for every block's sums: arrive after
+        // the chunks, wait once the other vertices are done
+        hub_chunk_sums(g, gather, bounds, gwave, nwaves, pre,
+                       [&](bool has, uint32_t c, uint32_t v, bool one, const Own &o, double s) {
+                           if (has && !one) a.hubpart[c] = s;
+                           finish(has && one, v, o, s);
+                       });
+        grid_signal(a.bar, xcc, gen, a.abort);
+        word_sums<kRows>(g, gather, bounds, gwave, nwaves, pre, finish);
+        ok = wide_hub_sums(g, a.hubpart, bounds, gwave, nwaves, [&]() { return grid_wait(a.bar, gen, a.abort); }, pre, finish);
         if (!ok) break;
-        while (h0 < g.nhubin) {
-            const Hub cur = hb;
-            h0 += nwaves * kHubs;
-            if (h0 < g.nhubin) hb = load_hub(h0);
-            double s = 0.0;
-            if (cur.chunks > 1 && cur.chunks <= kHubWave) {
-#pragma unroll 8
-                for (uint32_t k = (uint32_t)ln % kHubLanes; k < cur.chunks; k += kHubLanes) s += a.hubpart[cur.at + k];
-            }
-            s += dpp<kDppQuad1>(0.0, s);
-            s += dpp<kDppQuad2>(0.0, s);
-            s += dpp<kDppHalfMirror>(0.0, s);
-            uint64_t wide = ballot(cur.chunks > kHubWave);
-            while (wide) {
-                const int l = first_lane(wide);
-                const uint32_t at = lane_value(cur.at, l), chunks = lane_value(cur.chunks, l);
-                double t = 0.0;
-                for (uint32_t k = ln; k < chunks; k += kWave) t += a.hubpart[at + k];
-                t = wave_sum_f64(t);
-                if (ln / (int)kHubLanes == l / (int)kHubLanes) s = t;
-                wide &= ~(0xFFull << l);
-            }
-            if (ln % (int)kHubLanes == 0 && cur.chunks > 1) finish(cur.v, s, cur.xo, cur.dout);
-        }
         put_part(it + 1, r_acc, d_acc);
         it++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
@@ -591,12 +682,13 @@ struct PrDdArgs {
     CSum *y;           // unnormalised ranks [n], compensated FP32
     float *r;          // residuals [n]: r + rlo, the rounding error of every
     float *rlo;        // atomic addition into r collected in rlo
-    float *p;          // d r / outdeg of this round's active vertices [n]
+    float *p;          // 2 rows: d r / outdeg of this / the next round's active vertices
+    double *hubpart;   // [nhugein] chunk sums of pull rounds
     uint64_t *abit;    // 2 x W: active vertices of rounds k (k % 2)
     uint32_t *queue;   // 2 x qcap: vertices whose residual crossed theta
     uint32_t qcap;
     FrontierCtr *ctr;  // [0,1]: activation totals; [2,3,4]: queue appends
-    PrPart *part;      // kMaxBlocks partials for the final sums
+    PrPart *part;      // 2 x kMaxBlocks partials: pull rounds' counts, the final sums
     GridBarrier bar;
     uint32_t *abort;
     DevStats *stats;
@@ -606,7 +698,6 @@ struct PrDdArgs {
     int32_t force;     // -1 auto, 0 push, 1 pull
     uint32_t max_rounds;
     uint32_t probe;
-    uint32_t iterative;  // rounds chosen by the ITERATIVE scheme's predicted times
     int32_t it_force;    // ITERATIVE: -1, or the variant every round runs (kItPullTd...)
     float ticks_per_us;  // wall clock rate
     float cut;           // sample-based priority for ASYNC_PUSH_TD rounds (0: off)
@@ -697,11 +788,9 @@ struct IterativePolicy {
 };
 
 // In-hub chunks and slice rows a wave of a residual pull round keeps in flight.
-constexpr int kDdChunks = 2;
-constexpr int kDdRows = 8;
-
 struct DdRound {
     const PrDdArgs *a;
+    const float *p;    // this round's row
     double theta;
     Stager S;
     unsigned long long count;
@@ -709,30 +798,20 @@ struct DdRound {
     bool qdeg;
 };
 
-// Add `add` to v's residual (atomically when `atomic`), queueing v if this
-// addition took its residual across theta. An atomic addition returns the
-// old value, so the lane recomputes the rounded sum the atomic stored and
-// adds its rounding error (TwoSum, Knuth) to rlo[v]. Wave-convergent.
-__device__ __forceinline__ void dd_accumulate(DdRound &R, bool act, uint32_t v, CSum add, bool atomic)
+// Add `add` to v's residual atomically, queueing v if this addition took its
+// residual across theta. The addition returns the old value, so the lane
+// recomputes the rounded sum it stored and adds its rounding error (TwoSum,
+// Knuth) to rlo[v]. Wave-convergent.
+__device__ __forceinline__ void dd_accumulate(DdRound &R, bool act, uint32_t v, float add)
 {
     bool crossed = false;
-    const float ad = csum_value(add);
-    if (act && ad > 0.f) {
-        float old;
-        if (atomic) {
-            old = atomicAdd(&R.a->r[v], add.hi);
-            const float s = old + add.hi;
-            const float bb = s - old;
-            const float err = (old - (s - bb)) + (add.hi - bb) + add.lo;
-            if (err != 0.f) atomicAdd(&R.a->rlo[v], err);
-        } else {
-            CSum c{R.a->r[v], R.a->rlo[v]};
-            old = c.hi;
-            c = csum_merge(c, add);
-            R.a->r[v] = c.hi;
-            R.a->rlo[v] = c.lo;
-        }
-        crossed = (double)old < R.theta && (double)old + (double)ad >= R.theta;
+    if (act && add > 0.f) {
+        const float old = atomicAdd(&R.a->r[v], add);
+        const float s = old + add;
+        const float bb = s - old;
+        const float err = (old - (s - bb)) + (add - bb);
+        if (err != 0.f) atomicAdd(&R.a->rlo[v], err);
+        crossed = (double)old < R.theta && (double)old + (double)add >= R.theta;
         R.count += crossed;
         if (crossed && R.qdeg) R.qscout += R.a->g.row[v + 1] - R.a->g.row[v];
     }
@@ -753,7 +832,7 @@ __device__ __forceinline__ void dd_push_word(DdRound &R, uint64_t word, uint32_t
         b = g.row[u];
         dg = g.row[u + 1] - b;
         if (dg > kHugeDegree) dg = 0;
-        if (dg) pu = a.p[u];
+        if (dg) pu = R.p[u];
     }
     const uint32_t incl = wave_incl_scan(dg);
     const uint32_t total = lane_value(incl, kWave - 1);
@@ -765,11 +844,13 @@ __device__ __forceinline__ void dd_push_word(DdRound &R, uint64_t word, uint32_t
         const uint32_t e = shfl(off, k) + j;
         const float pk = __shfl(pu, k, kWave);
         const uint32_t v = act ? g.col[e] : 0u;
-        dd_accumulate(R, act, v, CSum{pk, 0.f}, true);
+        dd_accumulate(R, act, v, pk);
     }
 }
 
-template <int BS>
+// kIter: rounds chosen by the ITERATIVE scheme's predicted times. Its state is
+// not kept by the other runs' kernel, which has few registers to spare.
+template <int BS, bool kIter>
 __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
 {
     if (a.probe) {
@@ -792,14 +873,13 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
     FrontierCtr *act_ctr = a.ctr;       // 2 slots
     FrontierCtr *q_ctr = a.ctr + 2;     // 3 slots
 
-    __shared__ double s_smp[kPrioSort];
-    // pull rounds test the active bits of the lowest ids (in a degree-ordered
-    // graph the sources of most in-edges) in an LDS copy of the bitmap
+    __shared__ double s_smp[kIter ? kPrioSort : 1];
 #ifndef SG_PRDD_LDS
-#define SG_PRDD_LDS 8
+#define SG_PRDD_LDS 30
 #endif
-    constexpr uint32_t kAbLds = SG_PRDD_LDS * BS;
-    __shared__ uint64_t s_ab[kAbLds];
+    using Hot = Staged<BS, SG_PRDD_LDS>;
+    __shared__ __align__(16) float s_p[Hot::kLds + 4];
+    if (threadIdx.x == 0) s_p[Hot::kLds] = 0.f;
     __shared__ PrPart s_red2[WPB];
     __shared__ PrPart s_glob;
     __shared__ unsigned long long s_red[2][WPB];
@@ -820,7 +900,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
     }
     // stamped barriers: the block completing each one records the wall clock,
     // so every block derives the same round times for the ITERATIVE scheme
-    bool ok = grid_sync<true>(a.bar, xcc, gen, a.abort);
+    bool ok = grid_sync<kIter>(a.bar, xcc, gen, a.abort);
     __shared__ unsigned long long s_stamp;
     IterativePolicy ipol;
     unsigned long long stamp0 = 0, stamp_prev = 0;
@@ -830,10 +910,11 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
 
     uint32_t k = 0, pushes = 0, pulls = 0;
     unsigned long long ptrace = 0;
+    float *pc = a.p, *pn = a.p + contrib_stride(n);  // this round's and the next round's row of p
     while (ok) {
         if (a.max_rounds && k >= a.max_rounds) break;
         // ---- activation: move residual >= theta into y, set p and the bit
-        if (threadIdx.x == 0) s_stamp = barrier_stamp(a.bar);
+        if (kIter && threadIdx.x == 0) s_stamp = barrier_stamp(a.bar);
         read_counts(&q_ctr[k % 3], s_lvl);
         __syncthreads();
         const RoundCounts qc = unpack_counts(s_lvl, a.qcap);
@@ -842,7 +923,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
         // ITERATIVE: time the round that just ended, then pick this round's
         // variant (topology-driven ones rebuild the active set by a scan)
         int var = -1;
-        if (a.iterative) {
+        if (kIter) {
             if (k == 0) {
                 stamp0 = stamp;
             } else {
@@ -860,7 +941,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
             csum_add(yu, ru);
             a.y[u] = yu;
             const uint32_t dout = g.row[u + 1] - g.row[u];
-            if (dout) a.p[u] = df * ru / (float)dout;
+            if (dout) pc[u] = df * ru / (float)dout;
             scout += dout;
             cnt++;
         };
@@ -870,9 +951,10 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
         // or once the queue holds an eighth of the vertices (it holds every
         // residual >= theta, so a scan finds the same set): reading all residuals
         // in order then costs less than two returning atomics per entry
-        if (k == 0 || qc.overflow || held || var == kItPullTd || var == kItPushTd || qc.qlen > n / 8) {
+        const bool scan = k == 0 || qc.overflow || held || var == kItPullTd || var == kItPushTd || qc.qlen > n / 8;
+        if (scan) {
             double thr = theta;
-            if (var == kItPushTd && a.cut > 0.f) thr = fmax(theta, sampled_threshold<BS>(a, k, s_smp));
+            if (kIter && var == kItPushTd && a.cut > 0.f) thr = fmax(theta, sampled_threshold<BS>(a, k, s_smp));
             for (uint32_t w = gwave; w < W; w += nwaves) {
                 const uint32_t v = w * 64 + ln;
                 bool act = false;
@@ -884,6 +966,8 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                         a.r[v] = 0.f;
                         a.rlo[v] = 0.f;
                         activate(v, rv);
+                    } else {
+                        pc[v] = 0.f;  // a pull round reads every source's
                     }
                 }
                 const uint64_t m = ballot(act);
@@ -921,16 +1005,22 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
         __syncthreads();
         if (ac.count == 0 && !ac.has_huge) break;  // every residual is below theta
         held = ac.has_huge;
+        auto pulls_at = [&](unsigned long long sc) {
+            return a.force >= 0 ? a.force == 1 : (double)sc > a.total_wl / a.alpha;
+        };
         bool pull;
         if (var >= 0) pull = var == kItPullTd;
-        else if (a.force >= 0) pull = a.force == 1;
-        else pull = (double)ac.scout > a.total_wl / a.alpha;
-        if (pull) {
-            pulls++;
-            if (k < 64) ptrace |= 1ull << k;
-        } else {
-            pushes++;
-        }
+        else pull = pulls_at(ac.scout);
+        auto note_round = [&](bool was_pull, const RoundCounts &c) {
+            if (was_pull) {
+                pulls++;
+                if (k < 64) ptrace |= 1ull << k;
+            } else {
+                pushes++;
+            }
+            if (var < 0 && gtid == 0) write_trace(a.trace, k, was_pull, c.count, c.scout, t_start);
+        };
+        note_round(pull, ac);
         if (var >= 0) {
             // the reference's input workload: edges for a topology-driven
             // round, the worklist's out-degree sum for a data-driven one
@@ -944,23 +1034,162 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                 t.in_edges = ac.scout;
                 a.trace[k] = t;  // ticks filled in when the round's end is known
             }
-        } else if (gtid == 0) {
-            write_trace(a.trace, k, pull, ac.count, ac.scout, t_start);
         }
-        if (blockIdx.x == 0) {
-            clear_ctr(&act_ctr[(k + 1) & 1]);
-            clear_ctr(&q_ctr[(k + 2) % 3]);
-        }
-        uint64_t *ab_next = a.abit + (size_t)((k + 1) & 1) * W;
-        for (uint32_t w = gtid; w < W; w += nthreads) ab_next[w] = 0;
-
         DdRound R;
         R.a = &a;
         R.theta = theta;
-        R.S = Stager{a.queue + (size_t)((k + 1) & 1) * a.qcap, a.qcap, &q_ctr[(k + 1) % 3], s_q, &s_qn, kLdsQ};
-        R.count = 0;
-        R.qscout = 0;
-        R.qdeg = a.iterative != 0;
+        R.qdeg = kIter;
+        // counters and bitmap of the rounds to come, and the queue of the next
+        auto begin_round = [&]() {
+            if (blockIdx.x == 0) {
+                clear_ctr(&act_ctr[(k + 1) & 1]);
+                clear_ctr(&q_ctr[(k + 2) % 3]);
+            }
+            R.p = pc;
+            R.S = Stager{a.queue + (size_t)((k + 1) & 1) * a.qcap, a.qcap, &q_ctr[(k + 1) % 3], s_q, &s_qn, kLdsQ};
+            R.count = 0;
+            R.qscout = 0;
+        };
+        begin_round();
+        if (pull && !scan) {
+            // the round's row of p still holds earlier rounds' entries
+            for (uint32_t v = gtid; v < n; v += nthreads)
+                if (!test_bit(ab, v)) pc[v] = 0.f;
+            ok = grid_sync(a.bar, xcc, gen, a.abort);
+            if (!ok) break;
+        }
+        // ---- pull rounds: each vertex adds what its in-edges bring and, if
+        // that takes its residual to theta, is activated for the next round in
+        // the same pass (the next row of p), with no queue and no pass over the
+        // residuals in between: a round of two grid barriers and one reading of
+        // the edges, as one of the power iteration. Rounds of the ITERATIVE
+        // scheme, and the last one before max_rounds, leave activation out.
+        // RMAT graph of 100 003 vertices, 1.4 M edges, nearly all active: 19 us a
+        // round, 2.1 ms a run (45 and 4.8 with activation in a pass of its own);
+        // ~10 of the 19 are the two barriers, the counts and the LDS copy, 5 the
+        // words' chains of in-edge steps, 3 the hubs.
+        bool more = true;
+        const Bounds bounds(g, gwave, nwaves);
+        if (pull) Hot::take(s_p, pc, n);
+        while (pull) {
+            const bool act_next = !kIter && !(a.max_rounds && k + 1 >= a.max_rounds);
+            Hot::wait();
+            __syncthreads();
+            const Gather<Hot::kLds> gather{pc, s_p, n};
+            constexpr uint32_t kRows = BS > 512 ? 8 : 16;
+            unsigned long long nscout = 0, ncnt = 0;
+            struct Own {
+                uint32_t dout;
+                CSum r;
+            };
+            struct Later {};  // loaded at the end
+            auto pre = [&](bool has, uint32_t v) {
+                Own o{0u, CSum{0.f, 0.f}};
+                if (has) {
+                    o.dout = g.row[v + 1] - g.row[v];
+                    o.r = CSum{a.r[v], a.rlo[v]};
+                }
+                return o;
+            };
+            auto finish = [&](bool has, uint32_t v, const Own &o, double s) {
+                const CSum add{(float)s, (float)(s - (double)(float)s)};
+                CSum c = csum_merge(o.r, add);
+                const float ru = csum_value(c);
+                const bool active = has && act_next && (double)ru >= theta;
+                bool crossed = false;
+                if (has && act_next) {
+                    float pv = 0.f;
+                    if (active) {
+                        CSum yv = a.y[v];
+                        csum_add(yv, ru);
+                        a.y[v] = yv;
+                        if (o.dout) pv = df * ru / (float)o.dout;
+                        nscout += o.dout;
+                        ncnt++;
+                        c = CSum{0.f, 0.f};
+                    }
+                    pn[v] = pv;
+                }
+                if (has && (s > 0.0 || active)) {
+                    a.r[v] = c.hi;
+                    a.rlo[v] = c.lo;
+                    const float ad = csum_value(add);
+                    crossed = kIter && (double)o.r.hi < theta && (double)o.r.hi + (double)ad >= theta;
+                    R.count += crossed;
+                    if (crossed && R.qdeg) R.qscout += o.dout;
+                }
+                if (kIter) stage(R.S, crossed, v);
+            };
+            auto later = [](bool, uint32_t) { return Later{}; };
+            hub_chunk_sums(g, gather, bounds, gwave, nwaves, later,
+                           [&](bool has, uint32_t c, uint32_t v, bool one, Later, double s) {
+                               if (has && !one) a.hubpart[c] = s;
+                               finish(has && one, v, pre(has && one, v), s);
+                           });
+            grid_signal(a.bar, xcc, gen, a.abort);
+            word_sums<kRows>(g, gather, bounds, gwave, nwaves, pre, finish);
+            ok = wide_hub_sums(
+                g, a.hubpart, bounds, gwave, nwaves, [&]() { return grid_wait(a.bar, gen, a.abort); }, later,
+                [&](bool has, uint32_t v, Later, double s) { finish(has, v, pre(has, v), s); });
+            if (!ok || !act_next) break;
+            // the next round's totals, by blocks: no atomics, and every wave
+            // adds them by itself
+            nscout = wave_sum_u64(nscout);
+            ncnt = wave_sum_u64(ncnt);
+            if (ln == 0) {
+                s_red[0][threadIdx.x / kWave] = nscout;
+                s_red[1][threadIdx.x / kWave] = ncnt;
+            }
+            __syncthreads();
+            if (threadIdx.x < kWave) {
+                nscout = wave_sum_u64(ln < WPB ? s_red[0][ln] : 0ull);
+                ncnt = wave_sum_u64(ln < WPB ? s_red[1][ln] : 0ull);
+                if (ln == 0)
+                    ((ulonglong2 *)a.part)[(size_t)((k + 1) & 1) * kMaxBlocks + blockIdx.x] = make_ulonglong2(nscout, ncnt);
+            }
+            ok = grid_sync(a.bar, xcc, gen, a.abort);
+            if (!ok) break;
+            k++;
+            {
+                float *const t = pc;
+                pc = pn;
+                pn = t;
+            }
+            Hot::take(s_p, pc, n);  // in flight while the counts are added
+            RoundCounts nc{};
+            for (uint32_t i = ln; i < gridDim.x; i += kWave) {
+                const ulonglong2 q = ((const ulonglong2 *)a.part)[(size_t)(k & 1) * kMaxBlocks + i];
+                nc.scout += q.x;
+                nc.count += q.y;
+            }
+            nc.scout = wave_sum_u64(nc.scout);
+            nc.count = wave_sum_u64(nc.count);
+            if (nc.count == 0) {
+                more = false;  // every residual is below theta
+                Hot::wait();   // no copy into LDS outlives the block
+                break;
+            }
+            pull = pulls_at(nc.scout);
+            note_round(pull, nc);
+            if (!pull) {
+                // a push round reads the active set off its bitmap, and finds
+                // clear counters
+                if (blockIdx.x == 0) {
+                    for (int c = 0; c < 5; c++) clear_ctr(&a.ctr[c]);
+                }
+                ab = a.abit + (size_t)(k & 1) * W;
+                begin_round();
+                for (uint32_t w = gwave; w < W; w += nwaves) {
+                    const uint32_t v = w * 64 + ln;
+                    const uint64_t m = ballot(v < n && pc[v] != 0.f);
+                    if (ln == 0) ab[w] = m;
+                }
+                ok = grid_sync(a.bar, xcc, gen, a.abort);
+            }
+        }
+        if (!ok || !more) break;
+        uint64_t *ab_next = a.abit + (size_t)((k + 1) & 1) * W;
+        for (uint32_t w = gtid; w < W; w += nthreads) ab_next[w] = 0;
         if (!pull) {
             for (uint32_t c0 = 0; c0 < g.nhuge; c0 += nwaves * kWave) {
                 const uint32_t c = c0 + (uint32_t)ln * nwaves + gwave;
@@ -976,11 +1205,11 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                     mm &= mm - 1;
                     const uint32_t u = lane_value(dsc.x, t), beg = lane_value(dsc.y, t);
                     const uint32_t end = min(g.row[u + 1], beg + kHugeChunk);
-                    const float pu = a.p[u];
+                    const float pu = pc[u];
                     for (uint32_t e0 = beg; e0 < end; e0 += kWave) {
                         const uint32_t e = e0 + ln;
                         const bool act = e < end;
-                        dd_accumulate(R, act, act ? g.col[e] : 0u, CSum{pu, 0.f}, true);
+                        dd_accumulate(R, act, act ? g.col[e] : 0u, pu);
                     }
                 }
             }
@@ -988,107 +1217,11 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                 const uint64_t word = ab[w];
                 if (word) dd_push_word(R, word, w);
             }
-        } else {
-            const uint32_t nab = min(W, kAbLds);
-            for (uint32_t i = threadIdx.x; i < nab; i += BS) s_ab[i] = ab[i];
-            __syncthreads();
-            auto active = [&](uint32_t u) -> bool {
-                const uint32_t w = u >> 6;
-                return ((w < nab ? s_ab[w] : ab[w]) >> (u & 63)) & 1;
-            };
-            // in-hub chunks, kDdChunks per wave together with every load of a
-            // stage issued for all of them before any is used, their sums
-            // merged into the hubs by one lane each. A wave's chunks are
-            // nwaves apart, so a short list still spreads over every wave.
-            constexpr int kSteps = (int)(kPullChunk / kWave);
-            for (uint32_t c0 = gwave; c0 < g.nhugein; c0 += nwaves * kDdChunks) {
-                uint32_t cv[kDdChunks], cb[kDdChunks], ce[kDdChunks];
-#pragma unroll
-                for (int q = 0; q < kDdChunks; q++) {
-                    const uint32_t c = c0 + (uint32_t)q * nwaves;
-                    cv[q] = cb[q] = ce[q] = 0;
-                    if (c < g.nhugein) {
-                        const uint2 dsc = g.hugein[c];
-                        cv[q] = dsc.x;
-                        cb[q] = dsc.y;
-                        ce[q] = min(g.cstart[dsc.x + 1], dsc.y + kPullChunk);
-                    }
-                }
-                uint32_t u[kDdChunks][kSteps];
-#pragma unroll
-                for (int q = 0; q < kDdChunks; q++)
-#pragma unroll
-                    for (int t = 0; t < kSteps; t++) {
-                        const uint32_t e = cb[q] + (uint32_t)(t * kWave + ln);
-                        u[q][t] = e < ce[q] ? g.csrc[e] : 0xFFFFFFFFu;
-                    }
-                float pu[kDdChunks][kSteps];
-#pragma unroll
-                for (int q = 0; q < kDdChunks; q++)
-#pragma unroll
-                    for (int t = 0; t < kSteps; t++)
-                        pu[q][t] = u[q][t] != 0xFFFFFFFFu && active(u[q][t]) ? a.p[u[q][t]] : 0.f;
-                uint32_t hv = 0;
-                CSum hs{0.f, 0.f};
-#pragma unroll
-                for (int q = 0; q < kDdChunks; q++) {
-                    CSum s{0.f, 0.f};
-#pragma unroll
-                    for (int t = 0; t < kSteps; t++) csum_add(s, pu[q][t]);
-                    s = wave_csum(s);
-                    if (ln == q) {
-                        hv = cv[q];
-                        hs = s;
-                    }
-                }
-                dd_accumulate(R, ln < kDdChunks, hv, hs, true);
-            }
-            for (uint32_t w = gwave; w < W; w += nwaves) {
-                const uint32_t v = w * 64 + ln;
-                uint32_t b = 0, e = 0;
-                bool own = false;
-                if (v < n) {
-                    b = g.cstart[v];
-                    e = g.cstart[v + 1];
-                    own = e - b <= kPullHubDegree;
-                    if (!own) b = e;
-                }
-                CSum s{0.f, 0.f};
-                if (g.sell_src) {
-                    // by the sliced in-edges, a lane per vertex: its sum stays
-                    // in registers, with no edge scheduling and no segmented
-                    // scans. RMAT graph of 100 003 vertices, 1.4 M edges,
-                    // nearly all active: 95 -> 45 us a round, 9.6 -> 4.8 ms a run
-                    // (rows in flight 4, 8, 16: within 5 %)
-                    const uint32_t beg = g.sell_off[w];
-                    const uint32_t rows = (g.sell_off[w + 1] - beg) / kWave;
-                    const uint32_t *S = g.sell_src + beg + ln;
-                    const uint32_t deg = e - b;
-                    for (uint32_t j0 = 0; j0 < rows; j0 += kDdRows) {
-                        uint32_t u[kDdRows];
-                        float pu[kDdRows];
-#pragma unroll
-                        for (int q = 0; q < kDdRows; q++)
-                            u[q] = j0 + q < deg ? S[(size_t)(j0 + q) * kWave] : 0xFFFFFFFFu;
-#pragma unroll
-                        for (int q = 0; q < kDdRows; q++)
-                            pu[q] = u[q] != 0xFFFFFFFFu && active(u[q]) ? a.p[u[q]] : 0.f;
-#pragma unroll
-                        for (int q = 0; q < kDdRows; q++) csum_add(s, pu[q]);
-                    }
-                } else {
-                    s = wave_gather_csum(b, e, [&](uint32_t ed) {
-                        const uint32_t u = g.csrc[ed];
-                        return active(u) ? a.p[u] : 0.f;
-                    });
-                }
-                dd_accumulate(R, own, v, s, false);
-            }
         }
         publish_counts<WPB>(&q_ctr[(k + 1) % 3], R.qscout, R.count, false, s_red);
         flush_stage(R.S, s_flush);
         k++;
-        ok = grid_sync<true>(a.bar, xcc, gen, a.abort);
+        ok = grid_sync<kIter>(a.bar, xcc, gen, a.abort);
     }
 
     // ---- absorb what residual is left, then normalise
@@ -1107,12 +1240,13 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
             rsum += (double)rv + (double)rl;
         }
         const PrPart t = block_part<WPB>(rsum, ysum, s_red2);
-        if (threadIdx.x == 0) a.part[blockIdx.x] = t;
+        // (the set that no block reads any more)
+        if (threadIdx.x == 0) a.part[(size_t)((k + 1) & 1) * kMaxBlocks + blockIdx.x] = t;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
     PrPart tot{0.0, 1.f, 0.f};
     if (ok) {
-        tot = grid_part<BS>(a.part, gridDim.x, s_red2, &s_glob);
+        tot = grid_part<BS>(a.part + (size_t)((k + 1) & 1) * kMaxBlocks, gridDim.x, s_red2, &s_glob);
         const float ys = csum_value(CSum{tot.dhi, tot.dlo});
         const float inv = ys > 0.f ? 1.0f / ys : 0.f;
         for (uint32_t v = gtid; v < n; v += nthreads) a.x[v] = csum_value(a.y[v]) * inv;
@@ -1230,8 +1364,9 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
     } else {
         const int force = mode == SG_PR_ITERATIVE ? -1 : forced_direction(o);
         if (force < -1) SG_FAIL(SG_ERR_UNSUPPORTED, "sg_pagerank: data-driven mode takes push/pull DD variants only");
-        // y (n compensated floats) | r | rlo | p (n floats each) | partials
-        const uint64_t off_part = (n * 8 + 3 * n * 4 + 15) / 16 * 16;
+        // y (n compensated floats) | r | rlo (n floats each) | two rows of p | hubpart | partials
+        const uint64_t off_hub = n * 16 + 2ull * contrib_stride(d.n) * 4;
+        const uint64_t off_part = off_hub + ((uint64_t)d.nhugein * 8 + 15) / 16 * 16;
         if ((rc = engine_ensure_aux(e, off_part + part_bytes))) return rc;
         char *base = (char *)e->aux;
         PrDdArgs a{};
@@ -1241,6 +1376,7 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
         a.r = (float *)(base + n * 8);
         a.rlo = (float *)(base + n * 12);
         a.p = (float *)(base + n * 16);
+        a.hubpart = (double *)(base + off_hub);
         a.part = (PrPart *)(base + off_part);
         a.abit = e->bitmaps;
         a.queue = e->queues;
@@ -1256,7 +1392,7 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
         a.total_wl = (double)d.m * o.edge_factor;
         a.force = force;
         a.max_rounds = max_iter ? (uint32_t)max_iter : 100000u;
-        a.iterative = mode == SG_PR_ITERATIVE;
+        const bool it = mode == SG_PR_ITERATIVE;
         a.it_force = it_force;
         a.ticks_per_us = (float)(e->wall_khz / 1000.0);
         a.cut = 0.f;
@@ -1265,10 +1401,20 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
                 SG_FAIL(SG_ERR_RANGE, "sg_pagerank: sample-based priority needs 0 < cut_threshold < 1");
             a.cut = o.cut_threshold;
         }
-        switch (bs) {
-        case 256: rc = launch_persistent<PrDdArgs, k_pr_dd<256>>(e, a, 256); break;
-        case 512: rc = launch_persistent<PrDdArgs, k_pr_dd<512>>(e, a, 512); break;
-        default: rc = launch_persistent<PrDdArgs, k_pr_dd<1024>>(e, a, 1024); break;
+        // Up to 2^18 vertices a round is latency: blocks of 512 threads, whose
+        // waves have registers for 16 rows in flight and none to spill (100 003
+        // vertices 2124 us, of 1024 threads 2490; 400 001: 3611 and 3637). Beyond,
+        // twice the waves hide more (1 000 001: 7465 and 6969).
+        const int dbs = o.block_size || d.n > (1u << 18) ? bs : 512;
+        switch (dbs) {
+        case 256:
+            rc = it ? launch_persistent<PrDdArgs, k_pr_dd<256, true>>(e, a, 256) : launch_persistent<PrDdArgs, k_pr_dd<256, false>>(e, a, 256);
+            break;
+        case 512:
+            rc = it ? launch_persistent<PrDdArgs, k_pr_dd<512, true>>(e, a, 512) : launch_persistent<PrDdArgs, k_pr_dd<512, false>>(e, a, 512);
+            break;
+        default:
+            rc = it ? launch_persistent<PrDdArgs, k_pr_dd<1024, true>>(e, a, 1024) : launch_persistent<PrDdArgs, k_pr_dd<1024, false>>(e, a, 1024);
         }
     }
     if (rc) return rc;

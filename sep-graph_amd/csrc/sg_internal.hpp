@@ -210,7 +210,7 @@ struct sg_engine {
         // launches the kernel in residency-probe mode with a given grid
         std::function<int(int blocks, uint32_t *words)> probe;
     };
-    static constexpr int kMaxGrids = 32;
+    static constexpr int kMaxGrids = 64;
     PGrid grids[kMaxGrids];
     int ngrids = 0;
     bool needs_bar_reset = false;

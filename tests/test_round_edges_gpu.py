@@ -270,3 +270,39 @@ def test_calls_back_to_back_and_their_time(sg, gpu, call, k):
         assert np.allclose(got, want, rtol=1e-5, atol=1e-12)
     else:
         assert np.array_equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("block_size,n", [(256, 7679), (256, 7681), (512, 15361), (1024, 30719), (1024, 30721), (0, 20000)])
+def test_residual_pull_rounds_and_push_rounds_agree(sg, orc, gpu, block_size, n, relabel):
+    """Pull rounds activate in the pass that sums; push rounds in one of their
+    own. Stopped after the same number of rounds, whatever the directions, the
+    ranks are the same; run to the end they are the oracle's."""
+    rng = np.random.default_rng(n)
+    hubs = [d for d in (65, 256, 257, 2049, 16385, 20000) if d < n]
+    src = np.concatenate([rng.choice(n, d, replace=False) for d in hubs] + [rng.integers(0, n, 4 * n)])
+    dst = np.concatenate([np.full(d, i * 7) for i, d in enumerate(hubs)] + [rng.integers(0, n, 4 * n) // 2])
+    row, col = sg.build_csr(n, src.astype(np.uint32), dst.astype(np.uint32))
+    graph = sg.Graph(sg.HostGraph(n, row, col, None), relabel=relabel)
+    bound = 3 * 2.0**-24 / 0.15  # three FP32 roundings per rank and round, carried on by 1 / (1 - d)
+
+    def ranks(max_iter, tol, **opts):
+        e = sg.Engine(graph, block_size=block_size, **opts)
+        e.pagerank(0.85, tol, max_iter, sg.PR_PUSH_DD)
+        return e.gather(np.float32).astype(np.float64), e.stats()
+
+    for rounds in (1, 2, 3, 7):
+        push, ps = ranks(rounds, 1e-9, force_variant="async_push_dd")
+        pull, qs = ranks(rounds, 1e-9, force_variant="async_pull_dd")
+        assert ps["rounds"] == qs["rounds"] == rounds and ps["pull_rounds"] == 0 and qs["pull_rounds"] == rounds
+        assert np.abs(push - pull).sum() / push.sum() < bound
+    ref = orc.pagerank(row, col, 0.85, 1e-12)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    # thresholds from "every round pulls" to "none does": both directions, either after the other
+    mixed = 0
+    for alpha in (1e9, 1e4, 1e3, 300.0, 100.0, 30.0, 10.0, 1e-3):
+        got, st = ranks(0, 1e-9, alpha=alpha)
+        mixed += st["push_rounds"] > 0 and st["pull_rounds"] > 0
+        assert np.abs(got - ref).sum() / ref.sum() < bound
+    assert mixed
