@@ -676,6 +676,9 @@ struct MsBfsArgs {
     uint64_t *F;          // 3 x n level masks
     int32_t *out;         // levels of source s in row out_row(orow, s), -1 when unreached
     const uint32_t *orow;
+    uint8_t *lev;         // optional (with inv): level rows [n][lev_row(nsrc)], see LevelRows
+    const uint32_t *inv;  // optional: out is in the caller's order, vertex v there is inv[v] here
+    const uint32_t *perm; // (with inv) its inverse
     uint32_t *ring_v;     // 2 x n: entries of level L in half L % 2
     uint64_t *ring_m;
     uint32_t *ctl;        // [1] overflow, [2 + h] entries in ring half h
@@ -690,6 +693,56 @@ struct MsBfsArgs {
     uint32_t max_rounds;
     uint32_t probe;
 };
+
+// Levels in the caller's order, when that is another than the device's. A pass
+// over the finished rows that gathers them by `inv` reads 4 bytes from a line
+// of its own per level: RMAT-19, 64 sources, 100 of 533 us. Instead the levels
+// are kept as a row of bytes per vertex, one per source, and the kernel ends by
+// reading whole rows in the caller's order, 64 vertices a wave, and writing each
+// source's 64 levels together (408 us). Levels of 255 and more are written to
+// their place at once, and their bytes say so.
+constexpr uint32_t kDeepLevel = 255;
+
+__host__ __device__ constexpr uint32_t lev_row(uint32_t nsrc)
+{
+    uint32_t b = 4;  // at most 4 nsrc: the rows fit where nsrc rows of int32 do
+    while (b < nsrc) b *= 2;
+    return b;
+}
+
+// The four bytes of `x` that `bits` names become `b`'s.
+__device__ __forceinline__ uint32_t put_bytes(uint32_t x, uint32_t bits, uint32_t b)
+{
+    const uint32_t m = (((bits & 15u) * 0x00204081u) & 0x01010101u) * 0xFFu;
+    return (x & ~m) | (b & m);
+}
+
+// Byte `level` for the sources in `nw` into a vertex's row; `fresh`: none of
+// its bytes counts yet.
+__device__ __forceinline__ void put_levels(uint8_t *row, uint32_t bytes, uint64_t nw, bool fresh, uint32_t level)
+{
+    const uint32_t b = level * 0x01010101u;
+    if (bytes < 16) {
+        for (uint32_t d = 0; d < bytes / 4; d++) {
+            uint32_t *x = (uint32_t *)row + d;
+            const uint32_t bits = (uint32_t)(nw >> (4 * d)) & 15u;
+            if (bits) *x = put_bytes(fresh ? 0u : *x, bits, b);
+        }
+        return;
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < 4; c++) {
+        const uint32_t bits = (uint32_t)(nw >> (16 * c)) & 0xFFFFu;
+        if (16 * c >= bytes || !bits) continue;
+        uint4 x = make_uint4(0u, 0u, 0u, 0u);
+        if (!fresh) x = ((uint4 *)row)[c];
+        x.x = put_bytes(x.x, bits, b);
+        x.y = put_bytes(x.y, bits >> 4, b);
+        x.z = put_bytes(x.z, bits >> 8, b);
+        x.w = put_bytes(x.w, bits >> 12, b);
+        ((uint4 *)row)[c] = x;
+    }
+}
 
 template <int BS>
 __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
@@ -710,6 +763,7 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
     BarState gen = bar_begin(a.bar, xcc);
     const long long t_start = wall_clock64();
     const uint64_t bm = a.nsrc >= 64 ? ~0ull : ((1ull << a.nsrc) - 1);
+    const uint32_t lb = lev_row(a.nsrc);
 
     __shared__ unsigned long long s_red[2][WPB];
     __shared__ unsigned long long s_lvl[5];
@@ -745,7 +799,10 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
             }
         }
         const bool lead = has && firstl == ln;
-        if (has) a.out[out_row(a.orow, ln, n) + v] = 0;
+        if (has) {
+            if (a.lev) a.lev[(size_t)v * lb + ln] = 0;
+            else a.out[out_row(a.orow, ln, n) + v] = 0;
+        }
         if (lead) {
             a.seen[v] = m;
             a.F[v] = m;
@@ -801,9 +858,23 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
             const uint32_t v = w * 64 + ln;
             const uint64_t nw = v < n ? Fn[v] : 0ull;
             if (nw) {
-                a.seen[v] |= nw;
+                const uint64_t old = a.seen[v];
+                a.seen[v] = old | nw;
                 scout += g.row[v + 1] - g.row[v];
                 cnt++;
+                if (a.lev) put_levels(a.lev + (size_t)v * lb, lb, nw, old == 0, min(L + 1, kDeepLevel));
+            }
+            if (a.lev) {
+                if (L + 1 >= kDeepLevel) {
+                    uint64_t left = nw;
+                    const uint32_t at = nw ? a.perm[v] : 0u;
+                    while (left) {
+                        const int s = first_lane(left);
+                        left &= left - 1;
+                        a.out[out_row(a.orow, s, n) + at] = (int32_t)(L + 1);
+                    }
+                }
+                continue;
             }
             // one pass per source present in this word: lanes write consecutive vertices
             uint64_t any = wave_or_u64(nw);
@@ -821,7 +892,36 @@ __global__ __launch_bounds__(BS) void k_msbfs(MsBfsArgs a)
     }
     // -1 where no query of the batch came by (every block left the loop after
     // the same barrier, and `seen` holds all levels)
-    if (ok)
+    if (ok && a.lev) {
+        for (uint32_t w = gwave; w < W; w += nwaves) {
+            const uint32_t v = w * 64 + ln;
+            if (v >= n) break;
+            const uint32_t u = a.inv[v];
+            const uint64_t seen = a.seen[u];
+            const uint8_t *row = a.lev + (size_t)u * lb;
+            uint32_t x[16];
+            if (lb < 16) {
+                for (uint32_t d = 0; d < 4; d++) x[d] = d < lb / 4 && seen ? ((const uint32_t *)row)[d] : 0u;
+            } else {
+#pragma unroll
+                for (uint32_t c = 0; c < 4; c++) {
+                    uint4 y = make_uint4(0u, 0u, 0u, 0u);
+                    if (16 * c < lb && seen) y = ((const uint4 *)row)[c];
+                    x[4 * c] = y.x;
+                    x[4 * c + 1] = y.y;
+                    x[4 * c + 2] = y.z;
+                    x[4 * c + 3] = y.w;
+                }
+            }
+#pragma unroll
+            for (uint32_t s = 0; s < 64; s++) {
+                if (s >= a.nsrc) break;
+                const uint32_t b = (x[s / 4] >> (8 * (s % 4))) & 0xFFu;
+                const bool in = (seen >> s) & 1;
+                if (!in || b != kDeepLevel) a.out[out_row(a.orow, s, n) + v] = in ? (int32_t)b : -1;
+            }
+        }
+    } else if (ok)
         for (uint32_t w = gwave; w < W; w += nwaves) {
             const uint32_t v = w * 64 + ln;
             const uint64_t not_seen = v < n ? bm & ~a.seen[v] : 0ull;
@@ -1436,6 +1536,11 @@ int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, vo
         a.ctl = (uint32_t *)(base + L.off[4]);
         a.out = (int32_t *)out;
         a.orow = dev_orow;
+        if (inv) {
+            a.lev = (uint8_t *)e->work;
+            a.inv = inv;
+            a.perm = e->g->d_perm;
+        }
         a.alpha = alpha;
         a.beta = o.beta;
         a.total_wl = total_wl;
@@ -1519,9 +1624,13 @@ int ms_run(sg_engine *e, int kind, const uint32_t *sources, int32_t k, int32_t b
     const uint64_t n = d.n;
     const uint64_t rows = kind == kMsBcSum ? 1 : (uint64_t)k;
     void *res = nullptr;
-    // batched SSSP writes the caller's order itself
-    const bool direct = kind == kMsSssp;
-    if (direct) {
+    // batched BFS and SSSP write the caller's order themselves
+    const bool direct = kind == kMsSssp || kind == kMsBfs;
+    if (kind == kMsBfs) {
+        // (a relabelled graph's level rows are kept in the work rows)
+        if ((rc = engine_result_rows(e, rows, &res))) return rc;
+        res = e->value;
+    } else if (direct) {
         if ((rc = engine_ensure_value(e, rows * n * 4))) return rc;
         res = e->value;
     } else if ((rc = engine_result_rows(e, rows, &res))) {

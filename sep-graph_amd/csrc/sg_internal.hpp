@@ -252,7 +252,8 @@ int ms_prepare(sg_engine *e, int kind);
 // host), asynchronously on the engine's stream. Results: row dev_orow[i] (or i when null) of `out`, n
 // elements per row (int32 levels, uint32 distances, FP32 dependencies); for
 // kMsBcSum, `out` is the n-float BC sum written by the batch with `last`. Rows
-// are in device order; for kMsSssp, `inv` (optional) puts them in the caller's.
+// are in device order; for kMsBfs and kMsSssp, `inv` (optional) puts them in the
+// caller's (kMsBfs then keeps rows of its own in the engine's work rows).
 int ms_launch(sg_engine *e, int kind, const uint32_t *dev_src, uint32_t nsrc, void *out, const uint32_t *dev_orow,
               bool first, bool last, const uint32_t *inv = nullptr, const uint32_t *host_src = nullptr);
 

@@ -306,3 +306,34 @@ def test_residual_pull_rounds_and_push_rounds_agree(sg, orc, gpu, block_size, n,
         mixed += st["push_rounds"] > 0 and st["pull_rounds"] > 0
         assert np.abs(got - ref).sum() / ref.sum() < bound
     assert mixed
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nsrc", [1, 3, 4, 5, 8, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("graph", ["path", "random", "islands"])
+def test_bfs_batch_level_rows(sg, gpu, graph, nsrc):
+    """Levels of a renumbered graph, kept as bytes until the end: rows of each
+    width, levels around the last a byte holds, sources that share a vertex,
+    vertices that no source reaches."""
+    if graph == "path":
+        hg = path_graph(sg, 600)  # levels up to 599
+    elif graph == "random":
+        hg = random_graph(sg, 3001, 3, nsrc)
+    else:
+        v = np.arange(0, 900, 2, dtype=np.uint32)
+        row, col = sg.build_csr(901, v, v + 1, symmetrize=True)
+        hg = sg.HostGraph(901, row, col, None, undirected=True)
+    rng = np.random.default_rng(nsrc)
+    src = rng.integers(0, hg.n, nsrc).astype(np.uint32)
+    if nsrc > 2:
+        src[1] = src[0]
+        src[2] = 0
+    g = sg.Graph(hg, relabel=True)
+    e = sg.Engine(g)
+    one = sg.Engine(g)
+    for batch in (64, max(1, nsrc - 1)):
+        e.bfs_multi(src, batch)
+        got = e.gather(np.int32).reshape(nsrc, hg.n)
+        for i, s in enumerate(src):
+            one.bfs(int(s))
+            assert np.array_equal(got[i], one.gather(np.int32)), (batch, i)
