@@ -11,12 +11,14 @@
 // The ranks computed here are the normalised PageRank with uniform teleport
 // and uniform redistribution of dangling mass,
 //     x = (1-d)/n + d (P^T x + (sum of x over dangling vertices)/n),
-// stored as FP32. In the pull mode every sum (in-edges, dangling mass, L1
-// residual) is FP64, in a fixed order for a given grid, so repeated runs give
-// identical bits. In the residual mode the unnormalised ranks, the residuals
+// stored as FP32. Sums are compensated FP32 (hi + lo): in-edge sums and the
+// dangling mass, in the residual mode the unnormalised ranks, the residuals
 // (each atomic addition's rounding error, recomputed by the adding lane, goes
-// to a second FP32 array) and the normalising sum are compensated FP32 (hi +
-// lo, Neumaier); the residual mass absorbed at the end is reduced in FP64.
+// to a second FP32 array) and the normalising sum; only the L1 residual (pull)
+// and the residual mass absorbed at the end (DD) are reduced in FP64. In the
+// pull mode every reduction runs in a fixed order for a given grid, so repeated
+// runs give identical bits. (FP64 sums, two instructions per in-edge instead of
+// seven: RMAT-21 pull 1750 us and 1778, 100 003 vertices DD 2151 and 2182.)
 //
 // Pull TD: one lane per vertex sums x[u]/outdeg(u) (kept as an FP32 array
 // `contrib`, ping-ponged between iterations) over its in-edges, reading them
@@ -45,8 +47,9 @@ namespace {
 
 // ------------------------------------------- compensated FP32 accumulation
 // A sum kept as hi + lo, where lo collects the rounding error of every
-// addition into hi (Neumaier's variant of Kahan summation): FP32 storage and
-// arithmetic with an error close to one rounding of the final sum.
+// addition into hi (TwoSum, Knuth: exact, and without the comparison of
+// Neumaier's form): FP32 storage and arithmetic with an error close to one
+// rounding of the final sum.
 struct CSum {
     float hi, lo;
 };
@@ -54,7 +57,8 @@ struct CSum {
 __device__ __forceinline__ void csum_add(CSum &a, float x)
 {
     const float s = a.hi + x;
-    const float t = fabsf(a.hi) >= fabsf(x) ? (a.hi - s) + x : (x - s) + a.hi;
+    const float b = s - a.hi;
+    const float t = (a.hi - (s - b)) + (x - b);
     a.hi = s;
     a.lo += t;
 }
@@ -177,24 +181,23 @@ __device__ __forceinline__ CSum wave_gather_csum(uint32_t b, uint32_t e, F val)
 
 // ------------------------------------------------------------ pull TD kernel
 
-// Lanes of one row of 16 take each other's sums (every lane has the total).
-__device__ __forceinline__ double row_sum(double x)
+// The sum over each row of 16 lanes, in the row's first lane in a fixed order.
+__device__ __forceinline__ CSum row_csum(CSum x)
 {
-    x += dpp<kDppRowRor + 8>(0.0, x);
-    x += dpp<kDppRowRor + 4>(0.0, x);
-    x += dpp<kDppRowRor + 2>(0.0, x);
-    x += dpp<kDppRowRor + 1>(0.0, x);
+    const CSum none{0.f, 0.f};
+    x = csum_merge(x, dpp<kDppRowRor + 8>(none, x));
+    x = csum_merge(x, dpp<kDppRowRor + 4>(none, x));
+    x = csum_merge(x, dpp<kDppRowRor + 2>(none, x));
+    x = csum_merge(x, dpp<kDppRowRor + 1>(none, x));
     return x;
 }
 
-// (FP64 adds run at the rate of FP32 ones here: a conversion and an add per
-// in-edge where a compensated FP32 sum takes eight instructions.)
 // Four wave sums together: lane l gets that of s[l % 4]. Halves of the wave,
-// then rows of 16 lanes, trade places between two sums, so that three
-// additions leave one sum per row, where four scans would take 24.
-__device__ __forceinline__ double wave_sum4(const double (&s)[4])
+// then rows of 16 lanes, trade places between two sums, so that three merges
+// leave one sum per row and four more finish them, where four scans take 24.
+__device__ __forceinline__ CSum wave_csum4(const CSum (&s)[4])
 {
-    auto fold = [](double a, double b, bool half) {
+    auto fold = [](CSum a, CSum b, bool half) {
         uint32_t x[2], y[2];
         __builtin_memcpy(x, &a, 8);
         __builtin_memcpy(y, &b, 8);
@@ -207,11 +210,12 @@ __device__ __forceinline__ double wave_sum4(const double (&s)[4])
         }
         __builtin_memcpy(&a, x, 8);
         __builtin_memcpy(&b, y, 8);
-        return a + b;
+        return csum_merge(a, b);
     };
     // rows of (0, 2): 0 0 2 2; of (1, 3): 1 1 3 3; of both: 0 1 2 3
-    const double t = row_sum(fold(fold(s[0], s[2], true), fold(s[1], s[3], true), false));
-    return shfl(t, (lane() & 3) * 16);
+    const CSum t = row_csum(fold(fold(s[0], s[2], true), fold(s[1], s[3], true), false));
+    const int from = (lane() & 3) * 16;
+    return CSum{shfl(t.hi, from), shfl(t.lo, from)};
 }
 
 // ---------------------------------------------- sums over every in-edge list
@@ -355,21 +359,21 @@ __device__ __forceinline__ void hub_chunk_sums(const DevGraph &g, const G &gathe
                 }
             }
         };
-        double mine = 0.0;
+        CSum mine{0.f, 0.f};
         uint32_t u[kQ * kSteps], nu[kQ * kSteps];
         load(0, u);
         for (uint32_t j = 0; j < cnt; j += kQ) {
             if (j + kQ < cnt) load(j + kQ, nu);
             float cv[kQ * kSteps];
             gather.get(u, cv);
-            double s[kQ];
+            CSum s[kQ];
 #pragma unroll
             for (int q = 0; q < kQ; q++) {
-                s[q] = 0.0;
+                s[q] = CSum{0.f, 0.f};
 #pragma unroll
-                for (int t = 0; t < kSteps; t++) s[q] += (double)cv[q * kSteps + t];
+                for (int t = 0; t < kSteps; t++) csum_add(s[q], cv[q * kSteps + t]);
             }
-            const double t = wave_sum4(s);
+            const CSum t = wave_csum4(s);
             if ((uint32_t)ln / kQ == j / kQ) mine = t;
 #pragma unroll
             for (int q = 0; q < kQ * kSteps; q++) u[q] = nu[q];
@@ -403,7 +407,7 @@ __device__ __forceinline__ void word_sums(const DevGraph &g, const G &gather, co
             }
             const auto own = pre(has, v);
             const CSum s = wave_gather_csum(b, e, [&](uint32_t ed) { return gather.one(g.csrc[ed]); });
-            done(has, v, own, (double)s.hi + (double)s.lo);
+            done(has, v, own, s);
         }
         return;
     }
@@ -426,7 +430,7 @@ __device__ __forceinline__ void word_sums(const DevGraph &g, const G &gather, co
         uint32_t v = first * kWave + ln, nv = v, din = degree(v), ndin = din;
         auto own = pre(v < n, v), nown = own;
         load(0, 0, u);
-        double s = 0.0;
+        CSum s{0.f, 0.f};
         while (i < cnt) {
             if (j == 0 && i + 1 < cnt) {
                 nv = v + nwaves * kWave;
@@ -441,11 +445,11 @@ __device__ __forceinline__ void word_sums(const DevGraph &g, const G &gather, co
                 float cv[U];
                 gather.get(u, cv);
 #pragma unroll
-                for (uint32_t q = 0; q < U; q++) s += (double)cv[q];
+                for (uint32_t q = 0; q < U; q++) csum_add(s, cv[q]);
             }
             if (last) {
                 done(din <= kPullHubDegree, v, own, s);
-                s = 0.0;
+                s = CSum{0.f, 0.f};
                 v = nv;
                 din = ndin;
                 own = nown;
@@ -464,7 +468,7 @@ __device__ __forceinline__ void word_sums(const DevGraph &g, const G &gather, co
 // first ones' data is loaded before the wait. done(has, v, own, sum),
 // wave-convergent. Returns wait()'s result.
 template <typename Wait, typename Pre, typename Done>
-__device__ __forceinline__ bool wide_hub_sums(const DevGraph &g, const double *hubpart, const Bounds &bounds, uint32_t gwave,
+__device__ __forceinline__ bool wide_hub_sums(const DevGraph &g, const CSum *hubpart, const Bounds &bounds, uint32_t gwave,
                                               uint32_t nwaves, Wait wait, Pre pre, Done done)
 {
     constexpr uint32_t kHubLanes = Bounds::kHubLanes, kHubs = kWave / kHubLanes, kHubWave = 8 * kHubLanes;
@@ -481,21 +485,22 @@ __device__ __forceinline__ bool wide_hub_sums(const DevGraph &g, const double *h
             bd.hub(g, h0, nwaves);
             own = pre(bd.chunks > 1, bd.v);
         }
-        double s = 0.0;
+        CSum s{0.f, 0.f};
         if (cc > 1 && cc <= kHubWave) {
 #pragma unroll 8
-            for (uint32_t k = (uint32_t)ln % kHubLanes; k < cc; k += kHubLanes) s += hubpart[cat + k];
+            for (uint32_t k = (uint32_t)ln % kHubLanes; k < cc; k += kHubLanes) s = csum_merge(s, hubpart[cat + k]);
         }
-        s += dpp<kDppQuad1>(0.0, s);
-        s += dpp<kDppQuad2>(0.0, s);
-        s += dpp<kDppHalfMirror>(0.0, s);
+        const CSum none{0.f, 0.f};
+        s = csum_merge(s, dpp<kDppQuad1>(none, s));
+        s = csum_merge(s, dpp<kDppQuad2>(none, s));
+        s = csum_merge(s, dpp<kDppHalfMirror>(none, s));
         uint64_t wide = ballot(cc > kHubWave);
         while (wide) {
             const int l = first_lane(wide);
             const uint32_t wat = lane_value(cat, l), wc = lane_value(cc, l);
-            double t = 0.0;
-            for (uint32_t k = ln; k < wc; k += kWave) t += hubpart[wat + k];
-            t = wave_sum_f64(t);
+            CSum t{0.f, 0.f};
+            for (uint32_t k = ln; k < wc; k += kWave) t = csum_merge(t, hubpart[wat + k]);
+            t = wave_csum(t);
             if (ln / (int)kHubLanes == l / (int)kHubLanes) s = t;
             wide &= ~(0xFFull << l);
         }
@@ -508,8 +513,8 @@ struct PrArgs {
     DevGraph g;
     float *x;          // ranks [n]
     float *contrib;    // 2 rows: x[u] / outdeg(u) of the current / next iteration
-    double *hubpart;   // [nhugein] chunk sums
-    double2 *part;     // 2 x kMaxBlocks (residual, dangling) partials
+    CSum *hubpart;     // [nhugein] chunk sums
+    PrPart *part;      // 2 x kMaxBlocks (residual, dangling) partials
     GridBarrier bar;
     uint32_t *abort;
     DevStats *stats;
@@ -521,7 +526,7 @@ struct PrArgs {
 
 // What bounds an iteration: the in-edges whose source has no place in LDS,
 // each an L2 request for a line of which it needs 4 bytes. RMAT-21 (32.4 M
-// edges, 36 % of them such), 17 iterations: 1750 us, of which 1030 are these
+// edges, 36 % of them such), 17 iterations: 1778 us, of which 1030 are these
 // reads (11.7 M an iteration at 0.19 T/s; the L2s answer 0.27 T/s at most),
 // 210 the barriers, partial sums and LDS copy, the rest index reads, LDS reads
 // and the vertices' own data. It took 2640 us when each in-edge's LDS or L2 read
@@ -549,7 +554,7 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
     const float inv_nf = (float)(1.0 / (double)n);
     const uint64_t stride = contrib_stride(n);
 
-    __shared__ double2 s_red[WPB];
+    __shared__ PrPart s_red[WPB];
     // as many ids in LDS as fit beside the rest: with 32 per thread RMAT-21
     // took 1848 us, with 39 1803
 #ifndef SG_PR_LDS
@@ -559,26 +564,26 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
     __shared__ __align__(16) float s_cc[Hot::kLds + 4];
 
     // the block's (residual, dangling) partials, in a fixed order
-    auto put_part = [&](uint32_t it, double res, double dang) {
+    auto put_part = [&](uint32_t it, double res, CSum dang) {
         res = wave_sum_f64(res);
-        dang = wave_sum_f64(dang);
-        if (ln == 0) s_red[threadIdx.x / kWave] = make_double2(res, dang);
+        dang = wave_csum(dang);
+        if (ln == 0) s_red[threadIdx.x / kWave] = PrPart{res, dang.hi, dang.lo};
         __syncthreads();
         if (threadIdx.x < kWave) {
-            const double2 t = ln < WPB ? s_red[ln] : make_double2(0.0, 0.0);
-            res = wave_sum_f64(t.x);
-            dang = wave_sum_f64(t.y);
-            if (ln == 0) a.part[(size_t)(it & 1) * kMaxBlocks + blockIdx.x] = make_double2(res, dang);
+            const PrPart t = ln < WPB ? s_red[ln] : PrPart{0.0, 0.f, 0.f};
+            res = wave_sum_f64(t.res);
+            dang = wave_csum(CSum{t.dhi, t.dlo});
+            if (ln == 0) a.part[(size_t)(it & 1) * kMaxBlocks + blockIdx.x] = PrPart{res, dang.hi, dang.lo};
         }
     };
 
     // x = 1/n; contributions of iteration 0; dangling mass
-    double dang = 0.0;
+    CSum dang{0.f, 0.f};
     for (uint32_t v = gtid; v < n; v += nthreads) {
         a.x[v] = inv_nf;
         const uint32_t dout = g.row[v + 1] - g.row[v];
         a.contrib[v] = dout ? inv_nf / (float)dout : 0.0f;
-        if (!dout) dang += (double)inv_nf;
+        if (!dout) csum_add(dang, inv_nf);
     }
     if (threadIdx.x == 0) s_cc[Hot::kLds] = 0.f;
     put_part(0, 0.0, dang);
@@ -593,20 +598,21 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         // the LDS copy's loads are in flight while the partials are added
         Hot::take(s_cc, cc, n);
         // every wave adds the blocks' partials by itself: no wait for others
-        double2 gs = make_double2(0.0, 0.0);
+        double gres = 0.0;
+        CSum gdang{0.f, 0.f};
         for (uint32_t i = ln; i < gridDim.x; i += kWave) {
-            const double2 q = a.part[(size_t)(it & 1) * kMaxBlocks + i];
-            gs.x += q.x;
-            gs.y += q.y;
+            const PrPart q = a.part[(size_t)(it & 1) * kMaxBlocks + i];
+            gres += q.res;
+            gdang = csum_merge(gdang, CSum{q.dhi, q.dlo});
         }
-        gs.x = wave_sum_f64(gs.x);
-        gs.y = wave_sum_f64(gs.y);
-        if (it > 0) res = gs.x;
+        gres = wave_sum_f64(gres);
+        gdang = wave_csum(gdang);
+        if (it > 0) res = gres;
         if ((it > 0 && res < a.tol) || it >= a.max_iter) {
             Hot::wait();  // no copy into LDS outlives the block
             break;
         }
-        const float base = (1.0f - df) * inv_nf + df * (float)gs.y * inv_nf;
+        const float base = (1.0f - df) * inv_nf + df * csum_value(gdang) * inv_nf;
         if (gtid == 0 && it < kTraceRows) {
             DevTrace t;
             t.round = it;
@@ -620,8 +626,9 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         Hot::wait();
         __syncthreads();
         const Gather<Hot::kLds> gather{cc, s_cc, n};
-        constexpr uint32_t kRows = 8;  // RMAT-21 1774 us by 4, 1746 by 8; 15 001 vertices 226 and 210
-        double r_acc = 0.0, d_acc = 0.0;
+        constexpr uint32_t kRows = 8;  // RMAT-21 1774 us by 4, 1746 by 8; 15 001 vertices 226 and 210 (FP64 sums)
+        double r_acc = 0.0;
+        CSum d_acc{0.f, 0.f};
         struct Own {
             uint32_t dout;
             float xo;
@@ -630,19 +637,19 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
             return has ? Own{g.row[v + 1] - g.row[v], a.x[v]} : Own{0u, 0.f};
         };
         // x(v) from its in-edge sum, its last rank and its out-degree: FP32
-        // ranks and contributions, sums and the residual |x' - x| in FP64
-        auto finish = [&](bool has, uint32_t v, const Own &o, double s) {
+        // ranks and contributions, the residual |x' - x| summed in FP64
+        auto finish = [&](bool has, uint32_t v, const Own &o, const CSum &s) {
             if (!has) return;
-            const float xn = base + df * (float)s;
+            const float xn = base + df * csum_value(s);
             r_acc += fabs((double)xn - (double)o.xo);
             a.x[v] = xn;
             if (o.dout) cn[v] = xn / (float)o.dout;
-            else d_acc += (double)xn;
+            else csum_add(d_acc, xn);
         };
         // in-hubs of several chunks wait for every block's sums: arrive after
         // the chunks, wait once the other vertices are done
         hub_chunk_sums(g, gather, bounds, gwave, nwaves, pre,
-                       [&](bool has, uint32_t c, uint32_t v, bool one, const Own &o, double s) {
+                       [&](bool has, uint32_t c, uint32_t v, bool one, const Own &o, const CSum &s) {
                            if (has && !one) a.hubpart[c] = s;
                            finish(has && one, v, o, s);
                        });
@@ -683,7 +690,7 @@ struct PrDdArgs {
     float *r;          // residuals [n]: r + rlo, the rounding error of every
     float *rlo;        // atomic addition into r collected in rlo
     float *p;          // 2 rows: d r / outdeg of this / the next round's active vertices
-    double *hubpart;   // [nhugein] chunk sums of pull rounds
+    CSum *hubpart;     // [nhugein] chunk sums of pull rounds
     uint64_t *abit;    // 2 x W: active vertices of rounds k (k % 2)
     uint32_t *queue;   // 2 x qcap: vertices whose residual crossed theta
     uint32_t qcap;
@@ -1065,7 +1072,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
         // the edges, as one of the power iteration. Rounds of the ITERATIVE
         // scheme, and the last one before max_rounds, leave activation out.
         // RMAT graph of 100 003 vertices, 1.4 M edges, nearly all active: 19 us a
-        // round, 2.1 ms a run (45 and 4.8 with activation in a pass of its own);
+        // round, 2.2 ms a run (45 and 4.8 with activation in a pass of its own);
         // ~10 of the 19 are the two barriers, the counts and the LDS copy, 5 the
         // words' chains of in-edge steps, 3 the hubs.
         bool more = true;
@@ -1091,8 +1098,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                 }
                 return o;
             };
-            auto finish = [&](bool has, uint32_t v, const Own &o, double s) {
-                const CSum add{(float)s, (float)(s - (double)(float)s)};
+            auto finish = [&](bool has, uint32_t v, const Own &o, const CSum &add) {
                 CSum c = csum_merge(o.r, add);
                 const float ru = csum_value(c);
                 const bool active = has && act_next && (double)ru >= theta;
@@ -1110,10 +1116,10 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                     }
                     pn[v] = pv;
                 }
-                if (has && (s > 0.0 || active)) {
+                const float ad = csum_value(add);
+                if (has && (ad > 0.f || active)) {
                     a.r[v] = c.hi;
                     a.rlo[v] = c.lo;
-                    const float ad = csum_value(add);
                     crossed = kIter && (double)o.r.hi < theta && (double)o.r.hi + (double)ad >= theta;
                     R.count += crossed;
                     if (crossed && R.qdeg) R.qscout += o.dout;
@@ -1122,7 +1128,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
             };
             auto later = [](bool, uint32_t) { return Later{}; };
             hub_chunk_sums(g, gather, bounds, gwave, nwaves, later,
-                           [&](bool has, uint32_t c, uint32_t v, bool one, Later, double s) {
+                           [&](bool has, uint32_t c, uint32_t v, bool one, Later, const CSum &s) {
                                if (has && !one) a.hubpart[c] = s;
                                finish(has && one, v, pre(has && one, v), s);
                            });
@@ -1130,7 +1136,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
             word_sums<kRows>(g, gather, bounds, gwave, nwaves, pre, finish);
             ok = wide_hub_sums(
                 g, a.hubpart, bounds, gwave, nwaves, [&]() { return grid_wait(a.bar, gen, a.abort); }, later,
-                [&](bool has, uint32_t v, Later, double s) { finish(has, v, pre(has, v), s); });
+                [&](bool has, uint32_t v, Later, const CSum &s) { finish(has, v, pre(has, v), s); });
             if (!ok || !act_next) break;
             // the next round's totals, by blocks: no atomics, and every wave
             // adds them by itself
@@ -1347,8 +1353,8 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
         a.g = d;
         a.x = (float *)res;
         a.contrib = (float *)base;
-        a.hubpart = (double *)(base + off_hub);
-        a.part = (double2 *)(base + off_part);
+        a.hubpart = (CSum *)(base + off_hub);
+        a.part = (PrPart *)(base + off_part);
         a.bar.spin_limit = 1u << 22;
         a.abort = e->abort_flag;
         a.stats = e->stats;
@@ -1376,7 +1382,7 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
         a.r = (float *)(base + n * 8);
         a.rlo = (float *)(base + n * 12);
         a.p = (float *)(base + n * 16);
-        a.hubpart = (double *)(base + off_hub);
+        a.hubpart = (CSum *)(base + off_hub);
         a.part = (PrPart *)(base + off_part);
         a.abit = e->bitmaps;
         a.queue = e->queues;
