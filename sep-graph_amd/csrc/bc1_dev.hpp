@@ -488,7 +488,9 @@ __device__ __forceinline__ bool bc_phase(const Bc1Args &a, TeamLds &t, uint32_t 
     uint32_t members, rank;
     team_place(xcc, gen, members, rank);
     RoundState S{};
-    bool ok = true, left;
+    TeamEnd E{};
+    E.more = true;
+    bool ok = true;
     if (rank != ~0u) {
         const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
         BcTeam T;
@@ -505,7 +507,7 @@ __device__ __forceinline__ bool bc_phase(const Bc1Args &a, TeamLds &t, uint32_t 
         bc_level_bits(a, l - kStep, l - kStep, true, tid, nthreads);
         S.L = l;
     }
-    ok = team_rejoin<false>(a.f.bar, xcc, gen, a.f.abort, phase++, rank, true, S, left);
+    ok = team_rejoin<false>(a.f.bar, xcc, gen, a.f.abort, phase++, rank, S, E);
     l = S.L;
     return ok;
 }

@@ -513,17 +513,18 @@ __device__ __forceinline__ void team_pull(const BfsArgs &a, const BfsTeam &T, Te
 
 // A team phase: rounds from L on, by this member of the team, while they stay
 // small (kWhole, a graph the team runs whole: to the end). The state it leaves
-// is what a grid round expects: frontier L as a bitmap, counters saying that no
-// queue holds it; after the last round, what the epilogue leaves. Returns
-// false when a wait expired; `more`: rounds are left. At most `cap` rounds;
-// `t_start` is the trace's time 0. `order` (from level 0): receives the reached
+// is what a grid round expects: frontier L as a bitmap, its counts in E; after
+// the last round, what the epilogue leaves but for the counters. Returns
+// false when a wait expired; E.more: rounds are left. At most `cap` rounds;
+// `t_start` is the trace's time 0. `level1`: frontier L is round 0's, its levels
+// (1) not yet written. `order` (from level 0): receives the reached
 // vertices level by level, loff[l] the first position of level l.
 template <int BS, bool kWhole>
 __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, TeamBits *front, uint64_t *s_vis,
                                                uint32_t members,
                                                uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
-                                               long long t_start, uint32_t cap, bool &more, uint32_t *order = nullptr,
-                                               uint32_t *loff = nullptr)
+                                               long long t_start, uint32_t cap, bool level1, TeamEnd &E,
+                                               uint32_t *order = nullptr, uint32_t *loff = nullptr)
 {
     constexpr int WPB = BS / kWave;
     const uint32_t W = a.g.words;
@@ -557,13 +558,17 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, Tea
     unsigned long long count = rc.count, scout = rc.scout;
     bool hubs = rc.has_huge;
     uint32_t placed = 0;  // vertices of the levels before L
+    if (!kWhole && level1) {
+        const uint32_t *q1 = a.queue + (size_t)(L % 3) * a.qcap;
+        for (uint32_t i = tid; i < T.total; i += nthreads) a.level[caller_id(a, load_team(q1 + i))] = (int32_t)L;
+    }
     // a phase of narrow rounds keeps no bitmaps and leaves all three clear meanwhile
     if (!kWhole)
         for (uint32_t w = tid; w < W; w += nthreads) {
             a.fbit[(size_t)(L % 3) * W + w] = 0;
             a.fbit[(size_t)((L + 2) % 3) * W + w] = 0;
         }
-    more = ok;
+    bool more = ok;
     for (uint32_t r = 0; more && r < cap; r++) {
         const bool pull = S.next(count, scout);
         if (lead) write_trace(a.trace, L, pull, count, scout, t_start);
@@ -611,14 +616,10 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, Tea
     tag = T.tag;
     if (!ok) return false;
     uint64_t *fl = a.fbit + (size_t)(L % 3) * W;
-    if (!more) {
-        // the last round: bitmaps and counters are left clear for the next query
-        for (uint32_t w = tid; w < 3 * W && kWhole; w += nthreads) a.fbit[w] = 0;
-    } else if (kWhole) {
-        // the filter in memory takes frontier L and all before it
-        if (rank == 0)
-            for (uint32_t w = threadIdx.x; w < W; w += BS) a.vis[w] = T.s_vis[w] | load_team(fl + w);
-    } else {
+    if (kWhole) {
+        // the last round: bitmaps are left clear for the next query
+        for (uint32_t w = tid; w < 3 * W; w += nthreads) a.fbit[w] = 0;
+    } else if (more) {
         const uint32_t own = (uint32_t)((t.slot[rank] >> kTeamCountShift) & kTeamCountMask);
         const uint32_t *q = a.queue + (size_t)(L % 3) * a.qcap + (size_t)rank * T.seg;
         for (uint32_t i = threadIdx.x; i < own; i += BS) {
@@ -626,17 +627,10 @@ __device__ __forceinline__ bool bfs_team_phase(const BfsArgs &a, TeamLds &t, Tea
             atomicOr((unsigned long long *)&fl[u >> 6], 1ull << (u & 63));
         }
     }
-    if (rank == 0) {
-        for (int i = 0; i < 3; i++) clear_ctr(&a.ctr[i]);
-        block_sync_global();
-        if (threadIdx.x == 0 && more) {
-            FrontierCtr &c = a.ctr[L % 3];
-            c.overflow = 1;
-            c.has_huge = hubs;
-            c.stripe[0].scout = scout;
-            c.stripe[0].count = count;
-        }
-    }
+    E.count = count;
+    E.scout = scout;
+    E.hubs = hubs;
+    E.more = more;
     return true;
 }
 
@@ -665,7 +659,7 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint32_t
     if (threadIdx.x == 0) s_ok = bar_census(a.bar, xcc, gen, a.abort);
     team_place(xcc, gen, members, rank);
     RoundState S{{a.alpha, a.beta, a.total_workload0, g.n, a.force}, 0, 0, 0, 0};
-    bool ok = s_ok != 0u, more = true;
+    bool ok = s_ok != 0u;
     if (ok && rank == ~0u) return true;
     if (ok) {
         const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
@@ -683,7 +677,11 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint32_t
     }
     if (ok) {
         const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
-        ok = bfs_team_phase<BS, true>(a, t, &s_front, s_vis, members, rank, tag, S, rc, t_start, ~0u, more, order, loff);
+        TeamEnd E{};
+        ok = bfs_team_phase<BS, true>(a, t, &s_front, s_vis, members, rank, tag, S, rc, t_start, ~0u, false, E, order, loff);
+        // (the other blocks read no counters)
+        if (ok && rank == 0)
+            for (int i = 0; i < 3; i++) clear_ctr(&a.ctr[i]);
     }
     // (after a failed census no block's place is known: block 0 reports)
     if (!s_ok) rank = blockIdx.x ? ~0u : 0u;
@@ -811,41 +809,57 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         L = 1;
     }
 
+    // the grid's rounds use the counter slots in turn; the team's use none, and
+    // after a phase the counts come with its note
+    uint32_t slot = L;
+    bool noted = false;
     while (ok) {
-        read_counts(&a.ctr[L % 3], s_lvl);
+        if (!noted) read_counts(&a.ctr[slot % 3], s_lvl);
         if (threadIdx.x == 0) s_qn = 0;
         __syncthreads();
         const RoundCounts rc = unpack_counts(s_lvl, a.qcap);
         __syncthreads();
-        if (L == 1 && local0) {
+        noted = false;
+        const bool last = rc.count == 0 || (a.max_rounds && L >= a.max_rounds);
+        const bool team_phase_next = kTeamOk && !last && bfs_team_fits<kLeave>(a, S, rc);
+        const bool level1 = L == 1 && local0;
+        if (level1 && !team_phase_next) {
             // the source's out-neighbours found by block 0 (at most
-            // kLocalRound0, so the queue holds them all)
+            // kLocalRound0, so the queue holds them all); a team's rounds
+            // would overwrite the queue under a block that is late here, so
+            // before a phase its members write them
             const uint32_t *q1 = a.queue + (size_t)a.qcap;
             for (uint32_t i = gtid; i < rc.qlen; i += nthreads) a.level[caller_id(a, q1[i])] = 1;
         }
-        if (rc.count == 0) break;
-        if (a.max_rounds && L >= a.max_rounds) break;
+        if (last) break;
 
-        if (kTeamOk && bfs_team_fits<kLeave>(a, S, rc)) {
+        if (team_phase_next) {
             uint32_t members, rank;
             team_place(xcc, gen, members, rank);
-            bool more = true, left;
+            TeamEnd E{};
             if (rank != ~0u) {
                 // a failed wait set the abort flag, which ends the others' wait
                 const long long t0 = rank == 0 && threadIdx.x == 0 ? team_clock(a.bar) : 0ll;
-                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, nullptr, members, rank, tag, S, rc, t0, kTeamRounds, more);
+                ok = bfs_team_phase<BS, false>(a, s_t, nullptr, nullptr, members, rank, tag, S, rc, t0, kTeamRounds, level1,
+                                               E);
                 if (!ok) break;
-                if (kLeave && !more && rank == 0 && threadIdx.x == 0)
+                if (kLeave && !E.more && rank == 0 && threadIdx.x == 0)
                     write_final(a.trace, a.stats, L, S.pushes, S.pulls, S.ptrace, true, t0);
             }
-            ok = team_rejoin<kLeave>(a.bar, xcc, gen, a.abort, phase++, rank, more, S, left);
-            if (ok && left) return true;
+            ok = team_rejoin<kLeave>(a.bar, xcc, gen, a.abort, phase++, rank, S, E, s_lvl);
+            if (ok && E.left) {
+                // every block has read the counters: leave them clear for the next query
+                if (E.closed)
+                    for (int i = 0; i < 3; i++) clear_ctr(&a.ctr[i]);
+                return true;
+            }
+            noted = true;
             continue;
         }
 
         const bool pull = S.next(rc.count, rc.scout);
         if (gtid == 0) write_trace(a.trace, L, pull, rc.count, rc.scout, t_start);
-        if (brank == 0) clear_ctr(&a.ctr[(L + 2) % 3]);
+        if (brank == 0) clear_ctr(&a.ctr[(slot + 2) % 3]);
 
         Round R;
         R.a = &a;
@@ -857,7 +871,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
             uint64_t *fclr = a.fbit + (size_t)((L + 2) % 3) * W;
             for (uint32_t w = gtid; w < W; w += nthreads) fclr[w] = 0;
         }
-        R.S = Stager{a.queue + (size_t)((L + 1) % 3) * a.qcap, a.qcap, &a.ctr[(L + 1) % 3], s_q, &s_qn, kLdsQ};
+        R.S = Stager{a.queue + (size_t)((L + 1) % 3) * a.qcap, a.qcap, &a.ctr[(slot + 1) % 3], s_q, &s_qn, kLdsQ};
         R.scout = 0;
         R.count = 0;
         R.huge = false;
@@ -1008,6 +1022,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         flush_stage(R.S, s_flush);
         S.pol.pull_prev = pull;
         L++;
+        slot++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
 

@@ -523,50 +523,81 @@ __device__ __forceinline__ long long team_clock(const GridBarrier &gb)
     return (long long)load_team((const uint64_t *)(gb.words + kBarNote + 8));
 }
 
+// The end of a team phase, and what it hands to the grid round that follows it.
+struct TeamEnd {
+    unsigned long long count, scout;  // of frontier L, which its bitmap holds
+    bool hubs;
+    uint32_t cmin;   // SSSP: the smallest distance in it
+    bool more;       // rounds are left
+    bool left;       // (kLeave) none are: the block is done
+    bool closed;     // this block was the last to arrive at the phase's end
+};
+
 // The grid barrier that ends team phase number `phase`: the member of rank 0
 // leaves the rounds' state in a note (two in turn: a block may still be reading
 // the last phase's when the next phase's is written), from which every block
-// goes on. `more` (members): rounds are left. With kLeave, nothing follows the
+// goes on. The counts of frontier L are part of it (left in s_lvl as read_counts
+// does, its smallest distance's complement in *s_cmin), and a phase touches no
+// counter slot: blocks outside the team take no part in its rounds, so one of
+// them may still be reading the slot of the round that started the phase.
+// E.more (members): rounds are left. With kLeave, nothing follows the
 // last round: a member is done once it has arrived, and the others as soon as
-// they see the note, with no acquire; `left` tells them so. False when the wait
+// they see the note, with no acquire; E.left tells them so. False when the wait
 // expired or a block aborted.
 template <bool kLeave>
 __device__ __forceinline__ bool team_rejoin(const GridBarrier &gb, uint32_t xcc, BarState &gen, uint32_t *abort,
-                                            uint32_t phase, uint32_t rank, bool more, RoundState &S, bool &left)
+                                            uint32_t phase, uint32_t rank, RoundState &S, TeamEnd &E,
+                                            unsigned long long *s_lvl = nullptr, uint32_t *s_cmin = nullptr)
 {
-    __shared__ uint32_t s_note[8], s_ok;
+    // words 8 and 9 of the first note are team_clock's
+    constexpr int kWords = 14;
+    __shared__ uint32_t s_note[kWords], s_ok, s_closed;
     uint32_t *note = gb.words + kBarNote + 16 * (phase & 1u);
     if (rank == 0 && threadIdx.x == 0) {
         note[0] = S.L;
         note[1] = S.pol.total_wl;
-        note[2] = S.pol.pull_prev;
+        note[2] = (uint32_t)S.pol.pull_prev | (uint32_t)E.hubs << 1;
         note[3] = S.pushes;
         note[4] = S.pulls;
         note[5] = (uint32_t)S.ptrace;
         note[6] = (uint32_t)(S.ptrace >> 32);
-        note[7] = more;
+        note[7] = E.more;
+        note[10] = (uint32_t)E.scout;
+        note[11] = (uint32_t)(E.scout >> 32);
+        note[12] = E.cmin;
+        note[13] = (uint32_t)E.count;
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t gen0 = grid_arrive(gb, xcc, gen);
+        s_closed = 0u;
+        const uint32_t gen0 = grid_arrive(gb, xcc, gen, &s_closed);
         s_ok = 1u;
-        if (kLeave && rank != ~0u && !more) {
+        if (kLeave && rank != ~0u && !E.more) {
             s_note[7] = 0;
         } else {
             s_ok = spin_wait<true>(gb.words + kBarGen, gen0, true, gb.spin_limit, abort);
-            for (int i = 0; i < 8; i++) s_note[i] = poll_load(note + i);
+            for (int i = 0; i < kWords; i++) s_note[i] = poll_load(note + i);
             if (!kLeave || s_note[7]) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             __builtin_amdgcn_s_waitcnt(0);
+            if (s_lvl) {
+                s_lvl[0] = s_note[13];
+                s_lvl[1] = (unsigned long long)s_note[11] << 32 | s_note[10];
+                s_lvl[2] = 0;  // no queue
+                s_lvl[3] = 1;
+                s_lvl[4] = s_note[2] >> 1;
+            }
+            if (s_cmin) *s_cmin = ~s_note[12];
         }
     }
     __syncthreads();
-    left = kLeave && !s_note[7];
+    E.left = kLeave && !s_note[7];
+    E.closed = s_closed != 0u;
     if (!s_ok) return false;
-    if (!left) {
+    if (!E.left) {
         S.L = s_note[0];
         S.pol.total_wl = s_note[1];
-        S.pol.pull_prev = s_note[2] != 0u;
+        S.pol.pull_prev = (s_note[2] & 1u) != 0u;
         S.pushes = s_note[3];
         S.pulls = s_note[4];
         S.ptrace = (unsigned long long)s_note[6] << 32 | s_note[5];

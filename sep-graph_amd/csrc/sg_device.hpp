@@ -375,10 +375,12 @@ __device__ inline void residency_probe(uint32_t *words, uint32_t limit)
 
 // Arrival of this block at the grid barrier (thread 0, after the block's stores
 // have drained and the census is taken); returns the generation it ends.
+// `closed`: set when it was the last block's.
 // kStamp: the block that completes the barrier also records the wall clock
 // (barrier_stamp), so every block can time the grid's rounds identically.
 template <bool kStamp = false>
-__device__ __forceinline__ uint32_t grid_arrive(const GridBarrier &gb, uint32_t xcc, BarState &st)
+__device__ __forceinline__ uint32_t grid_arrive(const GridBarrier &gb, uint32_t xcc, BarState &st,
+                                                uint32_t *closed = nullptr)
 {
     uint32_t *w = gb.words;
     const uint32_t gen0 = st.gen;
@@ -400,6 +402,7 @@ __device__ __forceinline__ uint32_t grid_arrive(const GridBarrier &gb, uint32_t 
             }
             flag_store(w + kBarGen, gen0 + 1);
             flag_store(top, 0u);
+            if (closed) *closed = 1u;
         }
     }
     return gen0;

@@ -811,12 +811,12 @@ __device__ __forceinline__ void team_pull(const SsspArgs &a, SsspTeam &T, TeamLd
 }
 
 // A team phase: see bfs_team_phase. `cmin`: the smallest distance in frontier
-// S.L. Leaves the bitmaps and counters that a grid round expects.
+// S.L. Leaves the bitmaps that a grid round expects.
 template <int BS, bool kWhole>
 __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, TeamBits *front, uint64_t *s_next,
                                                 uint32_t members,
                                                 uint32_t rank, uint32_t &tag, RoundState &S, const RoundCounts &rc,
-                                                uint32_t cmin, long long t_start, uint32_t cap, bool &more)
+                                                uint32_t cmin, long long t_start, uint32_t cap, TeamEnd &E)
 {
     constexpr int WPB = BS / kWave;
     const uint32_t W = a.g.words;
@@ -848,7 +848,7 @@ __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, T
     }
     unsigned long long count = rc.count, scout = rc.scout;
     bool hubs = rc.has_huge;
-    more = ok;
+    bool more = ok;
     for (uint32_t r = 0; more && r < cap; r++) {
         const bool pull = S.next(count, scout);
         if (lead && a.trace) write_trace(a.trace, L, pull, count, scout, t_start);
@@ -887,18 +887,11 @@ __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, T
     }
     tag = T.tag;
     if (!ok) return false;
-    if (rank == 0) {
-        for (int i = 0; i < 3; i++) clear_ctr(&a.ctr[i]);
-        block_sync_global();
-        if (threadIdx.x == 0 && more) {
-            FrontierCtr &c = a.ctr[L % 3];
-            c.overflow = 1;
-            c.has_huge = hubs;
-            c.stripe[0].scout = scout;
-            c.stripe[0].count = count;
-            slot_cmin(&c) = ~cmin;
-        }
-    }
+    E.count = count;
+    E.scout = scout;
+    E.hubs = hubs;
+    E.cmin = cmin;
+    E.more = more;
     return true;
 }
 
@@ -921,7 +914,7 @@ __device__ __forceinline__ bool sssp_whole(const SsspArgs &a, uint32_t xcc, BarS
     uint32_t members, rank, tag = 0;
     team_place(xcc, gen, members, rank);
     RoundState S{{a.alpha, a.beta, a.total_workload0, g.n, a.force}, 0, 0, 0, 0};
-    bool ok = s_ok != 0u, more = true;
+    bool ok = s_ok != 0u;
     if (ok && rank == ~0u) return true;
     const uint32_t tid = rank * BS + threadIdx.x, nthreads = members * BS;
     if (ok) {
@@ -931,7 +924,8 @@ __device__ __forceinline__ bool sssp_whole(const SsspArgs &a, uint32_t xcc, BarS
     }
     if (ok) {
         const RoundCounts rc{1, sdeg, 1, false, sdeg > kHugeDegree};
-        ok = sssp_team_phase<BS, true>(a, t, &s_front, s_next, members, rank, tag, S, rc, 0, t_start, ~0u, more);
+        TeamEnd E{};
+        ok = sssp_team_phase<BS, true>(a, t, &s_front, s_next, members, rank, tag, S, rc, 0, t_start, ~0u, E);
     }
     // the last exchange ordered every distance before this
     if (ok && a.out)
@@ -1000,14 +994,20 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
 
     RoundState S{{a.alpha, a.beta, a.total_workload0, n, a.force}, 0, 0, 0, 0};
     uint32_t &L = S.L;
+    // the grid's rounds use the counter slots in turn; the team's use none, and
+    // after a phase the counts come with its note
+    uint32_t slot = L;
+    bool noted = false;
     while (ok) {
-        read_counts(&a.ctr[L % 3], s_lvl);
+        if (!noted) read_counts(&a.ctr[slot % 3], s_lvl);
         if (threadIdx.x == 0) {
             s_qn = 0;
-            s_cmin = __hip_atomic_load(&slot_cmin(&a.ctr[L % 3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!noted)
+                s_cmin = __hip_atomic_load(&slot_cmin(&a.ctr[slot % 3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
         const RoundCounts rc = unpack_counts(s_lvl, a.qcap);
+        noted = false;
         // priority mode: expand only the lowest delta-bucket present
         uint32_t thr = kInf;
         if (a.delta) {
@@ -1022,21 +1022,22 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
             if (sssp_team_fits(a, S, rc.count, rc.scout, rc.has_huge)) {
                 uint32_t members, rank;
                 team_place(xcc, gen, members, rank);
-                bool more = true, left;
+                TeamEnd E{};
                 if (rank != ~0u) {
                     // a failed wait set the abort flag, which ends the others' wait
                     const long long t0 = rank == 0 && threadIdx.x == 0 ? team_clock(a.bar) : 0ll;
                     ok = sssp_team_phase<BS, false>(a, s_t, nullptr, nullptr, members, rank, tag, S, rc,
-                                                    s_cmin ? ~s_cmin : 0u, t0, kTeamRounds, more);
+                                                    s_cmin ? ~s_cmin : 0u, t0, kTeamRounds, E);
                     if (!ok) break;
                 }
-                ok = team_rejoin<false>(a.bar, xcc, gen, a.abort, phase++, rank, more, S, left);
+                ok = team_rejoin<false>(a.bar, xcc, gen, a.abort, phase++, rank, S, E, s_lvl, &s_cmin);
+                noted = true;
                 continue;
             }
         }
         const bool pull = S.next(rc.count, rc.scout);
         if (gtid == 0 && a.trace) write_trace(a.trace, L, pull, rc.count, rc.scout, t_start);
-        if (brank == 0) clear_ctr(&a.ctr[(L + 2) % 3]);
+        if (brank == 0) clear_ctr(&a.ctr[(slot + 2) % 3]);
 
         Round R;
         R.a = &a;
@@ -1050,7 +1051,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
         // the bitmap for round L+2 is free (read in round L-1): clear it
         uint64_t *fclr = a.fbit + (size_t)((L + 2) % 3) * W;
         for (uint32_t w = gtid; w < W; w += nthreads) fclr[w] = 0;
-        R.S = Stager{a.queue + (size_t)((L + 1) % 3) * a.qcap, a.qcap, &a.ctr[(L + 1) % 3], s_q, &s_qn, kLdsQ};
+        R.S = Stager{a.queue + (size_t)((L + 1) % 3) * a.qcap, a.qcap, &a.ctr[(slot + 1) % 3], s_q, &s_qn, kLdsQ};
         R.scout = 0;
         R.count = 0;
         R.huge = false;
@@ -1162,6 +1163,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
         flush_stage(R.S, s_flush);
         S.pol.pull_prev = pull;
         L++;
+        slot++;
         ok = grid_sync(a.bar, xcc, gen, a.abort);
     }
 
