@@ -73,6 +73,14 @@ __device__ __forceinline__ CSum csum_merge(CSum a, const CSum &b)
 
 __device__ __forceinline__ float csum_value(const CSum &a) { return a.hi + a.lo; }
 
+// The same sum with its value in hi and what that rounds off in lo (TwoSum).
+__device__ __forceinline__ CSum csum_settle(const CSum &a)
+{
+    CSum s{a.hi, 0.f};
+    csum_add(s, a.lo);
+    return s;
+}
+
 // Wave sum, merged lower lanes first in a fixed order; every lane has the
 // same bits.
 __device__ __forceinline__ CSum wave_csum(CSum a)
@@ -808,7 +816,11 @@ struct DdRound {
 // Add `add` to v's residual atomically, queueing v if this addition took its
 // residual across theta. The addition returns the old value, so the lane
 // recomputes the rounded sum it stored and adds its rounding error (TwoSum,
-// Knuth) to rlo[v]. Wave-convergent.
+// Knuth) to rlo[v]. The crossing is told by r[v] alone, as stored before and
+// after: additions only raise it, so one of them sees it cross, and a vertex that is
+// left inactive is stored with its r below theta (csum_settle). Told by the
+// exact sum, or with hi >= theta > hi + lo left in place, a residual could get
+// past theta unseen and grow to the end of the run. Wave-convergent.
 __device__ __forceinline__ void dd_accumulate(DdRound &R, bool act, uint32_t v, float add)
 {
     bool crossed = false;
@@ -818,7 +830,7 @@ __device__ __forceinline__ void dd_accumulate(DdRound &R, bool act, uint32_t v, 
         const float bb = s - old;
         const float err = (old - (s - bb)) + (add - bb);
         if (err != 0.f) atomicAdd(&R.a->rlo[v], err);
-        crossed = (double)old < R.theta && (double)old + (double)add >= R.theta;
+        crossed = (double)old < R.theta && (double)s >= R.theta;
         R.count += crossed;
         if (crossed && R.qdeg) R.qscout += R.a->g.row[v + 1] - R.a->g.row[v];
     }
@@ -966,7 +978,8 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                 const uint32_t v = w * 64 + ln;
                 bool act = false;
                 if (v < n) {
-                    const float rv = a.r[v] + a.rlo[v];
+                    const CSum c{a.r[v], a.rlo[v]};
+                    const float rv = csum_value(c);
                     act = (double)rv >= thr;
                     waiting |= !act && (double)rv >= theta;
                     if (act) {
@@ -975,6 +988,11 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                         activate(v, rv);
                     } else {
                         pc[v] = 0.f;  // a pull round reads every source's
+                        if ((double)rv < theta && (double)c.hi >= theta) {
+                            const CSum s = csum_settle(c);
+                            a.r[v] = s.hi;
+                            a.rlo[v] = s.lo;
+                        }
                     }
                 }
                 const uint64_t m = ballot(act);
@@ -994,8 +1012,9 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                     atomicOr((unsigned long long *)&ab[u >> 6], 1ull << (u & 63));
                     activate(u, ru);
                 } else if (hi != 0.f || lo != 0.f) {
-                    atomicAdd(&a.r[u], hi);
-                    atomicAdd(&a.rlo[u], lo);
+                    const CSum c = hi != 0.f ? csum_settle(CSum{hi, lo}) : CSum{0.f, lo};
+                    atomicAdd(&a.r[u], c.hi);
+                    atomicAdd(&a.rlo[u], c.lo);
                 }
             }
         }
@@ -1116,11 +1135,11 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
                     }
                     pn[v] = pv;
                 }
-                const float ad = csum_value(add);
-                if (has && (ad > 0.f || active)) {
+                if (has && (csum_value(add) > 0.f || active)) {
+                    if (!active) c = csum_settle(c);
                     a.r[v] = c.hi;
                     a.rlo[v] = c.lo;
-                    crossed = kIter && (double)o.r.hi < theta && (double)o.r.hi + (double)ad >= theta;
+                    crossed = kIter && (double)o.r.hi < theta && (double)c.hi >= theta;
                     R.count += crossed;
                     if (crossed && R.qdeg) R.qscout += o.dout;
                 }
