@@ -284,7 +284,7 @@ typedef struct sg_stats {
     uint32_t reached;           /* n_r: vertices with a finite result */
     uint64_t reached_edges;     /* m_r: sum of out-degree over reached vertices */
     uint64_t policy_trace;      /* bit r = 1 if round r ran pull (first 64 rounds) */
-    double kernel_ms;           /* device time of the last run: first block's start to
+    double kernel_ms;           /* device time of the last run: block 0's start to the
                                  last block's end (HIP events around several kernels) */
     double residual;            /* PageRank: final L1 change (FP64 on device) */
     uint32_t iterations;        /* PageRank iterations */

@@ -276,12 +276,16 @@ __device__ __forceinline__ bool spin_wait(const uint32_t *p, uint32_t v, bool wa
 }
 
 // End of a persistent kernel that the engine times: the run took from block
-// 0's start to the last block's end. Two event records around the kernel took
+// 0's start to the end of the last block's last wave, its stores done. Reached
+// by every wave of the block. Two event records around the kernel took
 // 7 us of every call (RMAT-12 BFS 35.5 us with them, 28.3 without), these
 // stores cost none that could be measured.
 __device__ __forceinline__ void bar_end(const GridBarrier &gb)
 {
-    if (gb.clock && threadIdx.x == 0) gb.clock[1 + blockIdx.x] = (uint64_t)wall_clock64();
+    if (!gb.clock) return;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) gb.clock[1 + blockIdx.x] = (uint64_t)wall_clock64();
 }
 
 // Start of a persistent kernel (thread 0's copy is the one used): read the
