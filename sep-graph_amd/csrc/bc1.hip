@@ -71,7 +71,7 @@ int launch_bc1(sg_engine *e, Bc1KArgs &a)
     // (a forced push fixes the direction of every level pass: grid passes only)
     void (*kernel)(Bc1KArgs) = a.b.f.team && a.b.f.force != 0 ? k_bc1<BS, true> : k_bc1<BS, false>;
     int most = 0;
-    if (a.b.f.force != 0 && team_whole_graph(a.b.f.g)) {
+    if (team_whole_graph(a.b.f.g, kTeamBc, a.b.f.force, e->g->relabeled)) {
         kernel = k_bc1_whole<BS>;
         most = e->g->num_cus;
     }

@@ -42,7 +42,7 @@ int launch_bfs(sg_engine *e, BfsArgs &args)
 {
     void (*kernel)(BfsArgs) = k_bfs<BS, kStage>;
     int most = 0;
-    if (!kStage && args.team && team_whole_graph(args.g)) {
+    if (!kStage && args.team && team_whole_graph(args.g, kTeamBfs, args.force, e->g->relabeled)) {
         kernel = k_bfs_whole<BS>;
         most = e->g->num_cus;
     }
@@ -294,7 +294,9 @@ extern "C" int sg_bfs_noalloc(const sg_graph *g, uint32_t source, int32_t *level
     a.abort = (uint32_t *)(d.ptr + kNaOffAbort);
     a.stats = (DevStats *)(d.ptr + kNaOffStats);
     // (k_bfs_whole takes fewer registers and less LDS: k_bfs's grid is resident for it too)
-    void (*kernel)(BfsArgs) = a.team && team_whole_graph(dg) ? k_bfs_whole<kNaBlock> : k_bfs<kNaBlock, false>;
+    void (*kernel)(BfsArgs) = a.team && team_whole_graph(dg, kTeamBfs, force, g->relabeled)
+                                 ? k_bfs_whole<kNaBlock>
+                                 : k_bfs<kNaBlock, false>;
     hipLaunchKernelGGL(kernel, dim3(d.blocks), dim3(kNaBlock), 0, s, a);
     SG_HIP(hipGetLastError());
     d.launches++;

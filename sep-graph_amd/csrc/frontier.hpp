@@ -415,16 +415,12 @@ __device__ __forceinline__ void write_final(DevTrace *trace, DevStats *stats, ui
     *stats = s;
 }
 
-// A team runs every round of a graph of at most this many words and edges (see
-// bfs_whole).
+// A team runs every round of a graph of at most this many words (see bfs_whole
+// and team_whole_graph).
 #ifndef SG_TEAM_WORDS
 #define SG_TEAM_WORDS 256
 #endif
-#ifndef SG_TEAM_EDGES
-#define SG_TEAM_EDGES 1000000
-#endif
 constexpr uint32_t kTeamWords = SG_TEAM_WORDS;
-constexpr uint64_t kTeamEdges = SG_TEAM_EDGES;
 
 // What a narrow round may add to the next frontier at most: however it spreads
 // over the members, it has to fit one member's segment of the queue (an engine's
@@ -437,11 +433,36 @@ __device__ __forceinline__ uint32_t team_limit(uint32_t qcap, uint32_t most)
 // Rounds of one team phase: bounds the other blocks' wait.
 constexpr uint32_t kTeamRounds = 8192;
 
-// A graph so small that the team runs all of its rounds (kernels of their own:
-// a query this short is held up by code it does not run).
-__host__ __device__ __forceinline__ bool team_whole_graph(const DevGraph &g)
+// Whether a graph is so small that the team runs all of a query's rounds (kernels
+// of their own: a query this short is held up by code it does not run). The
+// team has an eighth of the CUs, so what counts beside the vertices is how many
+// edges the rounds walk. us by the team and by rounds of the whole grid:
+//  - alpha/beta rule, BFS: 4000 vertices 254 K edges 45 and 62, 504 K 85 and 64;
+//    8000 vertices 510 K 47 and 70, 952 K 65 and 62; skewed graphs of 16 384 vertices
+//    426 K 61 and 66, 777 K 77 and 64, of 8192 vertices 366 K 67 and 61. SSSP: 16 000
+//    vertices 511 K 212 and 276, 958 K 305 and 287; 4000 vertices 254 K 134 and 225,
+//    504 K 179 and 193. Single-source BC, whose passes walk every edge of a level:
+//    228 K 195 and 193, 366 K 247 and 167.
+//  - pull only: BFS and BC stop or skip early at any density (BFS 16 384 vertices,
+//    777 K: 73 and 1407); SSSP as above (16 000 vertices 511 K 209 and 297, 958 K
+//    392 and 318).
+//  - push only (the priority schedule too) walks every frontier edge with an atomic:
+//    BFS 62 K 81 and 98, 92 K 111 and 100; SSSP 22 K 188 and 211, 29 K 206 and 181,
+//    but with few edges a vertex, in narrow rounds, up to 4 a vertex (127 x 128
+//    grid, 58 K: 1148 and 1734; 16 000 vertices, 64 K 213 and 246, 96 K 272 and
+//    260); on skewed graphs 16 K 176 and 191, 23 K 254 and 203.
+enum TeamQuery { kTeamBfs, kTeamSssp, kTeamBc };
+inline bool team_whole_graph(const DevGraph &g, TeamQuery q, int32_t force, bool skewed)
 {
-    return g.words <= kTeamWords && g.m <= kTeamEdges;
+    if (g.words > kTeamWords) return false;
+    const uint64_t n = g.n, m = g.m;
+    if (force == 0) {
+        if (q == kTeamBfs) return m <= 65536;
+        return q == kTeamSssp && m <= (skewed ? 16384 : std::max<uint64_t>(24576, 4 * n));
+    }
+    if (force == 1 && q != kTeamSssp) return m <= 1000000;
+    if (q == kTeamBc) return m <= 1u << 18;
+    return m <= std::max<uint64_t>(1u << 18, (q == kTeamBfs && !skewed ? 64 : 32) * n);
 }
 
 // The frontier of a whole-graph phase as a bitmap in LDS, with the vertices

@@ -94,7 +94,7 @@ int launch_sssp(sg_engine *e, SsspArgs &args, uint32_t *group_words)
         SG_FAIL(SG_ERR_STATE, "sg_sssp: launch with unset device state");
     void (*kernel)(SsspArgs) = k_sssp<BS>;
     int most = 0;
-    if (!args.grouped && args.team && team_whole_graph(args.g)) {
+    if (!args.grouped && args.team && team_whole_graph(args.g, kTeamSssp, args.force, e->g->relabeled)) {
         kernel = k_sssp_whole<BS>;
         most = e->g->num_cus;
     }
