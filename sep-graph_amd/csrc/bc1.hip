@@ -128,6 +128,7 @@ int bc1_launch(sg_engine *e, uint32_t dev_source, float *dep, const uint32_t *pe
     a.b.last = last;
     a.acc = e->stats;
     a.b.f.team = e->g->relabeled ? 0u : 2u;
+    a.b.f.team_start = team_start(a.b.f.g, kTeamPushEdges);
     const int bs = e->opt.block_size ? e->opt.block_size : 1024;
     switch (bs) {
     case 256: return launch_bc1<256>(e, a);

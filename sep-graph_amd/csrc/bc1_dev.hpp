@@ -589,7 +589,7 @@ __device__ __forceinline__ bool bc1_run(const Bc1Args &a, uint32_t brank, uint32
         a.ctl[0] = 0;
         a.ctl[1] = 0;
     }
-    bool ok = bfs_run<BS, false, kTeamOk>(a.f, brank, nblocks, xcc, gen, &s_t, &tag, &phase);
+    bool ok = bfs_run<BS, false, kTeamOk, false, kTeamOk>(a.f, brank, nblocks, xcc, gen, &s_t, &tag, &phase);
     int32_t status = ok ? SG_OK : SG_ERR_TIMEOUT;
 
     // ---- per-level counts: block histograms, one atomic per block and level

@@ -7,7 +7,8 @@ using namespace bfsk;
 
 namespace {
 
-template <int BS, bool kStage>
+// kEven: the graph is not skewed (see bfs_run).
+template <int BS, bool kStage, bool kEven>
 __global__ SG_BFS_BOUNDS(BS) void k_bfs(BfsArgs a)
 {
     if (a.probe) {
@@ -16,7 +17,7 @@ __global__ SG_BFS_BOUNDS(BS) void k_bfs(BfsArgs a)
     }
     const uint32_t xcc = xcc_id();
     BarState gen = bar_begin<!kStage>(a.bar, xcc);
-    bfs_run<BS, kStage, !kStage, !kStage>(a, blockIdx.x, gridDim.x, xcc, gen);
+    bfs_run<BS, kStage, !kStage, !kStage, kEven>(a, blockIdx.x, gridDim.x, xcc, gen);
     bar_end(a.bar);
 }
 
@@ -40,7 +41,7 @@ __global__ SG_BFS_BOUNDS(BS) void k_bfs_whole(BfsArgs a)
 template <int BS, bool kStage>
 int launch_bfs(sg_engine *e, BfsArgs &args)
 {
-    void (*kernel)(BfsArgs) = k_bfs<BS, kStage>;
+    void (*kernel)(BfsArgs) = e->g->relabeled ? k_bfs<BS, kStage, false> : k_bfs<BS, kStage, !kStage>;
     int most = 0;
     if (!kStage && args.team && team_whole_graph(args.g, kTeamBfs, args.force, e->g->relabeled)) {
         kernel = k_bfs_whole<BS>;
@@ -110,6 +111,7 @@ int bfs_launch(sg_engine *e, uint32_t source, int32_t *out, bool traced)
     a.lb_push_none = o.lb_push == SG_LB_NONE;
     a.lb_pull_none = o.lb_pull == SG_LB_NONE;
     a.team = a.lb_push_none || a.lb_pull_none ? 0u : e->g->relabeled ? 1u : 2u;
+    a.team_start = team_start(a.g, kTeamPushEdges);
     e->last_algo = 0;
     const int bs = o.block_size ? o.block_size : 1024;
     switch (bs) {
@@ -181,7 +183,7 @@ constexpr int kNaMaxDevices = 64;
 
 struct NaDevice {
     char *ptr = nullptr;   // device address of `scratch` on this device
-    int blocks = 0;        // co-resident grid of k_bfs<kNaBlock, false>
+    int blocks = 0;        // co-resident grid, see na_setup
     uint64_t launches = 0; // runs on the barrier words (registration parity)
 };
 std::mutex g_na_mu[kNaMaxDevices];
@@ -200,7 +202,8 @@ int na_zero(hipStream_t s, char *p, size_t bytes)
 }
 
 // Once per device: the array's address, cleared counters, and the largest
-// blocks-per-CU grid of k_bfs<kNaBlock, false> whose blocks are all resident.
+// blocks-per-CU grid that the occupancy API allows every kernel of the call, and
+// whose blocks are all resident when one of them is probed.
 int na_setup(NaDevice &d, const sg_graph *g, hipStream_t s, const BfsArgs &proto)
 {
     void *p = nullptr;
@@ -209,8 +212,12 @@ int na_setup(NaDevice &d, const sg_graph *g, hipStream_t s, const BfsArgs &proto
     d.ptr = (char *)p;
     int rc = na_zero(s, d.ptr + kNaOffCtr, kNaBytes - kNaOffCtr);
     if (rc) return rc;
-    int per_cu = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_bfs<kNaBlock, false>, kNaBlock, 0));
+    int per_cu = INT_MAX;
+    for (void (*k)(BfsArgs) : {k_bfs<kNaBlock, false, true>, k_bfs<kNaBlock, false, false>, k_bfs_whole<kNaBlock>}) {
+        int blocks = 0;
+        SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, (const void *)k, kNaBlock, 0));
+        per_cu = std::min(per_cu, blocks);
+    }
     if (per_cu < 1) SG_FAIL(SG_ERR_HIP, "sg_bfs_noalloc: kernel cannot be resident");
     uint32_t *words = (uint32_t *)(d.ptr + kNaOffProbe);
     for (int pc = per_cu; pc >= 1; pc--) {
@@ -219,7 +226,7 @@ int na_setup(NaDevice &d, const sg_graph *g, hipStream_t s, const BfsArgs &proto
         BfsArgs pa = proto;
         pa.probe = 1;
         pa.bar.words = words;
-        hipLaunchKernelGGL((k_bfs<kNaBlock, false>), dim3(blocks), dim3(kNaBlock), 0, s, pa);
+        hipLaunchKernelGGL((k_bfs<kNaBlock, false, true>), dim3(blocks), dim3(kNaBlock), 0, s, pa);
         SG_HIP(hipGetLastError());
         uint32_t counts[kMaxXcd + 2];
         SG_HIP(hipMemcpyAsync(counts, words + bar_count(0), sizeof(counts), hipMemcpyDeviceToHost, s));
@@ -281,6 +288,7 @@ extern "C" int sg_bfs_noalloc(const sg_graph *g, uint32_t source, int32_t *level
     a.lb_push_none = o.lb_push == SG_LB_NONE;
     a.lb_pull_none = o.lb_pull == SG_LB_NONE;
     a.team = a.lb_push_none || a.lb_pull_none ? 0u : g->relabeled ? 1u : 2u;
+    a.team_start = team_start(dg, kTeamPushEdges);
     if (!d.ptr && (rc = na_setup(d, g, s, a))) return rc;
 
     uint64_t *bm = (uint64_t *)(d.ptr + kNaOffBitmaps);
@@ -293,10 +301,10 @@ extern "C" int sg_bfs_noalloc(const sg_graph *g, uint32_t source, int32_t *level
     a.bar.rset = (uint32_t)(d.launches & 1u);
     a.abort = (uint32_t *)(d.ptr + kNaOffAbort);
     a.stats = (DevStats *)(d.ptr + kNaOffStats);
-    // (k_bfs_whole takes fewer registers and less LDS: k_bfs's grid is resident for it too)
     void (*kernel)(BfsArgs) = a.team && team_whole_graph(dg, kTeamBfs, force, g->relabeled)
-                                 ? k_bfs_whole<kNaBlock>
-                                 : k_bfs<kNaBlock, false>;
+                              ? k_bfs_whole<kNaBlock>
+                              : g->relabeled ? k_bfs<kNaBlock, false, false>
+                                             : k_bfs<kNaBlock, false, true>;
     hipLaunchKernelGGL(kernel, dim3(d.blocks), dim3(kNaBlock), 0, s, a);
     SG_HIP(hipGetLastError());
     d.launches++;

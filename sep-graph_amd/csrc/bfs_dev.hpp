@@ -90,8 +90,9 @@ struct BfsArgs {
     // LoadBalancing::NONE (one lane per vertex, its edges in order, no hub
     // chunks) for push / pull rounds; otherwise the balanced schedulers
     uint32_t lb_push_none, lb_pull_none;
-    uint32_t team;  // rounds with little work may run on one XCD's blocks:
-                    // 1 (skewed graphs) after the first pull round, 2 from the start
+    uint32_t team;        // rounds with little work may run on one XCD's blocks:
+                          // 1 (skewed graphs) after the first pull round, 2 from the start
+    uint32_t team_start;  // (2) see team_start()
 };
 
 // Hub chunks whose heads a block stages in LDS at a time (with 64-edge
@@ -337,13 +338,15 @@ constexpr uint32_t kTeamPushEdges = SG_TEAM_PUSH_EDGES;
 // barrier and a frontier read back from its bitmap; and only when nothing
 // follows the traversal (kLeave): its last one to three rounds do not earn
 // the barrier back (the BFS of a BC query on 32 001 vertices: 230 us without, 238 with).
-template <bool kLeave>
-__device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const RoundState &S, const RoundCounts &rc)
+template <bool kLeave, bool kEven>
+__device__ __forceinline__ bool bfs_team_fits(const BfsArgs &a, const RoundState &S, const RoundCounts &rc, uint32_t prev)
 {
     if (!a.team) return false;
     const uint32_t limit = team_limit(a.qcap, kTeamPushEdges);
     DirectionPolicy p = S.pol;
-    return (a.team == 2 || (kLeave && S.pulls)) && !rc.has_huge && rc.count <= limit && rc.scout <= limit &&
+    const bool stays =
+        kEven ? team_stays(a.team_start, rc.count, prev, rc.scout) : a.team == 2 || (kLeave && S.pulls);
+    return stays && !rc.has_huge && rc.count <= limit && rc.scout <= limit &&
            !p.next(S.L, rc.count, rc.scout);
 }
 
@@ -707,9 +710,9 @@ __device__ __forceinline__ bool bfs_whole(const BfsArgs &a, TeamLds &t, uint32_t
 // kTeamOk: rounds with little work may run on the team (a.team; needs `gen`
 // from bar_begin<true> on a.bar, whose first barrier takes the census).
 // kLeave: nothing follows the traversal, so blocks may return before every
-// block has seen its end. team, team_tag, team_phase: the caller's own team
+// block has seen its end. kEven: the graph is not skewed (a.team 2 or 0). team, team_tag, team_phase: the caller's own team
 // state, when its team goes on after the traversal.
-template <int BS, bool kStage = false, bool kTeamOk = false, bool kLeave = false>
+template <int BS, bool kStage = false, bool kTeamOk = false, bool kLeave = false, bool kEven = false>
 __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32_t nblocks, uint32_t xcc,
                                         BarState &gen, TeamLds *team = nullptr, uint32_t *team_tag = nullptr,
                                         uint32_t *team_phase = nullptr)
@@ -812,16 +815,20 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
     // the grid's rounds use the counter slots in turn; the team's use none, and
     // after a phase the counts come with its note
     uint32_t slot = L;
+    __shared__ uint32_t s_prev;  // (kEven) see team_stays()
+    if (kEven && threadIdx.x == 0) s_prev = 0;
     bool noted = false;
     while (ok) {
         if (!noted) read_counts(&a.ctr[slot % 3], s_lvl);
         if (threadIdx.x == 0) s_qn = 0;
         __syncthreads();
         const RoundCounts rc = unpack_counts(s_lvl, a.qcap);
+        const uint32_t prev = kEven ? s_prev : 0u;
         __syncthreads();
-        noted = false;
         const bool last = rc.count == 0 || (a.max_rounds && L >= a.max_rounds);
-        const bool team_phase_next = kTeamOk && !last && bfs_team_fits<kLeave>(a, S, rc);
+        const bool team_phase_next = kTeamOk && !last && bfs_team_fits<kLeave, kEven>(a, S, rc, prev);
+        noted = false;
+        if (kEven && threadIdx.x == 0) s_prev = team_phase_next ? ~0u : (uint32_t)rc.count;
         const bool level1 = L == 1 && local0;
         if (level1 && !team_phase_next) {
             // the source's out-neighbours found by block 0 (at most

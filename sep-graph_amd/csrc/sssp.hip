@@ -14,7 +14,8 @@ namespace {
 // queries each keep their working set in one XCD's L2 and synchronise only
 // within it, which suits SSSP, whose rounds are latency-bound at far below
 // the bandwidth of the chip.
-template <int BS>
+// kEven: the graph is not skewed (see sssp_run).
+template <int BS, bool kEven>
 __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
 {
     if (a.probe) {
@@ -24,7 +25,7 @@ __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
     const uint32_t xcc = xcc_id();
     BarState st = bar_begin<true>(a.bar, xcc);
     if (!a.grouped) {
-        sssp_run<BS, SG_FRONT_LDS * BS, true>(a, blockIdx.x, gridDim.x, xcc, st);
+        sssp_run<BS, SG_FRONT_LDS * BS, true, kEven>(a, blockIdx.x, gridDim.x, xcc, st);
         bar_end(a.bar);
         return;
     }
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(BS) void k_sssp(SsspArgs a)
     b.bar.words = a.bar.words + (size_t)(xcc + 1) * kBarWords;
     BarState xs{0u, s_cnt, 1u, s_rank};
     if (threadIdx.x == 0) xs.gen = poll_load(b.bar.words + kBarGen);
-    sssp_run<BS, SG_FRONT_LDS * BS, true>(b, s_rank, s_cnt, xcc, xs);
+    sssp_run<BS, SG_FRONT_LDS * BS, true, kEven>(b, s_rank, s_cnt, xcc, xs);
     if (s_rank == 0 && threadIdx.x == 0) atomicMin(a.gr.status, b.stats->status);
 }
 
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(BS) void k_sssp_whole(SsspArgs a)
     bar_end(a.bar);
 }
 
-// Persistent grid for k_sssp<BS>; grouped launches take the barrier area
+// Persistent grid for k_sssp; grouped launches take the barrier area
 // `group_words` ((1 + kMaxXcd) areas) and give the XCDs holding blocks one
 // query each, in XCD order.
 template <int BS>
@@ -92,7 +93,7 @@ int launch_sssp(sg_engine *e, SsspArgs &args, uint32_t *group_words)
     if (!args.abort || !args.stats || (!args.dist && !args.grouped) || !args.fbit || !args.queue ||
         !args.ctr || (args.grouped && (!group_words || !args.gr.status)))
         SG_FAIL(SG_ERR_STATE, "sg_sssp: launch with unset device state");
-    void (*kernel)(SsspArgs) = k_sssp<BS>;
+    void (*kernel)(SsspArgs) = e->g->relabeled ? k_sssp<BS, false> : k_sssp<BS, true>;
     int most = 0;
     if (!args.grouped && args.team && team_whole_graph(args.g, kTeamSssp, args.force, e->g->relabeled)) {
         kernel = k_sssp_whole<BS>;
@@ -155,6 +156,7 @@ int sssp_args(sg_engine *e, SsspArgs &a)
     a.lb_push_none = o.lb_push == SG_LB_NONE;
     a.lb_pull_none = o.lb_pull == SG_LB_NONE;
     a.team = a.lb_push_none || a.lb_pull_none ? 0u : e->g->relabeled ? 1u : 2u;
+    a.team_start = team_start(a.g, kTeamPushWork);
     if (o.priority == SG_PRIO_LOW_HIGH) {
         // two-level priority (the reference's SetTwoLevelBasedPriority,
         // algo_variants.cuh:605-685) runs push rounds only; the bucket width

@@ -85,8 +85,9 @@ struct SsspArgs {
     // LoadBalancing::NONE (one lane per vertex, its edges in order, no hub
     // chunks) for push / pull rounds; otherwise the balanced schedulers
     uint32_t lb_push_none, lb_pull_none;
-    uint32_t team;  // rounds with little work may run on one XCD's blocks:
-                    // 1 (skewed graphs) after the first pull round, 2 from the start
+    uint32_t team;        // rounds with little work may run on one XCD's blocks:
+                          // 1 (skewed graphs) after the first pull round, 2 from the start
+    uint32_t team_start;  // (2) see team_start()
 };
 
 struct Round {
@@ -622,11 +623,12 @@ __device__ __forceinline__ void pull_hubs_sorted(Round &R, uint32_t first, uint3
 // the heads of its edges and the vertices it defers.
 constexpr uint32_t kTeamPushWork = 24576;
 
-// Whether round S.L, of a grid round's frontier, starts a team phase; evaluated
+// Whether round S.L is a narrow one, which goes on with a team phase, or starts
+// one where its frontier stays so (team_stays); evaluated
 // alike by every block. 1024 x 1024 grid with the
 // priority schedule (1844 rounds, up to 13 K edges): 11.6-14.9 us a round on the
 // whole grid, 4.6-8.1 on the team, 23.3 -> 11.6 ms a query.
-__device__ __forceinline__ bool sssp_team_fits(const SsspArgs &a, const RoundState &S, unsigned long long count,
+__device__ __forceinline__ bool sssp_narrow(const SsspArgs &a, const RoundState &S, unsigned long long count,
                                                unsigned long long scout, bool hubs)
 {
     if (!a.team || !(a.team == 2 || S.pulls) || hubs || count + scout > team_limit(a.qcap, kTeamPushWork)) return false;
@@ -883,7 +885,7 @@ __device__ __forceinline__ bool sssp_team_phase(const SsspArgs &a, TeamLds &t, T
         hubs = ballot((w >> kTeamFlagShift) & 1) != 0;
         cmin = wave_min_u32((uint32_t)lane() < kTeamMax ? (uint32_t)t.slot[kTeamMax + lane()] : kInf);
         more = count != 0 && !(a.max_rounds && L >= a.max_rounds);
-        if (more && !kWhole && !sssp_team_fits(a, S, count, scout, hubs)) break;
+        if (more && !kWhole && !sssp_narrow(a, S, count, scout, hubs)) break;
     }
     tag = T.tag;
     if (!ok) return false;
@@ -941,8 +943,8 @@ __device__ __forceinline__ bool sssp_whole(const SsspArgs &a, uint32_t xcc, BarS
 // is advanced by every barrier. kFrontWords: frontier bitmap words a pull
 // round copies into LDS (the first kFrontWords * 64 vertex ids). kTeamOk:
 // rounds with little work may run on the team (a.team; needs `gen` from
-// bar_begin<true> on a.bar).
-template <int BS, uint32_t kFrontWords = SG_FRONT_LDS * BS, bool kTeamOk = false>
+// bar_begin<true> on a.bar). kEven: the graph is not skewed (a.team 2 or 0).
+template <int BS, uint32_t kFrontWords = SG_FRONT_LDS * BS, bool kTeamOk = false, bool kEven = false>
 __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint32_t nblocks, uint32_t xcc,
                                          BarState &gen)
 {
@@ -997,6 +999,8 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
     // the grid's rounds use the counter slots in turn; the team's use none, and
     // after a phase the counts come with its note
     uint32_t slot = L;
+    __shared__ uint32_t s_prev;  // (kEven) see team_stays()
+    if (kEven && threadIdx.x == 0) s_prev = 0;
     bool noted = false;
     while (ok) {
         if (!noted) read_counts(&a.ctr[slot % 3], s_lvl);
@@ -1007,6 +1011,7 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
         }
         __syncthreads();
         const RoundCounts rc = unpack_counts(s_lvl, a.qcap);
+        const bool stays = !kEven || team_stays(a.team_start, rc.count, s_prev, rc.scout);
         noted = false;
         // priority mode: expand only the lowest delta-bucket present
         uint32_t thr = kInf;
@@ -1019,7 +1024,9 @@ __device__ __forceinline__ bool sssp_run(const SsspArgs &a, uint32_t brank, uint
         if (a.max_rounds && L >= a.max_rounds) break;
 
         if constexpr (kTeamOk) {
-            if (sssp_team_fits(a, S, rc.count, rc.scout, rc.has_huge)) {
+            const bool team = stays && sssp_narrow(a, S, rc.count, rc.scout, rc.has_huge);
+            if (kEven && threadIdx.x == 0) s_prev = team ? ~0u : (uint32_t)rc.count;
+            if (team) {
                 uint32_t members, rank;
                 team_place(xcc, gen, members, rank);
                 TeamEnd E{};
