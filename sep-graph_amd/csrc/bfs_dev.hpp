@@ -117,6 +117,7 @@ struct Round {
     unsigned long long scout, count;  // this lane's share of the next frontier
     bool huge;                        // this lane discovered a vertex above kHugeDegree
     bool levels = true;               // write discovered levels now (else the next round does)
+    bool even = false;                // bfs_run's kEven
 };
 
 __device__ __forceinline__ bool in_frontier(const Round &R, uint32_t u) { return test_bit(R.fcur, u); }
@@ -133,7 +134,7 @@ __device__ __forceinline__ void push_visit(Round &R, bool act, uint32_t v)
     // of L2-resident bits instead of the level array, with one atomic per
     // run of a wave's candidates in one word, none per edge.
     const bool cand = act && !test_bit(a.vis, v);
-    const bool found = wave_claim_bits(a.vis, cand, v, R.fnext);
+    const bool found = R.even ? wave_claim_bits<true>(a.vis, cand, v, R.fnext) : wave_claim_bits(a.vis, cand, v, R.fnext);
     if (found) {
         if (R.levels) a.level[caller_id(a, v)] = R.L + 1;
         const uint32_t dv = a.g.row[v + 1] - a.g.row[v];
@@ -882,6 +883,7 @@ __device__ __forceinline__ bool bfs_run(const BfsArgs &a, uint32_t brank, uint32
         R.scout = 0;
         R.count = 0;
         R.huge = false;
+        R.even = kEven;
         const uint32_t *qin = a.queue + (size_t)(L % 3) * a.qcap;
 
         if (!pull) {
