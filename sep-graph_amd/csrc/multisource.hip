@@ -1076,7 +1076,11 @@ constexpr int kMsPullRows = 8;
 // call 3180 us without pull rounds, 1759 with a ratio of 4, 1621 with 16, 1569
 // with 32 (64: 1541, but a 150 x 200 grid loses what that gains). Narrow groups walk too
 // few edges at a time: 8 queries on 60 001 vertices take 602 us pushing and 702
-// pulling, 16 take 859 and 703.
+// pulling, 16 take 859 and 703. Groups of 16 lanes walk an in-hub's chunk in 16 steps,
+// which a graph of few vertices has too little other work to hide: with in-hubs they
+// pull from kMsPullNarrow vertices on (16 queries on R-MAT graphs: 4096 vertices, 97 K
+// edges 607 us pulling and 428 pushing, 8192, 111 K 569 and 487, 16 384, 120 K 638 and 749;
+// without in-hubs, 8000 vertices of mean degree 15: 300 and 365).
 #ifndef SG_MS_PULL_RATIO
 #define SG_MS_PULL_RATIO 32
 #endif
@@ -1085,6 +1089,7 @@ constexpr uint32_t kMsPullRatio = SG_MS_PULL_RATIO;
 #define SG_MS_PULL_BITS 4
 #endif
 constexpr uint32_t kMsPullBits = SG_MS_PULL_BITS;
+constexpr uint32_t kMsPullNarrow = 12288;
 
 // In-edges a group is about to read the far ends of: one per lane.
 struct MsEdges {
@@ -1309,6 +1314,8 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
     }
     if (ok) ok = grid_sync(a.bar, xcc, gen, a.abort);
 
+    const bool pullable =
+        qbits > kMsPullBits || (qbits == kMsPullBits && (n >= kMsPullNarrow || g.nhugein == 0));
     uint32_t r = 0, prev_len = 0, pulls = 0;
     unsigned long long ptrace = 0;
     while (ok) {
@@ -1319,7 +1326,7 @@ __global__ __launch_bounds__(BS) void k_mssssp(MsSsspArgs a)
         const uint32_t len = rc.qlen;
         __syncthreads();
         if (rc.count == 0 || (a.max_rounds && r >= a.max_rounds)) break;
-        const bool pull = a.force != 0 && qbits >= kMsPullBits && rc.scout * kMsPullRatio >= g.m;
+        const bool pull = a.force != 0 && pullable && rc.scout * kMsPullRatio >= g.m;
         pulls += pull;
         if (pull && r < 64) ptrace |= 1ull << r;
         if (gtid == 0) write_trace(a.trace, r, pull, rc.count, rc.scout, t_start);
