@@ -422,9 +422,12 @@ int sg_bc_dependency(sg_engine *e, const uint32_t *sources, int32_t k, int32_t b
 int sg_bfs_multi(sg_engine *e, const uint32_t *sources, int32_t k, int32_t batch);
 
 /* SSSP from k sources, `batch` (1..64, 0 = 64) per launch: distance rows
- * [vertex][query] relaxed for every query of the batch at once (data-driven
- * push rounds, and pull rounds while most of the graph is in the frontier
- * unless a push variant is forced). The value array becomes k rows of n uint32 distances, row i
+ * [vertex][query] relaxed for every query of the batch at once in data-driven
+ * rounds. A round pushes, or pulls when the frontier's out-edges number at
+ * least 1/32 of all edges and the batch has more than 16 queries (more than 8
+ * on graphs of 12288 vertices and more, or with no in-degree above 64). Forcing
+ * a push variant rules pulling out; forcing a pull variant changes nothing
+ * here. The value array becomes k rows of n uint32 distances, row i
  * equal to sg_sssp from sources[i] (UINT32_MAX when unreached). No reference
  * counterpart (one source per run there); serves batched SSSP queries. */
 int sg_sssp_multi(sg_engine *e, const uint32_t *sources, int32_t k, int32_t batch);

@@ -43,8 +43,6 @@ using namespace sg;
 
 namespace {
 
-// ------------------------------------------------------------------ helpers
-
 // ------------------------------------------- compensated FP32 accumulation
 // A sum kept as hi + lo, where lo collects the rounding error of every
 // addition into hi (TwoSum, Knuth: exact, and without the comparison of
@@ -802,7 +800,7 @@ struct IterativePolicy {
     }
 };
 
-// In-hub chunks and slice rows a wave of a residual pull round keeps in flight.
+// What the propagation of one residual round shares.
 struct DdRound {
     const PrDdArgs *a;
     const float *p;    // this round's row
