@@ -95,10 +95,12 @@ int launch_sssp(sg_engine *e, SsspArgs &args, uint32_t *group_words)
         SG_FAIL(SG_ERR_STATE, "sg_sssp: launch with unset device state");
     void (*kernel)(SsspArgs) = e->g->relabeled ? k_sssp<BS, false> : k_sssp<BS, true>;
     // Three blocks of 256 threads fit a CU. Where rounds are short, two make the faster
-    // barriers: RMAT of 262 144 vertices 395 and 336 us, 1024 x 1024 grid 53.8 and
-    // 42.9 ms; 8 M edges over 1 M vertices 1245 and 1291 us, RMAT-21 by pushes 1218 and
-    // 1420. (Concurrent queries, whose barriers are an XCD's: always three.)
-    const bool short_rounds = args.g.m <= (4u << 20) || args.g.m < 6 * (uint64_t)args.g.n;
+    // barriers: RMAT of 262 144 vertices 395 and 336 us, of 1 048 576 507 and 489, 1024 x
+    // 1024 grid 53.8 and 42.9 ms; RMAT-21 by pushes 1218 and 1420 us, 4.8 M edges over
+    // 300 000 vertices 725 and 751. (Concurrent queries, whose barriers are an XCD's:
+    // always three.)
+    const bool short_rounds = args.g.m <= (e->g->relabeled && args.force != 0 ? 16u << 20 : 4u << 20) ||
+                              args.g.m < 6 * (uint64_t)args.g.n;
     int most = BS == 256 && !args.grouped && short_rounds ? 2 * e->g->num_cus : 0;
     if (!args.grouped && args.team && team_whole_graph(args.g, kTeamSssp, args.force, e->g->relabeled)) {
         kernel = k_sssp_whole<BS>;
