@@ -562,7 +562,7 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
 
     __shared__ PrPart s_red[WPB];
     // as many ids in LDS as fit beside the rest: with 32 per thread RMAT-21
-    // took 1848 us, with 39 1803
+    // takes 1752 us, with 39 1708, 400 001 vertices 500 and 480
 #ifndef SG_PR_LDS
 #define SG_PR_LDS 39
 #endif
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(BS) void k_pr_pull(PrArgs a)
         Hot::wait();
         __syncthreads();
         const Gather<Hot::kLds> gather{cc, s_cc, n};
-        constexpr uint32_t kRows = 8;  // RMAT-21 1774 us by 4, 1746 by 8; 15 001 vertices 226 and 210 (FP64 sums)
+        constexpr uint32_t kRows = 8;  // RMAT-21 1740 us by 4, 1708 by 8; 15 001 vertices 257 and 234
         double r_acc = 0.0;
         CSum d_acc{0.f, 0.f};
         struct Own {
@@ -1088,10 +1088,10 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
         // residuals in between: a round of two grid barriers and one reading of
         // the edges, as one of the power iteration. Rounds of the ITERATIVE
         // scheme, and the last one before max_rounds, leave activation out.
-        // RMAT graph of 100 003 vertices, 1.4 M edges, nearly all active: 19 us a
+        // RMAT graph of 100 003 vertices, 1.4 M edges, nearly all active: 21 us a
         // round, 2.2 ms a run (45 and 4.8 with activation in a pass of its own);
-        // ~10 of the 19 are the two barriers, the counts and the LDS copy, 5 the
-        // words' chains of in-edge steps, 3 the hubs.
+        // ~10 of them are the two barriers, the counts and the LDS copy, the rest the
+        // words' chains of in-edge steps and the hubs.
         bool more = true;
         const Bounds bounds(g, gwave, nwaves);
         if (pull) Hot::take(s_p, pc, n);
@@ -1100,7 +1100,7 @@ __global__ __launch_bounds__(BS) void k_pr_dd(PrDdArgs a)
             Hot::wait();
             __syncthreads();
             const Gather<Hot::kLds> gather{pc, s_p, n};
-            constexpr uint32_t kRows = BS > 512 ? 8 : 16;
+            constexpr uint32_t kRows = BS > 512 ? 8 : 16;  // 100 003 vertices, 512 threads: 2356 us by 8, 2255 by 16
             unsigned long long nscout = 0, ncnt = 0;
             struct Own {
                 uint32_t dout;
@@ -1426,8 +1426,8 @@ extern "C" int sg_pagerank(sg_engine *e, double damping, double tol, int32_t max
         }
         // Up to 2^18 vertices a round is latency: blocks of 512 threads, whose
         // waves have registers for 16 rows in flight and none to spill (100 003
-        // vertices 2124 us, of 1024 threads 2490; 400 001: 3611 and 3637). Beyond,
-        // twice the waves hide more (1 000 001: 7465 and 6969).
+        // vertices 2255 us, of 1024 threads 2564; 400 001: 3768 and 3777). Beyond,
+        // twice the waves hide more (1 000 001: 7340 and 6896).
         const int dbs = o.block_size || d.n > (1u << 18) ? bs : 512;
         switch (dbs) {
         case 256:
